@@ -8,6 +8,7 @@
 namespace gpdev {
 
 constexpr int kBlock = 256;  // 4 waves of 64 lanes
+constexpr int kWaves = kBlock / 64;
 
 __host__ inline unsigned grid_for(int64_t n, int block = kBlock) {
   int64_t g = (n + block - 1) / block;
@@ -50,6 +51,81 @@ __device__ inline void wave_max(int32_t* addr, int32_t v) {
 __device__ inline void wave_add1(int32_t* addr) {
   uint64_t m;
   if (wave_leader(&m)) atomicAdd(addr, static_cast<int32_t>(__popcll(m)));
+}
+
+// Orders a wave's LDS stores before its own later loads (and the reverse);
+// no other wave is met.
+__device__ inline void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// s + t[0] + t[1] + ..., added one after the other; t is 16-byte aligned LDS,
+// and where n is odd t[n] holds +0.  Eight pairs are on their way at a time.
+__device__ inline double add_in_order(double s, const double* t, int n) {
+  const double2* p = reinterpret_cast<const double2*>(t);
+  const int pairs = (n + 1) / 2;
+  int i = 0;
+  for (; i + 8 <= pairs; i += 8) {
+    double2 v[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = p[i + k];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      s += v[k].x;
+      s += v[k].y;
+    }
+  }
+  for (; i < pairs; ++i) {
+    const double2 v = p[i];
+    s += v.x;
+    s += v.y;
+  }
+  return s;
+}
+
+// Calls f(row, begin, end) in all lanes of a wave for every row of more than
+// `longer` entries that falls to it, in a launch whose blocks from
+// `first_block` on are given to long rows.  A wave looks at every waves-th group of g
+// neighbouring rows, so neighbouring long rows go to different waves: g = 1
+// up to 262,144 rows (a line of row pointers read for each, 16 MB of L2 reads
+// in all), past that the 16 rows of a line.  The row pointers of kLook groups
+// are loaded together: without a long row these blocks are gone in a few
+// memory round trips.
+inline unsigned long_row_blocks(int32_t m) {  // at most one a CU
+  const unsigned b = grid_for(m, kWaves);
+  return b < 256u ? b : 256u;
+}
+
+template <class F>
+__device__ __forceinline__ void wave_long_rows(const int32_t* __restrict__ ptr, int32_t m, int32_t longer,
+                                               int32_t first_block, F&& f) {
+  constexpr int kLook = 8;
+  const int lane = lane_id();
+  const int g = m <= 262144 ? 1 : 16;
+  const int64_t waves = static_cast<int64_t>(static_cast<int32_t>(gridDim.x) - first_block) * kWaves;
+  const int64_t w0 = (static_cast<int64_t>(static_cast<int32_t>(blockIdx.x) - first_block) * kWaves + (threadIdx.x >> 6)) * g;
+  const int64_t mine = (lane / g) * waves * g + lane % g;
+  for (int64_t look = w0; look < m; look += kLook * 64 * waves) {
+    bool any = false;
+#pragma unroll
+    for (int u = 0; u < kLook; ++u) {
+      const int64_t r = look + u * 64 * waves + mine;
+      any = any || (r < m && ptr[r + 1] - ptr[r] > longer);
+    }
+    if (__ballot(any) == 0) continue;
+#pragma unroll 1
+    for (int u = 0; u < kLook; ++u) {
+      const int64_t first = look + u * 64 * waves, r = first + mine;
+      const int32_t rb = r < m ? ptr[r] : 0, re = r < m ? ptr[r + 1] : 0;
+      uint64_t todo = __ballot(re - rb > longer);
+      while (todo) {
+        const int q = __ffsll(static_cast<unsigned long long>(todo)) - 1;
+        todo &= todo - 1;
+        f(first + (q / g) * waves * g + q % g, __shfl(rb, q, 64), __shfl(re, q, 64));
+      }
+    }
+  }
 }
 
 // Inclusive wave64 prefix sum of an int32.

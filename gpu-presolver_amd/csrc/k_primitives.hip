@@ -102,9 +102,17 @@ __global__ void k_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t
 // them; each thread then adds its own row's terms in CSR order, so every row
 // sum has exactly the sequential rounding of the reference kernel
 // (gpu_presolve_kernels.cu:18-66) for any row length.
+// A row of more than kActLong entries is left to act_long_row: its one
+// thread would add thousands of terms from LDS while the other 255 wait, and
+// neighbouring long rows (linking rows come last in most models) would queue
+// in one block.  200 adjacent rows of 3,000 entries behind 80,000 short rows
+// took 67 ms per call that way, and 42 us with a wave each.
 constexpr int kActRows = kBlock;
 constexpr int kActCap = 2048;
 constexpr int kActItems = kActCap / kBlock;
+// A wave of its own costs a row about 3 us of latency; a 128-entry row costs
+// its tile about as much (2 x 128 LDS reads and adds in one lane).
+constexpr int kActLong = 128;
 
 // (l, u) interleaved, so an activity term needs one 16-byte gather.
 __global__ void k_pack_lu(const double* __restrict__ l, const double* __restrict__ u, int32_t n,
@@ -113,30 +121,124 @@ __global__ void k_pack_lu(const double* __restrict__ l, const double* __restrict
   if (j < n) lu[j] = make_double2(l[j], u[j]);
 }
 
-__global__ __launch_bounds__(kBlock) void k_row_activity_lu(const int32_t* __restrict__ row_ptr,
+// A term of the activity sums; b = (l, u) of the entry's column.
+__device__ inline double act_min(double a, double2 b, bool on) { return on ? (a >= 0.0 ? a * b.x : a * b.y) : 0.0; }
+__device__ inline double act_max(double a, double2 b, bool on) { return on ? (a >= 0.0 ? a * b.y : a * b.x) : 0.0; }
+
+// One of the rows of more than kActLong entries, by a wave.  It loads 256
+// entries at a time (the next 256 on their way while these are summed) and
+// stages both terms in LDS; lane 0 adds the min terms and lane 1 the max terms
+// in CSR order, so the sums are those of one thread.  A term that is not
+// finite is counted and staged as 0: adding +0 to a sum that started at +0
+// leaves it as it is (no such sum is -0).  Bound by the add chain of the row,
+// about 10 us for 3,000 entries.
+constexpr int kActSteps = 4;
+constexpr int kActChunk = 64 * kActSteps;
+constexpr int kActPitch = kActChunk + 2;  // the min and max terms start in different banks
+static_assert(kWaves * 2 * kActPitch <= kActCap + 16, "the long rows' terms fit the tile's LDS");
+
+__device__ __forceinline__ void act_long_row(const int32_t* __restrict__ col_idx, const double* __restrict__ val,
+                                             int64_t row, int32_t b, int32_t e, const double2* __restrict__ lu,
+                                             double ztol, double* __restrict__ min_fin, double* __restrict__ max_fin,
+                                             int32_t* __restrict__ neg_inf, int32_t* __restrict__ pos_inf,
+                                             double* s_mn, double* s_mx) {
+  const int lane = lane_id();
+  double a[kActSteps];
+  int32_t j[kActSteps];
+#pragma unroll
+  for (int k = 0; k < kActSteps; ++k) {
+    const int32_t pc = min(b + 64 * k + lane, e - 1);
+    a[k] = val[pc];
+    j[k] = col_idx[pc];
+  }
+  double acc = 0.0;
+  int32_t ni = 0, pi = 0;
+  for (int32_t c = b; c < e; c += kActChunk) {
+    double2 lub[kActSteps];
+    bool on[kActSteps];
+#pragma unroll
+    for (int k = 0; k < kActSteps; ++k) {
+      on[k] = c + 64 * k + lane < e && fabs(a[k]) > ztol;
+      lub[k] = lu[on[k] ? j[k] : 0];
+    }
+    double tn[kActSteps], tx[kActSteps];
+#pragma unroll
+    for (int k = 0; k < kActSteps; ++k) {
+      tn[k] = act_min(a[k], lub[k], on[k]);
+      tx[k] = act_max(a[k], lub[k], on[k]);
+    }
+    // the next chunk's entries (the last entry again past the row's end)
+#pragma unroll
+    for (int k = 0; k < kActSteps; ++k) {
+      const int32_t pc = min(c + kActChunk + 64 * k + lane, e - 1);
+      a[k] = val[pc];
+      j[k] = col_idx[pc];
+    }
+#pragma unroll
+    for (int k = 0; k < kActSteps; ++k) {
+      const bool fn = isfinite(tn[k]), fx = isfinite(tx[k]);
+      ni += static_cast<int32_t>(__popcll(__ballot(!fn && tn[k] < 0.0)));
+      pi += static_cast<int32_t>(__popcll(__ballot(!fx && tx[k] > 0.0)));
+      s_mn[64 * k + lane] = fn ? tn[k] : 0.0;
+      s_mx[64 * k + lane] = fx ? tx[k] : 0.0;
+    }
+    wave_lds_fence();
+    if (lane < 2) acc = add_in_order(acc, lane == 0 ? s_mn : s_mx, min(kActChunk, e - c));
+    wave_lds_fence();
+  }
+  if (lane == 0) {
+    min_fin[row] = acc;
+    neg_inf[row] = ni;
+    pos_inf[row] = pi;
+  } else if (lane == 1) {
+    max_fin[row] = acc;
+  }
+}
+
+// At least six waves a SIMD: the gathers of the tiles are bound by how many
+// are in flight.
+__global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __restrict__ row_ptr,
                                                             const int32_t* __restrict__ col_idx,
                                                             const double* __restrict__ val, int32_t m,
                                                             const double2* __restrict__ lu, double ztol,
                                                             double* __restrict__ min_fin,
                                                             double* __restrict__ max_fin,
                                                             int32_t* __restrict__ neg_inf,
-                                                            int32_t* __restrict__ pos_inf) {
+                                                            int32_t* __restrict__ pos_inf,
+                                                            int32_t tiles) {
   // One term array (the min terms, then the max terms): 16 KB of LDS per
   // block, so eight blocks fit a CU and their load phases overlap.
-  __shared__ double s_t[kActCap];
-  __shared__ int32_t s_ptr[kActRows + 1];
-  const int32_t r0 = blockIdx.x * kActRows;
+  __shared__ __align__(16) double s_t[kActCap + 16];
+  __shared__ int32_t s_next;
+  if (static_cast<int32_t>(blockIdx.x) >= tiles) {
+    double* s_mn = s_t + (threadIdx.x >> 6) * 2 * kActPitch;
+    wave_long_rows(row_ptr, m, kActLong, tiles, [&](int64_t row, int32_t b, int32_t e) {
+      act_long_row(col_idx, val, row, b, e, lu, ztol, min_fin, max_fin, neg_inf, pos_inf, s_mn, s_mn + kActPitch);
+    });
+    return;
+  }
+  const int32_t r0 = static_cast<int32_t>(blockIdx.x) * kActRows;
   const int32_t rows = min(kActRows, m - r0);
   const int tid = threadIdx.x;
-  for (int t = tid; t <= rows; t += kBlock) s_ptr[t] = row_ptr[r0 + t];
-  __syncthreads();
-  const int32_t seg_b = s_ptr[0], seg_e = s_ptr[rows];
-  const int32_t my_b = tid < rows ? s_ptr[tid] : 0;
-  const int32_t my_e = tid < rows ? s_ptr[tid + 1] : 0;
+  const int32_t seg_b = row_ptr[r0], seg_e = row_ptr[r0 + rows];
+  const int32_t my_b = row_ptr[r0 + min(tid, rows)];
+  int32_t my_e = row_ptr[r0 + min(tid + 1, rows)];
+  const bool is_long = my_e - my_b > kActLong;
+  if (is_long) my_e = my_b;  // no entry of it is added here
+  const bool any_long = __syncthreads_or(is_long) != 0;
   double mn = 0.0, mx = 0.0;
   int32_t ni = 0, pi = 0;
   for (int32_t w = seg_b; w < seg_e; w += kActCap) {
+    if (any_long) {  // on to the next entry of a row that is added here
+      if (tid == 0) s_next = seg_e;
+      __syncthreads();
+      if (my_e > w && my_e > my_b) atomicMin(&s_next, max(my_b, w));
+      __syncthreads();
+      w = s_next;
+      if (w >= seg_e) break;
+    }
     const int32_t we = min(w + kActCap, seg_e);
+    const int32_t rb = max(my_b, w), re = min(my_e, we);
     double a[kActItems];
     double2 b[kActItems];
     int32_t j[kActItems];
@@ -154,14 +256,13 @@ __global__ __launch_bounds__(kBlock) void k_row_activity_lu(const int32_t* __res
       if (w + tid + k * kBlock >= we) a[k] = 0.0;
       b[k] = lu[fabs(a[k]) > ztol ? j[k] : 0];
     }
-    const int32_t rb = max(my_b, w), re = min(my_e, we);
     double tmx[kActItems];  // the max terms wait in registers while the min terms are summed
 #pragma unroll
     for (int k = 0; k < kActItems; ++k) {
       const int32_t p = w + tid + k * kBlock;
       const bool on = fabs(a[k]) > ztol;
-      tmx[k] = on ? (a[k] >= 0.0 ? a[k] * b[k].y : a[k] * b[k].x) : 0.0;
-      if (p < we) s_t[p - w] = on ? (a[k] >= 0.0 ? a[k] * b[k].x : a[k] * b[k].y) : 0.0;
+      tmx[k] = act_max(a[k], b[k], on);
+      if (p < we) s_t[p - w] = act_min(a[k], b[k], on);
     }
     __syncthreads();
     for (int32_t p = rb; p < re; ++p) {
@@ -179,9 +280,9 @@ __global__ __launch_bounds__(kBlock) void k_row_activity_lu(const int32_t* __res
       const double t = s_t[p - w];
       if (isfinite(t)) mx += t; else if (t > 0.0) ++pi;
     }
-    __syncthreads();
+    if (we < seg_e) __syncthreads();  // the next window restages
   }
-  if (tid < rows) {
+  if (tid < rows && !is_long) {
     min_fin[r0 + tid] = mn;
     max_fin[r0 + tid] = mx;
     neg_inf[r0 + tid] = ni;
@@ -1439,8 +1540,13 @@ hipError_t gpk_row_activity_lu(const int32_t* row_ptr, const int32_t* col_idx, c
                                const double* lu, double ztol, double* min_fin, double* max_fin, int32_t* neg_inf,
                                int32_t* pos_inf, hipStream_t s) {
   if (m <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_row_activity_lu, dim3(grid_for(m, kActRows)), dim3(kBlock), 0, s, row_ptr, col_idx,
-                     val, m, reinterpret_cast<const double2*>(lu), ztol, min_fin, max_fin, neg_inf, pos_inf);
+  // The tiles, then the blocks that look for long rows: on a matrix without
+  // one those end while the last tiles run.  (A launch of their own cost 2.6
+  // us more at 1M rows, and in front of the tiles they cost 1 us.)
+  const unsigned tiles = grid_for(m, kActRows);
+  hipLaunchKernelGGL(k_row_activity_lu, dim3(tiles + long_row_blocks(m)), dim3(kBlock), 0, s, row_ptr, col_idx, val, m,
+                     reinterpret_cast<const double2*>(lu), ztol, min_fin, max_fin, neg_inf, pos_inf,
+                     static_cast<int32_t>(tiles));
   return hipGetLastError();
 }
 

@@ -180,7 +180,7 @@ hipError_t gpk_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t* o
 /* Row activity (reference gpu_presolve_kernels.cu:18-111) over bounds packed
  * as lu[2j] = l[j], lu[2j+1] = u[j] (16-byte aligned, written by
  * gpk_pack_lu), so each entry needs one 16-byte gather; 256 rows per block,
- * each row summed in CSR order. */
+ * rows of more than 128 entries one wave each, every row summed in CSR order. */
 hipError_t gpk_pack_lu(const double* l, const double* u, int32_t n, double* lu, hipStream_t stream);
 hipError_t gpk_row_activity_lu(const int32_t* row_ptr, const int32_t* col_idx, const double* val, int32_t m,
                                const double* lu, double ztol, double* min_fin, double* max_fin, int32_t* neg_inf,

@@ -8,7 +8,7 @@ planted reductions of the workload description).  `value` is LPs presolved
 per second.
 
 Extra objects on the JSON line:
-  roofline           the compaction (k_build_rank, k_compact_map, the tile-offset
+  roofline           the compaction (k_apply_maps, k_compact_map, the chunk-offset
                      scan and k_compact_write; the largest share of presolve
                      kernel time after the replay) on the full A with
                      15% of rows and columns dropped, timed with HIP events
@@ -181,21 +181,37 @@ def compaction_compulsory_bytes(m, n, nnz, m_new, nnz_new):
     return 4 * (m + 1) + 4 * m + 4 * n + 12 * nnz + 12 * nnz_new + 4 * (m_new + 1)
 
 
-def measure_compaction(gp_ffi, dlp, lp, stream, launches, frac=0.15, seed=7):
-    """Times the compaction the presolve uses (gpk_build_rank, gpk_compact_map,
-    the tile-offset scan and gpk_compact_write, back to back on one stream)
-    on the full A with 15% of rows and columns dropped (a typical early
-    apply), each kernel also timed apart, and checks the output against the
-    host."""
+def compaction_case(gp_ffi, dlp, lp, frac, seed, with_at):
+    """The buffers and calls of a compaction of the LP's A (and, with_at, of
+    its transpose by the same maps) with `frac` of rows and columns dropped,
+    through the library's internal launchers, in the steps a plan application
+    takes: maps (keep maps, rank words, chunk rows), map (the map pass), scan
+    (the chunk offsets; the library skips it up to 2,048 chunks a side), write
+    (the write pass); check() compares with the host."""
     import ctypes as C
 
     import numpy as np
 
-    class Lookback(C.Structure):
-        _fields_ = [("status", C.c_void_p), ("ticket", C.c_void_p), ("error", C.c_void_p), ("epoch", C.c_uint32)]
+    vp = C.c_void_p
 
-    m, n = lp["m"], lp["n"]
-    nnz = len(lp["A_idx"])
+    class Lookback(C.Structure):
+        _fields_ = [("status", vp), ("ticket", vp), ("error", vp), ("epoch", C.c_uint32)]
+
+    class Side(C.Structure):
+        _fields_ = [("ptr", vp), ("idx", vp), ("val", vp), ("m_old", C.c_int32), ("m_new", C.c_int32),
+                    ("nnz", C.c_int32), ("pad", C.c_int32), ("row_map", vp), ("col_rank", vp), ("chunk_row", vp),
+                    ("jn", vp), ("mask", vp), ("word_pre", vp), ("out_ptr", vp), ("out_idx", vp), ("out_val", vp)]
+
+    class Gathers(C.Structure):
+        _fields_ = [("m", C.c_int32), ("n", C.c_int32)] + [(f"p{k}", vp) for k in range(20)]
+
+    class Maps(C.Structure):
+        _fields_ = [("m", C.c_int32), ("n", C.c_int32), ("keep_row", vp), ("keep_col", vp), ("l", vp), ("u", vp),
+                    ("row_map", vp), ("col_map", vp), ("fixed_mask", vp), ("fixed_tiles", vp), ("counts", vp),
+                    ("row_rank", vp), ("col_rank", vp), ("a_ptr", vp), ("at_ptr", vp), ("a_chunk", vp),
+                    ("at_chunk", vp), ("tile_counts", vp), ("chunk_shift", C.c_int32)]
+
+    m, n, nnz = lp["m"], lp["n"], len(lp["A_idx"])
     rng = np.random.default_rng(seed)
     keep_r = rng.random(m) >= frac
     keep_c = rng.random(n) >= frac
@@ -203,98 +219,109 @@ def measure_compaction(gp_ffi, dlp, lp, stream, launches, frac=0.15, seed=7):
     col_map = np.where(keep_c, np.cumsum(keep_c) - 1, -1).astype(np.int32)
     rows = np.repeat(np.arange(m), np.diff(lp["A_ptr"]))
     kept = keep_r[rows] & keep_c[lp["A_idx"]]
-    m_new, nnz_new = int(keep_r.sum()), int(kept.sum())
-    L = gp_ffi.lib()
-    vp = C.c_void_p
-    L.gpk_build_rank.argtypes = [vp, C.c_int32, vp, vp]
-    L.gpk_compact_map.argtypes = [vp, vp, C.c_int32, vp, vp, vp, vp, vp, vp]
-    L.gpk_compact_write.argtypes = [vp, vp, C.c_int32, vp, vp, vp, vp, C.c_int32, vp, vp, vp]
-    L.gpk_compact_tiles.restype = C.c_int32
-    L.gpk_compact_tiles.argtypes = [C.c_int32]
+    L, ck = gp_ffi.lib(), gp_ffi.hip_check
+    L.gpk_apply_maps.argtypes = [Maps, Lookback, vp]
+    L.gpk_apply_maps_tiles.restype = C.c_int64
+    L.gpk_apply_maps_tiles.argtypes = [C.c_int32, C.c_int32]
+    L.gpk_compact_chunks.argtypes = [C.c_int32]
+    L.gpk_compact_shift.argtypes = [C.c_int32]
+    L.gpk_compact_map.argtypes = [Side, Side, vp, vp, vp]
+    L.gpk_compact_write.argtypes = [Side, Side, vp, C.c_int32, Gathers, vp]
     L.gpk_scan_lb_i32.argtypes = [vp, vp, C.c_int64, Lookback, vp]
     L.gpk_lookback_tiles.restype = C.c_int64
     L.gpk_lookback_tiles.argtypes = [C.c_int64]
-    d_rm, d_cm = gp_ffi.DeviceArray(row_map), gp_ffi.DeviceArray(col_map)
-    d_rank = gp_ffi.DeviceArray(size=2 * ((n + 63) // 64), dtype=np.uint64)
-    jn = gp_ffi.DeviceArray(size=nnz, dtype=np.int32)
-    o_ptr = gp_ffi.DeviceArray(size=m_new + 1, dtype=np.int32)
-    o_idx = gp_ffi.DeviceArray(size=nnz, dtype=np.int32)
-    o_val = gp_ffi.DeviceArray(size=nnz)
-    tiles = L.gpk_compact_tiles(m)
-    t_off = gp_ffi.DeviceArray(size=tiles + 1, dtype=np.int32)
-    status = gp_ffi.DeviceArray(np.zeros(max(1, L.gpk_lookback_tiles(tiles)), np.uint64))
-    tickets = gp_ffi.DeviceArray(np.zeros(4 * launches + 16, np.int32))
-    err = gp_ffi.DeviceArray(np.zeros(1, np.int32))
-    A = dlp.A.g
+    D = gp_ffi.DeviceArray
+    chunks, shift = L.gpk_compact_chunks(nnz), L.gpk_compact_shift(nnz)
+    words, tiles = (chunks << shift) // 64, L.gpk_apply_maps_tiles(m, n)
+    keep = {"row": D(keep_r.astype(np.uint8)), "col": D(keep_c.astype(np.uint8))}
+    maps = {"row": D(size=m, dtype=np.int32), "col": D(size=n, dtype=np.int32)}
+    ranks = {"row": D(size=2 * ((m + 63) // 64), dtype=np.uint64), "col": D(size=2 * ((n + 63) // 64), dtype=np.uint64)}
+    counts, tile_counts = D(np.zeros(16, np.int32)), D(size=tiles, dtype=np.int32)
+    sides = []
+    for g, r_map, mine, other in ((dlp.A.g, row_map, "row", "col"), (dlp.AT.g, col_map, "col", "row"))[:2 if with_at else 1]:
+        b = {"chunk": D(size=chunks + 1, dtype=np.int32), "jn": D(size=nnz, dtype=np.int32),
+             "mask": D(size=words, dtype=np.uint64), "pre": D(size=words, dtype=np.int32),
+             "ptr": D(size=len(r_map) + 1, dtype=np.int32), "idx": D(size=nnz, dtype=np.int32), "val": D(size=nnz)}
+        b["new"] = int((r_map >= 0).sum())
+        b["side"] = Side(g.row_ptr, g.col_idx, g.val, len(r_map), b["new"], nnz, 0, maps[mine].ptr, ranks[other].ptr,
+                         b["chunk"].ptr, b["jn"].ptr, b["mask"].ptr, b["pre"].ptr, b["ptr"].ptr, b["idx"].ptr,
+                         b["val"].ptr)
+        sides.append(b)
+    margs = Maps(m, n, keep["row"].ptr, keep["col"].ptr, None, None, maps["row"].ptr, maps["col"].ptr, None, None,
+                 counts.ptr, ranks["row"].ptr, ranks["col"].ptr, dlp.A.g.row_ptr,
+                 dlp.AT.g.row_ptr if with_at else None, sides[0]["chunk"].ptr,
+                 sides[1]["chunk"].ptr if with_at else None, tile_counts.ptr, shift)
+    cnt = D(size=2 * chunks + 1, dtype=np.int32)
+    status = D(np.zeros(max(tiles, L.gpk_lookback_tiles(2 * chunks)), np.uint64))
+    tickets = D(np.zeros(1 << 16, np.int32))
+    err = D(np.zeros(1, np.int32))
     launch_no = [0]
-    ck = gp_ffi.hip_check
+    a, t = sides[0]["side"], sides[1]["side"] if with_at else Side()
 
-    def rank():
-        ck(L.gpk_build_rank(d_cm.ptr, n, d_rank.ptr, stream.ptr), "build rank")
-
-    def cmap():
-        ck(L.gpk_compact_map(A.row_ptr, A.col_idx, m, d_rm.ptr, d_rank.ptr, jn.ptr, o_ptr.ptr, t_off.ptr, stream.ptr),
-           "map")
-
-    def scan():
+    def lookback():
         k = launch_no[0]
         launch_no[0] += 1
-        lb = Lookback(status.ptr, tickets.ptr + 4 * k, err.ptr, k + 1)
-        ck(L.gpk_scan_lb_i32(t_off.ptr, t_off.ptr, tiles, lb, stream.ptr), "scan")
+        return Lookback(status.ptr, tickets.ptr + 4 * k, err.ptr, k + 1)
 
-    def write():
-        ck(L.gpk_compact_write(A.row_ptr, A.val, m, d_rm.ptr, jn.ptr, t_off.ptr, o_ptr.ptr, m_new, o_idx.ptr,
-                               o_val.ptr, stream.ptr), "write")
+    def keep_maps(stream):
+        ck(L.gpk_apply_maps(margs, lookback(), stream.ptr), "keep maps")
 
-    def whole():
-        rank()
-        cmap()
-        scan()
-        write()
+    def cmap(stream):
+        ck(L.gpk_compact_map(a, t, cnt.ptr, None, stream.ptr), "map")
 
+    def scan(stream):
+        ck(L.gpk_scan_lb_i32(cnt.ptr, cnt.ptr, chunks * len(sides), lookback(), stream.ptr), "scan")
+
+    def write(stream):
+        ck(L.gpk_compact_write(a, t, cnt.ptr, 0, Gathers(), stream.ptr), "write")
+
+    def check():
+        nnz_new = int(kept.sum())
+        want = [(lp["A_ptr"], lp["A_idx"], lp["A_val"], keep_r, keep_c, col_map),
+                (lp["AT_ptr"], lp["AT_idx"], lp["AT_val"], keep_c, keep_r, row_map)]
+        for b, (ptr, idx, val, kr, kc, c_map) in zip(sides, want):
+            r = np.repeat(np.arange(len(kr)), np.diff(ptr))
+            k = kr[r] & kc[idx]
+            w_ptr = np.concatenate([[0], np.cumsum(np.bincount(r[k], minlength=len(kr))[kr])]).astype(np.int32)
+            if (err.numpy()[0] != 0 or not np.array_equal(b["ptr"].numpy()[:b["new"] + 1], w_ptr)
+                    or not np.array_equal(b["idx"].numpy()[:nnz_new], c_map[idx[k]])
+                    or not np.array_equal(b["val"].numpy()[:nnz_new], val[k])):
+                raise SystemExit("bench.py: the compaction differs from the host")
+
+    return {"maps": keep_maps, "map": cmap, "scan": scan, "write": write, "check": check, "keep": (sides, keep, maps, ranks, counts),
+            "sizes": (m, n, nnz, sides[0]["new"], int(keep_c.sum()), int(kept.sum()))}
+
+
+def time_launches(gp_ffi, stream, launches, *calls):
     for _ in range(3):
-        whole()
+        for f in calls:
+            f(stream)
     stream.sync()
-    ev = [gp_ffi.Event() for _ in range(6)]
-    ev[0].record(stream)
+    e0, e1 = gp_ffi.Event(), gp_ffi.Event()
+    e0.record(stream)
     for _ in range(launches):
-        whole()
-    ev[1].record(stream)
-    us = 1e3 * ev[0].elapsed_ms(ev[1]) / launches
-    want_ptr = np.concatenate([[0], np.cumsum(np.bincount(rows[kept], minlength=m)[keep_r])]).astype(np.int32)
-    if (err.numpy()[0] != 0 or not np.array_equal(o_ptr.numpy(), want_ptr)
-            or not np.array_equal(o_idx.numpy()[:nnz_new], col_map[lp["A_idx"][kept]])
-            or not np.array_equal(o_val.numpy()[:nnz_new], lp["A_val"][kept])):
-        raise SystemExit("bench.py: the compaction differs from the host")
-    # Each kernel apart (the map needs the rank, the write the scanned offsets
-    # and the map's counts, so the write is timed after map + scan).
-    parts = {}
-    for name, f in (("k_build_rank", rank), ("k_compact_map", cmap), ("tile scan", None), ("k_compact_write", None)):
-        if name == "tile scan":
-            e0, e1 = gp_ffi.Event(), gp_ffi.Event()
-            e0.record(stream)
-            for _ in range(launches):
-                cmap()
-                scan()
-            e1.record(stream)
-            parts[name] = 1e3 * e0.elapsed_ms(e1) / launches - parts["k_compact_map"]
-            continue
-        if name == "k_compact_write":
-            e0, e1 = gp_ffi.Event(), gp_ffi.Event()
-            e0.record(stream)
-            for _ in range(launches):
-                cmap()
-                scan()
-                write()
-            e1.record(stream)
-            parts[name] = 1e3 * e0.elapsed_ms(e1) / launches - parts["k_compact_map"] - parts["tile scan"]
-            continue
-        e0, e1 = gp_ffi.Event(), gp_ffi.Event()
-        e0.record(stream)
-        for _ in range(launches):
-            f()
-        e1.record(stream)
-        parts[name] = 1e3 * e0.elapsed_ms(e1) / launches
+        for f in calls:
+            f(stream)
+    e1.record(stream)
+    return 1e3 * e0.elapsed_ms(e1) / launches
+
+
+def measure_compaction(gp_ffi, dlp, lp, stream, launches, frac=0.15, seed=7):
+    """Times the compaction the presolve uses (keep maps with their rank words
+    and chunk rows, map pass, chunk offsets and write pass, back to back on one stream) on the
+    full A with 15% of rows and columns dropped (a typical early apply), the
+    passes also by differences, and checks the output against the host."""
+    c = compaction_case(gp_ffi, dlp, lp, frac, seed, False)
+    m, n, nnz, m_new, _, nnz_new = c["sizes"]
+    steps = ("maps", "map", "scan", "write")
+    us = time_launches(gp_ffi, stream, launches, *[c[k] for k in steps])
+    c["check"]()
+    # The write pass needs the map's counts scanned once: its share is the
+    # difference of two runs.
+    parts = {"k_apply_maps": time_launches(gp_ffi, stream, launches, c["maps"]),
+             "k_compact_map": time_launches(gp_ffi, stream, launches, c["map"])}
+    parts["chunk scan"] = time_launches(gp_ffi, stream, launches, c["map"], c["scan"]) - parts["k_compact_map"]
+    parts["k_compact_write"] = us - sum(parts.values())
     nbytes = compaction_bytes(m, n, nnz, m_new, nnz_new)
     floor = compaction_compulsory_bytes(m, n, nnz, m_new, nnz_new)
     log("compaction kernels (us): " + ", ".join(f"{k} {v:.1f}" for k, v in parts.items()))
@@ -306,96 +333,13 @@ def measure_compaction(gp_ffi, dlp, lp, stream, launches, frac=0.15, seed=7):
 
 def measure_compaction_pair(gp_ffi, dlp, lp, stream, launches, frac=0.15, seed=7):
     """Times the compaction a presolve plan application runs: A and its
-    transpose by the same maps, with both rank-word arrays built, one map
-    launch over both matrices' tiles (gpk_compact_map_pair), one scan of both
-    sides' tile counts and one write launch (gpk_compact_write_pair), on the
-    full LP with 15% of rows and columns dropped; checks both outputs against
-    the host."""
-    import ctypes as C
-
-    import numpy as np
-
-    class Lookback(C.Structure):
-        _fields_ = [("status", C.c_void_p), ("ticket", C.c_void_p), ("error", C.c_void_p), ("epoch", C.c_uint32)]
-
-    vp = C.c_void_p
-
-    class Side(C.Structure):
-        _fields_ = [("ptr", vp), ("idx", vp), ("val", vp), ("m_old", C.c_int32), ("m_new", C.c_int32),
-                    ("row_map", vp), ("col_rank", vp), ("jn", vp), ("out_ptr", vp), ("out_idx", vp),
-                    ("out_val", vp)]
-
-    m, n = lp["m"], lp["n"]
-    nnz = len(lp["A_idx"])
-    rng = np.random.default_rng(seed)
-    keep_r = rng.random(m) >= frac
-    keep_c = rng.random(n) >= frac
-    row_map = np.where(keep_r, np.cumsum(keep_r) - 1, -1).astype(np.int32)
-    col_map = np.where(keep_c, np.cumsum(keep_c) - 1, -1).astype(np.int32)
-    rows = np.repeat(np.arange(m), np.diff(lp["A_ptr"]))
-    kept = keep_r[rows] & keep_c[lp["A_idx"]]
-    m_new, n_new, nnz_new = int(keep_r.sum()), int(keep_c.sum()), int(kept.sum())
-    L = gp_ffi.lib()
-    L.gpk_build_rank.argtypes = [vp, C.c_int32, vp, vp]
-    L.gpk_compact_map_pair.argtypes = [Side, Side, vp, vp, vp]
-    L.gpk_compact_write_pair.argtypes = [Side, Side, vp, C.c_int32, vp]
-    L.gpk_compact_tiles.restype = C.c_int32
-    L.gpk_compact_tiles.argtypes = [C.c_int32]
-    L.gpk_scan_lb_i32.argtypes = [vp, vp, C.c_int64, Lookback, vp]
-    L.gpk_lookback_tiles.restype = C.c_int64
-    L.gpk_lookback_tiles.argtypes = [C.c_int64]
-    d_rm, d_cm = gp_ffi.DeviceArray(row_map), gp_ffi.DeviceArray(col_map)
-    c_rank = gp_ffi.DeviceArray(size=2 * ((n + 63) // 64), dtype=np.uint64)
-    r_rank = gp_ffi.DeviceArray(size=2 * ((m + 63) // 64), dtype=np.uint64)
-    jn, t_jn = gp_ffi.DeviceArray(size=nnz, dtype=np.int32), gp_ffi.DeviceArray(size=nnz, dtype=np.int32)
-    o_ptr = gp_ffi.DeviceArray(size=m + 1, dtype=np.int32)
-    t_ptr = gp_ffi.DeviceArray(size=n + 1, dtype=np.int32)
-    o_idx, t_idx = gp_ffi.DeviceArray(size=nnz, dtype=np.int32), gp_ffi.DeviceArray(size=nnz, dtype=np.int32)
-    o_val, t_val = gp_ffi.DeviceArray(size=nnz), gp_ffi.DeviceArray(size=nnz)
-    ta, tt = L.gpk_compact_tiles(m), L.gpk_compact_tiles(n)
-    from_counts = ta <= 256 and tt <= 256
-    t_off = gp_ffi.DeviceArray(size=ta + tt + 1, dtype=np.int32)
-    status = gp_ffi.DeviceArray(np.zeros(max(1, L.gpk_lookback_tiles(ta + tt)), np.uint64))
-    tickets = gp_ffi.DeviceArray(np.zeros(4 * launches + 16, np.int32))
-    err = gp_ffi.DeviceArray(np.zeros(1, np.int32))
-    A, AT = dlp.A.g, dlp.AT.g
-    a = Side(A.row_ptr, A.col_idx, A.val, m, m_new, d_rm.ptr, c_rank.ptr, jn.ptr, o_ptr.ptr, o_idx.ptr, o_val.ptr)
-    t = Side(AT.row_ptr, AT.col_idx, AT.val, n, n_new, d_cm.ptr, r_rank.ptr, t_jn.ptr, t_ptr.ptr, t_idx.ptr,
-             t_val.ptr)
-    launch_no = [0]
-    ck = gp_ffi.hip_check
-
-    def whole():
-        ck(L.gpk_build_rank(d_cm.ptr, n, c_rank.ptr, stream.ptr), "build rank")
-        ck(L.gpk_build_rank(d_rm.ptr, m, r_rank.ptr, stream.ptr), "build rank")
-        ck(L.gpk_compact_map_pair(a, t, t_off.ptr, None, stream.ptr), "map pair")
-        if not from_counts:
-            k = launch_no[0]
-            launch_no[0] += 1
-            lb = Lookback(status.ptr, tickets.ptr + 4 * k, err.ptr, k + 1)
-            ck(L.gpk_scan_lb_i32(t_off.ptr, t_off.ptr, ta + tt, lb, stream.ptr), "scan")
-        ck(L.gpk_compact_write_pair(a, t, t_off.ptr, 1 if from_counts else 0, stream.ptr), "write pair")
-
-    for _ in range(3):
-        whole()
-    stream.sync()
-    e0, e1 = gp_ffi.Event(), gp_ffi.Event()
-    e0.record(stream)
-    for _ in range(launches):
-        whole()
-    e1.record(stream)
-    us = 1e3 * e0.elapsed_ms(e1) / launches
-    want_ptr = np.concatenate([[0], np.cumsum(np.bincount(rows[kept], minlength=m)[keep_r])]).astype(np.int32)
-    at_rows = np.repeat(np.arange(n), np.diff(lp["AT_ptr"]))
-    t_kept = keep_c[at_rows] & keep_r[lp["AT_idx"]]
-    want_tptr = np.concatenate([[0], np.cumsum(np.bincount(at_rows[t_kept], minlength=n)[keep_c])]).astype(np.int32)
-    if (err.numpy()[0] != 0 or not np.array_equal(o_ptr.numpy()[:m_new + 1], want_ptr)
-            or not np.array_equal(o_idx.numpy()[:nnz_new], col_map[lp["A_idx"][kept]])
-            or not np.array_equal(o_val.numpy()[:nnz_new], lp["A_val"][kept])
-            or not np.array_equal(t_ptr.numpy()[:n_new + 1], want_tptr)
-            or not np.array_equal(t_idx.numpy()[:nnz_new], row_map[lp["AT_idx"][t_kept]])
-            or not np.array_equal(t_val.numpy()[:nnz_new], lp["AT_val"][t_kept])):
-        raise SystemExit("bench.py: the paired compaction differs from the host")
+    transpose by the same maps: the keep maps, one map launch, one scan of both sides' chunk counts and one write
+    launch, on the full LP with 15% of rows and columns dropped; checks both
+    outputs against the host."""
+    c = compaction_case(gp_ffi, dlp, lp, frac, seed, True)
+    m, n, nnz, m_new, n_new, nnz_new = c["sizes"]
+    us = time_launches(gp_ffi, stream, launches, *[c[k] for k in ("maps", "map", "scan", "write")])
+    c["check"]()
     nbytes = compaction_bytes(m, n, nnz, m_new, nnz_new) + compaction_bytes(n, m, nnz, n_new, nnz_new)
     log(f"paired compaction (A and AT): {us:.1f} us/call, {nbytes / (us * 1e-6) / 1e9:.0f} GB/s")
     return {"us": us, "bytes": nbytes, "achieved": nbytes / (us * 1e-6) / 1e9,
@@ -596,8 +540,8 @@ def transpose_traffic():
 def compaction_traffic():
     """HBM bytes of one compaction call: the sum over its kernels in the
     committed PMC summary, or None when one of them is missing."""
-    parts = [profiled_traffic(k) for k in ("k_build_rank", "k_compact_map", "k_scan_small<int, 0>",
-                                           "k_compact_write<false>")]
+    parts = [profiled_traffic(k) for k in ("k_apply_counts", "k_apply_maps<2>", "k_compact_map<8>",
+                                           "k_scan_small<int>", "k_compact_write<8>")]
     return None if any(p is None for p in parts) else sum(parts)
 
 
@@ -1242,7 +1186,7 @@ def main():
                    "iterations": summary["iterations"], "postsolve_ms": post_ms,
                    "postsolve_prepare_ms": prep_ms, "postsolve_prepared_run_ms": plan_ms},
         "roofline": {"bound": "hbm",
-                     "kernel": "compaction: k_build_rank + k_compact_map + tile-offset scan + k_compact_write",
+                     "kernel": "compaction: k_apply_counts + k_apply_maps + k_compact_map + chunk-offset scan + k_compact_write",
                      "achieved": comp["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": comp["achieved"] / HBM_PEAK_GBS, "traffic": compaction_traffic(),
                      "us_per_call": comp["us"], "algorithmic_bytes": comp["bytes"],
@@ -1250,8 +1194,8 @@ def main():
                      "compulsory_frac": comp["compulsory_achieved"] / HBM_PEAK_GBS,
                      "workload": comp["workload"], "kernels_us": comp["kernels_us"]},
         "roofline_compaction_pair": {"bound": "hbm",
-                                     "kernel": "paired compaction of A and AT: 2 x k_build_rank + "
-                                               "k_compact_map_pair + tile-offset scan + k_compact_write_pair",
+                                     "kernel": "paired compaction of A and AT: k_apply_counts + k_apply_maps + "
+                                               "k_compact_map + chunk-offset scan + k_compact_write",
                                      "achieved": comp["pair"]["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                      "frac": comp["pair"]["achieved"] / HBM_PEAK_GBS, "traffic": None,
                                      "us_per_call": comp["pair"]["us"],

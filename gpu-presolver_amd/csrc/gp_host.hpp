@@ -437,51 +437,36 @@ double ordered_masked_sum(const uint8_t* mask, const double* vals, int32_t n);
 // wait and the addition runs at the next wait (Ctx::after_wait), in the
 // order of the calls; the mask and values may be released once this returns.
 void add_ordered_masked_sum(double* target, const uint8_t* mask, const double* vals, int32_t n);
-// Compacts A by row/column keep maps; the result owns fresh device arrays.
-// known_nnz >= 0 is the kept count when the caller knows it (the transpose
-// of a matrix compacted with the same maps): the read-back is skipped.
-// col_rank: the column map's rank words when the caller has them (unused
-// when n_new == A.cols: no column is dropped and col_map is the identity).
-presolve::DeviceCsrMatrix compact_csr(const presolve::DeviceCsrMatrix& A, const int32_t* row_map,
-                                      const int32_t* col_map, int32_t m_new, int32_t n_new, int32_t known_nnz = -1,
-                                      const gpk_rank_word* col_rank = nullptr);
+// Compacts A by its keep masks (device); the result owns fresh device arrays.
+presolve::DeviceCsrMatrix compact_csr(const presolve::DeviceCsrMatrix& A, const uint8_t* keep_row,
+                                      const uint8_t* keep_col);
 // The same compaction in two halves, for a caller that reads the new sizes
-// in its own wait: compact_start launches the map pass (and, past 256 tiles,
-// the tile-offset scan) while the sizes are still unknown (every kept column
-// goes through col_rank, which must be given); the map pass adds the kept
-// entry count to the device word `kept`, which the caller zeroes.
-// compact_finish then writes the compacted matrix.  The row-pointer array is
-// sized for A.rows + 1.
+// in its own wait, of A and (when AT is given: a transpose of A with sorted
+// rows) of AT by the same maps: compact_start launches the map pass while the
+// sizes are still unknown (every kept column goes through the rank words); it
+// adds A's kept entry count to the device word `kept`, which the caller
+// zeroes.  compact_add_transpose adds an AT that is known only after the wait.
+// compact_finish writes the compacted matrices and, when an AT takes part and
+// gathers are given, runs them in the same launch (out.gathered).  The maps,
+// rank words and chunk rows (gpk_apply_maps) stay allocated until then.
 struct CompactStart {
   const presolve::DeviceCsrMatrix* A = nullptr;
-  const int32_t* row_map = nullptr;
-  DBuf<int32_t> ptr, jn, tile_off;
-  bool few_tiles = false;  // tile_off holds raw counts (no scan launched)
+  const presolve::DeviceCsrMatrix* AT = nullptr;
+  gpk_compact_side a{}, t{};
+  DBuf<char> work;
+  int32_t* cnt = nullptr;  // chunk counts, A's then AT's; null: nothing to compact
 };
 CompactStart compact_start(const presolve::DeviceCsrMatrix& A, const int32_t* row_map, const gpk_rank_word* col_rank,
-                           int32_t* kept);
-presolve::DeviceCsrMatrix compact_finish(CompactStart& st, int32_t m_new, int32_t n_new, int32_t nnz_new);
-// The two halves for A and a transpose of it with sorted rows, compacted by
-// the same maps (AT's rows by col_map, its columns by the row rank words):
-// compact_start_pair launches one map pass over both matrices' tiles and, past
-// 256 tiles on either side, one scan of both sides' tile counts;
-// compact_finish_pair writes both in one launch.  `kept` receives A's kept
-// count as in compact_start.
-struct CompactPairStart {
-  const presolve::DeviceCsrMatrix* A = nullptr;
-  const presolve::DeviceCsrMatrix* AT = nullptr;
-  const int32_t* row_map = nullptr;
-  const int32_t* col_map = nullptr;
-  DBuf<int32_t> ptr, t_ptr, jn, t_jn, tile_off;
-  bool from_counts = false;  // tile_off holds raw counts (no scan launched)
+                           const int32_t* chunk_row, int32_t* kept, const presolve::DeviceCsrMatrix* AT,
+                           const int32_t* col_map, const gpk_rank_word* row_rank, const int32_t* t_chunk_row);
+void compact_add_transpose(CompactStart& st, const presolve::DeviceCsrMatrix& AT, const int32_t* col_map,
+                           const gpk_rank_word* row_rank, const int32_t* t_chunk_row);
+struct CompactOut {
+  presolve::DeviceCsrMatrix A, AT;  // AT null arrays when none took part
+  bool gathered = false;
 };
-CompactPairStart compact_start_pair(const presolve::DeviceCsrMatrix& A, const int32_t* row_map,
-                                    const gpk_rank_word* col_rank, const presolve::DeviceCsrMatrix& AT,
-                                    const int32_t* col_map, const gpk_rank_word* row_rank, int32_t* kept);
-// {compacted A, compacted AT}; both hold nnz_new entries.
-std::pair<presolve::DeviceCsrMatrix, presolve::DeviceCsrMatrix> compact_finish_pair(CompactPairStart& st,
-                                                                                     int32_t m_new, int32_t n_new,
-                                                                                     int32_t nnz_new);
+CompactOut compact_finish(CompactStart& st, int32_t m_new, int32_t n_new, int32_t nnz_new,
+                          const gpk_apply_gathers_args* gathers);
 // Stable transpose (rows of the result sorted); fresh device arrays.
 presolve::DeviceCsrMatrix transpose_csr(const presolve::DeviceCsrMatrix& A);
 void free_csr(presolve::DeviceCsrMatrix& A) noexcept;
@@ -543,8 +528,6 @@ struct PipelineReport {
 PipelineReport presolve_solve(const presolve::LPInfoGpu& lp, const presolve::PresolveParams& prm,
                               const PdhgOptions& solve, double* x, double* y, double* z);
 void screen_structural_l1(const presolve::LPInfoGpu& lp, const presolve::PresolveParams& prm);
-// old_to_new map of a keep mask; returns the kept count.
-int32_t build_old_to_new(const uint8_t* mask, int32_t n, DBuf<int32_t>& map);
 // FixedCol records and the long-double objective delta
 // (fixed_col_tape.cu:107-267).
 double fixed_col_tape(presolve::PostsolveTape* tape, const uint8_t* fixed_mask, const uint8_t* excluded,

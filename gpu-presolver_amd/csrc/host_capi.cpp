@@ -414,10 +414,7 @@ gp_status gp_compact_csr(const gp_csr* A, const uint8_t* keep_row, const uint8_t
     require((A->rows == 0 || keep_row) && (A->cols == 0 || keep_col), "null keep mask");
     require_device();
     amd::check(hipDeviceSynchronize(), "entry synchronize");
-    amd::DBuf<int32_t> row_map, col_map;
-    const int32_t m_new = amd::build_old_to_new(keep_row, A->rows, row_map);
-    const int32_t n_new = amd::build_old_to_new(keep_col, A->cols, col_map);
-    const DeviceCsrMatrix r = amd::compact_csr(to_csr(*A), row_map, col_map, m_new, n_new);
+    const DeviceCsrMatrix r = amd::compact_csr(to_csr(*A), keep_row, keep_col);
     amd::ctx().sync("gp_compact_csr");
     *out = from_csr(r);
   });

@@ -507,15 +507,6 @@ void add_ordered_masked_sum(double* target, const uint8_t* mask, const double* v
   });
 }
 
-int32_t build_old_to_new(const uint8_t* mask, int32_t n, DBuf<int32_t>& map) {
-  map.alloc(static_cast<int64_t>(n) + 1, "old_to_new");
-  if (n == 0) return 0;
-  Ctx& c = ctx();
-  int32_t* count = map.get() + n;  // spare word after the map
-  check(gpk_mask_to_map(mask, map, n, count, c.lookback(gpk_lookback_tiles(n)), c.stream()), "old_to_new");
-  return c.scalar_to_host(count, "old_to_new count");
-}
-
 void free_csr(DeviceCsrMatrix& A) noexcept {
   hipStream_t s = ctx().stream();
   dev_free(A.rowPtr, s);
@@ -526,189 +517,154 @@ void free_csr(DeviceCsrMatrix& A) noexcept {
   A.nzVal = nullptr;
 }
 
-// compact_csr_by_masks_gpu (gpu_presolve.cu:1881-1978): the column map in
-// rank form, one mapping pass over the entries (per-entry new column and
-// per-row kept counts), an exclusive scan into the row pointers, then the
-// coalesced write of the kept entries.
-// Up to this many 256-row tiles the write pass derives the tile offsets
-// itself (gpk_compact_write_counts), one launch fewer.
-constexpr int32_t kCompactFewTiles = 256;
-
-DeviceCsrMatrix compact_csr(const DeviceCsrMatrix& A, const int32_t* row_map, const int32_t* col_map, int32_t m_new,
-                            int32_t n_new, int32_t known_nnz, const gpk_rank_word* col_rank) {
-  Ctx& c = ctx();
-  DeviceCsrMatrix out;
-  out.rows = m_new;
-  out.cols = n_new;
-  DBuf<int32_t> ptr(static_cast<int64_t>(m_new) + 1, "compact rowPtr");
-  if (m_new == 0 || n_new == 0 || A.nnz == 0) {
-    check(hipMemsetAsync(ptr.get(), 0, sizeof(int32_t) * (static_cast<size_t>(m_new) + 1), c.stream()),
-          "compact empty rowPtr");
-    out.rowPtr = ptr.release();
-    return out;
-  }
-  const int32_t m_old = A.rows;
-  DBuf<gpk_rank_word> rank;
-  DBuf<int32_t> jn(A.nnz, "compact entry map");
-  hipStream_t s = c.stream();
-  if (n_new == A.cols) {
-    col_rank = nullptr;  // no column dropped: every entry keeps its column index
-  } else if (col_rank == nullptr) {
-    rank.alloc((static_cast<int64_t>(A.cols) + 63) / 64, "compact column rank");
-    check(gpk_build_rank(col_map, A.cols, rank, s), "compact column rank");
-    col_rank = rank.get();
-  }
-  const int32_t tiles = gpk_compact_tiles(m_old);
-  DBuf<int32_t> tile_off(static_cast<int64_t>(tiles) + 1, "compact tile offsets");
-  check(gpk_compact_map(A.rowPtr, A.colVal, m_old, row_map, col_rank, jn, ptr, tile_off, s), "compact map");
-  const bool few_tiles = tiles <= kCompactFewTiles;
-  if (!few_tiles)
-    check(gpk_scan_lb_i32(tile_off, tile_off, tiles, c.lookback(gpk_lookback_tiles(tiles)), s),
-          "compact tile offsets");
-  // Kept entries are at most A.nnz: the outputs are sized for that and the
-  // kept count is read back once the entries are written.
-  DBuf<int32_t> idx(A.nnz, "compact colVal");
-  DBuf<double> val(A.nnz, "compact nzVal");
-  if (few_tiles)
-    check(gpk_compact_write_counts(A.rowPtr, A.nzVal, m_old, row_map, jn, tile_off, ptr, m_new, idx, val, s),
-          "compact write");
-  else
-    check(gpk_compact_write(A.rowPtr, A.nzVal, m_old, row_map, jn, tile_off, ptr, m_new, idx, val, s),
-          "compact write");
-  out.nnz = known_nnz >= 0 ? known_nnz : c.scalar_to_host(ptr.get() + m_new, "compact kept count");
-  out.rowPtr = ptr.release();
-  out.colVal = idx.release();
-  out.nzVal = val.release();
-  return out;
-}
-
-CompactStart compact_start(const DeviceCsrMatrix& A, const int32_t* row_map, const gpk_rank_word* col_rank,
-                           int32_t* kept) {
-  Ctx& c = ctx();
-  hipStream_t s = c.stream();
-  CompactStart st;
-  st.A = &A;
-  st.row_map = row_map;
-  st.ptr.alloc(static_cast<int64_t>(A.rows) + 1, "compact rowPtr");
-  if (A.rows == 0 || A.nnz == 0) return st;  // *kept stays as the caller zeroed it
-  if (col_rank == nullptr) throw std::logic_error("compact_start: the column rank words are required");
-  const int32_t tiles = gpk_compact_tiles(A.rows);
-  st.jn.alloc(A.nnz, "compact entry map");
-  st.tile_off.alloc(static_cast<int64_t>(tiles) + 1, "compact tile offsets");
-  check(gpk_compact_map_total(A.rowPtr, A.colVal, A.rows, row_map, col_rank, st.jn, st.ptr, st.tile_off, kept, s),
-        "compact map");
-  st.few_tiles = tiles <= kCompactFewTiles;  // the write pass derives the offsets from the raw counts
-  if (!st.few_tiles)
-    check(gpk_scan_lb_i32(st.tile_off, st.tile_off, tiles, c.lookback(gpk_lookback_tiles(tiles)), s),
-          "compact tile offsets");
-  return st;
-}
-
-DeviceCsrMatrix compact_finish(CompactStart& st, int32_t m_new, int32_t n_new, int32_t nnz_new) {
-  Ctx& c = ctx();
-  hipStream_t s = c.stream();
-  const DeviceCsrMatrix& A = *st.A;
-  DeviceCsrMatrix out;
-  out.rows = m_new;
-  out.cols = n_new;
-  if (m_new == 0 || n_new == 0 || A.nnz == 0 || st.jn.get() == nullptr) {
-    CopyBatch().zero(st.ptr.get(), static_cast<int64_t>(m_new) + 1).run("compact empty rowPtr");
-    out.rowPtr = st.ptr.release();
-    return out;
-  }
-  DBuf<int32_t> idx(A.nnz, "compact colVal");
-  DBuf<double> val(A.nnz, "compact nzVal");
-  if (st.few_tiles)
-    check(gpk_compact_write_counts(A.rowPtr, A.nzVal, A.rows, st.row_map, st.jn, st.tile_off, st.ptr, m_new, idx, val,
-                                   s),
-          "compact write");
-  else
-    check(gpk_compact_write(A.rowPtr, A.nzVal, A.rows, st.row_map, st.jn, st.tile_off, st.ptr, m_new, idx, val, s),
-          "compact write");
-  out.nnz = nnz_new;
-  out.rowPtr = st.ptr.release();
-  out.colVal = idx.release();
-  out.nzVal = val.release();
-  return out;
-}
-
+// ---- compaction (compact_csr_by_masks_gpu, gpu_presolve.cu:1881-1978) -------
 namespace {
+size_t align256(size_t b) { return (b + 255) & ~size_t{255}; }
+size_t compact_words(int32_t nnz) {
+  return (static_cast<size_t>(gpk_compact_chunks(nnz)) << gpk_compact_shift(nnz)) / 64;
+}
+// A side's entry map, kept-entry words and their prefix sums.
+size_t compact_work_bytes(int32_t nnz) {
+  const size_t words = compact_words(nnz);
+  return align256(sizeof(int32_t) * static_cast<size_t>(nnz)) + align256(sizeof(uint64_t) * words) +
+         align256(sizeof(int32_t) * words);
+}
 gpk_compact_side compact_side(const DeviceCsrMatrix& M, const int32_t* row_map, const gpk_rank_word* col_rank,
-                              int32_t* jn, int32_t* out_ptr) {
-  return gpk_compact_side{M.rowPtr, M.colVal, M.nzVal, M.rows, 0, row_map, col_rank, jn, out_ptr, nullptr, nullptr};
+                              const int32_t* chunk_row, char* work) {
+  const size_t words = compact_words(M.nnz);
+  gpk_compact_side s{};
+  s.ptr = M.rowPtr;
+  s.idx = M.colVal;
+  s.val = M.nzVal;
+  s.m_old = M.rows;
+  s.nnz = M.nnz;
+  s.row_map = row_map;
+  s.col_rank = col_rank;
+  s.chunk_row = chunk_row;
+  s.jn = reinterpret_cast<int32_t*>(work);
+  work += align256(sizeof(int32_t) * static_cast<size_t>(M.nnz));
+  s.mask = reinterpret_cast<uint64_t*>(work);
+  work += align256(sizeof(uint64_t) * words);
+  s.word_pre = reinterpret_cast<int32_t*>(work);
+  return s;
 }
 }  // namespace
 
-CompactPairStart compact_start_pair(const DeviceCsrMatrix& A, const int32_t* row_map, const gpk_rank_word* col_rank,
-                                    const DeviceCsrMatrix& AT, const int32_t* col_map, const gpk_rank_word* row_rank,
-                                    int32_t* kept) {
-  Ctx& c = ctx();
-  hipStream_t s = c.stream();
-  if (AT.rows != A.cols || AT.cols != A.rows || AT.nnz != A.nnz)
-    throw std::logic_error("compact_start_pair: AT is not the transpose shape of A");
-  CompactPairStart st;
+CompactStart compact_start(const DeviceCsrMatrix& A, const int32_t* row_map, const gpk_rank_word* col_rank,
+                           const int32_t* chunk_row, int32_t* kept, const DeviceCsrMatrix* AT, const int32_t* col_map,
+                           const gpk_rank_word* row_rank, const int32_t* t_chunk_row) {
+  if (AT != nullptr && (AT->rows != A.cols || AT->cols != A.rows || AT->nnz != A.nnz))
+    throw std::logic_error("compact_start: AT is not the transpose shape of A");
+  CompactStart st;
   st.A = &A;
-  st.AT = &AT;
-  st.row_map = row_map;
-  st.col_map = col_map;
-  st.ptr.alloc(static_cast<int64_t>(A.rows) + 1, "compact rowPtr");
-  st.t_ptr.alloc(static_cast<int64_t>(AT.rows) + 1, "compact AT rowPtr");
-  if (A.rows == 0 || AT.rows == 0 || A.nnz == 0) return st;  // *kept stays as the caller zeroed it
-  if (col_rank == nullptr || row_rank == nullptr)
-    throw std::logic_error("compact_start_pair: both sides' rank words are required");
-  const int32_t ta = gpk_compact_tiles(A.rows), tt = gpk_compact_tiles(AT.rows);
-  st.jn.alloc(A.nnz, "compact entry map");
-  st.t_jn.alloc(AT.nnz, "compact AT entry map");
-  st.tile_off.alloc(static_cast<int64_t>(ta) + tt + 1, "compact tile offsets");
-  check(gpk_compact_map_pair(compact_side(A, row_map, col_rank, st.jn, st.ptr),
-                             compact_side(AT, col_map, row_rank, st.t_jn, st.t_ptr), st.tile_off, kept, s),
-        "compact map pair");
-  st.from_counts = ta <= kCompactFewTiles && tt <= kCompactFewTiles;
-  if (!st.from_counts)
-    check(gpk_scan_lb_i32(st.tile_off, st.tile_off, ta + tt, c.lookback(gpk_lookback_tiles(ta + tt)), s),
-          "compact tile offsets");
+  st.AT = AT;
+  if (A.rows == 0 || A.cols == 0 || A.nnz == 0) return st;  // *kept stays as the caller zeroed it
+  const int32_t chunks = gpk_compact_chunks(A.nnz);
+  const size_t side = compact_work_bytes(A.nnz);
+  // Room for the transpose as well: it may be added after the sizes are read.
+  st.work.alloc(static_cast<int64_t>(2 * side + sizeof(int32_t) * (2 * static_cast<size_t>(chunks) + 1)),
+                "compact work");
+  st.cnt = reinterpret_cast<int32_t*>(st.work.get() + 2 * side);
+  st.a = compact_side(A, row_map, col_rank, chunk_row, st.work.get());
+  if (AT != nullptr) st.t = compact_side(*AT, col_map, row_rank, t_chunk_row, st.work.get() + side);
+  check(gpk_compact_map(st.a, st.t, st.cnt, kept, ctx().stream()), "compact map");
   return st;
 }
 
-std::pair<DeviceCsrMatrix, DeviceCsrMatrix> compact_finish_pair(CompactPairStart& st, int32_t m_new, int32_t n_new,
-                                                                int32_t nnz_new) {
+void compact_add_transpose(CompactStart& st, const DeviceCsrMatrix& AT, const int32_t* col_map,
+                           const gpk_rank_word* row_rank, const int32_t* t_chunk_row) {
+  if (AT.rows != st.A->cols || AT.cols != st.A->rows || AT.nnz != st.A->nnz)
+    throw std::logic_error("compact_add_transpose: AT is not the transpose shape of A");
+  st.AT = &AT;
+  if (st.cnt == nullptr) return;
+  st.t = compact_side(AT, col_map, row_rank, t_chunk_row, st.work.get() + compact_work_bytes(AT.nnz));
+  check(gpk_compact_map(gpk_compact_side{}, st.t, st.cnt + gpk_compact_chunks(AT.nnz), nullptr, ctx().stream()),
+        "compact map of the transpose");
+}
+
+CompactOut compact_finish(CompactStart& st, int32_t m_new, int32_t n_new, int32_t nnz_new,
+                          const gpk_apply_gathers_args* gathers) {
   Ctx& c = ctx();
   hipStream_t s = c.stream();
-  const DeviceCsrMatrix& A = *st.A;
-  const DeviceCsrMatrix& AT = *st.AT;
-  DeviceCsrMatrix a_out, t_out;
-  a_out.rows = m_new;
-  a_out.cols = n_new;
-  t_out.rows = n_new;
-  t_out.cols = m_new;
-  if (m_new == 0 || n_new == 0 || A.nnz == 0 || st.jn.get() == nullptr) {
-    CopyBatch()
-        .zero(st.ptr.get(), static_cast<int64_t>(m_new) + 1)
-        .zero(st.t_ptr.get(), static_cast<int64_t>(n_new) + 1)
-        .run("compact empty rowPtr");
-    a_out.rowPtr = st.ptr.release();
-    t_out.rowPtr = st.t_ptr.release();
-    return {a_out, t_out};
+  CompactOut out;
+  out.A.rows = out.AT.cols = m_new;
+  out.A.cols = out.AT.rows = n_new;
+  DBuf<int32_t> ptr(static_cast<int64_t>(m_new) + 1, "compact rowPtr"), t_ptr;
+  if (st.AT != nullptr) t_ptr.alloc(static_cast<int64_t>(n_new) + 1, "compact AT rowPtr");
+  if (m_new == 0 || n_new == 0 || st.cnt == nullptr) {
+    CopyBatch zeros;
+    zeros.zero(ptr.get(), static_cast<int64_t>(m_new) + 1);
+    if (st.AT != nullptr) zeros.zero(t_ptr.get(), static_cast<int64_t>(n_new) + 1);
+    zeros.run("compact empty rowPtr");
+    out.A.rowPtr = ptr.release();
+    out.AT.rowPtr = t_ptr.release();
+    return out;
   }
-  DBuf<int32_t> idx(A.nnz, "compact colVal"), t_idx(AT.nnz, "compact AT colVal");
-  DBuf<double> val(A.nnz, "compact nzVal"), t_val(AT.nnz, "compact AT nzVal");
-  gpk_compact_side a = compact_side(A, st.row_map, nullptr, st.jn, st.ptr);
-  gpk_compact_side t = compact_side(AT, st.col_map, nullptr, st.t_jn, st.t_ptr);
-  a.m_new = m_new;
-  a.out_idx = idx;
-  a.out_val = val;
-  t.m_new = n_new;
-  t.out_idx = t_idx;
-  t.out_val = t_val;
-  check(gpk_compact_write_pair(a, t, st.tile_off, st.from_counts ? 1 : 0, s), "compact write pair");
-  a_out.nnz = t_out.nnz = nnz_new;
-  a_out.rowPtr = st.ptr.release();
-  a_out.colVal = idx.release();
-  a_out.nzVal = val.release();
-  t_out.rowPtr = st.t_ptr.release();
-  t_out.colVal = t_idx.release();
-  t_out.nzVal = t_val.release();
-  return {a_out, t_out};
+  const int32_t nnz = st.A->nnz, chunks = gpk_compact_chunks(nnz);
+  const int32_t scanned = chunks * (st.AT != nullptr ? 2 : 1);
+  const bool from_counts = chunks <= GPK_COMPACT_COUNT_CHUNKS;
+  if (!from_counts)
+    check(gpk_scan_lb_i32(st.cnt, st.cnt, scanned, c.lookback(gpk_lookback_tiles(scanned)), s),
+          "compact chunk offsets");
+  DBuf<int32_t> idx(nnz, "compact colVal"), t_idx;
+  DBuf<double> val(nnz, "compact nzVal"), t_val;
+  gpk_apply_gathers_args g{};
+  st.a.m_new = m_new;
+  st.a.out_ptr = ptr;
+  st.a.out_idx = idx;
+  st.a.out_val = val;
+  if (st.AT != nullptr) {
+    t_idx.alloc(nnz, "compact AT colVal");
+    t_val.alloc(nnz, "compact AT nzVal");
+    st.t.m_new = n_new;
+    st.t.out_ptr = t_ptr;
+    st.t.out_idx = t_idx;
+    st.t.out_val = t_val;
+    if (gathers != nullptr) {
+      g = *gathers;
+      out.gathered = true;
+    }
+  }
+  check(gpk_compact_write(st.a, st.t, st.cnt, from_counts ? 1 : 0, g, s), "compact write");
+  out.A.nnz = nnz_new;
+  out.A.rowPtr = ptr.release();
+  out.A.colVal = idx.release();
+  out.A.nzVal = val.release();
+  if (st.AT != nullptr) {
+    out.AT.nnz = nnz_new;
+    out.AT.rowPtr = t_ptr.release();
+    out.AT.colVal = t_idx.release();
+    out.AT.nzVal = t_val.release();
+  }
+  return out;
+}
+
+DeviceCsrMatrix compact_csr(const DeviceCsrMatrix& A, const uint8_t* keep_row, const uint8_t* keep_col) {
+  Ctx& c = ctx();
+  DBuf<int32_t> row_map(A.rows, "row map"), col_map(A.cols, "column map");
+  DBuf<gpk_rank_word> col_rank((static_cast<int64_t>(A.cols) + 63) / 64, "column rank");
+  DBuf<int32_t> chunk_row(static_cast<int64_t>(gpk_compact_chunks(A.nnz)) + 1, "chunk rows");
+  const int64_t tiles = gpk_apply_maps_tiles(A.rows, A.cols);
+  DBuf<int32_t> tile_counts(tiles, "map tile counts");
+  int32_t* counts = c.flags();
+  gpk_apply_maps_args maps{};
+  maps.m = A.rows;
+  maps.n = A.cols;
+  maps.keep_row = keep_row;
+  maps.keep_col = keep_col;
+  maps.row_map = row_map;
+  maps.col_map = col_map;
+  maps.counts = counts;
+  maps.col_rank = col_rank;
+  maps.a_ptr = A.rowPtr;
+  maps.a_chunk = chunk_row;
+  maps.tile_counts = tile_counts;
+  maps.chunk_shift = gpk_compact_shift(A.nnz);
+  check(gpk_apply_maps(maps, c.lookback(tiles), c.stream()), "keep maps");
+  CompactStart st = compact_start(A, row_map, col_rank, chunk_row, counts + 4, nullptr, nullptr, nullptr, nullptr);
+  int32_t h[5];
+  std::memcpy(h, c.read_flags(5), sizeof(h));
+  return compact_finish(st, h[0], h[1], h[4], nullptr).A;
 }
 
 // Stable transpose: LSD radix sort of the column indices (entries already in

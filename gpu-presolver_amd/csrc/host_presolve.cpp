@@ -389,12 +389,14 @@ void append_global_tape(RecordState& rs, const PostsolveTape& src) {
 }
 
 // update_record_from_plan (gpu_presolve.cu:1535-1802).
-// fixed: the removed columns with a finite fixed interval (mask and its
-// old-to-new map, k of them), computed by apply_plan with the keep maps.
+// fixed: the removed columns with a finite fixed interval (mask and its counts
+// per map tile, k of them), computed by apply_plan with the keep maps.
 struct FixedCols {
   DBuf<uint8_t> mask;
-  DBuf<int32_t> map;
+  DBuf<int32_t> tiles;
   int32_t k = 0;
+  DBuf<int32_t> idx;  // the k records: global index and midpoint
+  DBuf<double> val;
 };
 
 // row_r2o_next / col_r2o_next: the maps already gathered through row_map /
@@ -406,19 +408,15 @@ void update_record(RecordState& rs, const PresolvePlanGpu& p, int32_t m, int32_t
   hipStream_t s = c.stream();
   PresolveRecordGpu& rec = *rs.rec;
   if (fixed.k > 0) {
-    // Removed columns with a finite fixed interval become (global index, midpoint).
+    // Removed columns with a finite fixed interval, packed by apply_plan.
     const int32_t k = fixed.k;
-    DBuf<int32_t> oi(k);
-    DBuf<double> ov(k);
-    check(gpk_pack_fixed_records(n, fixed.mask, fixed.map, rs.col_r2o, p.new_l, p.new_u, oi, ov, s),
-          "fixed records");
     const size_t base = rec.fixed_idx.size();
     rec.fixed_idx.resize(base + static_cast<size_t>(k));
     rec.fixed_val.resize(base + static_cast<size_t>(k));
     // Land at the context's next wait, like the tape indices below.
     c.begin_copy_group();
-    c.download(rec.fixed_idx.data() + base, oi.get(), sizeof(int32_t) * k, "fixed records idx");
-    c.download(rec.fixed_val.data() + base, ov.get(), sizeof(double) * k, "fixed records val");
+    c.download(rec.fixed_idx.data() + base, fixed.idx.get(), sizeof(int32_t) * k, "fixed records idx");
+    c.download(rec.fixed_val.data() + base, fixed.val.get(), sizeof(double) * k, "fixed records val");
     c.end_copy_group("fixed records");
   }
   append_global_tape(rs, p.tape);
@@ -457,39 +455,47 @@ void apply_plan(WorkLp& cur, const PresolvePlanGpu& p, RecordState& rs, const De
   DBuf<int32_t> row_map(static_cast<int64_t>(m) + 1), col_map(static_cast<int64_t>(n) + 1);
   FixedCols fixed;
   fixed.mask.alloc(n);
-  fixed.map.alloc(static_cast<int64_t>(n) + 1);
+  fixed.tiles.alloc(gpk_apply_maps_tiles(0, n));
   int32_t* counts = c.flags();
   // Rank words of both maps (the column map's for compacting A, the row
-  // map's for compacting AT) come out of the same launch.
+  // map's for compacting AT) and the chunk rows of the matrices to compact
+  // come out of the same launch.
   DBuf<gpk_rank_word> row_rank((static_cast<int64_t>(m) + 63) / 64), col_rank((static_cast<int64_t>(n) + 63) / 64);
+  const DeviceCsrMatrix& src = p.has_new_A ? p.new_A : cur.lp.A;
+  // An AT with sorted rows that is the exact transpose of the A being
+  // compacted (the working AT, the caller's AT when sorted, the rebuilding
+  // rule's AT of a new A) is compacted with the maps swapped, which gives
+  // the transpose of the compacted A; otherwise the compacted A is
+  // re-transposed.
+  const DeviceCsrMatrix* at = p.has_new_A ? new_at : &cur.lp.AT;
+  const int32_t chunks = gpk_compact_chunks(src.nnz);
+  DBuf<int32_t> a_chunk(static_cast<int64_t>(chunks) + 1), at_chunk(static_cast<int64_t>(chunks) + 1);
+  const int64_t tiles = gpk_apply_maps_tiles(m, n);
+  DBuf<int32_t> tile_counts(tiles);
   const gpk_apply_maps_args maps{m, n, p.keep_row_mask, p.keep_col_mask, p.new_l, p.new_u, row_map, col_map,
-                                 fixed.mask, fixed.map, counts, row_rank.get(), col_rank.get()};
-  check(gpk_apply_maps(maps, c.lookback(gpk_apply_maps_tiles(m, n)), s), "keep maps");
+                                 fixed.mask, fixed.tiles, counts, row_rank.get(), col_rank.get(),
+                                 src.rowPtr, at != nullptr ? at->rowPtr : nullptr, a_chunk, at_chunk, tile_counts,
+                                 gpk_compact_shift(src.nnz)};
+  check(gpk_apply_maps(maps, c.lookback(tiles), s), "keep maps");
   // The caller's AT (first change) is compacted like a working AT when its
   // rows are sorted; the flag comes back with the counts.
   const bool callers_at = !cur.owns && !p.has_new_A;
   if (callers_at && cur.lp.AT.rows > 0 && cur.lp.AT.nnz > 1)
     check(gpk_rows_unsorted(cur.lp.AT.rowPtr, cur.lp.AT.colVal, cur.lp.AT.rows, counts + 3, s), "AT sorted check");
   // A plan that may drop rows or columns (or rebuilt A) has A's map pass
-  // and tile scan launched before the sizes are read, so the kept entry
-  // count comes back in the same wait as the three counts.
-  const DeviceCsrMatrix& src = p.has_new_A ? p.new_A : cur.lp.A;
+  // launched before the sizes are read, so the kept entry count comes back in
+  // the same wait as the three counts; AT's goes out with it when the AT to
+  // compact is known by then.
   const bool early = p.has_new_A || p.has_row_action || p.has_col_action;
-  // When the AT to compact is known before the wait (the working AT, or the
-  // rebuilding rule's transpose of its new A), both matrices' map passes go
-  // out in one launch now and both write passes in one launch after it.
-  const DeviceCsrMatrix* at_early = !early ? nullptr : p.has_new_A ? new_at : cur.owns ? &cur.lp.AT : nullptr;
-  amd::CompactStart a_start;
-  amd::CompactPairStart pair_start;
-  if (at_early)
-    pair_start =
-        amd::compact_start_pair(src, row_map, col_rank.get(), *at_early, col_map, row_rank.get(), counts + 4);
-  else if (early)
-    a_start = amd::compact_start(src, row_map, col_rank.get(), counts + 4);
+  const bool at_early = early && at != nullptr && !callers_at;
+  amd::CompactStart start;
+  if (early)
+    start = amd::compact_start(src, row_map, col_rank, a_chunk, counts + 4, at_early ? at : nullptr, col_map, row_rank,
+                               at_chunk);
   const int32_t* h = c.read_flags(early ? 5 : 4);
-  const bool callers_at_sorted = callers_at && h[3] == 0;
+  if (callers_at && h[3] != 0) at = nullptr;
   const int32_t m_new = h[0], n_new = h[1];
-  const int32_t a_nnz = early ? h[4] : -1;
+  int32_t a_nnz = early ? h[4] : src.nnz;
   fixed.k = h[2];
   const double obj_new = cur.lp.obj_constant + p.obj_constant_delta;
   if (cur.owns && !p.has_new_A && m_new == m && n_new == n) {
@@ -505,23 +511,11 @@ void apply_plan(WorkLp& cur, const PresolvePlanGpu& p, RecordState& rs, const De
     return;
   }
   LPInfoGpu next;
-  if (at_early) {
-    std::tie(next.A, next.AT) = amd::compact_finish_pair(pair_start, m_new, n_new, a_nnz);
-  } else {
-    next.A = early ? amd::compact_finish(a_start, m_new, n_new, a_nnz)
-                   : amd::compact_csr(src, row_map, col_map, m_new, n_new, -1, col_rank.get());
-    // An AT with sorted rows that is the exact transpose of the A being
-    // compacted (the working AT, the caller's AT when sorted, the rebuilding
-    // rule's AT of a new A) is compacted with the maps swapped, which gives
-    // the transpose of the compacted A; otherwise the compacted A is
-    // re-transposed.
-    const DeviceCsrMatrix* at_src = p.has_new_A ? new_at : (cur.owns || callers_at_sorted ? &cur.lp.AT : nullptr);
-    if (at_src != nullptr) {
-      next.AT = amd::compact_csr(*at_src, col_map, row_map, n_new, m_new, next.A.nnz, row_rank.get());
-    } else {
-      next.AT = amd::transpose_csr(next.A);
-    }
+  if (!early) {
+    start = amd::compact_start(src, row_map, col_rank, a_chunk, counts + 4, nullptr, nullptr, nullptr, nullptr);
+    if (m_new != m || n_new != n) a_nnz = c.read_flags(5)[4];
   }
+  if (!at_early && at != nullptr) amd::compact_add_transpose(start, *at, col_map, row_rank, at_chunk);
   next.c = pool_f64(n_new, "working c");
   next.l = pool_f64(n_new, "working l");
   next.u = pool_f64(n_new, "working u");
@@ -533,11 +527,19 @@ void apply_plan(WorkLp& cur, const PresolvePlanGpu& p, RecordState& rs, const De
   DBuf<int32_t> row_r2o_next, col_r2o_next;
   if (m_new < m) row_r2o_next.alloc(m_new);
   if (n_new < n) col_r2o_next.alloc(n_new);
+  if (fixed.k > 0) {
+    fixed.idx.alloc(fixed.k);
+    fixed.val.alloc(fixed.k);
+  }
   const gpk_apply_gathers_args ga{m, n, col_map, p.new_c, p.new_l, p.new_u, rs.col_r2o,
                                   next.c, next.l, next.u, n_new < n ? col_r2o_next.get() : nullptr,
                                   row_map, p.new_AL, p.new_AU, rs.row_r2o,
-                                  next.AL, next.AU, m_new < m ? row_r2o_next.get() : nullptr};
-  check(gpk_apply_gathers(ga, s), "gather vectors");
+                                  next.AL, next.AU, m_new < m ? row_r2o_next.get() : nullptr,
+                                  fixed.k > 0 ? fixed.mask.get() : nullptr, fixed.tiles, fixed.idx, fixed.val};
+  const amd::CompactOut out = amd::compact_finish(start, m_new, n_new, a_nnz, &ga);
+  next.A = out.A;
+  next.AT = at != nullptr ? out.AT : amd::transpose_csr(next.A);
+  if (!out.gathered) check(gpk_apply_gathers(ga, s), "gather vectors");
   update_record(rs, p, m, n, row_map, col_map, m_new, n_new, fixed, m_new < m ? &row_r2o_next : nullptr,
                 n_new < n ? &col_r2o_next : nullptr);
   next.obj_constant = obj_new;

@@ -313,12 +313,6 @@ __global__ void k_csr_stats(const int32_t* ptr, const int32_t* idx, const double
 }
 
 // ---------------------------------------------------------- compaction ----
-// A tile's entry segment is processed in chunks of kCompChunk entries,
-// striped: entry c + 256k + t goes to thread t, so every load instruction of
-// a wave reads 64 consecutive entries.
-constexpr int kCompItems = 8;
-constexpr int kCompChunk = kBlock * kCompItems;
-
 __device__ inline int find_row(const int32_t* s_ptr, int rows, int32_t p) {
   int lo = 0, hi = rows;  // s_ptr[lo] <= p < s_ptr[hi]
   while (hi - lo > 1) {
@@ -411,13 +405,10 @@ __device__ inline int32_t lb_ticket(const gpk_lookback& lb) {
   return s_tile;
 }
 
-// Exclusive scan, 2048 items per tile (8 consecutive per thread).  mode 0:
-// out = prefix (out[n] = total); mode 1 (mask input): out = prefix or -1 for
-// unset entries, *count = total.
-template <class In, int kMode>
-__global__ __launch_bounds__(kBlock) void k_scan_lb(const In* in, int32_t* out, int64_t n, int32_t* count,
-                                                    gpk_lookback lb) {
-  constexpr int kWaves = kBlock / 64;
+// Exclusive scan, 2048 items per tile (8 consecutive per thread); out[n] =
+// total.
+template <class In>
+__global__ __launch_bounds__(kBlock) void k_scan_lb(const In* in, int32_t* out, int64_t n, gpk_lookback lb) {
   __shared__ int32_t s_wbase[kScanItems * kWaves];
   __shared__ int32_t s_excl;
   const int32_t tile = lb_ticket(lb);
@@ -451,10 +442,7 @@ __global__ __launch_bounds__(kBlock) void k_scan_lb(const In* in, int32_t* out, 
     const int32_t e = lb_exclusive(lb, tile, total);
     if (tid == 0) s_excl = e;
     const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-    if (tid == 0 && tile == tiles - 1) {
-      if (kMode == 1) *count = e + total;
-      else out[n] = e + total;
-    }
+    if (tid == 0 && tile == tiles - 1) out[n] = e + total;
   }
   __syncthreads();
   const int32_t excl = s_excl;
@@ -462,90 +450,219 @@ __global__ __launch_bounds__(kBlock) void k_scan_lb(const In* in, int32_t* out, 
   for (int k = 0; k < kScanItems; ++k) {
     const int64_t i = base + k * kBlock;
     const int32_t prefix = excl + s_wbase[k * kWaves + wave] + inc[k] - v[k];
-    if (i < n) out[i] = kMode == 1 ? (v[k] ? prefix : -1) : prefix;
+    if (i < n) out[i] = prefix;
   }
 }
 
-// The three keep maps of one plan application in one launch
-// (build_old_to_new for rows and columns, gpu_presolve.cu:878-934, and the
-// map of removed columns with a fixed interval): three look-back chains in
-// one status array, ticket order rows, then columns, then fixed columns.
-// The fixed-column mask is computed from keep_col, l and u on the way and
-// stored (removed, both bounds finite, |u - l| <= 1e-9).
-__global__ __launch_bounds__(kBlock) void k_apply_maps(gpk_apply_maps_args a, int32_t row_tiles, int32_t col_tiles,
+// Bit b of the result: byte b of the word is not zero.
+__device__ inline uint32_t nonzero_bytes(uint64_t x) {
+  constexpr uint64_t k7f = 0x7f7f7f7f7f7f7f7full;
+  const uint64_t hi = (((x & k7f) + k7f) | x) & ~k7f;  // bit 7 of every byte that is set
+  return static_cast<uint32_t>(((hi >> 7) * 0x0102040810204080ull) >> 56);
+}
+
+// Eight mask entries from i on as bits (none past n); mask + i is 8-byte
+// aligned when `aligned`.
+__device__ inline uint32_t mask_bits8(const uint8_t* __restrict__ mask, int64_t i, int64_t n, bool aligned) {
+  if (aligned && i + 8 <= n) return nonzero_bytes(*reinterpret_cast<const uint64_t*>(mask + i));
+  uint32_t b = 0;
+#pragma unroll 1
+  for (int k = 0; k < 8 && i + k < n; ++k) b |= (mask[i + k] != 0 ? 1u : 0u) << k;
+  return b;
+}
+
+// Set entries of mask[0, n), n a multiple of 16 and mask 16-byte aligned,
+// counted by the thread's share of the block; four loads on their way at a
+// time.
+__device__ inline int32_t mask_count_share(const uint8_t* __restrict__ mask, int64_t n) {
+  constexpr int U = 4;
+  const ulonglong2* w = reinterpret_cast<const ulonglong2*>(mask);
+  const int64_t words = n / 16;
+  int32_t c = 0;
+#pragma unroll 1
+  for (int64_t i = threadIdx.x; i < words; i += U * kBlock) {
+    ulonglong2 v[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) v[k] = i + k * kBlock < words ? w[i + k * kBlock] : make_ulonglong2(0, 0);
+#pragma unroll
+    for (int k = 0; k < U; ++k) c += __popc(nonzero_bytes(v[k].x)) + __popc(nonzero_bytes(v[k].y));
+  }
+  return c;
+}
+
+// The two keep maps of one plan application in one launch (build_old_to_new
+// for rows and columns, gpu_presolve.cu:878-934): chains of 2048-item tiles,
+// rows, then columns, eight consecutive items a thread (one 8-byte load of the
+// mask, two 16-byte stores of the map; these kernels are bound by their chain
+// of loads and by fetching their code, so both are kept short).  With l, the
+// column tiles also mark the removed columns with a fixed interval, store how
+// many each tile has and add them up.  A tile's offset comes from (kMode)
+//   kMapRecount  the tile counting the chain's mask up to itself: one byte an
+//                item, so at 262,144 items (GPK_MAP_RECOUNT_MAX) the last tile
+//                reads 64 16-byte words a thread.  No tile waits for another,
+//                as in look-back, whose status words cross the XCDs through
+//                memory: 10.3 us on average over the applications of the 1M x
+//                1.5M presolve, 13.5 before (8.7 at 12,000 x 23,000);
+//   kMapCounts   the counts that k_apply_counts left, summed by the tile
+//                (up to GPK_MAP_COUNT_TILES of them), 17.4 us for both launches
+//                at 1M x 1.5M against 57 with look-back; at 200,000 items both
+//                routes take 13 us;
+//   kMapLookback decoupled look-back, for more tiles than that.
+// The row pointers of the matrices to compact are walked on the way: entry
+// q << chunk_shift of A lies in row a_chunk[q] (and of AT in row at_chunk[q]).
+enum { kMapLookback = 0, kMapRecount = 1, kMapCounts = 2 };
+
+__global__ __launch_bounds__(kBlock) void k_apply_counts(gpk_apply_maps_args a, int32_t row_tiles, int32_t aligned) {
+  const int32_t tile = static_cast<int32_t>(blockIdx.x);
+  const bool rows = tile < row_tiles;
+  const int64_t i0 = static_cast<int64_t>(rows ? tile : tile - row_tiles) * kScanTile + 8 * threadIdx.x;
+  int32_t total;
+  (void)block_exclusive_sum(__popc(mask_bits8(rows ? a.keep_row : a.keep_col, i0, rows ? a.m : a.n, aligned != 0)),
+                            &total);
+  if (threadIdx.x == 0) a.tile_counts[tile] = total;
+}
+
+template <int kMode>
+__global__ __launch_bounds__(kBlock) void k_apply_maps(gpk_apply_maps_args a, int32_t row_tiles, int32_t aligned,
                                                        gpk_lookback lb) {
-  constexpr int kWaves = kBlock / 64;
-  __shared__ int32_t s_wbase[kScanItems * kWaves];
   __shared__ int32_t s_excl;
-  const int32_t tile = lb_ticket(lb);
-  if (tile >= static_cast<int32_t>(gridDim.x)) {  // the ticket word was not zeroed
-    if (threadIdx.x == 0) __hip_atomic_store(lb.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    return;
+  __shared__ __align__(8) uint8_t s_bits[kBlock];
+  __shared__ int32_t s_first[kBlock / 8];
+  int32_t tile = static_cast<int32_t>(blockIdx.x);
+  if constexpr (kMode == kMapLookback) {
+    tile = lb_ticket(lb);
+    if (tile >= static_cast<int32_t>(gridDim.x)) {  // the ticket word was not zeroed
+      if (threadIdx.x == 0) __hip_atomic_store(lb.error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      return;
+    }
   }
-  const int chain = tile < row_tiles ? 0 : (tile < row_tiles + col_tiles ? 1 : 2);
-  const int32_t first = chain == 0 ? 0 : (chain == 1 ? row_tiles : row_tiles + col_tiles);
-  const int64_t n = chain == 0 ? a.m : a.n;
-  int32_t* out = chain == 0 ? a.row_map : (chain == 1 ? a.col_map : a.fixed_map);
-  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
-  const int64_t base = static_cast<int64_t>(tile - first) * kScanTile + tid;
-  int32_t v[kScanItems], inc[kScanItems];
+  const bool rows = tile < row_tiles;
+  const int32_t first = rows ? 0 : row_tiles, last = rows ? row_tiles - 1 : static_cast<int32_t>(gridDim.x) - 1;
+  const int64_t n = rows ? a.m : a.n;
+  const uint8_t* mask = rows ? a.keep_row : a.keep_col;
+  const int32_t* ptr = rows ? a.a_ptr : a.at_ptr;
+  const int tid = threadIdx.x;
+  const int64_t base = static_cast<int64_t>(tile - first) * kScanTile, i0 = base + 8 * tid;
+  const int64_t i1 = i0 + 8 < n ? i0 + 8 : n;
+  const bool any = i0 < n;
+  const int32_t pb = ptr != nullptr && any ? ptr[i0] : 0, pe = ptr != nullptr && any ? ptr[i1] : 0;
+  const uint32_t bits = mask_bits8(mask, i0, n, aligned != 0);
+  int32_t share = 0;  // of the set entries before the tile
+  if constexpr (kMode == kMapRecount) {
+    share = mask_count_share(mask, base);
+  } else if constexpr (kMode == kMapCounts) {
+#pragma unroll 1
+    for (int32_t t = first + tid; t < tile; t += kBlock) share += a.tile_counts[t];
+  }
+  int32_t total, excl = 0;
+  const int32_t before = block_exclusive_sum(__popc(bits), &total);  // in the tile
+  if constexpr (kMode == kMapLookback) {
+    if (tid < 64) {
+      const int32_t e = lb_exclusive(lb, tile, total, first);
+      if (tid == 0) s_excl = e;
+    }
+    __syncthreads();
+    excl = s_excl;
+  } else {
+    (void)block_exclusive_sum(share, &excl);
+  }
+  if (tid == 0 && tile == last) a.counts[rows ? 0 : 1] = excl + total;
+  if (ptr != nullptr) {
+    // Chunk starts among the thread's entries: each lies in the last row that
+    // begins at or before it.
+    int32_t* chunk_row = rows ? a.a_chunk : a.at_chunk;
+    const int shift = a.chunk_shift;
+    int64_t r = i0;
+#pragma unroll 1
+    for (int64_t q = (pb + (int64_t{1} << shift) - 1) >> shift; q << shift < pe; ++q) {
+#pragma unroll 1
+      while (r + 1 < i1 && ptr[r + 1] <= q << shift) ++r;
+      chunk_row[q] = static_cast<int32_t>(r);
+    }
+    if (tile == last && i1 == n && any)
+      chunk_row[(pe >> shift) + ((pe & ((1 << shift) - 1)) != 0 ? 1 : 0)] = static_cast<int32_t>(n) - 1;
+  }
+  if (!rows && a.l != nullptr) {
+    // Removed, both bounds finite and within 1e-9 of each other.
+    uint32_t fixed = 0;
+    if (bits != 255u && any) {
 #pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    const int64_t i = base + k * kBlock;
-    int32_t x = 0;
-    if (i < n) {
-      if (chain == 0) {
-        x = a.keep_row[i] != 0;
-      } else if (chain == 1) {
-        x = a.keep_col[i] != 0;
-      } else {
+      for (int k = 0; k < 8; ++k) {
+        const int64_t i = i0 + k < n ? i0 + k : n - 1;
         const double lo = a.l[i], hi = a.u[i];
-        x = (!a.keep_col[i] && isfinite(lo) && isfinite(hi) && fabs(lo - hi) <= 1.0e-9) ? 1 : 0;
-        a.fixed_mask[i] = static_cast<uint8_t>(x);
+        fixed |= (isfinite(lo) && isfinite(hi) && fabs(lo - hi) <= 1.0e-9 ? 1u : 0u) << k;
       }
+      fixed &= ~bits & (i1 - i0 == 8 ? 255u : (1u << (i1 - i0)) - 1u);
     }
-    v[k] = x;
-  }
+    if (i1 - i0 == 8) {  // the mask is the library's own (aligned)
+      uint64_t bytes = 0;
 #pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    inc[k] = wave_inclusive_sum(v[k]);
-    if (lane == 63) s_wbase[k * kWaves + wave] = inc[k];
-  }
-  __syncthreads();
-  if (tid < 64) {
-    const int32_t c = tid < kScanItems * kWaves ? s_wbase[tid] : 0;
-    const int32_t ci = wave_inclusive_sum(c);
-    if (tid < kScanItems * kWaves) s_wbase[tid] = ci - c;
-    const int32_t total = __shfl(ci, 63, 64);
-    const int32_t e = lb_exclusive(lb, tile, total, first);
-    if (tid == 0) s_excl = e;
-    const int32_t last = chain == 0 ? row_tiles - 1 : (chain == 1 ? row_tiles + col_tiles - 1 : gridDim.x - 1);
-    if (tid == 0 && tile == last) a.counts[chain] = e + total;
-  }
-  __syncthreads();
-  const int32_t excl = s_excl;
-  gpk_rank_word* rank = chain == 0 ? a.row_rank : (chain == 1 ? a.col_rank : nullptr);
-#pragma unroll
-  for (int k = 0; k < kScanItems; ++k) {
-    const int64_t i = base + k * kBlock;
-    const int32_t prefix = excl + s_wbase[k * kWaves + wave] + inc[k] - v[k];
-    if (i < n) out[i] = v[k] ? prefix : -1;
-    if (rank) {
-      // A wave's 64 items of slice k are 64 consecutive, 64-aligned entries:
-      // one rank word (kept bits and the new index of the first kept one).
-      const uint64_t bits = __ballot(v[k] != 0);
-      const int lead = bits ? __ffsll(static_cast<unsigned long long>(bits)) - 1 : 0;
-      const int32_t first_new = __shfl(prefix, lead, 64);
-      const int64_t i0 = i - lane;
-      if (lane == 0 && i0 < n) {
-        gpk_rank_word w;
-        w.bits = bits;
-        w.base = bits ? first_new : 0;
-        w.pad = 0;
-        rank[i0 >> 6] = w;
-      }
+      for (int k = 0; k < 8; ++k) bytes |= static_cast<uint64_t>((fixed >> k) & 1u) << (8 * k);
+      *reinterpret_cast<uint64_t*>(a.fixed_mask + i0) = bytes;
+    } else {
+#pragma unroll 1
+      for (int64_t i = i0; i < i1; ++i) a.fixed_mask[i] = (fixed >> (i - i0)) & 1u;
+    }
+    int32_t c;
+    (void)block_exclusive_sum(__popc(fixed), &c);
+    if (tid == 0) {
+      a.fixed_tiles[tile - first] = c;
+      if (c != 0) atomicAdd(&a.counts[2], c);
     }
   }
+  int32_t* out = rows ? a.row_map : a.col_map;
+  int32_t v[8], run = excl + before;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    v[k] = (bits >> k) & 1u ? run : -1;
+    run += (bits >> k) & 1u;
+  }
+  if (i1 - i0 == 8) {  // the maps are the library's own (16-byte aligned)
+    reinterpret_cast<int4*>(out + i0)[0] = make_int4(v[0], v[1], v[2], v[3]);
+    reinterpret_cast<int4*>(out + i0)[1] = make_int4(v[4], v[5], v[6], v[7]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < 8; ++k)
+      if (i0 + k < n) out[i0 + k] = v[k];
+  }
+  gpk_rank_word* rank = rows ? a.row_rank : a.col_rank;
+  if (rank == nullptr) return;
+  // Eight threads make a rank word: kept bits and the new index of the first
+  // kept one.
+  s_bits[tid] = static_cast<uint8_t>(bits);
+  if ((tid & 7) == 0) s_first[tid >> 3] = excl + before;
+  __syncthreads();
+  if (tid < kBlock / 8 && base + 64 * tid < n) {
+    const uint64_t b = reinterpret_cast<const uint64_t*>(s_bits)[tid];
+    gpk_rank_word w;
+    w.bits = b;
+    w.base = b ? s_first[tid] : 0;
+    w.pad = 0;
+    rank[(base >> 6) + tid] = w;
+  }
+}
+
+// Exclusive scan (out[n] = total) of a 16-byte aligned mask of up to
+// GPK_MAP_RECOUNT_MAX entries, a tile's offset as in k_apply_maps with
+// kMapRecount: 5.1 us at 23,000 entries against 9.9 with look-back, and 4.4 at
+// 12,000 against 9.4 in one workgroup.  `out` holds n + 1 entries and may
+// start anywhere.
+__global__ __launch_bounds__(kBlock) void k_mask_scan(const uint8_t* __restrict__ mask, int32_t* __restrict__ out,
+                                                      int32_t n) {
+  const int tid = threadIdx.x;
+  const int32_t base = static_cast<int32_t>(blockIdx.x) * kScanTile, i0 = base + 8 * tid;
+  const uint32_t bits = mask_bits8(mask, i0, n, true);
+  const int32_t share = mask_count_share(mask, base);
+  int32_t total, excl;
+  int32_t run = block_exclusive_sum(__popc(bits), &total);
+  (void)block_exclusive_sum(share, &excl);
+  run += excl;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    if (i0 + k < n) out[i0 + k] = run;
+    run += (bits >> k) & 1u;
+  }
+  if (blockIdx.x == gridDim.x - 1 && tid == 0) out[n] = excl + total;
 }
 
 // Small scans in one workgroup (no tickets, no look-back): 1024 threads walk
@@ -554,8 +671,8 @@ __global__ __launch_bounds__(kBlock) void k_apply_maps(gpk_apply_maps_args a, in
 constexpr int kSmallBlock = 1024;
 constexpr int64_t kSmallScanMax = 16384;
 
-template <class In, int kMode>
-__global__ __launch_bounds__(kSmallBlock) void k_scan_small(const In* in, int32_t* out, int64_t n, int32_t* count) {
+template <class In>
+__global__ __launch_bounds__(kSmallBlock) void k_scan_small(const In* in, int32_t* out, int64_t n) {
   constexpr int kWaves = kSmallBlock / 64;
   constexpr int kSlots = kScanItems * kWaves;  // 128
   __shared__ int32_t s_w[kSlots];
@@ -587,48 +704,35 @@ __global__ __launch_bounds__(kSmallBlock) void k_scan_small(const In* in, int32_
     for (int k = 0; k < kScanItems; ++k) {
       const int64_t i = c + k * kSmallBlock + tid;
       const int32_t prefix = carry + s_w[k * kWaves + wave] + inc[k] - v[k];
-      if (i < n) out[i] = kMode == 1 ? (v[k] ? prefix : -1) : prefix;
+      if (i < n) out[i] = prefix;
     }
     carry += s_total;
     __syncthreads();  // s_w and s_total are rewritten by the next chunk
   }
-  if (tid == 0) {
-    if (kMode == 1) *count = carry;
-    else out[n] = carry;
-  }
+  if (tid == 0) out[n] = carry;
 }
 
-// Compaction (gpu_presolve.cu:1881-1978): after the column map's rank
-// words, three launches over tiles of 256 old rows: k_compact_map maps
-// every entry once (row kept and column rank,
-// one cache-resident rank gather per entry; with no rank words, when no
-// column is dropped, the column keeps its index), stores the new column index or
-// -1 per entry, each kept row's kept count at out_ptr[new row] and the
-// tile's kept count; an exclusive scan of the tile counts (one small array,
-// m/256 entries) gives every tile its output offset; k_compact_write turns
-// its rows' counts into row pointers (a block scan plus the tile offset),
-// then streams the mapped indices and the values and writes the kept
-// entries, positioned by wave ballots and staged in LDS for coalesced stores.
-constexpr int kCompRows = kBlock;
-
-// Rank form of a keep map (map[j] = new index or -1), one 16-byte word per 64
-// entries: bit b of word w is set when entry 64w + b is kept, and base is the
-// new index of the word's first kept entry.  A lookup then reads one small,
-// cache-resident word instead of gathering from the n-entry map.
-__global__ void k_build_rank(const int32_t* __restrict__ map, int32_t n, gpk_rank_word* __restrict__ out) {
-  const int32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  const int32_t v = j < n ? map[j] : -1;
-  const uint64_t bits = __ballot(v >= 0);
-  const int first = bits ? __ffsll(static_cast<unsigned long long>(bits)) - 1 : 0;
-  const int32_t base = __shfl(v, first, 64);
-  if (lane_id() == 0 && (j >> 6) <= ((n - 1) >> 6)) {
-    gpk_rank_word w;
-    w.bits = bits;
-    w.base = bits ? base : 0;
-    w.pad = 0;
-    out[j >> 6] = w;
-  }
-}
+// Compaction (gpu_presolve.cu:1881-1978) over chunks of entries, whatever the
+// rows: a tile of 256 rows gives a block-structured LP's 200 linking rows of
+// 3,000 entries to one block (1.58 ms a map pass, 0.59 ms a write pass on
+// 80,200 x 120,000; 14.5 and 15.4 us by chunks), and the popular columns of AT
+// to few (121 us the map pass of the pair on 1M x 1.5M; 67 by chunks).
+//   k_compact_map    maps every entry once (row kept and column rank, one
+//     cache-resident rank gather per entry; with no rank words, when no column
+//     is dropped, the column keeps its index), stores the new column index or
+//     -1 per entry, the chunk's kept entries as words of bits with their
+//     prefix sums, and its kept count;
+//   k_compact_write  moves the chunk's kept entries to their places (chunk
+//     offset, word prefix, bits below), staged in LDS for coalesced stores;
+//     further blocks turn every kept row's first entry into its row pointer
+//     through the same words, and gather the LP's vectors on the way.
+// A chunk's offset is the sum of the counts before it: added up by each block
+// from the raw counts (up to GPK_COMPACT_COUNT_CHUNKS a side), or scanned by a
+// launch in between.
+// kI entries a thread: 8 (chunks of 2048) on large matrices, 2 (chunks of 512)
+// up to GPK_COMPACT_SMALL_NNZ entries, where the chip is far from full and a
+// block's own chain of loads is what counts (26,000 entries: 4.2 us a map pass
+// against 8.7 with 2048).
 
 // One 16-byte load of the word, then the rank; -1 when entry j is dropped.
 __device__ inline uint4 rank_word(const gpk_rank_word* __restrict__ rank, int32_t j) {
@@ -641,246 +745,290 @@ __device__ inline int32_t rank_of(uint4 w, int32_t j) {
   return (bits & bit) ? r : -1;
 }
 
-// Per-row kept counts of one striped item per lane: the lanes of a wave that
-// hold entries of the same row are consecutive, so the first lane of each
-// run adds the run's kept count with one LDS atomic.
-__device__ inline void comp_count_run(int row, bool valid, bool kept, int32_t* s_cnt) {
-  const int lane = lane_id();
-  const uint64_t kb = __ballot(kept);
-  const int prev = __shfl_up(row, 1, 64);
-  const bool head = valid && (lane == 0 || prev != row);
-  const uint64_t hb = __ballot(head);
-  if (!head) return;
-  const uint64_t after = lane == 63 ? 0ull : (hb & (~0ull << (lane + 1)));
-  const int next = after ? __ffsll(static_cast<unsigned long long>(after)) - 1 : 64;
-  const uint64_t run = (next == 64 ? ~0ull : ((1ull << next) - 1)) & ~lanemask_lt(lane);
-  const int c = static_cast<int>(__popcll(kb & run));
-  if (c) atomicAdd(&s_cnt[row], c);
-}
-
-// The map pass of one 256-row tile (tile_cnt[tile]: its kept count).
-__device__ __forceinline__ void compact_map_tile(int32_t tile, const int32_t* __restrict__ ptr,
-                                                 const int32_t* __restrict__ idx, int32_t m_old,
-                                                 const int32_t* __restrict__ row_map,
-                                                 const gpk_rank_word* __restrict__ col_rank,
-                                                 int32_t* __restrict__ jn_out, int32_t* __restrict__ out_ptr,
-                                                 int32_t* __restrict__ tile_cnt, int32_t* __restrict__ kept_total) {
-  __shared__ int32_t s_cnt[kCompRows];
-  __shared__ int32_t s_wsum[kBlock / 64];
-  __shared__ uint8_t s_keep[kCompRows];
-  __shared__ uint8_t s_row[kCompChunk];  // tile-local row of each entry of the chunk
-  static_assert(kCompRows <= 256, "tile-local rows are stored in one byte");
-  const int32_t r0 = tile * kCompRows;
-  const int rows = min(kCompRows, m_old - r0);
-  const int tid = threadIdx.x;
-  const int32_t my_new_row = tid < rows ? row_map[r0 + tid] : -1;
-  const int32_t my_b = tid < rows ? ptr[r0 + tid] : 0;
-  const int32_t my_e = tid < rows ? ptr[r0 + tid + 1] : 0;
-  s_cnt[tid] = 0;
-  s_keep[tid] = my_new_row >= 0 ? 1 : 0;
-  const int32_t seg_b = ptr[r0], seg_e = ptr[r0 + rows];
-  for (int32_t c = seg_b; c < seg_e; c += kCompChunk) {
-    // Each thread labels its row's entries of the chunk; then rows and
-    // liveness come from LDS, and every load goes out at once (a register a
-    // load is still writing is never assigned).
-    for (int32_t q = max(my_b, c); q < min(my_e, c + kCompChunk); ++q) s_row[q - c] = static_cast<uint8_t>(tid);
-    __syncthreads();
-    int rr[kCompItems];
-    bool live[kCompItems];
-#pragma unroll
-    for (int k = 0; k < kCompItems; ++k) {
-      const int32_t p = c + k * kBlock + tid;
-      rr[k] = p < seg_e ? static_cast<int>(s_row[p - c]) : -1;
-      live[k] = rr[k] >= 0 && s_keep[rr[k]] != 0;
-    }
-    int32_t cj[kCompItems];
-#pragma unroll
-    for (int k = 0; k < kCompItems; ++k) cj[k] = idx[min(c + k * kBlock + tid, seg_e - 1)];
-    uint4 w[kCompItems];
-    if (col_rank != nullptr) {
-#pragma unroll
-      for (int k = 0; k < kCompItems; ++k) w[k] = rank_word(col_rank, live[k] ? cj[k] : 0);
-    }
-#pragma unroll
-    for (int k = 0; k < kCompItems; ++k) {
-      const int32_t p = c + k * kBlock + tid;
-      const int32_t jn = !live[k] ? -1 : col_rank != nullptr ? rank_of(w[k], cj[k]) : cj[k];
-      if (p < seg_e) jn_out[p] = jn;
-      comp_count_run(rr[k], rr[k] >= 0, jn >= 0, s_cnt);
-    }
-    __syncthreads();  // s_row is relabelled for the next chunk
-  }
-  const int32_t mine = my_new_row >= 0 ? s_cnt[tid] : 0;
-  if (my_new_row >= 0) out_ptr[my_new_row] = mine;
-  const int32_t inc = wave_inclusive_sum(mine);
-  if (lane_id() == 63) s_wsum[tid >> 6] = inc;
-  __syncthreads();
-  if (tid == 0) {
-    int32_t t = 0;
-    for (int w = 0; w < kBlock / 64; ++w) t += s_wsum[w];
-    tile_cnt[tile] = t;
-    if (kept_total != nullptr && t != 0) atomicAdd(kept_total, t);  // integer: order-free
+// Sets bits [b, e) of an LDS bitmap.
+__device__ inline void set_bits(uint32_t* words, int b, int e) {
+  for (int w = b >> 5; w <= (e - 1) >> 5; ++w) {
+    const int lo = max(b - 32 * w, 0), hi = min(e - 32 * w, 32);
+    atomicOr(&words[w], (hi == 32 ? ~0u : (1u << hi) - 1u) & ~((1u << lo) - 1u));
   }
 }
 
-__global__ __launch_bounds__(kBlock) void k_compact_map(const int32_t* __restrict__ ptr,
-                                                        const int32_t* __restrict__ idx, int32_t m_old,
-                                                        const int32_t* __restrict__ row_map,
-                                                        const gpk_rank_word* __restrict__ col_rank,
-                                                        int32_t* __restrict__ jn_out, int32_t* __restrict__ out_ptr,
-                                                        int32_t* __restrict__ tile_cnt,
-                                                        int32_t* __restrict__ kept_total) {
-  compact_map_tile(static_cast<int32_t>(blockIdx.x), ptr, idx, m_old, row_map, col_rank, jn_out, out_ptr, tile_cnt,
-                   kept_total);
-}
+// Rows of a chunk (its entries' rows and the empty ones between) up to which
+// the block marks kept rows in the bitmap; past that every entry looks its row
+// up by bisection, so a chunk that spans a million empty rows costs 20 loads
+// an entry instead of 4,000 a thread.
+constexpr int kCompMarkRows = 8192;
 
-// A and its transpose compacted with the same maps in one launch: blocks
-// [0, tiles_a) map A's tiles, the rest AT's; the tile counts go to one array
-// (A's, then AT's), so one scan serves both.
-__global__ __launch_bounds__(kBlock) void k_compact_map_pair(gpk_compact_side a, gpk_compact_side t,
-                                                             int32_t tiles_a, int32_t* __restrict__ tile_cnt,
-                                                             int32_t* __restrict__ kept_total) {
-  const int32_t b = static_cast<int32_t>(blockIdx.x);
-  if (b < tiles_a)
-    compact_map_tile(b, a.ptr, a.idx, a.m_old, a.row_map, a.col_rank, a.jn, a.out_ptr, tile_cnt, kept_total);
-  else
-    compact_map_tile(b - tiles_a, t.ptr, t.idx, t.m_old, t.row_map, t.col_rank, t.jn, t.out_ptr,
-                     tile_cnt + tiles_a, nullptr);
-}
-
-// The write pass of tile `tile` of `ntiles`.  seg: the tiles' raw kept
-// counts (from_counts; ntiles <= kBlock) or an exclusive scan of them whose
-// first word is subtracted (a segment of a longer scan).
-__device__ __forceinline__ void compact_write_tile(int32_t tile, int32_t ntiles, bool from_counts,
-                                                   const int32_t* __restrict__ ptr, const double* __restrict__ val,
-                                                   int32_t m_old, const int32_t* __restrict__ row_map,
-                                                   const int32_t* __restrict__ jn_in,
-                                                   const int32_t* __restrict__ seg, int32_t* __restrict__ out_ptr,
-                                                   int32_t m_new, int32_t* __restrict__ out_idx,
-                                                   double* __restrict__ out_val) {
-  constexpr int kWaves = kBlock / 64;
-  __shared__ int32_t s_oidx[kCompChunk];
-  __shared__ double s_oval[kCompChunk];
-  __shared__ int32_t s_wcnt[kCompItems * kWaves];
-  __shared__ int32_t s_wsum[kWaves];
-  __shared__ int32_t s_total;
-  const int32_t r0 = tile * kCompRows;
-  const int rows = min(kCompRows, m_old - r0);
-  const int tid = threadIdx.x;
-  const int lane = lane_id(), wave = tid >> 6;
-  const int32_t my_new_row = tid < rows ? row_map[r0 + tid] : -1;
-  int32_t base;
-  if (from_counts) {
-    // Few tiles (ntiles <= kBlock): seg holds the raw per-tile kept counts
-    // and each block sums those of the tiles before it (and the last block
-    // all of them) instead of waiting for a scan launch.
-    const int32_t t = tid < ntiles ? seg[tid] : 0;
-    const int32_t before = wave_inclusive_sum(tid < tile ? t : 0);
-    const int32_t all = wave_inclusive_sum(t);
-    if (lane == 63) {
-      s_wsum[wave] = before;
-      s_wcnt[wave] = all;  // s_wcnt is free until the chunk loop
+template <int kI>
+__device__ __forceinline__ void compact_map_chunk(int32_t q, const gpk_compact_side& s, int32_t* __restrict__ chunk_cnt,
+                                                  int32_t* __restrict__ kept_total) {
+  constexpr int kChunk = kBlock * kI, kWords = kChunk / 64, kAhead = 2;
+  __shared__ uint32_t s_live[2 * kWords];
+  __shared__ uint64_t s_mask[kWords];
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+  const int32_t c0 = q * kChunk;
+  const int32_t c1 = min(s.nnz - c0, kChunk);  // entries of the chunk
+  const int32_t r_lo = s.chunk_row[q], r_hi = s.chunk_row[q + 1];
+  int32_t cj[kI];
+#pragma unroll
+  for (int k = 0; k < kI; ++k) cj[k] = s.idx[c0 + min(k * kBlock + tid, c1 - 1)];
+  if (tid < 2 * kWords) s_live[tid] = 0;
+  if (r_hi - r_lo < kCompMarkRows) {
+    // The first rows' pointers and fates are loaded together.
+    int32_t b[kAhead], e[kAhead], to[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int32_t r = min(r_lo + tid + k * kBlock, r_hi);
+      b[k] = s.ptr[r];
+      e[k] = s.ptr[r + 1];
+      to[k] = s.row_map[r];
     }
     __syncthreads();
-    int32_t b = 0, a = 0;
-    for (int w = 0; w < kWaves; ++w) {
-      b += s_wsum[w];
-      a += s_wcnt[w];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int lo = max(b[k] - c0, 0), hi = min(e[k] - c0, c1);
+      if (r_lo + tid + k * kBlock <= r_hi && lo < hi && to[k] >= 0) set_bits(s_live, lo, hi);
     }
-    base = b;
-    if (tile == ntiles - 1 && tid == 0) out_ptr[m_new] = a;
-    __syncthreads();  // s_wsum is reused below
+    for (int32_t r = r_lo + tid + kAhead * kBlock; r <= r_hi; r += kBlock) {
+      const int lo = max(s.ptr[r] - c0, 0), hi = min(s.ptr[r + 1] - c0, c1);
+      if (lo < hi && s.row_map[r] >= 0) set_bits(s_live, lo, hi);
+    }
   } else {
-    const int32_t s0 = seg[0];
-    base = seg[tile] - s0;
-    if (tile == ntiles - 1 && tid == 0) out_ptr[m_new] = seg[ntiles] - s0;
-  }
-  {  // row pointers of the tile's kept rows: tile offset + block exclusive scan of the counts
-    const int32_t cnt = my_new_row >= 0 ? out_ptr[my_new_row] : 0;
-    const int32_t inc = wave_inclusive_sum(cnt);
-    if (lane == 63) s_wsum[wave] = inc;
     __syncthreads();
-    int32_t before = 0, all = 0;
-    for (int w = 0; w < kWaves; ++w) {
-      before += w < wave ? s_wsum[w] : 0;
-      all += s_wsum[w];
-    }
-    if (my_new_row >= 0) out_ptr[my_new_row] = base + before + inc - cnt;
-    if (all == 0) return;  // no kept entry in the tile (the same in every thread)
-  }
-  const int32_t seg_b = ptr[r0], seg_e = ptr[r0 + rows];
-  const uint64_t below = lanemask_lt(lane);
-  for (int32_t c = seg_b; c < seg_e; c += kCompChunk) {
-    int32_t jn[kCompItems];
-    double v[kCompItems];
-#pragma unroll
-    for (int k = 0; k < kCompItems; ++k) {
-      const int32_t pc = min(c + k * kBlock + tid, seg_e - 1);
-      jn[k] = jn_in[pc];
-      v[k] = val[pc];
-    }
-    uint64_t ball[kCompItems];
-#pragma unroll
-    for (int k = 0; k < kCompItems; ++k) {
-      const bool keep = c + k * kBlock + tid < seg_e && jn[k] >= 0;
-      ball[k] = __ballot(keep);
-    }
-    if (lane == 0) {
-#pragma unroll
-      for (int k = 0; k < kCompItems; ++k) s_wcnt[k * kWaves + wave] = static_cast<int32_t>(__popcll(ball[k]));
-    }
-    __syncthreads();
-    if (tid < 64) {  // exclusive prefix over (slice, wave) in entry order
-      const int32_t cnt = tid < kCompItems * kWaves ? s_wcnt[tid] : 0;
-      const int32_t inc = wave_inclusive_sum(cnt);
-      if (tid < kCompItems * kWaves) s_wcnt[tid] = inc - cnt;
-      if (tid == 63) s_total = inc;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < kCompItems; ++k) {
-      if ((ball[k] >> lane) & 1ull) {
-        const int32_t pos = s_wcnt[k * kWaves + wave] + static_cast<int32_t>(__popcll(ball[k] & below));
-        s_oidx[pos] = jn[k];
-        s_oval[pos] = v[k];
+    for (int k = 0; k < kI; ++k) {
+      const int32_t p = k * kBlock + tid;
+      if (p >= c1) break;
+      int32_t lo = r_lo, hi = r_hi + 1;  // ptr[lo] <= c0 + p < ptr[hi]
+      while (hi - lo > 1) {
+        const int32_t mid = lo + (hi - lo) / 2;
+        if (s.ptr[mid] <= c0 + p) lo = mid; else hi = mid;
       }
+      if (s.row_map[lo] >= 0) atomicOr(&s_live[p >> 5], 1u << (p & 31));
     }
-    __syncthreads();
-    const int32_t total = s_total;
-    for (int t = tid; t < total; t += kBlock) {
-      out_idx[base + t] = s_oidx[t];
-      out_val[base + t] = s_oval[t];
+  }
+  __syncthreads();
+  // Slice k of a wave is word k * kWaves + wave of the chunk.
+  bool live[kI];
+  uint4 w[kI];
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    const int p = k * kBlock + tid;
+    live[k] = (s_live[p >> 5] >> (p & 31)) & 1u;
+  }
+  if (s.col_rank != nullptr) {
+#pragma unroll
+    for (int k = 0; k < kI; ++k) w[k] = rank_word(s.col_rank, live[k] ? cj[k] : 0);
+  }
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    const int p = k * kBlock + tid;
+    const int32_t jn = !live[k] ? -1 : s.col_rank != nullptr ? rank_of(w[k], cj[k]) : cj[k];
+    if (p < c1) s.jn[c0 + p] = jn;
+    const uint64_t kept = __ballot(jn >= 0);  // entries past the chunk are not live
+    if (lane == 0) s_mask[k * kWaves + wave] = kept;
+  }
+  __syncthreads();
+  if (tid < 64) {
+    const uint64_t bits = tid < kWords ? s_mask[tid] : 0ull;
+    const int32_t c = static_cast<int32_t>(__popcll(bits));
+    const int32_t inc = wave_inclusive_sum(c);
+    if (tid < kWords) {
+      s.mask[static_cast<int64_t>(q) * kWords + tid] = bits;
+      s.word_pre[static_cast<int64_t>(q) * kWords + tid] = inc - c;
     }
-    base += total;
-    __syncthreads();
+    if (tid == 63) {
+      chunk_cnt[q] = inc;
+      if (kept_total != nullptr && inc != 0) atomicAdd(kept_total, inc);  // integer: order-free
+    }
   }
 }
 
-template <bool kOffsetsFromCounts>
-__global__ __launch_bounds__(kBlock) void k_compact_write(const int32_t* __restrict__ ptr,
-                                                          const double* __restrict__ val, int32_t m_old,
-                                                          const int32_t* __restrict__ row_map,
-                                                          const int32_t* __restrict__ jn_in,
-                                                          const int32_t* __restrict__ tile_off,
-                                                          int32_t* __restrict__ out_ptr, int32_t m_new,
-                                                          int32_t* __restrict__ out_idx,
-                                                          double* __restrict__ out_val) {
-  compact_write_tile(static_cast<int32_t>(blockIdx.x), static_cast<int32_t>(gridDim.x), kOffsetsFromCounts, ptr, val,
-                     m_old, row_map, jn_in, tile_off, out_ptr, m_new, out_idx, out_val);
+// A's chunks, then those of its transpose, compacted with the same maps.
+template <int kI>
+__global__ __launch_bounds__(kBlock) void k_compact_map(gpk_compact_side a, gpk_compact_side t, int32_t chunks_a,
+                                                        int32_t* __restrict__ chunk_cnt,
+                                                        int32_t* __restrict__ kept_total) {
+  const int32_t b = static_cast<int32_t>(blockIdx.x);
+  if (b < chunks_a) compact_map_chunk<kI>(b, a, chunk_cnt, kept_total);
+  else compact_map_chunk<kI>(b - chunks_a, t, chunk_cnt + chunks_a, nullptr);
 }
 
-// Both write passes of a pair map (k_compact_map_pair) in one launch.
-__global__ __launch_bounds__(kBlock) void k_compact_write_pair(gpk_compact_side a, gpk_compact_side t,
-                                                               int32_t tiles_a, int32_t tiles_t,
-                                                               const int32_t* __restrict__ tile_off,
-                                                               int32_t from_counts) {
+// The vector gathers of one plan application: c, l, u, the column
+// reduced-to-original map and the record of a removed fixed column for column
+// i (fixed_at: its place among them, or -1); AL, AU and the row map for row i
+// (dst[map[i]] = src[i] for map[i] >= 0; a null destination is skipped).
+__device__ __forceinline__ void gather_col(const gpk_apply_gathers_args& a, int32_t i, int32_t j, int32_t fixed_at) {
+  if (j >= 0) {
+    a.c_out[j] = a.c_in[i];
+    a.l_out[j] = a.l_in[i];
+    a.u_out[j] = a.u_in[i];
+    if (a.col_r2o_out) a.col_r2o_out[j] = a.col_r2o_in[i];
+  } else if (fixed_at >= 0) {
+    a.fixed_idx[fixed_at] = a.col_r2o_in[i];
+    a.fixed_val[fixed_at] = 0.5 * (a.l_in[i] + a.u_in[i]);
+  }
+}
+__device__ __forceinline__ void gather_row(const gpk_apply_gathers_args& a, int32_t i, int32_t r) {
+  if (r < 0) return;
+  a.al_out[r] = a.al_in[i];
+  a.au_out[r] = a.au_in[i];
+  if (a.row_r2o_out) a.row_r2o_out[r] = a.row_r2o_in[i];
+}
+
+// The column's place among the removed fixed columns (-1: not one), for the
+// kBlock columns from block * kBlock on: the tiles' counts before its map
+// tile, the mask up to the block, then the block's own prefix.
+static_assert(kScanTile % kBlock == 0, "a block of columns lies in one map tile");
+__device__ __forceinline__ int32_t fixed_place(const gpk_apply_gathers_args& a, int32_t block) {
+  const int tid = threadIdx.x;
+  const int64_t at = static_cast<int64_t>(block) * kBlock;
+  const int32_t j0 = at < a.n ? static_cast<int32_t>(at) : a.n, tile = j0 / kScanTile;  // past the columns: none
+  const int32_t f = at + tid < a.n ? a.fixed_mask[at + tid] : 0;
+  int32_t c = 0, before, mine;
+#pragma unroll 1
+  for (int32_t t = tid; t < tile; t += kBlock) c += a.fixed_tiles[t];
+#pragma unroll 1
+  for (int32_t j = tile * kScanTile + tid; j < j0; j += kBlock) c += a.fixed_mask[j];
+  (void)block_exclusive_sum(c, &before);
+  const int32_t excl = block_exclusive_sum(f, &mine);
+  return f ? before + excl : -1;
+}
+
+__global__ __launch_bounds__(kBlock) void k_apply_gathers(gpk_apply_gathers_args a) {
   const int32_t b = static_cast<int32_t>(blockIdx.x);
-  if (b < tiles_a)
-    compact_write_tile(b, tiles_a, from_counts != 0, a.ptr, a.val, a.m_old, a.row_map, a.jn, tile_off, a.out_ptr,
-                       a.m_new, a.out_idx, a.out_val);
-  else
-    compact_write_tile(b - tiles_a, tiles_t, from_counts != 0, t.ptr, t.val, t.m_old, t.row_map, t.jn,
-                       tile_off + tiles_a, t.out_ptr, t.m_new, t.out_idx, t.out_val);
+  const int64_t i = static_cast<int64_t>(b) * kBlock + threadIdx.x;
+  const int32_t at = a.fixed_mask != nullptr ? fixed_place(a, b) : -1;
+  if (i < a.n) gather_col(a, static_cast<int32_t>(i), a.col_map[i], at);
+  if (i < a.m) gather_row(a, static_cast<int32_t>(i), a.row_map[i]);
+}
+
+// The kept entries of chunk q; off: the side's raw chunk counts (from_counts)
+// or their exclusive scan (whose first word is subtracted: a segment of a
+// longer scan).
+template <int kI>
+__device__ __forceinline__ void compact_write_chunk(int32_t q, bool from_counts, const gpk_compact_side& s,
+                                                    const int32_t* __restrict__ off, double* s_oval, int32_t* s_oidx) {
+  constexpr int kChunk = kBlock * kI, kWords = kChunk / 64;
+  const int tid = threadIdx.x, lane = lane_id(), wave = tid >> 6;
+  const int32_t c0 = q * kChunk;
+  const int32_t c1 = min(s.nnz - c0, kChunk);
+  const int64_t word0 = static_cast<int64_t>(q) * kWords + wave;
+  int32_t jn[kI], pre[kI];
+  uint64_t bits[kI];
+  double v[kI];
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    const int32_t p = c0 + min(k * kBlock + tid, c1 - 1);
+    jn[k] = s.jn[p];
+    v[k] = s.val[p];
+    bits[k] = s.mask[word0 + k * kWaves];
+    pre[k] = s.word_pre[word0 + k * kWaves];
+  }
+  int32_t base, total;
+  if (from_counts) {
+    int32_t c = 0;
+    total = off[q];
+    for (int32_t i = tid; i < q; i += kBlock) c += off[i];
+    (void)block_exclusive_sum(c, &base);
+  } else {
+    const int32_t first = off[0];
+    base = off[q] - first;
+    total = off[q + 1] - first - base;
+  }
+  if (total == 0) return;
+  const uint64_t below = lanemask_lt(lane);
+#pragma unroll
+  for (int k = 0; k < kI; ++k) {
+    if ((bits[k] >> lane) & 1ull) {
+      const int32_t pos = pre[k] + static_cast<int32_t>(__popcll(bits[k] & below));
+      s_oidx[pos] = jn[k];
+      s_oval[pos] = v[k];
+    }
+  }
+  __syncthreads();
+  for (int t = tid; t < total; t += kBlock) {
+    s.out_idx[base + t] = s_oidx[t];
+    s.out_val[base + t] = s_oval[t];
+  }
+}
+
+// The row pointers of kBlock old rows; returns the thread's new row (-1:
+// dropped or past the end).
+template <int kI>
+__device__ __forceinline__ int32_t compact_row(int32_t block, int32_t chunks, bool from_counts,
+                                               const gpk_compact_side& s, const int32_t* __restrict__ off,
+                                               int32_t* s_off) {
+  constexpr int kChunk = kBlock * kI;
+  const int tid = threadIdx.x;
+  const int64_t r = static_cast<int64_t>(block) * kBlock + tid;
+  const int32_t nr = r < s.m_old ? s.row_map[r] : -1;
+  const int32_t p = r < s.m_old ? s.ptr[r] : s.nnz;
+  int32_t local = 0;
+  if (p < s.nnz)
+    local = s.word_pre[p >> 6] + static_cast<int32_t>(__popcll(s.mask[p >> 6] & ((1ull << (p & 63)) - 1ull)));
+  int32_t first = 0;  // the word subtracted from an offset
+  if (from_counts) {
+    constexpr int kPer = GPK_COMPACT_COUNT_CHUNKS / kBlock;
+    int32_t c[kPer], sum = 0, all;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      c[k] = tid * kPer + k < chunks ? off[tid * kPer + k] : 0;
+      sum += c[k];
+    }
+    int32_t run = block_exclusive_sum(sum, &all);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      s_off[tid * kPer + k] = run;
+      run += c[k];
+    }
+    if (tid == 0) s_off[GPK_COMPACT_COUNT_CHUNKS] = all;
+    __syncthreads();
+  } else {
+    first = off[0];
+  }
+  auto offset = [&](int32_t q) {
+    return from_counts ? s_off[q < chunks ? q : GPK_COMPACT_COUNT_CHUNKS] : off[q] - first;
+  };
+  // empty rows at the end start at the kept count
+  if (nr >= 0) s.out_ptr[nr] = offset(p < s.nnz ? p / kChunk : chunks) + local;
+  if (block == 0 && tid == 0) s.out_ptr[s.m_new] = offset(chunks);
+  return nr;
+}
+
+// Blocks: A's chunks, AT's chunks, A's rows, AT's rows.
+template <int kI>
+__global__ __launch_bounds__(kBlock) void k_compact_write(gpk_compact_side a, gpk_compact_side t, int32_t chunks_a,
+                                                          int32_t chunks_t, int32_t row_blocks_a,
+                                                          const int32_t* __restrict__ off, int32_t from_counts,
+                                                          gpk_apply_gathers_args g) {
+  constexpr int kChunk = kBlock * kI;
+  constexpr int kLds = kChunk * 12 > (GPK_COMPACT_COUNT_CHUNKS + 1) * 4 ? kChunk * 12 : (GPK_COMPACT_COUNT_CHUNKS + 2) * 4;
+  __shared__ __align__(16) char s_buf[kLds];
+  double* s_oval = reinterpret_cast<double*>(s_buf);
+  int32_t* s_oidx = reinterpret_cast<int32_t*>(s_buf + sizeof(double) * kChunk);
+  int32_t* s_off = reinterpret_cast<int32_t*>(s_buf);
+  int32_t b = static_cast<int32_t>(blockIdx.x);
+  if (b < chunks_a) {
+    compact_write_chunk<kI>(b, from_counts != 0, a, off, s_oval, s_oidx);
+    return;
+  }
+  b -= chunks_a;
+  if (b < chunks_t) {
+    compact_write_chunk<kI>(b, from_counts != 0, t, off + chunks_a, s_oval, s_oidx);
+    return;
+  }
+  b -= chunks_t;
+  const bool rows = b < row_blocks_a;
+  if (!rows) b -= row_blocks_a;
+  const int32_t to = rows ? compact_row<kI>(b, chunks_a, from_counts != 0, a, off, s_off)
+                          : compact_row<kI>(b, chunks_t, from_counts != 0, t, off + chunks_a, s_off);
+  const int64_t i = static_cast<int64_t>(b) * kBlock + threadIdx.x;
+  if (rows) {
+    if (g.m > 0) gather_row(g, static_cast<int32_t>(i), to);
+  } else if (g.n > 0) {
+    const int32_t at = g.fixed_mask != nullptr ? fixed_place(g, b) : -1;
+    if (i < g.n) gather_col(g, static_cast<int32_t>(i), to, at);
+  }
 }
 
 __global__ void k_mail(const uint32_t* __restrict__ src, int32_t words, uint32_t* mail, uint32_t seq) {
@@ -913,45 +1061,6 @@ __global__ __launch_bounds__(kBlock) void k_copy_many(CopyList list) {
   else if ((a & 7u) == 0) copy_units<uint2>(g);
   else if ((a & 3u) == 0) copy_units<uint32_t>(g);
   else copy_units<uint8_t>(g);
-}
-
-// The vector gathers of one plan application in one launch: c, l, u and
-// the column reduced-to-original map through col_map; AL, AU and the row
-// map through row_map (dst[map[i]] = src[i] for map[i] >= 0; a null
-// destination is skipped).
-__global__ void k_apply_gathers(gpk_apply_gathers_args a) {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < a.n) {
-    const int32_t j = a.col_map[i];
-    if (j >= 0) {
-      a.c_out[j] = a.c_in[i];
-      a.l_out[j] = a.l_in[i];
-      a.u_out[j] = a.u_in[i];
-      if (a.col_r2o_out) a.col_r2o_out[j] = a.col_r2o_in[i];
-    }
-  }
-  if (i < a.m) {
-    const int32_t r = a.row_map[i];
-    if (r >= 0) {
-      a.al_out[r] = a.al_in[i];
-      a.au_out[r] = a.au_in[i];
-      if (a.row_r2o_out) a.row_r2o_out[r] = a.row_r2o_in[i];
-    }
-  }
-}
-
-__global__ void k_gather5(const int32_t* map, int32_t n_old, const double* s0, double* d0, const double* s1,
-                          double* d1, const double* s2, double* d2, const double* s3, double* d3,
-                          const double* s4, double* d4) {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n_old) return;
-  const int32_t t = map[i];
-  if (t < 0) return;
-  if (s0) d0[t] = s0[i];
-  if (s1) d1[t] = s1[i];
-  if (s2) d2[t] = s2[i];
-  if (s3) d3[t] = s3[i];
-  if (s4) d4[t] = s4[i];
 }
 
 __global__ void k_gather_i32(const int32_t* map, int32_t n_old, const int32_t* src, int32_t* dst) {
@@ -1311,7 +1420,7 @@ hipError_t scan_impl(const In* in, int32_t* out, int64_t n, int32_t* scratch, hi
     return hipMemsetAsync(out, 0, sizeof(int32_t), s);
   }
   if (n <= kSmallScanMax) {
-    hipLaunchKernelGGL((k_scan_small<In, 0>), dim3(1), dim3(kSmallBlock), 0, s, in, out, n, nullptr);
+    hipLaunchKernelGGL((k_scan_small<In>), dim3(1), dim3(kSmallBlock), 0, s, in, out, n);
     return hipGetLastError();
   }
   const int64_t tiles = (n + kScanTile - 1) / kScanTile;
@@ -1408,119 +1517,88 @@ int64_t gpk_lookback_tiles(int64_t n) { return n > 0 ? (n + kScanTile - 1) / kSc
 hipError_t gpk_scan_lb_i32(const int32_t* in, int32_t* out, int64_t n, gpk_lookback lb, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (n <= kSmallScanMax) {
-    hipLaunchKernelGGL((k_scan_small<int32_t, 0>), dim3(1), dim3(kSmallBlock), 0, s, in, out, n, nullptr);
+    hipLaunchKernelGGL((k_scan_small<int32_t>), dim3(1), dim3(kSmallBlock), 0, s, in, out, n);
     return hipGetLastError();
   }
   const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL((k_scan_lb<int32_t, 0>), dim3(static_cast<unsigned>(tiles)), dim3(kBlock), 0, s, in, out, n,
-                     nullptr, lb);
+  hipLaunchKernelGGL((k_scan_lb<int32_t>), dim3(static_cast<unsigned>(tiles)), dim3(kBlock), 0, s, in, out, n,
+                     lb);
   return hipGetLastError();
 }
 
 hipError_t gpk_scan_lb_mask(const uint8_t* mask, int32_t* out, int64_t n, gpk_lookback lb, hipStream_t s) {
   if (n <= 0) return hipSuccess;
+  if (n <= GPK_MAP_RECOUNT_MAX && (reinterpret_cast<uintptr_t>(mask) & 15u) == 0) {
+    hipLaunchKernelGGL(k_mask_scan, dim3(grid_for(n, kScanTile)), dim3(kBlock), 0, s, mask, out,
+                       static_cast<int32_t>(n));
+    return hipGetLastError();
+  }
   if (n <= kSmallScanMax) {
-    hipLaunchKernelGGL((k_scan_small<uint8_t, 0>), dim3(1), dim3(kSmallBlock), 0, s, mask, out, n, nullptr);
+    hipLaunchKernelGGL((k_scan_small<uint8_t>), dim3(1), dim3(kSmallBlock), 0, s, mask, out, n);
     return hipGetLastError();
   }
   const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL((k_scan_lb<uint8_t, 0>), dim3(static_cast<unsigned>(tiles)), dim3(kBlock), 0, s, mask, out, n,
-                     nullptr, lb);
+  hipLaunchKernelGGL((k_scan_lb<uint8_t>), dim3(static_cast<unsigned>(tiles)), dim3(kBlock), 0, s, mask, out, n,
+                     lb);
   return hipGetLastError();
 }
 
 int64_t gpk_apply_maps_tiles(int32_t m, int32_t n) {
-  const int64_t rt = m > 0 ? (m + kScanTile - 1) / kScanTile : 0;
-  const int64_t ct = n > 0 ? (n + kScanTile - 1) / kScanTile : 0;
-  return rt + 2 * ct;
+  const int64_t rt = m > 0 ? (static_cast<int64_t>(m) + kScanTile - 1) / kScanTile : 0;
+  const int64_t ct = n > 0 ? (static_cast<int64_t>(n) + kScanTile - 1) / kScanTile : 0;
+  return rt + ct;
 }
 
 hipError_t gpk_apply_maps(gpk_apply_maps_args args, gpk_lookback lb, hipStream_t s) {
-  const int64_t rt = args.m > 0 ? (args.m + kScanTile - 1) / kScanTile : 0;
-  const int64_t ct = args.n > 0 ? (args.n + kScanTile - 1) / kScanTile : 0;
-  const int64_t tiles = rt + 2 * ct;
+  const int64_t tiles = gpk_apply_maps_tiles(args.m, args.n);
   if (tiles == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_apply_maps, dim3(static_cast<unsigned>(tiles)), dim3(kBlock), 0, s, args,
-                     static_cast<int32_t>(rt), static_cast<int32_t>(ct), lb);
-  return hipGetLastError();
-}
-
-hipError_t gpk_mask_to_map(const uint8_t* mask, int32_t* map, int64_t n, int32_t* count, gpk_lookback lb,
-                           hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  if (n <= kSmallScanMax) {
-    hipLaunchKernelGGL((k_scan_small<uint8_t, 1>), dim3(1), dim3(kSmallBlock), 0, s, mask, map, n, count);
-    return hipGetLastError();
+  const dim3 grid(static_cast<unsigned>(tiles));
+  const int32_t r = static_cast<int32_t>(gpk_apply_maps_tiles(args.m, 0));
+  const bool aligned =
+      ((reinterpret_cast<uintptr_t>(args.keep_row) | reinterpret_cast<uintptr_t>(args.keep_col)) & 15u) == 0;
+  const int32_t al = aligned ? 1 : 0;
+  if (aligned && args.m <= GPK_MAP_RECOUNT_MAX && args.n <= GPK_MAP_RECOUNT_MAX) {
+    hipLaunchKernelGGL(k_apply_maps<kMapRecount>, grid, dim3(kBlock), 0, s, args, r, al, lb);
+  } else if (tiles <= GPK_MAP_COUNT_TILES) {
+    hipLaunchKernelGGL(k_apply_counts, grid, dim3(kBlock), 0, s, args, r, al);
+    hipLaunchKernelGGL(k_apply_maps<kMapCounts>, grid, dim3(kBlock), 0, s, args, r, al, lb);
+  } else {
+    hipLaunchKernelGGL(k_apply_maps<kMapLookback>, grid, dim3(kBlock), 0, s, args, r, al, lb);
   }
-  const int64_t tiles = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL((k_scan_lb<uint8_t, 1>), dim3(static_cast<unsigned>(tiles)), dim3(kBlock), 0, s, mask, map, n,
-                     count, lb);
   return hipGetLastError();
 }
 
+int32_t gpk_compact_shift(int32_t nnz) { return nnz <= GPK_COMPACT_SMALL_NNZ ? 9 : 11; }
 
-
-hipError_t gpk_build_rank(const int32_t* map, int32_t n, gpk_rank_word* out, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_build_rank, dim3(grid_for(n)), dim3(kBlock), 0, s, map, n, out);
-  return hipGetLastError();
+int32_t gpk_compact_chunks(int32_t nnz) {
+  const int32_t shift = gpk_compact_shift(nnz);
+  return (nnz >> shift) + ((nnz & ((1 << shift) - 1)) != 0 ? 1 : 0);
 }
 
-int32_t gpk_compact_tiles(int32_t m_old) { return m_old > 0 ? static_cast<int32_t>(grid_for(m_old, kCompRows)) : 0; }
-
-hipError_t gpk_compact_map(const int32_t* ptr, const int32_t* idx, int32_t m_old, const int32_t* row_map,
-                           const gpk_rank_word* col_rank, int32_t* jn, int32_t* out_ptr, int32_t* tile_cnt,
+hipError_t gpk_compact_map(gpk_compact_side a, gpk_compact_side t, int32_t* chunk_cnt, int32_t* kept_total,
                            hipStream_t s) {
-  return gpk_compact_map_total(ptr, idx, m_old, row_map, col_rank, jn, out_ptr, tile_cnt, nullptr, s);
-}
-
-hipError_t gpk_compact_map_total(const int32_t* ptr, const int32_t* idx, int32_t m_old, const int32_t* row_map,
-                                 const gpk_rank_word* col_rank, int32_t* jn, int32_t* out_ptr, int32_t* tile_cnt,
-                                 int32_t* kept_total, hipStream_t s) {
-  if (m_old <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_compact_map, dim3(grid_for(m_old, kCompRows)), dim3(kBlock), 0, s, ptr, idx, m_old, row_map,
-                     col_rank, jn, out_ptr, tile_cnt, kept_total);
+  const int32_t ca = gpk_compact_chunks(a.nnz), ct = gpk_compact_chunks(t.nnz);
+  if (ca + ct == 0) return hipSuccess;
+  if (gpk_compact_shift(a.nnz > t.nnz ? a.nnz : t.nnz) == 9)
+    hipLaunchKernelGGL(k_compact_map<2>, dim3(ca + ct), dim3(kBlock), 0, s, a, t, ca, chunk_cnt, kept_total);
+  else
+    hipLaunchKernelGGL(k_compact_map<8>, dim3(ca + ct), dim3(kBlock), 0, s, a, t, ca, chunk_cnt, kept_total);
   return hipGetLastError();
 }
 
-hipError_t gpk_compact_write(const int32_t* ptr, const double* val, int32_t m_old, const int32_t* row_map,
-                             const int32_t* jn, const int32_t* tile_off, int32_t* out_ptr, int32_t m_new,
-                             int32_t* out_idx, double* out_val, hipStream_t s) {
-  if (m_old <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_compact_write<false>, dim3(grid_for(m_old, kCompRows)), dim3(kBlock), 0, s, ptr, val, m_old,
-                     row_map, jn, tile_off, out_ptr, m_new, out_idx, out_val);
-  return hipGetLastError();
-}
-
-hipError_t gpk_compact_map_pair(gpk_compact_side a, gpk_compact_side t, int32_t* tile_cnt, int32_t* kept_total,
-                                hipStream_t s) {
-  if (a.m_old < 0 || t.m_old < 0) return hipErrorInvalidValue;
-  const int32_t ta = a.m_old > 0 ? static_cast<int32_t>(grid_for(a.m_old, kCompRows)) : 0;
-  const int32_t tt = t.m_old > 0 ? static_cast<int32_t>(grid_for(t.m_old, kCompRows)) : 0;
-  if (ta + tt == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_compact_map_pair, dim3(ta + tt), dim3(kBlock), 0, s, a, t, ta, tile_cnt, kept_total);
-  return hipGetLastError();
-}
-
-hipError_t gpk_compact_write_pair(gpk_compact_side a, gpk_compact_side t, const int32_t* tile_off, int32_t from_counts,
-                                  hipStream_t s) {
-  if (a.m_old < 0 || t.m_old < 0) return hipErrorInvalidValue;
-  const int32_t ta = a.m_old > 0 ? static_cast<int32_t>(grid_for(a.m_old, kCompRows)) : 0;
-  const int32_t tt = t.m_old > 0 ? static_cast<int32_t>(grid_for(t.m_old, kCompRows)) : 0;
-  if (ta + tt == 0) return hipSuccess;
-  if (from_counts && (ta > kBlock || tt > kBlock)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_compact_write_pair, dim3(ta + tt), dim3(kBlock), 0, s, a, t, ta, tt, tile_off, from_counts);
-  return hipGetLastError();
-}
-
-hipError_t gpk_compact_write_counts(const int32_t* ptr, const double* val, int32_t m_old, const int32_t* row_map,
-                                    const int32_t* jn, const int32_t* tile_cnt, int32_t* out_ptr, int32_t m_new,
-                                    int32_t* out_idx, double* out_val, hipStream_t s) {
-  if (m_old <= 0) return hipSuccess;
-  const unsigned tiles = grid_for(m_old, kCompRows);
-  if (tiles > static_cast<unsigned>(kBlock)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_compact_write<true>, dim3(tiles), dim3(kBlock), 0, s, ptr, val, m_old, row_map, jn, tile_cnt,
-                     out_ptr, m_new, out_idx, out_val);
+hipError_t gpk_compact_write(gpk_compact_side a, gpk_compact_side t, const int32_t* chunk_off, int32_t from_counts,
+                             gpk_apply_gathers_args gathers, hipStream_t s) {
+  if (a.nnz > 0 && t.nnz > 0 && a.nnz != t.nnz) return hipErrorInvalidValue;
+  const int32_t ca = gpk_compact_chunks(a.nnz), ct = gpk_compact_chunks(t.nnz);
+  if (from_counts && (ca > GPK_COMPACT_COUNT_CHUNKS || ct > GPK_COMPACT_COUNT_CHUNKS)) return hipErrorInvalidValue;
+  const int32_t ra = ca > 0 ? static_cast<int32_t>(grid_for(a.m_old)) : 0;
+  const int32_t rt = ct > 0 ? static_cast<int32_t>(grid_for(t.m_old)) : 0;
+  if (ca + ct == 0) return hipSuccess;
+  const dim3 grid(ca + ct + ra + rt);
+  if (gpk_compact_shift(a.nnz > t.nnz ? a.nnz : t.nnz) == 9)
+    hipLaunchKernelGGL(k_compact_write<2>, grid, dim3(kBlock), 0, s, a, t, ca, ct, ra, chunk_off, from_counts, gathers);
+  else
+    hipLaunchKernelGGL(k_compact_write<8>, grid, dim3(kBlock), 0, s, a, t, ca, ct, ra, chunk_off, from_counts, gathers);
   return hipGetLastError();
 }
 
@@ -1593,15 +1671,6 @@ hipError_t gpk_apply_gathers(gpk_apply_gathers_args args, hipStream_t s) {
   const int32_t len = args.m > args.n ? args.m : args.n;
   if (len <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_apply_gathers, dim3(grid_for(len)), dim3(kBlock), 0, s, args);
-  return hipGetLastError();
-}
-
-hipError_t gpk_gather5(const int32_t* map, int32_t n_old, const double* s0, double* d0, const double* s1, double* d1,
-                       const double* s2, double* d2, const double* s3, double* d3, const double* s4, double* d4,
-                       hipStream_t s) {
-  if (n_old <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_gather5, dim3(grid_for(n_old)), dim3(kBlock), 0, s, map, n_old, s0, d0, s1, d1, s2, d2, s3,
-                     d3, s4, d4);
   return hipGetLastError();
 }
 

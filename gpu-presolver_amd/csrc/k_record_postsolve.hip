@@ -1,5 +1,4 @@
-// Record maintenance (device-resident red2org maps, fixed-column records,
-// tape index globalization) and postsolve kernels: scatter of the reduced
+// Record maintenance (tape index globalization) and postsolve kernels: scatter of the reduced
 // solution, fixed-value restore, reverse tape replay and the column-dual
 // projection.
 #include <hip/hip_runtime.h>
@@ -17,24 +16,6 @@ using namespace gpdev;
 namespace {
 
 // ------------------------------------------------------------ record ----
-// Removed columns whose bounds are finite and within 1e-9 (gpu_presolve.cu:1005-1043).
-__global__ void k_removed_fixed_mask(int32_t n, const uint8_t* keep_col, const double* l, const double* u,
-                                     uint8_t* mask) {
-  const int32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n) return;
-  const double lo = l[j], hi = u[j];
-  mask[j] = (!keep_col[j] && isfinite(lo) && isfinite(hi) && fabs(lo - hi) <= 1.0e-9) ? 1 : 0;
-}
-
-__global__ void k_pack_fixed_records(int32_t n, const uint8_t* mask, const int32_t* prefix, const int32_t* red2org,
-                                     const double* l, const double* u, int32_t* out_idx, double* out_val) {
-  const int32_t j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= n || !mask[j]) return;
-  const int32_t r = prefix[j];
-  out_idx[r] = red2org[j];
-  out_val[r] = 0.5 * (l[j] + u[j]);
-}
-
 // kind: 1 = row index, 2 = column index, 0 = not an index.  Out-of-range
 // values are left unchanged (gpu_presolve.cu:1347-1361).
 __global__ void k_map_tape_indices(int32_t count, int32_t* idx, const uint8_t* kind, const int32_t* row_red2org,
@@ -668,15 +649,6 @@ __global__ void k_protect(gp_tape_dev T, int32_t n, uint8_t* prot) {
 
 extern "C" {
 
-hipError_t gpk_removed_fixed_mask(int32_t n, const uint8_t* keep_col, const double* l, const double* u,
-                                  uint8_t* mask, hipStream_t stream) {
-  GPK_LAUNCH(k_removed_fixed_mask, n, n, keep_col, l, u, mask);
-}
-hipError_t gpk_pack_fixed_records(int32_t n, const uint8_t* mask, const int32_t* prefix, const int32_t* red2org,
-                                  const double* l, const double* u, int32_t* out_idx, double* out_val,
-                                  hipStream_t stream) {
-  GPK_LAUNCH(k_pack_fixed_records, n, n, mask, prefix, red2org, l, u, out_idx, out_val);
-}
 hipError_t gpk_map_tape_indices(int32_t count, int32_t* idx, const uint8_t* kind, const int32_t* row_red2org,
                                 int32_t m, const int32_t* col_red2org, int32_t n, hipStream_t stream) {
   GPK_LAUNCH(k_map_tape_indices, count, count, idx, kind, row_red2org, m, col_red2org, n);

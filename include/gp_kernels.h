@@ -59,98 +59,132 @@ int64_t gpk_lookback_tiles(int64_t n);
 hipError_t gpk_scan_lb_i32(const int32_t* in, int32_t* out, int64_t n, gpk_lookback lb, hipStream_t stream);
 /* Same over (mask[i] != 0). */
 hipError_t gpk_scan_lb_mask(const uint8_t* mask, int32_t* out, int64_t n, gpk_lookback lb, hipStream_t stream);
-/* map[i] = mask[i] ? (number of set mask entries before i) : -1; *count = total. */
-hipError_t gpk_mask_to_map(const uint8_t* mask, int32_t* map, int64_t n, int32_t* count, gpk_lookback lb,
-                           hipStream_t stream);
 /* Rank form of an old-to-new map, one word per 64 entries: bit b of word w
  * is set when entry 64w + b is kept; base is the new index of the word's
- * first kept entry.  gpk_build_rank writes ceil(n / 64) words. */
+ * first kept entry: a lookup reads one small, cache-resident word instead of
+ * gathering from the n-entry map. */
 typedef struct __attribute__((aligned(16))) gpk_rank_word {
   uint64_t bits;
   int32_t base;
   int32_t pad;
 } gpk_rank_word;
-hipError_t gpk_build_rank(const int32_t* map, int32_t n, gpk_rank_word* out, hipStream_t stream);
-/* The three keep maps of a plan application in one launch (three look-back
- * chains): row_map from keep_row (m), col_map from keep_col (n), and
- * fixed_map from the removed columns with a fixed finite interval
- * (!keep_col && |u - l| <= 1e-9; the mask is stored in fixed_mask);
- * map[i] = rank among the set entries or -1; counts[0..2] = the three totals;
- * row_rank / col_rank, when given, receive the maps' rank words (as
- * gpk_build_rank).
- * The look-back workspace covers gpk_apply_maps_tiles(m, n) tiles. */
+/* Sizes up to which a map tile counts its mask again, sums its chain's tile
+ * counts, a compaction sums its chunks' counts per block, and its chunks are
+ * small (the kernels say why). */
+#define GPK_MAP_RECOUNT_MAX 262144
+#define GPK_MAP_COUNT_TILES 4096
+#define GPK_COMPACT_COUNT_CHUNKS 2048
+#define GPK_COMPACT_SMALL_NNZ (GPK_COMPACT_COUNT_CHUNKS * 512)
+/* The keep maps of a plan application (chains of one launch): row_map from
+ * keep_row (m) and col_map from keep_col (n); map[i] = rank among the set
+ * entries or -1; counts[0..1] = the totals; row_rank / col_rank, when given,
+ * receive the maps' rank words.  With l: fixed_mask marks
+ * the removed columns with a fixed finite interval (!keep_col && |u - l| <=
+ * 1e-9), fixed_tiles[t] counts those of columns [2048 t, 2048 (t + 1)) and
+ * counts[2] all of them (the caller zeroes it).  a_chunk / at_chunk, when a_ptr
+ * / at_ptr (row pointers over the m rows / n columns) are given, receive the
+ * chunk rows of a compaction: entry q << chunk_shift lies in row a_chunk[q],
+ * and the word after the last chunk's holds the last row.
+ * The look-back workspace and tile_counts cover gpk_apply_maps_tiles(m, n)
+ * tiles, fixed_tiles gpk_apply_maps_tiles(0, n). */
 typedef struct gpk_apply_maps_args {
   int32_t m, n;
   const uint8_t* keep_row;
   const uint8_t* keep_col;
-  const double* l;
+  const double* l; /* optional */
   const double* u;
   int32_t* row_map;
   int32_t* col_map;
   uint8_t* fixed_mask;
-  int32_t* fixed_map;
+  int32_t* fixed_tiles;
   int32_t* counts;
   gpk_rank_word* row_rank; /* optional: rank words of row_map ((m + 63) / 64) */
   gpk_rank_word* col_rank; /* optional: rank words of col_map ((n + 63) / 64) */
+  const int32_t* a_ptr;    /* optional */
+  const int32_t* at_ptr;   /* optional */
+  int32_t* a_chunk;
+  int32_t* at_chunk;
+  int32_t* tile_counts;
+  int32_t chunk_shift;
 } gpk_apply_maps_args;
 int64_t gpk_apply_maps_tiles(int32_t m, int32_t n);
 hipError_t gpk_apply_maps(gpk_apply_maps_args args, gpk_lookback lb, hipStream_t stream);
 
+/* The vector gathers of a plan application (gpu_presolve.cu:2021-2147): c, l,
+ * u and the column reduced-to-original map through col_map (n); AL, AU and the
+ * row map through row_map (m).  Null r2o outputs are skipped.  With fixed_mask
+ * (and fixed_tiles, both as gpk_apply_maps leaves them), the removed fixed
+ * columns are recorded as well, in column order (gpu_presolve.cu:1005-1043):
+ * fixed_idx = col_r2o_in[j], fixed_val the interval's middle. */
+typedef struct gpk_apply_gathers_args {
+  int32_t m, n;
+  const int32_t* col_map;
+  const double* c_in;
+  const double* l_in;
+  const double* u_in;
+  const int32_t* col_r2o_in;
+  double* c_out;
+  double* l_out;
+  double* u_out;
+  int32_t* col_r2o_out;
+  const int32_t* row_map;
+  const double* al_in;
+  const double* au_in;
+  const int32_t* row_r2o_in;
+  double* al_out;
+  double* au_out;
+  int32_t* row_r2o_out;
+  const uint8_t* fixed_mask;
+  const int32_t* fixed_tiles;
+  int32_t* fixed_idx;
+  double* fixed_val;
+} gpk_apply_gathers_args;
+hipError_t gpk_apply_gathers(gpk_apply_gathers_args args, hipStream_t stream);
+
 /* Stable compaction of a CSR by an old-to-new row map and the rank form of
- * the column map, over tiles of 256 old rows (gpk_compact_tiles(m_old)):
+ * the column map, over gpk_compact_chunks(nnz) chunks of 1 <<
+ * gpk_compact_shift(nnz) entries, for a matrix and, in the same launches, its
+ * transpose t by the same maps (nnz 0: the matrix alone):
  *   gpk_compact_map    jn[p] = new column of entry p, or -1 when its row or
- *                      column is dropped; out_ptr[new row] = kept count;
- *                      tile_cnt[t] = kept entries of tile t;
- *   gpk_scan_lb_i32(tile_cnt, tile_cnt, tiles, ...) makes the tile counts
- *                      exclusive offsets (tile_cnt[tiles] = kept entries);
- *   gpk_compact_write  turns out_ptr into the new row pointers
- *                      (out_ptr[m_new] = kept entries) and writes the kept
- *                      (column, value) pairs.
- * jn holds one int32 per entry of A, tile_cnt tiles + 1.  col_rank NULL
- * means no column is dropped (every kept entry keeps its column index). */
-int32_t gpk_compact_tiles(int32_t m_old);
-hipError_t gpk_compact_map(const int32_t* ptr, const int32_t* idx, int32_t m_old, const int32_t* row_map,
-                           const gpk_rank_word* col_rank, int32_t* jn, int32_t* out_ptr, int32_t* tile_cnt,
-                           hipStream_t stream);
-hipError_t gpk_compact_write(const int32_t* ptr, const double* val, int32_t m_old, const int32_t* row_map,
-                             const int32_t* jn, const int32_t* tile_off, int32_t* out_ptr, int32_t m_new,
-                             int32_t* out_idx, double* out_val, hipStream_t stream);
-/* gpk_compact_map that also adds the kept entry count to *kept_total (one
- * integer atomic per tile; the caller zeroes it), so the count is known
- * before any scan. */
-hipError_t gpk_compact_map_total(const int32_t* ptr, const int32_t* idx, int32_t m_old, const int32_t* row_map,
-                                 const gpk_rank_word* col_rank, int32_t* jn, int32_t* out_ptr, int32_t* tile_cnt,
-                                 int32_t* kept_total, hipStream_t stream);
-/* A CSR and its transpose compacted with the same two maps (A by row_map
- * and the column rank words, AT by the column map and the row rank words)
- * in one map launch and one write launch.  tile_cnt holds
- * gpk_compact_tiles(a.m_old) + gpk_compact_tiles(t.m_old) + 1 words: A's tile
- * counts, then AT's.  The write pass takes either those raw counts
- * (from_counts, allowed when each side has at most 256 tiles)
- * or one exclusive scan of them (gpk_scan_lb_i32 over both sides' tiles).
- * kept_total (optional, zeroed by the caller) receives A's kept count. */
+ *                      column is dropped; mask and word_pre (a word per 64
+ *                      entries, whole chunks): the kept entries and the kept
+ *                      ones of the chunk before each word; chunk_cnt: the kept
+ *                      entries of a's chunks, then t's; kept_total (optional,
+ *                      zeroed by the caller) receives a's;
+ *   gpk_compact_write  the new row pointers (m_new + 1), columns and values,
+ *                      from chunk_cnt (from_counts, at most
+ *                      GPK_COMPACT_COUNT_CHUNKS chunks a side) or one exclusive
+ *                      scan of it (gpk_scan_lb_i32 over both sides' chunks);
+ *                      with gathers.m / gathers.n above 0 also
+ *                      gpk_apply_gathers' rows / columns (through a's / t's
+ *                      row_map).
+ * chunk_row holds the chunk rows (gpk_apply_maps).  col_rank NULL means no
+ * column is dropped.  nnz above 0, and every array given, on a side that takes
+ * part; both sides hold the same number of entries. */
 typedef struct gpk_compact_side {
   const int32_t* ptr;
   const int32_t* idx;
   const double* val;
   int32_t m_old;
   int32_t m_new;
+  int32_t nnz;
+  int32_t pad;
   const int32_t* row_map;
   const gpk_rank_word* col_rank;
+  const int32_t* chunk_row;
   int32_t* jn;
+  uint64_t* mask;
+  int32_t* word_pre;
   int32_t* out_ptr;
   int32_t* out_idx;
   double* out_val;
 } gpk_compact_side;
-hipError_t gpk_compact_map_pair(gpk_compact_side a, gpk_compact_side t, int32_t* tile_cnt, int32_t* kept_total,
-                                hipStream_t stream);
-hipError_t gpk_compact_write_pair(gpk_compact_side a, gpk_compact_side t, const int32_t* tile_off,
-                                  int32_t from_counts, hipStream_t stream);
-/* The same without the scan, for at most 256 tiles (m_old <= 65,536): it
- * takes the raw tile counts of gpk_compact_map and derives the offsets. */
-hipError_t gpk_compact_write_counts(const int32_t* ptr, const double* val, int32_t m_old, const int32_t* row_map,
-                                    const int32_t* jn, const int32_t* tile_cnt, int32_t* out_ptr, int32_t m_new,
-                                    int32_t* out_idx, double* out_val, hipStream_t stream);
+int32_t gpk_compact_shift(int32_t nnz);
+int32_t gpk_compact_chunks(int32_t nnz);
+hipError_t gpk_compact_map(gpk_compact_side a, gpk_compact_side t, int32_t* chunk_cnt, int32_t* kept_total,
+                           hipStream_t stream);
+hipError_t gpk_compact_write(gpk_compact_side a, gpk_compact_side t, const int32_t* chunk_off, int32_t from_counts,
+                             gpk_apply_gathers_args gathers, hipStream_t stream);
 
 /* Up to GPK_COPY_MAX copies (src != NULL) or zero fills (src == NULL) of
  * device byte ranges in one launch (block row y serves segment y; the unit
@@ -199,35 +233,7 @@ hipError_t gpk_csr_stats(const int32_t* ptr, const int32_t* idx, const double* v
                          int32_t* nnz_out, uint8_t* empty_mask, uint8_t* singleton_mask,
                          int32_t* singleton_idx, double* singleton_val, hipStream_t stream);
 
-/* ---- compaction helpers ---------------------------------------------- */
-/* The gathers of a plan application in one launch (gpu_presolve.cu:2021-2147):
- * c, l, u and the column reduced-to-original map through col_map (n); AL, AU
- * and the row map through row_map (m).  Null r2o outputs are skipped. */
-typedef struct gpk_apply_gathers_args {
-  int32_t m, n;
-  const int32_t* col_map;
-  const double* c_in;
-  const double* l_in;
-  const double* u_in;
-  const int32_t* col_r2o_in;
-  double* c_out;
-  double* l_out;
-  double* u_out;
-  int32_t* col_r2o_out;
-  const int32_t* row_map;
-  const double* al_in;
-  const double* au_in;
-  const int32_t* row_r2o_in;
-  double* al_out;
-  double* au_out;
-  int32_t* row_r2o_out;
-} gpk_apply_gathers_args;
-hipError_t gpk_apply_gathers(gpk_apply_gathers_args args, hipStream_t stream);
-/* dst[map[i]] = src[i] for map[i] >= 0, for up to 5 vectors of the same length. */
-hipError_t gpk_gather5(const int32_t* map, int32_t n_old, const double* s0, double* d0,
-                       const double* s1, double* d1, const double* s2, double* d2,
-                       const double* s3, double* d3, const double* s4, double* d4,
-                       hipStream_t stream);
+/* dst[map[i]] = src[i] for map[i] >= 0. */
 hipError_t gpk_gather_i32(const int32_t* map, int32_t n_old, const int32_t* src, int32_t* dst,
                           hipStream_t stream);
 

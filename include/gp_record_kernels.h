@@ -2,7 +2,6 @@
  * Internal C-ABI launchers for record maintenance and postsolve
  * (part of the same thin layer as gp_kernels.h).
  *
- *   gpk_removed_fixed_mask / gpk_pack_fixed_records
  *       append_removed_fixed_bound_records (reference gpu_presolve.cu:1005-1233)
  *   gpk_map_tape_indices
  *       append_globalized_postsolve_tape (reference gpu_presolve.cu:1363-1533)
@@ -47,11 +46,6 @@ typedef struct gp_orig_dev {
   const double* u;
 } gp_orig_dev;
 
-hipError_t gpk_removed_fixed_mask(int32_t n, const uint8_t* keep_col, const double* l, const double* u,
-                                  uint8_t* mask, hipStream_t stream);
-hipError_t gpk_pack_fixed_records(int32_t n, const uint8_t* mask, const int32_t* prefix, const int32_t* red2org,
-                                  const double* l, const double* u, int32_t* out_idx, double* out_val,
-                                  hipStream_t stream);
 hipError_t gpk_map_tape_indices(int32_t count, int32_t* idx, const uint8_t* kind, const int32_t* row_red2org,
                                 int32_t m, const int32_t* col_red2org, int32_t n, hipStream_t stream);
 hipError_t gpk_scatter(const double* src, const int32_t* red2org, int32_t n_red, double* dst, hipStream_t stream);

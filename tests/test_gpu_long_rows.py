@@ -1,6 +1,8 @@
 """Rows far longer than their neighbours: the kernels that give such a row a
 wave (or a tile of its own entries) against the oracle, bit for bit, at the
 lengths where the split happens and with neighbouring long rows."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -46,4 +48,62 @@ def test_row_activity_long_rows(lengths):
     got = gp_ffi.row_activity(m, n, ptr, idx, val, l, u, 1e-10)
     want = O.row_activity(m, n, ptr, idx, val, l, u, 1e-10)
     for name, a, b in zip(("min_fin", "max_fin", "neg_inf", "pos_inf"), got, want):
+        assert_same_array(name, a, b)
+
+
+def compact_lengths(case):
+    rng = np.random.default_rng(11)
+    if case == "edges":  # chunks of 2,048 entries: rows that end, start and straddle there
+        return [2048, 2048, 2047, 1, 4096, 0, 0, 1, 2046, 1, 3, 5000, 0, 2049] + [0] * 300 + [7]
+    if case == "long":
+        return lengths_with_long_rows(12)
+    if case == "empty-gap":  # one chunk spans more empty rows than it marks in its bitmap
+        return [3] * 100 + [0] * 20000 + [5, 0, 900] + [0] * 9000
+    if case == "empty-ends":
+        return [0] * 5000 + [1] * 4100 + [0] * 5000
+    if case == "counts":  # more rows than a tile counts again
+        return list(rng.integers(0, 3, 262144 + 4001))
+    if case == "scan":  # more chunks than a block sums
+        return [1400] * 3010
+    if case == "large-chunks":  # the first size of 2,048-entry chunks
+        return [1024] * 1024 + [1]
+    if case == "small-chunks":
+        return [1024] * 1024
+    return list(rng.integers(0, 9, 40000))  # "recount"
+
+
+@pytest.mark.parametrize("case", ["edges", "long", "empty-gap", "empty-ends", "counts", "scan", "recount",
+                                  "large-chunks", "small-chunks"])
+@pytest.mark.parametrize("drop", [0.0, 0.3, 1.0])
+def test_compaction_by_chunks(case, drop):
+    lengths = compact_lengths(case)
+    m, n = len(lengths), 5001
+    ptr, idx, val = csr_of_lengths([min(int(k), n) for k in lengths], n, 13)
+    rng = np.random.default_rng(14)
+    kr, kc = (rng.random(m) >= drop).astype(np.uint8), (rng.random(n) >= drop / 2).astype(np.uint8)
+    got = gp_ffi.compact_csr(m, n, ptr, idx, val, kr, kc)
+    want = O.compact_csr(m, n, ptr, idx, val, kr, kc)
+    assert got[:2] == want[:2]
+    for name, a, b in zip(("ptr", "idx", "val"), got[2:], want[2:]):
+        assert_same_array(name, a, b)
+
+
+@pytest.mark.parametrize("m", [2048, 5000, 9_000_000])
+def test_compaction_masks_at_an_odd_address(m):
+    """Masks that no 16-byte load can read; 9,000,000 rows take the look-back."""
+    rng = np.random.default_rng(m)
+    lengths = np.zeros(m, np.int64)
+    lengths[rng.choice(m, 1500, replace=False)] = rng.integers(1, 6, 1500)
+    n = 777
+    ptr, idx, val = csr_of_lengths(lengths if m < 10000 else lengths[lengths > 0], n, 15)
+    ptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    kr, kc = (rng.random(m) < 0.6).astype(np.uint8), (rng.random(n) < 0.6).astype(np.uint8)
+    A = gp_ffi.DeviceCsr(m, n, ptr, idx, val)
+    dr, dc = gp_ffi.DeviceArray(np.concatenate([[9], kr]).astype(np.uint8)), gp_ffi.DeviceArray(np.concatenate([[9], kc]).astype(np.uint8))
+    out = gp_ffi.T.GpCsr()
+    gp_ffi._check(gp_ffi.lib().gp_compact_csr(C.byref(A.g), dr.ptr + 1, dc.ptr + 1, C.byref(out)))
+    got = (out.rows, out.cols) + gp_ffi._take_csr(out)
+    want = O.compact_csr(m, n, ptr, idx, val, kr, kc)
+    assert got[:2] == want[:2]
+    for name, a, b in zip(("ptr", "idx", "val"), got[2:], want[2:]):
         assert_same_array(name, a, b)

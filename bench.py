@@ -118,7 +118,7 @@ def measure_activity_kernels(gp_ffi, dlp, lp, stream, launches, want_mn, want_mx
     L = gp_ffi.lib()
     vp = C.c_void_p
     L.gpk_pack_lu.argtypes = [vp, vp, C.c_int32, vp, vp]
-    L.gpk_row_activity_lu.argtypes = [vp, vp, vp, C.c_int32, vp, C.c_double, vp, vp, vp, vp, vp]
+    L.gpk_row_activity_lu.argtypes = [vp, vp, vp, C.c_int32, C.c_int32, vp, C.c_double, vp, vp, vp, vp, vp]
     lu = gp_ffi.DeviceArray(size=2 * n)
     mn, mx = gp_ffi.DeviceArray(size=m), gp_ffi.DeviceArray(size=m)
     ni, pi = gp_ffi.DeviceArray(size=m, dtype=np.int32), gp_ffi.DeviceArray(size=m, dtype=np.int32)
@@ -128,7 +128,7 @@ def measure_activity_kernels(gp_ffi, dlp, lp, stream, launches, want_mn, want_mx
         gp_ffi.hip_check(L.gpk_pack_lu(dlp.vec["l"].ptr, dlp.vec["u"].ptr, n, lu.ptr, stream.ptr), "pack lu")
 
     def act():
-        gp_ffi.hip_check(L.gpk_row_activity_lu(A.row_ptr, A.col_idx, A.val, m, lu.ptr, 1e-10, mn.ptr, mx.ptr,
+        gp_ffi.hip_check(L.gpk_row_activity_lu(A.row_ptr, A.col_idx, A.val, m, nnz, lu.ptr, 1e-10, mn.ptr, mx.ptr,
                                                ni.ptr, pi.ptr, stream.ptr), "activity lu")
 
     pack()

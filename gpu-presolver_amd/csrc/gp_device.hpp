@@ -92,10 +92,17 @@ __device__ inline double add_in_order(double s, const double* t, int n) {
 // in all), past that the 16 rows of a line.  The row pointers of kLook groups
 // are loaded together: without a long row these blocks are gone in a few
 // memory round trips.
-inline unsigned long_row_blocks(int32_t m) {  // at most one a CU
-  const unsigned b = grid_for(m, kWaves);
-  return b < 256u ? b : 256u;
+// One such block a CU, or eight where rows are long on average (100,000 rows
+// of 200 entries are 12 for each wave then).
+inline unsigned long_row_blocks(int32_t m, int64_t nnz) {
+  const unsigned b = grid_for(m, kWaves), most = nnz >= 32 * static_cast<int64_t>(m) ? 2048u : 256u;
+  return b < most ? b : most;
 }
+
+// Rows of more entries than this get a wave each in the kernels that otherwise
+// give a row to a thread: a thread walks a row at a few hundred ns an entry
+// (1.3 ms for 3,000), a wave needs about 3 us for a row and 10 ns an entry.
+constexpr int kLongRow = 128;
 
 template <class F>
 __device__ __forceinline__ void wave_long_rows(const int32_t* __restrict__ ptr, int32_t m, int32_t longer,
@@ -126,6 +133,57 @@ __device__ __forceinline__ void wave_long_rows(const int32_t* __restrict__ ptr, 
       }
     }
   }
+}
+
+// The entries [b, e) of a row walked by a wave, kRowChunk at a time (the next
+// ones on their way meanwhile): load(column, in_range) gathers, term(value,
+// gathered, in_range, t) forms kSums terms of the entry, each kind of which is
+// added in the order of the entries; lane k < kSums returns the sum of kind k.
+// term returns false for an entry that adds nothing: its terms must be +0,
+// which leaves a sum that started at +0 as it is (no such sum is -0).
+// s_t: kSums * kRowPitch doubles of LDS, 16-byte aligned, the wave's own.
+// Bound by the chain of adds, about 3 ns an entry.
+constexpr int kRowSteps = 4;
+constexpr int kRowChunk = 64 * kRowSteps;
+constexpr int kRowPitch = kRowChunk + 2;  // the kinds start in different banks
+
+template <int kSums, class G, class Load, class Term>
+__device__ __forceinline__ double wave_row_sums(const int32_t* __restrict__ idx, const double* __restrict__ val,
+                                                int32_t b, int32_t e, double* s_t, Load&& load, Term&& term) {
+  const int lane = lane_id();
+  double a[kRowSteps], acc = 0.0;
+  int32_t j[kRowSteps];
+#pragma unroll
+  for (int k = 0; k < kRowSteps; ++k) {
+    const int32_t p = min(b + 64 * k + lane, e - 1);
+    a[k] = val[p];
+    j[k] = idx[p];
+  }
+#pragma unroll 1
+  for (int32_t c = b; c < e; c += kRowChunk) {
+    G g[kRowSteps];
+#pragma unroll
+    for (int k = 0; k < kRowSteps; ++k) g[k] = load(j[k], a[k], c + 64 * k + lane < e);
+    double t[kRowSteps][kSums];
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < kRowSteps; ++k) any = term(a[k], g[k], c + 64 * k + lane < e, t[k]) || any;
+#pragma unroll
+    for (int k = 0; k < kRowSteps; ++k) {  // the last entry again past the row's end
+      const int32_t p = min(c + kRowChunk + 64 * k + lane, e - 1);
+      a[k] = val[p];
+      j[k] = idx[p];
+    }
+    if (__ballot(any) == 0) continue;
+#pragma unroll
+    for (int k = 0; k < kRowSteps; ++k)
+#pragma unroll
+      for (int q = 0; q < kSums; ++q) s_t[q * kRowPitch + 64 * k + lane] = t[k][q];
+    wave_lds_fence();
+    if (lane < kSums) acc = add_in_order(acc, s_t + lane * kRowPitch, min(kRowChunk, e - c));
+    wave_lds_fence();
+  }
+  return acc;
 }
 
 // Inclusive wave64 prefix sum of an int32.

@@ -419,7 +419,7 @@ int64_t plan_reuses();
 // Row activity (gpu_presolve_kernels.cu:18-111) on `stream`: the bounds are
 // first interleaved into a pool block (one 16-byte gather per entry), then
 // k_row_activity_lu runs; enqueue only.
-void row_activity(const int32_t* ptr, const int32_t* idx, const double* val, int32_t m, int32_t n, const double* l,
+void row_activity(const int32_t* ptr, const int32_t* idx, const double* val, int32_t m, int32_t n, int32_t nnz, const double* l,
                   const double* u, double ztol, double* min_fin, double* max_fin, int32_t* neg_inf, int32_t* pos_inf,
                   hipStream_t stream);
 // Exclusive scan of a uint8 mask into out[0..n]; returns the count.

@@ -354,7 +354,7 @@ gp_status gp_row_activity(const gp_csr* A, const double* l, const double* u, dou
     require(A->cols == 0 || (l && u), "null bounds");
     if (stream != nullptr) {
       if (A->rows == 0) return;
-      amd::row_activity(A->row_ptr, A->col_idx, A->val, A->rows, A->cols, l, u, zero_tol, row_min_fin, row_max_fin,
+      amd::row_activity(A->row_ptr, A->col_idx, A->val, A->rows, A->cols, A->nnz, l, u, zero_tol, row_min_fin, row_max_fin,
                         row_min_neg_inf_count, row_max_pos_inf_count, static_cast<hipStream_t>(stream));
       return;
     }
@@ -382,7 +382,7 @@ gp_status gp_row_activity_noalloc(const gp_csr* A, const double* l, const double
     if (A->rows == 0) return;
     require_device();
     hipStream_t s = static_cast<hipStream_t>(stream);
-    amd::check(gpk_row_activity_noalloc(A->row_ptr, A->col_idx, A->val, A->rows, A->cols, l, u, zero_tol,
+    amd::check(gpk_row_activity_noalloc(A->row_ptr, A->col_idx, A->val, A->rows, A->cols, A->nnz, l, u, zero_tol,
                                         row_min_fin, row_max_fin, row_min_neg_inf_count, row_max_pos_inf_count, s),
                "gp_row_activity_noalloc");
     if (s == nullptr) amd::check(hipStreamSynchronize(nullptr), "gp_row_activity_noalloc synchronize");

@@ -404,14 +404,14 @@ void dev_free(void* p, hipStream_t stream) noexcept {
   (void)hipFree(p);
 }
 
-void row_activity(const int32_t* ptr, const int32_t* idx, const double* val, int32_t m, int32_t n, const double* l,
+void row_activity(const int32_t* ptr, const int32_t* idx, const double* val, int32_t m, int32_t n, int32_t nnz, const double* l,
                   const double* u, double ztol, double* min_fin, double* max_fin, int32_t* neg_inf, int32_t* pos_inf,
                   hipStream_t stream) {
   if (m <= 0) return;
   void* lu = dev_alloc(sizeof(double) * 2 * static_cast<size_t>(n > 0 ? n : 1), stream, "packed bounds");
   hipError_t st = gpk_pack_lu(l, u, n, static_cast<double*>(lu), stream);
   if (st == hipSuccess)
-    st = gpk_row_activity_lu(ptr, idx, val, m, static_cast<const double*>(lu), ztol, min_fin, max_fin, neg_inf,
+    st = gpk_row_activity_lu(ptr, idx, val, m, nnz, static_cast<const double*>(lu), ztol, min_fin, max_fin, neg_inf,
                              pos_inf, stream);
   dev_free(lu, stream);  // stream-ordered reuse: later work on `stream` runs after the kernels
   check(st, "row activity");
@@ -722,8 +722,13 @@ void check_lp_arrays(const presolve::LPInfoGpu& lp, const char* who) {
   if (lp.A.rows <= 0 && lp.AT.rows <= 0) return;
   Ctx& c = ctx();
   int32_t* f = c.flags();
-  check(gpk_csr_check(lp.A.rowPtr, lp.A.colVal, lp.A.rows, lp.A.cols, lp.A.nnz, f, c.stream()), "check A");
-  check(gpk_csr_check(lp.AT.rowPtr, lp.AT.colVal, lp.AT.rows, lp.AT.cols, lp.AT.nnz, f + 4, c.stream()), "check AT");
+  const int32_t chunks = gpk_csr_check_chunks(lp.A.nnz);
+  DBuf<int32_t> chunk_row(static_cast<int64_t>(chunks) + gpk_csr_check_chunks(lp.AT.nnz));
+  const auto side = [](const DeviceCsrMatrix& M, int32_t* chunk_rows, int32_t* flags) {
+    return gpk_csr_check_side{M.rowPtr, M.colVal, M.rows, M.cols, M.nnz, 0, chunk_rows, flags};
+  };
+  check(gpk_csr_check(side(lp.A, chunk_row.get(), f), side(lp.AT, chunk_row.get() + chunks, f + 4), c.stream()),
+        "check A and AT");
   int32_t h[8];
   std::memcpy(h, c.read_flags(8), sizeof(h));
   const bool a_again = h[0] == 0 && h[2] == 0 && h[3] != 0, at_again = h[4] == 0 && h[6] == 0 && h[7] != 0;

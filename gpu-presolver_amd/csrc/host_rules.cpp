@@ -84,7 +84,7 @@ void compute_row_activity_summary(double* row_min_fin, double* row_max_fin, std:
                                   const double* u, double zero_tol) {
   amd::AbandonOnThrow abandon_guard;
   if (A_csr.rows == 0) return;
-  row_activity(A_csr.rowPtr, A_csr.colVal, A_csr.nzVal, A_csr.rows, A_csr.cols, l, u, zero_tol, row_min_fin,
+  row_activity(A_csr.rowPtr, A_csr.colVal, A_csr.nzVal, A_csr.rows, A_csr.cols, A_csr.nnz, l, u, zero_tol, row_min_fin,
                row_max_fin, row_min_neg_inf_count, row_max_pos_inf_count, ctx().stream());
 }
 
@@ -228,7 +228,7 @@ void apply_rule_implied_variable_bounds(PresolvePlanGpu& plan, const LPInfoGpu& 
   const gpk_csr A = csr_view(lp.A), AT = csr_view(lp.AT);
   DBuf<double> rmin(m), rmax(m);
   DBuf<int32_t> rni(m), rpi(m);
-  row_activity(A.ptr, A.idx, A.val, m, n, plan.new_l, plan.new_u, prm.zero_tol, rmin, rmax, rni, rpi, s);
+  row_activity(A.ptr, A.idx, A.val, m, n, A.nnz, plan.new_l, plan.new_u, prm.zero_tol, rmin, rmax, rni, rpi, s);
   DBuf<gpk_implied_row> rows(m);
   check(gpk_implied_pack_rows(m, P, stats.row_nnz, rmin, rmax, rni, rpi, rows, s), "implied bounds row records");
   DBuf<double> cl(n), cu(n), vmax(n);

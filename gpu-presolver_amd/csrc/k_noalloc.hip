@@ -55,7 +55,7 @@ hipError_t scratch_ptr(double** out) {
 extern "C" {
 
 hipError_t gpk_row_activity_noalloc(const int32_t* row_ptr, const int32_t* col_idx, const double* val, int32_t m,
-                                    int32_t n, const double* l, const double* u, double ztol, double* min_fin,
+                                    int32_t n, int32_t nnz, const double* l, const double* u, double ztol, double* min_fin,
                                     double* max_fin, int32_t* neg_inf, int32_t* pos_inf, hipStream_t s) {
   if (m <= 0) return hipSuccess;
   if (n < 0 || n > kNoAllocMaxCols) return hipErrorInvalidValue;
@@ -64,7 +64,7 @@ hipError_t gpk_row_activity_noalloc(const int32_t* row_ptr, const int32_t* col_i
   if (e != hipSuccess) return e;
   e = gpk_pack_lu(l, u, n, lu, s);
   if (e != hipSuccess) return e;
-  return gpk_row_activity_lu(row_ptr, col_idx, val, m, lu, ztol, min_fin, max_fin, neg_inf, pos_inf, s);
+  return gpk_row_activity_lu(row_ptr, col_idx, val, m, nnz, lu, ztol, min_fin, max_fin, neg_inf, pos_inf, s);
 }
 
 }  // extern "C"

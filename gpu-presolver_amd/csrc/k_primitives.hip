@@ -102,7 +102,7 @@ __global__ void k_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t
 // them; each thread then adds its own row's terms in CSR order, so every row
 // sum has exactly the sequential rounding of the reference kernel
 // (gpu_presolve_kernels.cu:18-66) for any row length.
-// A row of more than kActLong entries is left to act_long_row: its one
+// A row of more than kLongRow entries is left to act_long_row: its one
 // thread would add thousands of terms from LDS while the other 255 wait, and
 // neighbouring long rows (linking rows come last in most models) would queue
 // in one block.  200 adjacent rows of 3,000 entries behind 80,000 short rows
@@ -110,9 +110,6 @@ __global__ void k_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t
 constexpr int kActRows = kBlock;
 constexpr int kActCap = 2048;
 constexpr int kActItems = kActCap / kBlock;
-// A wave of its own costs a row about 3 us of latency; a 128-entry row costs
-// its tile about as much (2 x 128 LDS reads and adds in one lane).
-constexpr int kActLong = 128;
 
 // (l, u) interleaved, so an activity term needs one 16-byte gather.
 __global__ void k_pack_lu(const double* __restrict__ l, const double* __restrict__ u, int32_t n,
@@ -125,67 +122,30 @@ __global__ void k_pack_lu(const double* __restrict__ l, const double* __restrict
 __device__ inline double act_min(double a, double2 b, bool on) { return on ? (a >= 0.0 ? a * b.x : a * b.y) : 0.0; }
 __device__ inline double act_max(double a, double2 b, bool on) { return on ? (a >= 0.0 ? a * b.y : a * b.x) : 0.0; }
 
-// One of the rows of more than kActLong entries, by a wave.  It loads 256
-// entries at a time (the next 256 on their way while these are summed) and
-// stages both terms in LDS; lane 0 adds the min terms and lane 1 the max terms
-// in CSR order, so the sums are those of one thread.  A term that is not
-// finite is counted and staged as 0: adding +0 to a sum that started at +0
-// leaves it as it is (no such sum is -0).  Bound by the add chain of the row,
-// about 10 us for 3,000 entries.
-constexpr int kActSteps = 4;
-constexpr int kActChunk = 64 * kActSteps;
-constexpr int kActPitch = kActChunk + 2;  // the min and max terms start in different banks
-static_assert(kWaves * 2 * kActPitch <= kActCap + 16, "the long rows' terms fit the tile's LDS");
+// One of the rows of more than kLongRow entries, by a wave; lane 0 adds the min
+// terms and lane 1 the max terms.
+static_assert(kWaves * 2 * kRowPitch <= kActCap + 16, "the long rows' terms fit the tile's LDS");
 
 __device__ __forceinline__ void act_long_row(const int32_t* __restrict__ col_idx, const double* __restrict__ val,
                                              int64_t row, int32_t b, int32_t e, const double2* __restrict__ lu,
                                              double ztol, double* __restrict__ min_fin, double* __restrict__ max_fin,
                                              int32_t* __restrict__ neg_inf, int32_t* __restrict__ pos_inf,
-                                             double* s_mn, double* s_mx) {
-  const int lane = lane_id();
-  double a[kActSteps];
-  int32_t j[kActSteps];
-#pragma unroll
-  for (int k = 0; k < kActSteps; ++k) {
-    const int32_t pc = min(b + 64 * k + lane, e - 1);
-    a[k] = val[pc];
-    j[k] = col_idx[pc];
-  }
-  double acc = 0.0;
+                                             double* s_t) {
   int32_t ni = 0, pi = 0;
-  for (int32_t c = b; c < e; c += kActChunk) {
-    double2 lub[kActSteps];
-    bool on[kActSteps];
-#pragma unroll
-    for (int k = 0; k < kActSteps; ++k) {
-      on[k] = c + 64 * k + lane < e && fabs(a[k]) > ztol;
-      lub[k] = lu[on[k] ? j[k] : 0];
-    }
-    double tn[kActSteps], tx[kActSteps];
-#pragma unroll
-    for (int k = 0; k < kActSteps; ++k) {
-      tn[k] = act_min(a[k], lub[k], on[k]);
-      tx[k] = act_max(a[k], lub[k], on[k]);
-    }
-    // the next chunk's entries (the last entry again past the row's end)
-#pragma unroll
-    for (int k = 0; k < kActSteps; ++k) {
-      const int32_t pc = min(c + kActChunk + 64 * k + lane, e - 1);
-      a[k] = val[pc];
-      j[k] = col_idx[pc];
-    }
-#pragma unroll
-    for (int k = 0; k < kActSteps; ++k) {
-      const bool fn = isfinite(tn[k]), fx = isfinite(tx[k]);
-      ni += static_cast<int32_t>(__popcll(__ballot(!fn && tn[k] < 0.0)));
-      pi += static_cast<int32_t>(__popcll(__ballot(!fx && tx[k] > 0.0)));
-      s_mn[64 * k + lane] = fn ? tn[k] : 0.0;
-      s_mx[64 * k + lane] = fx ? tx[k] : 0.0;
-    }
-    wave_lds_fence();
-    if (lane < 2) acc = add_in_order(acc, lane == 0 ? s_mn : s_mx, min(kActChunk, e - c));
-    wave_lds_fence();
-  }
+  const double acc = wave_row_sums<2, double2>(
+      col_idx, val, b, e, s_t,
+      [&](int32_t j, double a, bool in) { return lu[in && fabs(a) > ztol ? j : 0]; },
+      [&](double a, double2 lub, bool in, double* t) {
+        const bool on = in && fabs(a) > ztol;
+        const double tn = act_min(a, lub, on), tx = act_max(a, lub, on);
+        const bool fn = isfinite(tn), fx = isfinite(tx);
+        ni += static_cast<int32_t>(__popcll(__ballot(!fn && tn < 0.0)));
+        pi += static_cast<int32_t>(__popcll(__ballot(!fx && tx > 0.0)));
+        t[0] = fn ? tn : 0.0;
+        t[1] = fx ? tx : 0.0;
+        return true;
+      });
+  const int lane = lane_id();
   if (lane == 0) {
     min_fin[row] = acc;
     neg_inf[row] = ni;
@@ -211,9 +171,9 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
   __shared__ __align__(16) double s_t[kActCap + 16];
   __shared__ int32_t s_next;
   if (static_cast<int32_t>(blockIdx.x) >= tiles) {
-    double* s_mn = s_t + (threadIdx.x >> 6) * 2 * kActPitch;
-    wave_long_rows(row_ptr, m, kActLong, tiles, [&](int64_t row, int32_t b, int32_t e) {
-      act_long_row(col_idx, val, row, b, e, lu, ztol, min_fin, max_fin, neg_inf, pos_inf, s_mn, s_mn + kActPitch);
+    double* s_row = s_t + (threadIdx.x >> 6) * 2 * kRowPitch;
+    wave_long_rows(row_ptr, m, kLongRow, tiles, [&](int64_t row, int32_t b, int32_t e) {
+      act_long_row(col_idx, val, row, b, e, lu, ztol, min_fin, max_fin, neg_inf, pos_inf, s_row);
     });
     return;
   }
@@ -223,7 +183,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
   const int32_t seg_b = row_ptr[r0], seg_e = row_ptr[r0 + rows];
   const int32_t my_b = row_ptr[r0 + min(tid, rows)];
   int32_t my_e = row_ptr[r0 + min(tid + 1, rows)];
-  const bool is_long = my_e - my_b > kActLong;
+  const bool is_long = my_e - my_b > kLongRow;
   if (is_long) my_e = my_b;  // no entry of it is added here
   const bool any_long = __syncthreads_or(is_long) != 0;
   double mn = 0.0, mx = 0.0;
@@ -1085,7 +1045,9 @@ constexpr int kRsWaves = kBlock / 64;
 // (256 x tiles words) instead of waiting for a scan launch.
 constexpr int kRsHistTilesMax = 64;
 
-template <class K>
+// kTileMajor: one tile's 256 counts together (for k_radix_scatter from the raw
+// histogram), else one digit's tiles together (for the scan).
+template <class K, bool kTileMajor>
 __global__ __launch_bounds__(kBlock) void k_radix_hist(const K* __restrict__ keys, int32_t n, int shift,
                                                       int32_t tiles, int32_t* __restrict__ hist) {
   __shared__ int32_t s_h[256];
@@ -1097,12 +1059,15 @@ __global__ __launch_bounds__(kBlock) void k_radix_hist(const K* __restrict__ key
     if (e < n) atomicAdd(&s_h[static_cast<int>((keys[e] >> shift) & 255u)], 1);
   }
   __syncthreads();
-  hist[static_cast<int64_t>(threadIdx.x) * tiles + blockIdx.x] = s_h[threadIdx.x];
+  hist[kTileMajor ? static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x
+                  : static_cast<int64_t>(threadIdx.x) * tiles + blockIdx.x] = s_h[threadIdx.x];
 }
 
-// kFromHist: offs is the raw histogram (digit-major, tiles per digit) and
-// every block derives its own digit offsets from it (for few tiles, this
-// saves the separate scan launch); otherwise offs is the scanned histogram.
+// kFromHist: offs is the raw histogram (tile-major) and every block derives its
+// own digit offsets from it, 16 tiles' loads on their way at a time (for few
+// tiles, this saves the separate scan launch; one load after the other took
+// 18 us at 59 tiles, 11 now); otherwise offs is the scanned histogram
+// (digit-major).
 template <class K, bool kFromHist>
 __global__ __launch_bounds__(kBlock) void k_radix_scatter(const K* __restrict__ kin, const int32_t* __restrict__ vin,
                                                          K* __restrict__ kout, int32_t* __restrict__ vout,
@@ -1119,11 +1084,18 @@ __global__ __launch_bounds__(kBlock) void k_radix_scatter(const K* __restrict__ 
   for (int i = tid; i < kRsWaves * 256; i += kBlock) s_cnt[i >> 8][i & 255] = 0;
   if (kFromHist) {
     static_assert(kBlock == 256, "one thread per digit");
+    constexpr int U = 16;
     int32_t total = 0, before = 0;
-    for (int32_t t = 0; t < tiles; ++t) {
-      const int32_t h = offs[static_cast<int64_t>(tid) * tiles + t];
-      total += h;
-      before += t < static_cast<int32_t>(blockIdx.x) ? h : 0;
+#pragma unroll 1
+    for (int32_t t0 = 0; t0 < tiles; t0 += U) {
+      int32_t h[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) h[k] = t0 + k < tiles ? offs[(t0 + k) * 256 + tid] : 0;
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        total += h[k];
+        before += t0 + k < static_cast<int32_t>(blockIdx.x) ? h[k] : 0;
+      }
     }
     const int32_t inc = wave_inclusive_sum(total);
     if ((tid & 63) == 63) s_wsum[tid >> 6] = inc;
@@ -1247,53 +1219,95 @@ __global__ void k_transpose_gather(const int32_t* __restrict__ perm, const gpk_r
   at_val[k] = __hiloint2double(w.w, w.z);
 }
 
-// CSR checks over tiles of 256 rows with one thread per entry, so a long
-// row (a popular column of AT) is shared by the whole tile instead of walked
-// by one thread.  The tile's row pointers go to LDS; every entry finds its
-// row by a binary search of them and is compared with the entry before it in
-// the same row.  kFull: flags[0] bad row pointers (not monotone, not from 0
-// to nnz: the tile then reads no entry), flags[1] a column outside [0, cols),
-// flags[2] two equal neighbours, flags[3] a descending pair.  Otherwise the
-// pointers are trusted and only a descending pair is flagged, in flags[0].
-template <bool kFull>
-__global__ __launch_bounds__(kBlock) void k_csr_tiles(const int32_t* __restrict__ ptr,
-                                                      const int32_t* __restrict__ idx, int32_t rows, int32_t cols,
-                                                      int32_t nnz, int32_t* flags) {
+// CSR checks.  The row pointers are checked first, one row a thread
+// (flags[0]: not monotone, not from 0 to nnz), and leave the chunk rows of the
+// matrix (its last row past the last chunk); then chunks of 2048 entries are
+// checked, 8 a thread, whatever the rows (tiles of 256 rows, each entry
+// finding its row by bisection, took 1.35 ms on 200 adjacent rows of 3,000
+// entries, and 98 us for A and AT of the 1M x 1.5M LP; 10 and 37 us for both
+// launches by chunks).  A
+// chunk marks the first entry of each of its rows in a bitmap; every other
+// entry is compared with the one before it: flags[1] a column outside
+// [0, cols), flags[2] two equal neighbours, flags[3] a descending pair.  No
+// entry is read of a matrix whose pointers are bad.
+constexpr int kChkItems = 8;
+constexpr int kChkChunk = kBlock * kChkItems;
+
+__global__ __launch_bounds__(kBlock) void k_csr_check_ptr(gpk_csr_check_side a, gpk_csr_check_side t,
+                                                          int32_t blocks_a) {
+  const bool first = static_cast<int32_t>(blockIdx.x) < blocks_a;
+  const gpk_csr_check_side& s = first ? a : t;
+  const int64_t i = static_cast<int64_t>(first ? blockIdx.x : blockIdx.x - blocks_a) * kBlock + threadIdx.x;
+  if (i >= s.rows) return;
+  const int32_t b = s.ptr[i], e = s.ptr[i + 1];
+  if ((i == 0 && b != 0) || (i == s.rows - 1 && e != s.nnz) || b > e || b < 0 || e > s.nnz) {
+    wave_set_flag(s.flags);
+    return;
+  }
+#pragma unroll 1
+  for (int64_t q = (static_cast<int64_t>(b) + kChkChunk - 1) / kChkChunk; q * kChkChunk < e; ++q)
+    s.chunk_row[q] = static_cast<int32_t>(i);
+}
+
+__global__ __launch_bounds__(kBlock) void k_csr_check_entries(gpk_csr_check_side a, gpk_csr_check_side t,
+                                                              int32_t chunks_a, int32_t chunks_t) {
+  __shared__ uint32_t s_head[kChkChunk / 32];
+  const int32_t blk = static_cast<int32_t>(blockIdx.x);
+  const bool first = blk < chunks_a;
+  const gpk_csr_check_side& s = first ? a : t;
+  const int32_t q = first ? blk : blk - chunks_a, chunks = first ? chunks_a : chunks_t;
+  const int tid = threadIdx.x;
+  if (*s.flags != 0) return;  // the pointers are bad (set by the launch before)
+  const int32_t c0 = q * kChkChunk, c1 = min(s.nnz - c0, kChkChunk);
+  int32_t j[kChkItems];
+#pragma unroll
+  for (int k = 0; k < kChkItems; ++k) j[k] = s.idx[c0 + min(k * kBlock + tid, c1 - 1)];
+  const int32_t edge = s.idx[c0 > 0 ? c0 - 1 : 0];
+  const int32_t r_lo = s.chunk_row[q], r_hi = q + 1 < chunks ? s.chunk_row[q + 1] : s.rows - 1;
+  if (tid < kChkChunk / 32) s_head[tid] = 0;
+  __syncthreads();
+#pragma unroll 1
+  for (int64_t r = r_lo + tid; r <= r_hi; r += kBlock) {
+    const int32_t b = s.ptr[r] - c0;
+    if (b >= 0 && b < c1) atomicOr(&s_head[b >> 5], 1u << (b & 31));  // empty rows mark their successor's
+  }
+  __syncthreads();
+  bool range = false, equal = false, desc = false;
+#pragma unroll
+  for (int k = 0; k < kChkItems; ++k) {
+    const int p = k * kBlock + tid;
+    // The entry before: the lane below, or for a wave's first lane from memory.
+    int32_t before = __shfl_up(j[k], 1, 64);
+    if (lane_id() == 0 && p < c1) before = p == 0 ? edge : s.idx[c0 + p - 1];
+    if (p >= c1) continue;
+    range = range || j[k] < 0 || j[k] >= s.cols;
+    if (((s_head[p >> 5] >> (p & 31)) & 1u) == 0) {
+      equal = equal || j[k] == before;
+      desc = desc || j[k] < before;
+    }
+  }
+  if (range) wave_set_flag(s.flags + 1);
+  if (equal) wave_set_flag(s.flags + 2);
+  if (desc) wave_set_flag(s.flags + 3);
+}
+
+// Rows sorted by column, over tiles of 256 rows with one thread per entry (the
+// pointers are trusted): every entry finds its row by a bisection of the tile's
+// row pointers in LDS and is compared with the entry before it in the same
+// row.
+__global__ __launch_bounds__(kBlock) void k_csr_unsorted(const int32_t* __restrict__ ptr,
+                                                         const int32_t* __restrict__ idx, int32_t rows,
+                                                         int32_t* flag) {
   __shared__ int32_t s_ptr[kBlock + 1];
-  __shared__ int32_t s_bad;
   const int32_t r0 = blockIdx.x * kBlock;
   const int nr = min(kBlock, rows - r0);
   const int tid = threadIdx.x;
-  if (tid == 0) s_bad = 0;
   for (int t = tid; t <= nr; t += kBlock) s_ptr[t] = ptr[r0 + t];
   __syncthreads();
-  if (kFull && tid < nr) {
-    const int32_t b = s_ptr[tid], e = s_ptr[tid + 1];
-    if ((r0 + tid == 0 && b != 0) || (r0 + tid == rows - 1 && e != nnz) || b > e || b < 0 || e > nnz) s_bad = 1;
-  }
-  __syncthreads();
-  if (s_bad != 0) {
-    if (tid == 0) __hip_atomic_store(flags, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return;
-  }
-  bool range = false, equal = false, desc = false;
-  for (int32_t p = s_ptr[0] + tid; p < s_ptr[nr]; p += kBlock) {
-    const int row = find_row(s_ptr, nr, p);
-    const int32_t j = idx[p];
-    if (kFull) range = range || j < 0 || j >= cols;
-    if (p > s_ptr[row]) {
-      const int32_t q = idx[p - 1];
-      equal = equal || j == q;
-      desc = desc || j < q;
-    }
-  }
-  if (kFull) {
-    if (range) wave_set_flag(flags + 1);
-    if (equal) wave_set_flag(flags + 2);
-    if (desc) wave_set_flag(flags + 3);
-  } else if (desc) {
-    wave_set_flag(flags);
-  }
+  bool desc = false;
+  for (int32_t p = s_ptr[0] + tid; p < s_ptr[nr]; p += kBlock)
+    if (p > s_ptr[find_row(s_ptr, nr, p)]) desc = desc || idx[p] < idx[p - 1];
+  if (desc) wave_set_flag(flag);
 }
 
 // Input check of a CSR matrix, one row per thread (for matrices whose rows
@@ -1450,11 +1464,12 @@ hipError_t radix_impl(K* keys, int32_t* vals, K* keys_alt, int32_t* vals_alt, in
   int32_t* vb = vals_alt;
   for (int pass = 0; pass < passes; ++pass) {
     const int shift = pass * 8;
-    hipLaunchKernelGGL(k_radix_hist<K>, dim3(tiles), dim3(kBlock), 0, s, ka, n, shift, tiles, hist);
     if (from_hist) {
+      hipLaunchKernelGGL((k_radix_hist<K, true>), dim3(tiles), dim3(kBlock), 0, s, ka, n, shift, tiles, hist);
       hipLaunchKernelGGL((k_radix_scatter<K, true>), dim3(tiles), dim3(kBlock), 0, s, ka, va, kb, vb, n, shift,
                          tiles, static_cast<const int32_t*>(hist));
     } else {
+      hipLaunchKernelGGL((k_radix_hist<K, false>), dim3(tiles), dim3(kBlock), 0, s, ka, n, shift, tiles, hist);
       hipError_t e = scan_impl<int32_t>(hist, hist, static_cast<int64_t>(256) * tiles, scan_scratch, s);
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL((k_radix_scatter<K, false>), dim3(tiles), dim3(kBlock), 0, s, ka, va, kb, vb, n, shift,
@@ -1615,14 +1630,14 @@ hipError_t gpk_pack_lu(const double* l, const double* u, int32_t n, double* lu, 
 }
 
 hipError_t gpk_row_activity_lu(const int32_t* row_ptr, const int32_t* col_idx, const double* val, int32_t m,
-                               const double* lu, double ztol, double* min_fin, double* max_fin, int32_t* neg_inf,
+                               int32_t nnz, const double* lu, double ztol, double* min_fin, double* max_fin, int32_t* neg_inf,
                                int32_t* pos_inf, hipStream_t s) {
   if (m <= 0) return hipSuccess;
   // The tiles, then the blocks that look for long rows: on a matrix without
   // one those end while the last tiles run.  (A launch of their own cost 2.6
   // us more at 1M rows, and in front of the tiles they cost 1 us.)
   const unsigned tiles = grid_for(m, kActRows);
-  hipLaunchKernelGGL(k_row_activity_lu, dim3(tiles + long_row_blocks(m)), dim3(kBlock), 0, s, row_ptr, col_idx, val, m,
+  hipLaunchKernelGGL(k_row_activity_lu, dim3(tiles + long_row_blocks(m, nnz)), dim3(kBlock), 0, s, row_ptr, col_idx, val, m,
                      reinterpret_cast<const double2*>(lu), ztol, min_fin, max_fin, neg_inf, pos_inf,
                      static_cast<int32_t>(tiles));
   return hipGetLastError();
@@ -1719,11 +1734,12 @@ hipError_t gpk_transpose_sort(const int32_t* col, int32_t nnz, int32_t key_bits,
   int32_t* vout = va;
   for (int pass = 0; pass < passes; ++pass) {
     const int shift = pass * 8;
-    hipLaunchKernelGGL(k_radix_hist<uint32_t>, dim3(tiles), dim3(kBlock), 0, s, kin, nnz, shift, tiles, hist);
     if (from_hist) {
+      hipLaunchKernelGGL((k_radix_hist<uint32_t, true>), dim3(tiles), dim3(kBlock), 0, s, kin, nnz, shift, tiles, hist);
       hipLaunchKernelGGL((k_radix_scatter<uint32_t, true>), dim3(tiles), dim3(kBlock), 0, s, kin, vin, kout, vout, nnz,
                          shift, tiles, static_cast<const int32_t*>(hist));
     } else {
+      hipLaunchKernelGGL((k_radix_hist<uint32_t, false>), dim3(tiles), dim3(kBlock), 0, s, kin, nnz, shift, tiles, hist);
       hipError_t e = scan_impl<int32_t>(hist, hist, static_cast<int64_t>(256) * tiles, scan_scratch, s);
       if (e != hipSuccess) return e;
       hipLaunchKernelGGL((k_radix_scatter<uint32_t, false>), dim3(tiles), dim3(kBlock), 0, s, kin, vin, kout, vout,
@@ -1760,14 +1776,20 @@ hipError_t gpk_transpose_gather(const int32_t* perm, const gpk_row_val* rv, int3
 
 hipError_t gpk_rows_unsorted(const int32_t* ptr, const int32_t* idx, int32_t rows, int32_t* flag, hipStream_t s) {
   if (rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_csr_tiles<false>, dim3(grid_for(rows)), dim3(kBlock), 0, s, ptr, idx, rows, 0, 0, flag);
+  hipLaunchKernelGGL(k_csr_unsorted, dim3(grid_for(rows)), dim3(kBlock), 0, s, ptr, idx, rows, flag);
   return hipGetLastError();
 }
 
-hipError_t gpk_csr_check(const int32_t* ptr, const int32_t* idx, int32_t rows, int32_t cols, int32_t nnz,
-                         int32_t* flags, hipStream_t s) {
-  if (rows <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_csr_tiles<true>, dim3(grid_for(rows)), dim3(kBlock), 0, s, ptr, idx, rows, cols, nnz, flags);
+int32_t gpk_csr_check_chunks(int32_t nnz) { return nnz > 0 ? static_cast<int32_t>(grid_for(nnz, kChkChunk)) : 0; }
+
+hipError_t gpk_csr_check(gpk_csr_check_side a, gpk_csr_check_side t, hipStream_t s) {
+  const int32_t ba = a.rows > 0 ? static_cast<int32_t>(grid_for(a.rows)) : 0;
+  const int32_t bt = t.rows > 0 ? static_cast<int32_t>(grid_for(t.rows)) : 0;
+  if (ba + bt == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_csr_check_ptr, dim3(ba + bt), dim3(kBlock), 0, s, a, t, ba);
+  const int32_t ca = ba > 0 ? gpk_csr_check_chunks(a.nnz) : 0, ct = bt > 0 ? gpk_csr_check_chunks(t.nnz) : 0;
+  if (ca + ct > 0)
+    hipLaunchKernelGGL(k_csr_check_entries, dim3(ca + ct), dim3(kBlock), 0, s, a, t, ca, ct);
   return hipGetLastError();
 }
 

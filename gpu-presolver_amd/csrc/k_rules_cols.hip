@@ -164,16 +164,61 @@ __global__ void k_cs_precheck(int32_t n, int32_t m, gpk_plan p, const uint8_t* m
 // The row is walked U entries at a time: their columns and values load
 // together, then the columns' keep flags and bounds, and the terms are then
 // added in CSR order (the sums are those of the entry-by-entry loop).
-__global__ __launch_bounds__(kBlock) void k_cs_activity_cache(gpk_csr A, gpk_plan p, const uint8_t* needed,
+__global__ __launch_bounds__(kBlock) void k_cs_activity_cache(int32_t row_blocks, gpk_csr A, gpk_plan p,
+                                                              const uint8_t* needed,
                                                               gpk_row_cache rc) {
+  if (static_cast<int32_t>(blockIdx.x) >= row_blocks) {
+    __shared__ __align__(16) double s_terms[kWaves][2 * kRowPitch];
+    double* s_t = s_terms[threadIdx.x >> 6];
+    struct Col {
+      double l, u;
+      bool kept;
+    };
+    wave_long_rows(A.ptr, A.rows, kLongRow, row_blocks, [&](int64_t i, int32_t b, int32_t e) {
+      if (!needed[i]) return;
+      int32_t mn = 0, mp = 0, xn = 0, xp = 0;
+      bool invalid = false;
+      double sum = 0.0;
+      if (p.keep_row[i])
+        sum = wave_row_sums<2, Col>(
+            A.idx, A.val, b, e, s_t,
+            [&](int32_t j, double, bool in) { return Col{p.l[j], p.u[j], in && p.keep_col[j] != 0}; },
+            [&](double a, const Col& c, bool, double* t) {
+              const double tmin = a >= 0.0 ? a * c.l : a * c.u;
+              const double tmax = a >= 0.0 ? a * c.u : a * c.l;
+              const bool bad = isnan(tmin) || isnan(tmax), on = c.kept && !bad;
+              const bool imin = on && isinf(tmin), imax = on && isinf(tmax);
+              invalid = invalid || __ballot(c.kept && bad) != 0;
+              mn += static_cast<int32_t>(__popcll(__ballot(imin && tmin < 0.0)));
+              mp += static_cast<int32_t>(__popcll(__ballot(imin && tmin > 0.0)));
+              xn += static_cast<int32_t>(__popcll(__ballot(imax && tmax < 0.0)));
+              xp += static_cast<int32_t>(__popcll(__ballot(imax && tmax > 0.0)));
+              t[0] = on && !imin ? tmin : 0.0;
+              t[1] = on && !imax ? tmax : 0.0;
+              return on;
+            });
+      if (lane_id() == 0) {
+        rc.fmin[i] = sum;
+        rc.mn[i] = mn;
+        rc.mp[i] = mp;
+        rc.xn[i] = xn;
+        rc.xp[i] = xp;
+        rc.invalid[i] = invalid ? 1 : 0;
+      } else if (lane_id() == 1) {
+        rc.fmax[i] = sum;
+      }
+    });
+    return;
+  }
   constexpr int U = 8;
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= A.rows || !needed[i]) return;
+  const int32_t qb = A.ptr[i], qe = A.ptr[i + 1];
+  if (qe - qb > kLongRow) return;
   double fmn = 0.0, fmx = 0.0;
   int32_t mn = 0, mp = 0, xn = 0, xp = 0;
   bool invalid = false;
   if (p.keep_row[i]) {
-    const int32_t qb = A.ptr[i], qe = A.ptr[i + 1];
     for (int32_t q0 = qb; q0 < qe; q0 += U) {
       int32_t cc[U];
       double av[U];
@@ -929,28 +974,85 @@ __device__ inline bool dbl_is_delta(const gpk_dbl_cols& cols, int32_t i, int32_t
   return cols.is_elim[j] && cols.row_of[j] != i && fabs(a) > zt;
 }
 
-__global__ void k_dbl_delta_count(gpk_csr A, gpk_plan p, gpk_dbl_cols cols, double zt, int32_t* counts) {
+__global__ __launch_bounds__(kBlock) void k_dbl_delta_count(int32_t row_blocks, gpk_csr A, gpk_plan p,
+                                                            gpk_dbl_cols cols, double zt, int32_t* counts) {
+  if (static_cast<int32_t>(blockIdx.x) >= row_blocks) {
+    wave_long_rows(A.ptr, A.rows, kLongRow, row_blocks, [&](int64_t i, int32_t b, int32_t e) {
+      int32_t cnt = 0;
+      if (p.keep_row[i])
+#pragma unroll 4
+        for (int32_t q = b + lane_id(); q < e; q += 64)
+          cnt += dbl_is_delta(cols, static_cast<int32_t>(i), A.idx[q], A.val[q], zt) ? 1 : 0;
+      cnt = __shfl(wave_inclusive_sum(cnt), 63, 64);
+      if (lane_id() == 0) counts[i] = cnt;
+    });
+    return;
+  }
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= A.rows) return;
+  const int32_t b = A.ptr[i], e = A.ptr[i + 1];
+  if (e - b > kLongRow) return;
   int32_t cnt = 0;
   if (p.keep_row[i])
-    for (int32_t q = A.ptr[i]; q < A.ptr[i + 1]; ++q) cnt += dbl_is_delta(cols, i, A.idx[q], A.val[q], zt) ? 1 : 0;
+    for (int32_t q = b; q < e; ++q) cnt += dbl_is_delta(cols, i, A.idx[q], A.val[q], zt) ? 1 : 0;
   counts[i] = cnt;
 }
 
 // Row shift of one batch: fixed keep columns first, then substituted columns,
 // each in CSR order along the row; applied to every row.
-__global__ void k_dbl_shift(gpk_csr A, gpk_plan p, gpk_dbl_cols cols, double zt, int32_t include_subst) {
+__global__ __launch_bounds__(kBlock) void k_dbl_shift(int32_t row_blocks, gpk_csr A, gpk_plan p, gpk_dbl_cols cols,
+                                                      double zt, int32_t include_subst) {
+  if (static_cast<int32_t>(blockIdx.x) >= row_blocks) {
+    __shared__ __align__(16) double s_terms[kWaves][2 * kRowPitch];
+    wave_long_rows(A.ptr, A.rows, kLongRow, row_blocks, [&](int64_t i, int32_t b, int32_t e) {
+      double s = 0.0;
+      if (p.keep_row[i]) {
+        // The fixed columns' terms, then in a second walk (where the row has
+        // any) the substituted ones', added to that sum one by one.
+        bool subst = false;
+        s = wave_row_sums<1, double2>(
+            A.idx, A.val, b, e, s_terms[threadIdx.x >> 6],
+            [&](int32_t j, double a, bool in) {
+              subst = subst || (in && dbl_is_delta(cols, static_cast<int32_t>(i), j, a, zt));
+              const bool on = in && cols.is_fixed_keep[j] && fabs(a) > zt;
+              return make_double2(on ? 1.0 : 0.0, on ? cols.fixed_val_of[j] : 0.0);
+            },
+            [&](double a, double2 v, bool, double* t) {
+              t[0] = v.x != 0.0 ? a * v.y : 0.0;
+              return v.x != 0.0;
+            });
+        if (include_subst && __ballot(subst) != 0) {
+          for (int32_t c = b; c < e; c += 64) {
+            const int32_t q = min(c + lane_id(), e - 1), j = A.idx[q];
+            const double a = A.val[q];
+            const bool on = c + lane_id() < e && dbl_is_delta(cols, static_cast<int32_t>(i), j, a, zt);
+            const double v = on ? a * cols.beta_of[j] : 0.0;
+            for (uint64_t m = __ballot(on); m; m &= m - 1) {
+              const double x = __shfl(v, __ffsll(static_cast<unsigned long long>(m)) - 1, 64);
+              if (lane_id() == 0) s += x;
+            }
+          }
+        }
+      }
+      if (lane_id() == 0) {
+        p.AL[i] -= s;
+        p.AU[i] -= s;
+      }
+    });
+    return;
+  }
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= A.rows) return;
+  const int32_t b = A.ptr[i], e = A.ptr[i + 1];
+  if (e - b > kLongRow) return;
   double s = 0.0;
   if (p.keep_row[i]) {
-    for (int32_t q = A.ptr[i]; q < A.ptr[i + 1]; ++q) {
+    for (int32_t q = b; q < e; ++q) {
       const int32_t j = A.idx[q];
       if (cols.is_fixed_keep[j] && fabs(A.val[q]) > zt) s += A.val[q] * cols.fixed_val_of[j];
     }
     if (include_subst)
-      for (int32_t q = A.ptr[i]; q < A.ptr[i + 1]; ++q) {
+      for (int32_t q = b; q < e; ++q) {
         const int32_t j = A.idx[q];
         if (dbl_is_delta(cols, i, j, A.val[q], zt)) s += A.val[q] * cols.beta_of[j];
       }
@@ -959,41 +1061,92 @@ __global__ void k_dbl_shift(gpk_csr A, gpk_plan p, gpk_dbl_cols cols, double zt,
   p.AU[i] -= s;
 }
 
-// Delta entries (keep column, alpha * a) of each live row, sorted by column.
-__global__ void k_dbl_delta_fill(gpk_csr A, gpk_plan p, gpk_dbl_cols cols, double zt, const int32_t* dptr,
-                                 int32_t* dcol, double* dval) {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= A.rows || !p.keep_row[i]) return;
-  const int32_t b = dptr[i];
-  int32_t o = b;
-  for (int32_t q = A.ptr[i]; q < A.ptr[i + 1]; ++q) {
+// Delta entries (keep column, alpha * a) of each live row, sorted by column
+// (equal columns in CSR order).  A long row's wave packs them into LDS and
+// places each by its rank; more than kDblLds of them go in order of insertion,
+// as in the thread's path.
+constexpr int kDblLds = 512;
+
+__device__ inline void dbl_insert(int32_t b, int32_t o, int32_t kc, double v, int32_t* dcol, double* dval) {
+  int32_t w = o - 1;
+  while (w >= b && dcol[w] > kc) {
+    dcol[w + 1] = dcol[w];
+    dval[w + 1] = dval[w];
+    --w;
+  }
+  dcol[w + 1] = kc;
+  dval[w + 1] = v;
+}
+
+__device__ inline void dbl_fill_serial(const gpk_csr& A, const gpk_dbl_cols& cols, double zt, int32_t i, int32_t b,
+                                       int32_t e, int32_t o0, int32_t* dcol, double* dval) {
+  int32_t o = o0;
+  for (int32_t q = b; q < e; ++q) {
     const int32_t j = A.idx[q];
     if (!dbl_is_delta(cols, i, j, A.val[q], zt)) continue;
-    const int32_t kc = cols.keep_of[j];
-    const double v = cols.alpha_of[j] * A.val[q];
-    int32_t w = o - 1;
-    while (w >= b && dcol[w] > kc) {
-      dcol[w + 1] = dcol[w];
-      dval[w + 1] = dval[w];
-      --w;
-    }
-    dcol[w + 1] = kc;
-    dval[w + 1] = v;
+    dbl_insert(o0, o, cols.keep_of[j], cols.alpha_of[j] * A.val[q], dcol, dval);
     ++o;
   }
 }
 
+__global__ __launch_bounds__(kBlock) void k_dbl_delta_fill(int32_t row_blocks, gpk_csr A, gpk_plan p,
+                                                           gpk_dbl_cols cols, double zt, const int32_t* dptr,
+                                                           int32_t* dcol, double* dval) {
+  if (static_cast<int32_t>(blockIdx.x) >= row_blocks) {
+    __shared__ int32_t s_col[kWaves][kDblLds];
+    __shared__ double s_val[kWaves][kDblLds];
+    int32_t* sc = s_col[threadIdx.x >> 6];
+    double* sv = s_val[threadIdx.x >> 6];
+    const int lane = lane_id();
+    wave_long_rows(A.ptr, A.rows, kLongRow, row_blocks, [&](int64_t i, int32_t b, int32_t e) {
+      if (!p.keep_row[i]) return;
+      const int32_t o0 = dptr[i], total = dptr[i + 1] - o0;
+      if (total == 0) return;
+      if (total > kDblLds) {
+        if (lane == 0) dbl_fill_serial(A, cols, zt, static_cast<int32_t>(i), b, e, o0, dcol, dval);
+        return;
+      }
+      int32_t n = 0;
+#pragma unroll 1
+      for (int32_t c = b; c < e; c += 64) {
+        const int32_t q = min(c + lane, e - 1), j = A.idx[q];
+        const double a = A.val[q];
+        const bool on = c + lane < e && dbl_is_delta(cols, static_cast<int32_t>(i), j, a, zt);
+        const uint64_t m = __ballot(on);
+        if (on) {
+          const int at = n + static_cast<int>(__popcll(m & lanemask_lt(lane)));
+          if (at < kDblLds) {
+            sc[at] = cols.keep_of[j];
+            sv[at] = cols.alpha_of[j] * a;
+          }
+        }
+        n += static_cast<int>(__popcll(m));
+      }
+      wave_lds_fence();
+      for (int32_t t = lane; t < total; t += 64) {
+        const int32_t kc = sc[t];
+        int32_t rank = 0;
+#pragma unroll 1
+        for (int32_t k = 0; k < total; ++k) rank += sc[k] < kc || (sc[k] == kc && k < t) ? 1 : 0;
+        dcol[o0 + rank] = kc;
+        dval[o0 + rank] = sv[t];
+      }
+      wave_lds_fence();
+    });
+    return;
+  }
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= A.rows || !p.keep_row[i]) return;
+  const int32_t b = A.ptr[i], e = A.ptr[i + 1];
+  if (e - b > kLongRow) return;
+  dbl_fill_serial(A, cols, zt, i, b, e, dptr[i], dcol, dval);
+}
+
 // Sorted merge of a row with its deltas (rule_doubleton_equations.cu:1129-1218);
 // count mode when out_idx is null.
-__global__ void k_dbl_merge(gpk_csr A, const int32_t* dptr, const int32_t* dcol, const double* dval, double zt,
-                            const int32_t* out_ptr, int32_t* counts, int32_t* out_idx, double* out_val) {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= A.rows) return;
-  int32_t q = A.ptr[i];
-  const int32_t qe = A.ptr[i + 1];
-  int32_t r = dptr[i];
-  const int32_t re = dptr[i + 1];
-  int32_t w = out_idx ? out_ptr[i] : 0;
+__device__ inline void dbl_merge_serial(const gpk_csr& A, int32_t q, int32_t qe, int32_t r, int32_t re,
+                                        const int32_t* dcol, const double* dval, double zt, int32_t w, int32_t* count,
+                                        int32_t* out_idx, double* out_val) {
   int32_t cnt = 0;
   while (q < qe || r < re) {
     const int32_t sc = q < qe ? A.idx[q] : INT_MAX;
@@ -1011,9 +1164,134 @@ __global__ void k_dbl_merge(gpk_csr A, const int32_t* dptr, const int32_t* dcol,
       ++cnt;
     }
   }
-  if (!out_idx) counts[i] = cnt;
+  if (!out_idx) *count = cnt;
 }
 
+// First position in a[lo, hi) (ascending) whose entry is not below c.
+__device__ inline int32_t lower_bound(const int32_t* __restrict__ a, int32_t lo, int32_t hi, int32_t c) {
+  while (lo < hi) {
+    const int32_t mid = lo + (hi - lo) / 2;
+    if (a[mid] < c) lo = mid + 1; else hi = mid;
+  }
+  return lo;
+}
+
+// A long row's merge by a wave: its own entries and the columns that only the
+// deltas have are each formed by one lane (the entry, then its deltas in
+// order), which finds its partner by bisection; an output's place is the kept
+// ones of its own kind before it plus those of the other kind below its
+// column.  The kept bits of the row (up to kDblRowMax entries) and the kept
+// counts along the deltas (up to kDblLds) are in LDS; longer ones, and rows
+// that are not ascending, are merged by one lane as in the thread's path.
+constexpr int kDblRowMax = 16384;
+
+__device__ __forceinline__ void dbl_merge_wave(const gpk_csr& A, int32_t qb, int32_t qe, int32_t rb, int32_t re,
+                                               const int32_t* dcol, const double* dval, double zt, int32_t w,
+                                               int32_t* count, int32_t* out_idx, double* out_val, uint64_t* s_bits,
+                                               int32_t* s_pre, int32_t* s_new) {
+  const int lane = lane_id();
+  const uint64_t below = lanemask_lt(lane);
+  bool ascending = true;
+#pragma unroll 1
+  for (int32_t q = qb + 1 + lane; q < qe; q += 64) ascending = ascending && A.idx[q - 1] < A.idx[q];
+  if (qe - qb > kDblRowMax || re - rb > kDblLds || __ballot(!ascending) != 0) {
+    if (lane == 0) dbl_merge_serial(A, qb, qe, rb, re, dcol, dval, zt, w, count, out_idx, out_val);
+    return;
+  }
+  // The columns of the deltas that the row does not have.
+  int32_t fresh = 0;
+#pragma unroll 1
+  for (int32_t r0 = rb; r0 < re; r0 += 64) {
+    const int32_t r = r0 + lane;
+    bool keep = false;
+    if (r < re) {
+      const int32_t c = dcol[r];
+      if (r == rb || dcol[r - 1] != c) {
+        const int32_t q = lower_bound(A.idx, qb, qe, c);
+        if (q == qe || A.idx[q] != c) {
+          double merged = 0.0;
+          for (int32_t t = r; t < re && dcol[t] == c; ++t) merged += dval[t];
+          keep = fabs(merged) > zt;
+        }
+      }
+      if (r - rb < kDblLds) s_new[r - rb] = fresh + static_cast<int32_t>(__popcll(__ballot(keep) & below)) + (keep ? (1 << 30) : 0);
+    }
+    const uint64_t m = __ballot(keep);
+    fresh += static_cast<int32_t>(__popcll(m));
+  }
+  wave_lds_fence();
+  int32_t kept = 0;
+#pragma unroll 1
+  for (int32_t q0 = qb; q0 < qe; q0 += 64) {
+    const int32_t q = q0 + lane;
+    bool keep = false;
+    double merged = 0.0;
+    int32_t c = 0, r = rb;
+    if (q < qe) {
+      c = A.idx[q];
+      merged += A.val[q];
+      r = lower_bound(dcol, rb, re, c);
+      for (int32_t t = r; t < re && dcol[t] == c; ++t) merged += dval[t];
+      keep = fabs(merged) > zt;
+    }
+    const uint64_t m = __ballot(keep);
+    if (out_idx) {
+      if (lane == 0) {
+        s_bits[(q0 - qb) >> 6] = m;
+        s_pre[(q0 - qb) >> 6] = kept;
+      }
+      if (keep) {
+        const int32_t at = w + kept + static_cast<int32_t>(__popcll(m & below)) +
+                           (r < re ? s_new[r - rb] & ((1 << 30) - 1) : fresh);
+        out_idx[at] = c;
+        out_val[at] = merged;
+      }
+    }
+    kept += static_cast<int32_t>(__popcll(m));
+  }
+  if (!out_idx) {
+    if (lane == 0) *count = kept + fresh;
+    return;
+  }
+  wave_lds_fence();
+#pragma unroll 1
+  for (int32_t r = rb + lane; r < re; r += 64) {
+    if ((s_new[r - rb] >> 30) == 0) continue;
+    const int32_t c = dcol[r], q = lower_bound(A.idx, qb, qe, c) - qb;
+    double merged = 0.0;
+    for (int32_t t = r; t < re && dcol[t] == c; ++t) merged += dval[t];
+    const int32_t own = q >= qe - qb ? kept
+                                     : s_pre[q >> 6] + static_cast<int32_t>(__popcll(s_bits[q >> 6] &
+                                                                                     ((1ull << (q & 63)) - 1ull)));
+    const int32_t at = w + (s_new[r - rb] & ((1 << 30) - 1)) + own;
+    out_idx[at] = c;
+    out_val[at] = merged;
+  }
+  wave_lds_fence();
+}
+
+__global__ __launch_bounds__(kBlock) void k_dbl_merge(int32_t row_blocks, gpk_csr A, const int32_t* dptr,
+                                                      const int32_t* dcol, const double* dval, double zt,
+                                                      const int32_t* out_ptr, int32_t* counts, int32_t* out_idx,
+                                                      double* out_val) {
+  if (static_cast<int32_t>(blockIdx.x) >= row_blocks) {
+    __shared__ uint64_t s_bits[kWaves][kDblRowMax / 64];
+    __shared__ int32_t s_pre[kWaves][kDblRowMax / 64];
+    __shared__ int32_t s_new[kWaves][kDblLds];
+    const int wave = threadIdx.x >> 6;
+    wave_long_rows(A.ptr, A.rows, kLongRow, row_blocks, [&](int64_t i, int32_t b, int32_t e) {
+      dbl_merge_wave(A, b, e, dptr[i], dptr[i + 1], dcol, dval, zt, out_idx ? out_ptr[i] : 0, counts + (counts ? i : 0),
+                     out_idx, out_val, s_bits[wave], s_pre[wave], s_new[wave]);
+    });
+    return;
+  }
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= A.rows) return;
+  const int32_t b = A.ptr[i], e = A.ptr[i + 1];
+  if (e - b > kLongRow) return;
+  dbl_merge_serial(A, b, e, dptr[i], dptr[i + 1], dcol, dval, zt, out_idx ? out_ptr[i] : 0, counts + (counts ? i : 0),
+                   out_idx, out_val);
+}
 
 // Single-doubleton rebuild of A (rule_doubleton_equations.cu:1094-1127,
 // 1779-1858): every row but the target gets keep += alpha * a_elim; the keep
@@ -1165,6 +1443,16 @@ __global__ void k_rb_apply(int32_t n, gpk_plan p, const uint8_t* sl, const uint8
 
 }  // namespace
 
+// One thread a row, then the blocks that give long rows a wave.
+#define GPK_LAUNCH_ROWS(kernel, A, ...)                                                                    \
+  do {                                                                                                     \
+    const unsigned row_blocks = grid_for((A).rows);                                                        \
+    if ((A).rows > 0)                                                                                      \
+      hipLaunchKernelGGL(kernel, dim3(row_blocks + long_row_blocks((A).rows, (A).nnz)), dim3(kBlock), 0, stream, \
+                         static_cast<int32_t>(row_blocks), A, __VA_ARGS__);                                \
+    return hipGetLastError();                                                                              \
+  } while (0)
+
 #define GPK_LAUNCH(kernel, n, ...)                                                      \
   do {                                                                                  \
     if ((n) > 0) hipLaunchKernelGGL(kernel, dim3(grid_for(n)), dim3(kBlock), 0, stream, __VA_ARGS__); \
@@ -1190,7 +1478,7 @@ hipError_t gpk_cs_precheck(int32_t n, int32_t m, gpk_plan plan, const uint8_t* m
 }
 hipError_t gpk_cs_activity_cache(gpk_csr A, gpk_plan plan, const uint8_t* needed, gpk_row_cache cache,
                                  hipStream_t stream) {
-  GPK_LAUNCH(k_cs_activity_cache, A.rows, A, plan, needed, cache);
+  GPK_LAUNCH_ROWS(k_cs_activity_cache, A, plan, needed, cache);
 }
 hipError_t gpk_cs_owner(gpk_csr A, gpk_plan plan, const uint8_t* mask, const int32_t* srow, const double* sval,
                         gpk_row_cache cache, double tol, double zero_tol, int32_t eq_mode, int32_t* owner,
@@ -1284,20 +1572,20 @@ hipError_t gpk_dbl_apply(int32_t k, const int32_t* sel, gpk_plan plan, gpk_dbl d
 }
 hipError_t gpk_dbl_delta_count(gpk_csr A, gpk_plan plan, gpk_dbl_cols cols, double zero_tol, int32_t* counts,
                                hipStream_t stream) {
-  GPK_LAUNCH(k_dbl_delta_count, A.rows, A, plan, cols, zero_tol, counts);
+  GPK_LAUNCH_ROWS(k_dbl_delta_count, A, plan, cols, zero_tol, counts);
 }
 hipError_t gpk_dbl_shift(gpk_csr A, gpk_plan plan, gpk_dbl_cols cols, double zero_tol, int32_t include_subst,
                          hipStream_t stream) {
-  GPK_LAUNCH(k_dbl_shift, A.rows, A, plan, cols, zero_tol, include_subst);
+  GPK_LAUNCH_ROWS(k_dbl_shift, A, plan, cols, zero_tol, include_subst);
 }
 hipError_t gpk_dbl_delta_fill(gpk_csr A, gpk_plan plan, gpk_dbl_cols cols, double zero_tol, const int32_t* delta_ptr,
                               int32_t* dcol, double* dval, hipStream_t stream) {
-  GPK_LAUNCH(k_dbl_delta_fill, A.rows, A, plan, cols, zero_tol, delta_ptr, dcol, dval);
+  GPK_LAUNCH_ROWS(k_dbl_delta_fill, A, plan, cols, zero_tol, delta_ptr, dcol, dval);
 }
 hipError_t gpk_dbl_merge(gpk_csr A, const int32_t* delta_ptr, const int32_t* dcol, const double* dval,
                          double zero_tol, const int32_t* out_ptr, int32_t* counts, int32_t* out_idx, double* out_val,
                          hipStream_t stream) {
-  GPK_LAUNCH(k_dbl_merge, A.rows, A, delta_ptr, dcol, dval, zero_tol, out_ptr, counts, out_idx, out_val);
+  GPK_LAUNCH_ROWS(k_dbl_merge, A, delta_ptr, dcol, dval, zero_tol, out_ptr, counts, out_idx, out_val);
 }
 hipError_t gpk_dbl_scalar_rows(gpk_csr A, int32_t target, int32_t ec, int32_t kc, double alpha, double zero_tol,
                                const int32_t* out_ptr, int32_t* counts, int32_t* out_idx, double* out_val,

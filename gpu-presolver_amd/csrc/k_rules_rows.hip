@@ -17,17 +17,49 @@ using namespace gpdev;
 namespace {
 
 // ------------------------------------------------------------ generic ----
-__global__ void k_row_shift(gpk_csr A, const uint8_t* keep_row, const uint8_t* col_flag, const double* col_val,
-                            double abs_min, double* AL, double* AU) {
+// LDS of the waves that walk long rows, kSums kinds of terms each.
+#define GPK_ROW_TERMS(kSums)                                            \
+  __shared__ __align__(16) double s_terms[kWaves][(kSums) * kRowPitch]; \
+  double* s_t = s_terms[threadIdx.x >> 6]
+
+// The blocks from row_blocks on take the rows of more than kLongRow entries (as
+// in every kernel below with row_blocks).
+__global__ __launch_bounds__(kBlock) void k_row_shift(int32_t row_blocks, gpk_csr A, const uint8_t* keep_row,
+                                                      const uint8_t* col_flag, const double* col_val, double abs_min,
+                                                      double* AL, double* AU) {
+  const auto adds = [&](double a) { return !(abs_min >= 0.0 && !(fabs(a) > abs_min)); };
+  if (static_cast<int32_t>(blockIdx.x) >= row_blocks) {
+    GPK_ROW_TERMS(1);
+    wave_long_rows(A.ptr, A.rows, kLongRow, row_blocks, [&](int64_t i, int32_t b, int32_t e) {
+      if (keep_row != nullptr && keep_row[i] == 0) e = b;
+      const double shift = e == b ? 0.0 : wave_row_sums<1, double2>(
+          A.idx, A.val, b, e, s_t,
+          [&](int32_t j, double a, bool in) {  // (whether the entry adds, its column's value)
+            const bool on = in && col_flag[j] != 0 && adds(a);
+            return make_double2(on ? 1.0 : 0.0, on ? col_val[j] : 0.0);
+          },
+          [&](double a, double2 v, bool, double* t) {
+            t[0] = v.x != 0.0 ? a * v.y : 0.0;
+            return v.x != 0.0;
+          });
+      if (lane_id() == 0) {
+        AL[i] -= shift;
+        AU[i] -= shift;
+      }
+    });
+    return;
+  }
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= A.rows) return;
+  const int32_t b = A.ptr[i], e = A.ptr[i + 1];
+  if (e - b > kLongRow) return;
   double shift = 0.0;
   if (keep_row == nullptr || keep_row[i] != 0) {
-    for (int32_t p = A.ptr[i]; p < A.ptr[i + 1]; ++p) {
+    for (int32_t p = b; p < e; ++p) {
       const int32_t j = A.idx[p];
       if (!col_flag[j]) continue;
       const double a = A.val[p];
-      if (abs_min >= 0.0 && !(fabs(a) > abs_min)) continue;
+      if (!adds(a)) continue;
       shift += a * col_val[j];
     }
   }
@@ -142,29 +174,9 @@ __global__ void k_singleton_rows_commit(int32_t m, int32_t n, gpk_plan p, const 
 
 // -------------------------------------------------- redundant rows ----
 // flags[0] infeasible, flags[1] any action.
-__global__ void k_redundant_rows_classify(gpk_csr A, gpk_plan p, const int32_t* row_nnz, double tol, uint8_t* full,
-                                          uint8_t* dlo, uint8_t* dhi, int32_t* flags) {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= A.rows) return;
-  full[i] = 0;
-  dlo[i] = 0;
-  dhi[i] = 0;
-  if (!p.keep_row[i] || row_nnz[i] <= 1) return;
-  const double lo = p.AL[i], hi = p.AU[i];
+__device__ inline void redundant_row(double lo, double hi, double rmin, double rmax, double tol, int64_t i,
+                                     uint8_t* full, uint8_t* dlo, uint8_t* dhi, int32_t* flags) {
   const bool lf = isfinite(lo), hf = isfinite(hi);
-  if (lf && hf && fabs(hi - lo) <= tol) return;
-  double rmin = 0.0, rmax = 0.0;
-  for (int32_t q = A.ptr[i]; q < A.ptr[i + 1]; ++q) {
-    const int32_t j = A.idx[q];
-    const double a = A.val[q];
-    if (a >= 0.0) {
-      rmin += a * p.l[j];
-      rmax += a * p.u[j];
-    } else {
-      rmin += a * p.u[j];
-      rmax += a * p.l[j];
-    }
-  }
   if ((lf && rmax < lo - tol) || (hf && rmin > hi + tol)) {
     wave_set_flag(&flags[0]);
     return;
@@ -181,6 +193,57 @@ __global__ void k_redundant_rows_classify(gpk_csr A, gpk_plan p, const int32_t* 
     dhi[i] = 1;
     wave_set_flag(&flags[1]);
   }
+}
+
+// The row's activity does not matter: it is gone, short or an equality.
+__device__ inline bool redundant_skips(const gpk_plan& p, const int32_t* row_nnz, int64_t i, double tol) {
+  if (!p.keep_row[i] || row_nnz[i] <= 1) return true;
+  const double lo = p.AL[i], hi = p.AU[i];
+  return isfinite(lo) && isfinite(hi) && fabs(hi - lo) <= tol;
+}
+
+__global__ __launch_bounds__(kBlock) void k_redundant_rows_classify(int32_t row_blocks, gpk_csr A, gpk_plan p,
+                                                                    const int32_t* row_nnz, double tol, uint8_t* full,
+                                                                    uint8_t* dlo, uint8_t* dhi, int32_t* flags) {
+  if (static_cast<int32_t>(blockIdx.x) >= row_blocks) {
+    GPK_ROW_TERMS(2);
+    wave_long_rows(A.ptr, A.rows, kLongRow, row_blocks, [&](int64_t i, int32_t b, int32_t e) {
+      const bool lead = lane_id() == 0;
+      if (lead) full[i] = dlo[i] = dhi[i] = 0;
+      if (redundant_skips(p, row_nnz, i, tol)) return;
+      const double sum = wave_row_sums<2, double2>(
+          A.idx, A.val, b, e, s_t, [&](int32_t j, double, bool) { return make_double2(p.l[j], p.u[j]); },
+          [&](double a, double2 lu, bool in, double* t) {
+            t[0] = in ? (a >= 0.0 ? a * lu.x : a * lu.y) : 0.0;
+            t[1] = in ? (a >= 0.0 ? a * lu.y : a * lu.x) : 0.0;
+            return true;
+          });
+      const double rmin = __shfl(sum, 0, 64), rmax = __shfl(sum, 1, 64);
+      if (lead) redundant_row(p.AL[i], p.AU[i], rmin, rmax, tol, i, full, dlo, dhi, flags);
+    });
+    return;
+  }
+  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= A.rows) return;
+  const int32_t qb = A.ptr[i], qe = A.ptr[i + 1];
+  if (qe - qb > kLongRow) return;
+  full[i] = 0;
+  dlo[i] = 0;
+  dhi[i] = 0;
+  if (redundant_skips(p, row_nnz, i, tol)) return;
+  double rmin = 0.0, rmax = 0.0;
+  for (int32_t q = qb; q < qe; ++q) {
+    const int32_t j = A.idx[q];
+    const double a = A.val[q];
+    if (a >= 0.0) {
+      rmin += a * p.l[j];
+      rmax += a * p.u[j];
+    } else {
+      rmin += a * p.u[j];
+      rmax += a * p.l[j];
+    }
+  }
+  redundant_row(p.AL[i], p.AU[i], rmin, rmax, tol, i, full, dlo, dhi, flags);
 }
 
 __global__ void k_redundant_rows_apply(int32_t m, gpk_plan p, const uint8_t* full, const uint8_t* dlo,
@@ -499,15 +562,50 @@ constexpr uint64_t kFnvPrime = 0x100000001b3ULL;
 __device__ inline uint64_t fnv_mix(uint64_t h, uint64_t x) { return (h ^ x) * kFnvPrime; }
 __device__ inline uint64_t dbits(double v) { return static_cast<uint64_t>(__double_as_longlong(v)); }
 
-// rule_duplicate_rows.cu:78-114 (sequential FNV over len, col, a/a_first).
-__global__ void k_dup_row_hash(gpk_csr A, const uint8_t* keep_row, double ctol, uint64_t* hash) {
+// rule_duplicate_rows.cu:78-114 (sequential FNV over len, col, a/a_first).  A
+// long row's words are formed by a wave, 64 entries at a time, and mixed one
+// after the other from its lanes: the chain of multiplies is what is left.
+__global__ __launch_bounds__(kBlock) void k_dup_row_hash(int32_t row_blocks, gpk_csr A, const uint8_t* keep_row,
+                                                         double ctol, uint64_t* hash) {
+  if (static_cast<int32_t>(blockIdx.x) >= row_blocks) {
+    wave_long_rows(A.ptr, A.rows, kLongRow, row_blocks, [&](int64_t i, int32_t b, int32_t e) {
+      uint64_t h;
+      const double piv = A.val[b];
+      if (!keep_row[i]) {
+        h = static_cast<uint64_t>(i);
+      } else if (fabs(piv) <= ctol) {
+        h = fnv_mix(kFnvOffset, static_cast<uint64_t>(i));
+      } else {
+        h = fnv_mix(kFnvOffset, static_cast<uint64_t>(e - b));
+        int32_t j = A.idx[min(b + lane_id(), e - 1)];
+        double a = A.val[min(b + lane_id(), e - 1)];
+#pragma unroll 1
+        for (int32_t c = b; c < e; c += 64) {
+          const uint64_t w = dbits(a / piv);
+          const int lo = static_cast<int>(w), hi = static_cast<int>(w >> 32), col = j;
+          j = A.idx[min(c + 64 + lane_id(), e - 1)];
+          a = A.val[min(c + 64 + lane_id(), e - 1)];
+          const int n = min(64, e - c);
+#pragma unroll 1
+          for (int t = 0; t < n; ++t) {
+            h = fnv_mix(h, static_cast<uint64_t>(static_cast<int64_t>(__builtin_amdgcn_readlane(col, t))));
+            h = fnv_mix(h, static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(lo, t))) |
+                               (static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(hi, t))) << 32));
+          }
+        }
+      }
+      if (lane_id() == 0) hash[i] = h;
+    });
+    return;
+  }
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= A.rows) return;
+  const int32_t b = A.ptr[i], e = A.ptr[i + 1];
+  if (e - b > kLongRow) return;
   if (!keep_row[i]) {
     hash[i] = static_cast<uint64_t>(i);
     return;
   }
-  const int32_t b = A.ptr[i], e = A.ptr[i + 1];
   if (e - b <= 0 || fabs(A.val[b]) <= ctol) {
     hash[i] = fnv_mix(kFnvOffset, static_cast<uint64_t>(i));
     return;
@@ -788,6 +886,16 @@ __global__ void k_closure_mark_rows(gpk_csr A, gpk_plan plan, gpk_plan seen, uin
 
 }  // namespace
 
+// One thread a row, then the blocks that give long rows a wave.
+#define GPK_LAUNCH_ROWS(kernel, A, ...)                                                                    \
+  do {                                                                                                     \
+    const unsigned row_blocks = grid_for((A).rows);                                                        \
+    if ((A).rows > 0)                                                                                      \
+      hipLaunchKernelGGL(kernel, dim3(row_blocks + long_row_blocks((A).rows, (A).nnz)), dim3(kBlock), 0, stream, \
+                         static_cast<int32_t>(row_blocks), A, __VA_ARGS__);                                \
+    return hipGetLastError();                                                                              \
+  } while (0)
+
 #define GPK_LAUNCH(kernel, n, ...)                                                      \
   do {                                                                                  \
     if ((n) > 0) hipLaunchKernelGGL(kernel, dim3(grid_for(n)), dim3(kBlock), 0, stream, __VA_ARGS__); \
@@ -798,7 +906,7 @@ extern "C" {
 
 hipError_t gpk_row_shift(gpk_csr A, const uint8_t* keep_row, const uint8_t* col_flag, const double* col_val,
                          double abs_min, double* AL, double* AU, hipStream_t stream) {
-  GPK_LAUNCH(k_row_shift, A.rows, A, keep_row, col_flag, col_val, abs_min, AL, AU);
+  GPK_LAUNCH_ROWS(k_row_shift, A, keep_row, col_flag, col_val, abs_min, AL, AU);
 }
 hipError_t gpk_pack_f64(const uint8_t* mask, const double* vals, const int32_t* prefix, int32_t n, double* out,
                         hipStream_t stream) {
@@ -838,7 +946,7 @@ hipError_t gpk_singleton_rows_commit(int32_t m, int32_t n, gpk_plan plan, const 
 }
 hipError_t gpk_redundant_rows_classify(gpk_csr A, gpk_plan plan, const int32_t* row_nnz, double tol, uint8_t* full,
                                        uint8_t* dlo, uint8_t* dhi, int32_t* flags, hipStream_t stream) {
-  GPK_LAUNCH(k_redundant_rows_classify, A.rows, A, plan, row_nnz, tol, full, dlo, dhi, flags);
+  GPK_LAUNCH_ROWS(k_redundant_rows_classify, A, plan, row_nnz, tol, full, dlo, dhi, flags);
 }
 hipError_t gpk_redundant_rows_apply(int32_t m, gpk_plan plan, const uint8_t* full, const uint8_t* dlo,
                                     const uint8_t* dhi, hipStream_t stream) {
@@ -902,7 +1010,7 @@ hipError_t gpk_dup_row_hash(gpk_csr A, const uint8_t* keep_row, double coeff_tol
                          stream, A, keep_row, coeff_tol, hash);
     return hipGetLastError();
   }
-  GPK_LAUNCH(k_dup_row_hash, A.rows, A, keep_row, coeff_tol, hash);
+  GPK_LAUNCH_ROWS(k_dup_row_hash, A, keep_row, coeff_tol, hash);
 }
 hipError_t gpk_dup_row_groups(gpk_csr A, gpk_plan plan, const uint64_t* sorted_hash, const int32_t* sorted_rows,
                               double coeff_tol, double interval_tol, uint8_t* row_delete, int32_t* merge_to,

@@ -217,7 +217,7 @@ hipError_t gpk_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t* o
  * rows of more than 128 entries one wave each, every row summed in CSR order. */
 hipError_t gpk_pack_lu(const double* l, const double* u, int32_t n, double* lu, hipStream_t stream);
 hipError_t gpk_row_activity_lu(const int32_t* row_ptr, const int32_t* col_idx, const double* val, int32_t m,
-                               const double* lu, double ztol, double* min_fin, double* max_fin, int32_t* neg_inf,
+                               int32_t nnz, const double* lu, double ztol, double* min_fin, double* max_fin, int32_t* neg_inf,
                                int32_t* pos_inf, hipStream_t stream);
 hipError_t gpk_col_max_abs(const int32_t* at_ptr, const double* at_val, int32_t n, double* out,
                            hipStream_t stream);
@@ -226,7 +226,7 @@ hipError_t gpk_col_max_abs(const int32_t* at_ptr, const double* at_val, int32_t 
  * GP_ROW_ACTIVITY_NOALLOC_MAX_COLS (hipErrorInvalidValue beyond).  Calls that
  * overlap on one GPU share that array and race. */
 hipError_t gpk_row_activity_noalloc(const int32_t* row_ptr, const int32_t* col_idx, const double* val, int32_t m,
-                                    int32_t n, const double* l, const double* u, double ztol, double* min_fin,
+                                    int32_t n, int32_t nnz, const double* l, const double* u, double ztol, double* min_fin,
                                     double* max_fin, int32_t* neg_inf, int32_t* pos_inf, hipStream_t stream);
 /* Row stats of a CSR (counts include explicit zeros; singleton = first entry). */
 hipError_t gpk_csr_stats(const int32_t* ptr, const int32_t* idx, const double* val, int32_t rows,
@@ -271,14 +271,22 @@ typedef struct gpk_row_val {
 hipError_t gpk_expand_rows(const int32_t* ptr, const double* val, int32_t m, gpk_row_val* rv, hipStream_t stream);
 hipError_t gpk_transpose_gather(const int32_t* perm, const gpk_row_val* rv, int32_t nnz, int32_t* at_idx,
                                 double* at_val, hipStream_t stream);
-/* Input check of a CSR matrix, one thread per entry over tiles of 256 rows:
- * flags[0] bad row pointers, flags[1] a column index outside [0, cols),
- * flags[2] two equal neighbours in a row, flags[3] a row not sorted by column
- * (flags are set to 1, never cleared).  A row that is not sorted can repeat a
+/* Input check of two CSR matrices (rows 0: none), flags[0] bad row pointers
+ * (no entry of that matrix is read then), flags[1] a column index outside
+ * [0, cols), flags[2] two equal neighbours in a row, flags[3] a row not sorted
+ * by column (flags are set to 1, never cleared).  chunk_row is scratch of
+ * gpk_csr_check_chunks(nnz) words.  A row that is not sorted can repeat a
  * column at a distance: gpk_csr_check_rows (one thread per row, every pair of
  * an unsorted row) sets flags[2] for those as well. */
-hipError_t gpk_csr_check(const int32_t* ptr, const int32_t* idx, int32_t rows, int32_t cols, int32_t nnz,
-                         int32_t* flags, hipStream_t stream);
+typedef struct gpk_csr_check_side {
+  const int32_t* ptr;
+  const int32_t* idx;
+  int32_t rows, cols, nnz, pad;
+  int32_t* chunk_row;
+  int32_t* flags;
+} gpk_csr_check_side;
+int32_t gpk_csr_check_chunks(int32_t nnz);
+hipError_t gpk_csr_check(gpk_csr_check_side a, gpk_csr_check_side t, hipStream_t stream);
 hipError_t gpk_csr_check_rows(const int32_t* ptr, const int32_t* idx, int32_t rows, int32_t cols, int32_t nnz,
                               int32_t* flags, hipStream_t stream);
 /* flag[0] = 1 if some row of the CSR is not sorted by column (row pointers

@@ -9,7 +9,7 @@ import pytest
 import gp_ffi
 import lp_synth
 import oracle_ffi as O
-from helpers import assert_same_array
+from helpers import assert_same_array, assert_same_lp, assert_same_record
 
 pytestmark = pytest.mark.gpu
 
@@ -107,3 +107,66 @@ def test_compaction_masks_at_an_odd_address(m):
     assert got[:2] == want[:2]
     for name, a, b in zip(("ptr", "idx", "val"), got[2:], want[2:]):
         assert_same_array(name, a, b)
+
+
+def with_dense_rows(lp, lengths, seed):
+    """The LP with further rows of the given lengths (wide or one-sided
+    bounds), every third one a scaled copy of the one before it."""
+    rng = np.random.default_rng(seed)
+    m, n = lp["m"], lp["n"]
+    rows, cols, vals, AL, AU = [], [], [], [], []
+    for k, length in enumerate(lengths):
+        if k % 3 == 2:
+            f = -2.0
+            c, v, lo, hi = cols[-1], f * vals[-1], f * AU[-1], f * AL[-1]
+        else:
+            c = np.sort(rng.choice(n, size=min(length, n), replace=False))
+            v = np.round(rng.uniform(0.5, 2.0, len(c)) * 8) / 8 * rng.choice([-1.0, 1.0], len(c))
+            lo, hi = (-np.inf, 2.0 ** 21) if k % 2 else (-2.0 ** 21, 2.0 ** 21)
+        rows.append(np.full(len(c), m + k))
+        cols.append(c)
+        vals.append(v)
+        AL.append(lo)
+        AU.append(hi)
+    r0 = np.repeat(np.arange(m), np.diff(lp["A_ptr"]))
+    M = m + len(lengths)
+    ptr, idx, val = lp_synth.csr_from_coo(M, n, np.concatenate([r0] + rows), np.concatenate([lp["A_idx"]] + cols),
+                                          np.concatenate([lp["A_val"]] + vals))
+    tptr, tidx, tval = lp_synth.transpose_csr(M, n, ptr, idx, val)
+    return dict(lp, m=M, A_ptr=ptr, A_idx=idx, A_val=val, AT_ptr=tptr, AT_idx=tidx, AT_val=tval,
+                AL=np.concatenate([lp["AL"], AL]), AU=np.concatenate([lp["AU"], AU]))
+
+
+@pytest.mark.parametrize("lengths,kw", [
+    ([127, 128, 128, 129, 130, 130, 255, 256, 257] * 3, {}),
+    ([2500, 2500, 2500, 600, 300, 300] * 4, dict(record_postsolve_tape_cpu=1)),
+    # more deltas in a row than a wave places by rank, and more columns than its bitmap holds
+    ([4400, 4000, 4000] * 3, dict(doubleton_equations_min_selected_per_batch=1,
+                                  doubleton_equations_min_selected_ratio=0.0)),
+    ([17000, 16384, 16385, 9000, 200], dict(doubleton_equations_min_selected_per_batch=1,
+                                            doubleton_equations_min_selected_ratio=0.0)),
+    ([700] * 60, dict(use_tiered_scheduler=0)),
+])
+def test_presolve_with_dense_rows(lengths, kw):
+    big = max(lengths) > 4400
+    lp = lp_synth.generate(14000 if big else 3000, 18000 if big else 4500, seed=31, mean_row_len=4.0,
+                           frac_doubleton=0.25, frac_fixed_cols=0.05, frac_singleton_cols=0.15)
+    lp = with_dense_rows(lp, lengths, 32)
+    kw = dict(kw, enable_structure_specific_rules=0, doubleton_equations_max_fill_in_proxy=100000)
+    sg, rg, lg = gp_ffi.presolve(lp, gp_ffi.params(**kw), True)
+    so, ro, lo = O.presolve(lp, O.params(**kw), True)
+    assert (sg["reduced_rows"], sg["reduced_cols"], sg["reduced_nnz"]) == (so["reduced_rows"], so["reduced_cols"],
+                                                                           so["reduced_nnz"])
+    assert sg["obj_constant_delta"] == so["obj_constant_delta"]
+    assert_same_record(rg, ro)
+    assert_same_lp(lg, lo)
+
+
+@pytest.mark.parametrize("n", [4097, 2048 * 16, 2048 * 16 + 1, 2048 * 17 - 1, 2048 * 64, 2048 * 64 + 1])
+def test_radix_sort_at_histogram_batches(n):
+    rng = np.random.default_rng(n)
+    keys, vals = rng.integers(0, 1 << 20, n).astype(np.uint64), np.arange(n, dtype=np.int32)
+    k, v = gp_ffi.radix_sort(keys, vals, 20)
+    order = np.argsort(keys, kind="stable")
+    assert_same_array("keys", k, keys[order])
+    assert_same_array("vals", v, order.astype(np.int32))

@@ -125,8 +125,8 @@ Lines gather_lines(const int32_t* ptr, const int32_t* idx, int32_t lines_total, 
   return L;
 }
 
-// Levels [first, first + count): one grid launch (a single large level) or
-// one workgroup that steps through a run of smaller levels.
+// Parts [first, first + count) of levels: one grid launch (a single large
+// level) or one workgroup that steps through a run of smaller levels.
 struct Segment {
   int32_t first, count;
   bool grid;
@@ -134,11 +134,17 @@ struct Segment {
 
 struct Schedule {
   std::vector<int32_t> order;        // record indices, level by level
-  std::vector<int32_t> level_start;  // levels + 1 offsets into order
+  std::vector<int32_t> level_start;  // offsets into order of the levels' parts, and its end
   std::vector<Segment> segs;
+  int32_t levels = 0;
 };
 
-constexpr int32_t kGridLevelMin = 2048;
+// Levels of at least this many records get a launch of their own (about 10 us
+// with the gap, and as much to start the next run of levels); in a run, a level
+// takes about 3 us for each 64 records.
+constexpr int32_t kGridLevelMin = 512;
+constexpr int32_t kTypes = 15;       // PostsolveReductionType
+constexpr int32_t kWaveRecords = 4;  // sixteen lanes each
 
 [[noreturn]] void bad_tape(int32_t k, const char* what) {
   throw std::runtime_error("postsolve_gpu: tape record " + std::to_string(k) + ": " + what);
@@ -306,6 +312,9 @@ class TapeScanner {
     }
   }
 
+  // The type of a record that takes part in a pass.
+  int32_t type(int32_t k) const { return t_.types[k]; }
+
   // Original rows (type 12) and columns (types 5 and 13 without a row
   // payload) whose index lists the dual pass walks.
   void pattern_lines(std::vector<int32_t>& rows, std::vector<int32_t>& cols) const {
@@ -356,24 +365,40 @@ Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, int32_t
     level[k - lo] = lv;
     levels = std::max(levels, lv + 1);
   }
-  std::vector<int32_t> start(static_cast<size_t>(levels) + 1, 0);
-  for (int32_t k = 0; k < span; ++k)
-    if (level[k] >= 0) ++start[level[k] + 1];
-  for (int32_t l = 0; l < levels; ++l) start[l + 1] += start[l];
+  // Records of a level in the order of their types, and in a level that one
+  // workgroup replays each type from a new wave on (empty slots, -1, between):
+  // a wave runs the branches of its records' types one after the other.  Such
+  // a level is given to the workgroup in parts of its slots.
+  std::vector<int32_t> size(static_cast<size_t>(levels) * kTypes, 0);
+  for (int32_t k = lo; k < hi; ++k)
+    if (level[k - lo] >= 0) ++size[static_cast<size_t>(level[k - lo]) * kTypes + scan.type(k)];
   Schedule sch;
-  sch.order.resize(start[levels]);
-  std::vector<int32_t> fill(start.begin(), start.end() - 1);
-  for (int32_t k = hi - 1; k >= lo; --k)
-    if (level[k - lo] >= 0) sch.order[fill[level[k - lo]]++] = k;  // descending k within a level
+  sch.levels = levels;
+  std::vector<int32_t>& start = sch.level_start;
+  start.push_back(0);
+  std::vector<int32_t> fill(static_cast<size_t>(levels) * kTypes);
   for (int32_t l = 0; l < levels; ++l) {
-    const bool big = start[l + 1] - start[l] >= kGridLevelMin;
-    if (!big && !sch.segs.empty() && !sch.segs.back().grid) {
-      ++sch.segs.back().count;
-    } else {
-      sch.segs.push_back(Segment{l, 1, big});
+    const size_t f = static_cast<size_t>(l) * kTypes;
+    int32_t records = 0, at = start.back();
+    for (int32_t t = 0; t < kTypes; ++t) records += size[f + t];
+    const bool grid = records >= kGridLevelMin;
+    for (int32_t t = 0; t < kTypes; ++t) {
+      fill[f + t] = at;
+      at += grid ? size[f + t] : (size[f + t] + kWaveRecords - 1) / kWaveRecords * kWaveRecords;
     }
+    const int32_t first = static_cast<int32_t>(start.size()) - 1;
+    if (!grid)
+      while (at - start.back() > GPK_REPLAY_SLOTS) start.push_back(start.back() + GPK_REPLAY_SLOTS);
+    start.push_back(at);
+    const int32_t parts = static_cast<int32_t>(start.size()) - 1 - first;
+    if (!grid && !sch.segs.empty() && !sch.segs.back().grid)
+      sch.segs.back().count += parts;
+    else
+      sch.segs.push_back(Segment{first, parts, grid});
   }
-  sch.level_start = std::move(start);
+  sch.order.assign(static_cast<size_t>(start.back()), -1);
+  for (int32_t k = hi - 1; k >= lo; --k)
+    if (level[k - lo] >= 0) sch.order[fill[static_cast<size_t>(level[k - lo]) * kTypes + scan.type(k)]++] = k;
   return sch;
 }
 
@@ -745,8 +770,8 @@ PostsolvePlan::Shape PostsolvePlan::shape() const {
   out.records = d_->records;
   out.tape_bytes = d_->tape_bytes;
   for (const auto& st : d_->primal)
-    out.primal_levels += static_cast<int32_t>(st.sched.level_start.empty() ? 0 : st.sched.level_start.size() - 1);
-  out.dual_levels = static_cast<int32_t>(d_->dual.level_start.empty() ? 0 : d_->dual.level_start.size() - 1);
+    out.primal_levels += st.sched.levels;
+  out.dual_levels = d_->dual.levels;
   return out;
 }
 

@@ -144,131 +144,263 @@ __device__ void dbl_recover_z(double xk, double zk_hat, double al, double okl, d
   else { *zk = zk_hat; *ze = 0.0; }
 }
 
-// s (+/-)= sum over q in [0, count) with idx[q] != skip of val[q] * vec[idx[q]],
-// accumulated in q order exactly as the plain loop would (every product
-// rounded, then added or subtracted one at a time).  The indices, values and
-// gathered entries of eight terms are loaded before they are used, so a long
-// column costs count / 8 memory round trips instead of count.
-template <bool kSub, int U = 8>
-__device__ inline double dot_in_order(double s, const int32_t* __restrict__ idx, const double* __restrict__ val,
-                                      const double* __restrict__ vec, int32_t count, int32_t skip) {
-  int32_t q = 0;
-  for (; q + U <= count; q += U) {
-    int32_t j[U];
-    double a[U], v[U];
+// Sixteen lanes (a DPP row) work on a record: its index words, its values and
+// the entries of the line it walks are one to a lane.  A level's time is that
+// of the instructions of one wave and of its round trips to memory: with a lane
+// per record the entries of a line are that many loads, branches and divides
+// one after the other (9.3 us a level even with all of them loaded ahead), so
+// they are side by side instead.
+constexpr int kRecLanes = 16;
+constexpr int kRecChunks = 2;  // chunks of 16 entries of a line loaded ahead
+
+// Lane k's value of the 16 lanes, k a constant.
+template <int k>
+__device__ __forceinline__ int32_t row_lane(int32_t v) {
+  return __builtin_amdgcn_update_dpp(v, v, 0x150 + k, 0xf, 0xf, true);  // row_newbcast
+}
+template <int k>
+__device__ __forceinline__ double row_lane(double v) {
+  const long long b = __double_as_longlong(v);
+  return __hiloint2double(row_lane<k>(static_cast<int32_t>(b >> 32)), row_lane<k>(static_cast<int32_t>(b)));
+}
+// s + (lane 0's term) + (lane 1's term) + ..., added one after the other.  A
+// lane without a term holds -0, which leaves any sum as it is.
+__device__ __forceinline__ double row_add(double s, double t) {
+  s += row_lane<0>(t);
+  s += row_lane<1>(t);
+  s += row_lane<2>(t);
+  s += row_lane<3>(t);
+  s += row_lane<4>(t);
+  s += row_lane<5>(t);
+  s += row_lane<6>(t);
+  s += row_lane<7>(t);
+  s += row_lane<8>(t);
+  s += row_lane<9>(t);
+  s += row_lane<10>(t);
+  s += row_lane<11>(t);
+  s += row_lane<12>(t);
+  s += row_lane<13>(t);
+  s += row_lane<14>(t);
+  s += row_lane<15>(t);
+  return s;
+}
+
+// s += sum over q in [0, count) with idx[q] != skip of sign * val[q] * vec[idx[q]]
+// (sign 1 or -1), accumulated in q order exactly as the plain loop would (every
+// product rounded, then added or subtracted one at a time).
+__device__ inline double dot_in_order(double s, double sign, const int32_t* __restrict__ idx,
+                                      const double* __restrict__ val, const double* vec, int32_t count, int32_t skip) {
+  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
+#pragma unroll 1
+  for (int32_t q = 0; q < count; q += 2 * kRecLanes) {
+    double p[2];
 #pragma unroll
-    for (int k = 0; k < U; ++k) {
-      j[k] = idx[q + k];
-      a[k] = val[q + k];
+    for (int c = 0; c < 2; ++c) {
+      const int32_t e = q + c * kRecLanes + t;
+      const int32_t j = e < count ? idx[e] : skip;
+      const double a = e < count ? val[e] : 0.0;
+      p[c] = e < count && j != skip ? sign * (a * vec[j]) : -0.0;
     }
-#pragma unroll
-    for (int k = 0; k < U; ++k) v[k] = vec[j[k]];
-#pragma unroll
-    for (int k = 0; k < U; ++k)
-      if (j[k] != skip) s = kSub ? s - a[k] * v[k] : s + a[k] * v[k];
-  }
-  for (; q < count; ++q) {
-    const int32_t j = idx[q];
-    if (j != skip) s = kSub ? s - val[q] * vec[j] : s + val[q] * vec[j];
+    s = row_add(s, p[0]);
+    if (q + kRecLanes < count) s = row_add(s, p[1]);
   }
   return s;
 }
 
-// Where a record's indices and values sit in the tape (immutable, so it can
-// be loaded ahead of the record's turn).
-// The header also carries the record's first three index words (-1 past
-// its end), so a prefetched header leaves the record's variables one load
-// away.
+// What a record's turn needs of the tape and of the original model, none of
+// which the replay writes: it can be loaded before the turn comes, and then
+// only the loads of x, y, z and zret are left to it.  Four steps, each one
+// memory round trip behind the one before: where the record's indices and
+// values sit; its first 16 index words (-1 past its end); the line of entries
+// it walks; its first 16 values (0 past its end) and the line's first entries.
 struct RecHead {
-  int32_t type, i0, i1, v0, v1;
-  int32_t a0, a1, a2;
+  int32_t type, i0, i1, v0, v1;  // type -1: an empty slot
 };
+struct RecLine {
+  int32_t qi, qv, n;  // the line's first index and first value, its length
+};
+struct RecEntries {
+  double v;  // the lane's value
+  int32_t j[kRecChunks];
+  double a[kRecChunks];
+};
+
 __device__ inline RecHead load_head(const gp_tape_dev& T, int32_t k) {
-  RecHead h{T.types[k], T.index_starts[k], T.index_starts[k + 1] - 1, T.value_starts[k], T.value_starts[k + 1] - 1,
-            -1, -1, -1};
-  if (h.i0 <= h.i1) h.a0 = T.indices[h.i0];
-  if (h.i0 + 1 <= h.i1) h.a1 = T.indices[h.i0 + 1];
-  if (h.i0 + 2 <= h.i1) h.a2 = T.indices[h.i0 + 2];
-  return h;
+  if (k < 0) return RecHead{-1, 0, -1, 0, -1};
+  return RecHead{T.types[k], T.index_starts[k], T.index_starts[k + 1] - 1, T.value_starts[k],
+                 T.value_starts[k + 1] - 1};
+}
+__device__ inline int32_t load_word(const gp_tape_dev& T, const RecHead& h, int t) {
+  return h.i0 + t <= h.i1 ? T.indices[h.i0 + t] : -1;
 }
 
-// Dot products inside a record keep this many entries' loads in flight.
-constexpr int kRecDotU = 32;
+__device__ inline bool has_payload(const RecHead& h) { return h.i1 >= h.i0 + 3 && h.v1 >= h.v0 + 11; }
+// Where the line sits: in the tape, in the columns or in the rows of the model.
+enum : int { LINE_TAPE, LINE_COL, LINE_ROW };
+__device__ inline int line_kind(const RecHead& h) {
+  if (h.type == 12 || h.type == 4) return LINE_ROW;
+  return h.type == 5 || (h.type == 13 && !has_payload(h)) ? LINE_COL : LINE_TAPE;
+}
+// The lines of types 0, 4, 5 and 13 are walked for y, and a line's place is
+// checked by the host only where there is a y.
+template <bool kDual>
+__device__ inline RecLine load_line(const gp_orig_dev& O, const RecHead& h, int32_t word, bool has_y) {
+  const int32_t type = h.type;
+  if (!kDual && type == 2) return RecLine{h.i0 + 3, h.v0 + 6, row_lane<2>(word)};
+  if (kDual && type == 0 && has_y) return RecLine{h.i0 + 1, h.v0 + 2, h.i1 - h.i0};
+  if (kDual && O.present != 0 && (has_y || type == 12)) {
+    const int kind = line_kind(h);
+    if (type == 13 && kind == LINE_TAPE) return RecLine{h.i0 + 4, h.v0 + 12, row_lane<3>(word)};
+    const int32_t line = type == 13 || type == 4 ? row_lane<0>(word) : row_lane<1>(word);
+    if (kind != LINE_TAPE && line >= 0) {
+      const int32_t* ptr = kind == LINE_ROW ? O.a_ptr : O.at_ptr;
+      const int32_t b = ptr[line];
+      return RecLine{b, b, ptr[line + 1] - b};
+    }
+  }
+  return RecLine{0, 0, 0};
+}
+__device__ inline const int32_t* line_idx(const gp_tape_dev& T, const gp_orig_dev& O, int kind) {
+  return kind == LINE_TAPE ? T.indices : kind == LINE_COL ? O.at_idx : O.a_idx;
+}
+__device__ inline const double* line_val(const gp_tape_dev& T, const gp_orig_dev& O, int kind) {
+  return kind == LINE_TAPE ? T.vals : kind == LINE_COL ? O.at_val : O.a_val;
+}
+__device__ inline RecEntries load_entries(const gp_tape_dev& T, const gp_orig_dev& O, const RecHead& h,
+                                          const RecLine& ln, int t) {
+  RecEntries r;
+  r.v = h.v0 + t <= h.v1 ? T.vals[h.v0 + t] : 0.0;
+  const int kind = line_kind(h);
+  const int32_t* idx = line_idx(T, O, kind);
+  const double* val = line_val(T, O, kind);
+#pragma unroll
+  for (int c = 0; c < kRecChunks; ++c) {
+    const int32_t e = c * kRecLanes + t;
+    r.j[c] = e < ln.n ? idx[ln.qi + e] : -1;
+    r.a[c] = e < ln.n ? val[ln.qv + e] : 0.0;
+  }
+  return r;
+}
+
+// The column and the row whose values a record reads besides its line's.
+__device__ inline int32_t column_read(int32_t type, int32_t w0, int32_t w1) {
+  return type == 3 || type == 13 || type == 5 ? w1 : type == 12 ? w0 : -1;
+}
+__device__ inline int32_t row_read(int32_t type, int32_t w0, int32_t w1) {
+  return type == 2 || type == 12 ? w1 : type == 10 || type == 4 ? w0 : -1;
+}
 
 // One record of the reverse replay (_kernel_replay_postsolve_tape,
-// gpu_postsolve.cu:605-1046).
-__device__ void replay_one(const gp_tape_dev& T, const gp_orig_dev& O, double* x, double* y, double* z,
-                           uint8_t* zret, const RecHead& h, bool primal, bool dual, double tol) {
+// gpu_postsolve.cu:605-1046); all sixteen lanes come with the same record.
+// kDual picks the pass.  All loads of x, y, z and zret that the record's type
+// needs go out together at the top: a wave waits for one round trip, for two
+// where a decision comes before a row is read.
+template <bool kDual>
+__device__ __forceinline__ void replay_one(const gp_tape_dev& T, const gp_orig_dev& O, double* x, double* y, double* z,
+                                           uint8_t* zret, const RecHead& h, int32_t word, const RecLine& ln,
+                                           RecEntries r, double tol) {
   const bool has_orig = O.present != 0;
   const int32_t type = h.type;
-  const int32_t i0 = h.i0, i1 = h.i1;
-  const int32_t v0 = h.v0, v1 = h.v1;
+  if (type < 0) return;
+  constexpr bool primal = !kDual, dual = kDual;
+  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
+  const bool first = t == 0;  // the lane that stores what the record has one of
+  const int32_t i0 = h.i0;
+  const int32_t v0 = h.v0;
   const int32_t* I = T.indices;
   const double* V = T.vals;
-  if (type == 3) {  // DuplicateColumn
-    const int32_t from = I[i0], to = I[i0 + 1];
-    const double r = V[v0];
-    if (primal) {
-      double xf = 0.0, xt = x[to];
-      recover_dup_col(x[to], z ? z[to] : 0.0, r, V[v0 + 1], V[v0 + 2], V[v0 + 3], V[v0 + 4], tol, &xf, &xt);
-      x[from] = xf;
-      x[to] = xt;
+  // The record's first index words and values.
+  const int32_t w0 = row_lane<0>(word), w1 = row_lane<1>(word), w2 = row_lane<2>(word);
+  const double W0 = row_lane<0>(r.v), W1 = row_lane<1>(r.v), W2 = row_lane<2>(r.v), W3 = row_lane<3>(r.v),
+               W4 = row_lane<4>(r.v), W5 = row_lane<5>(r.v);
+
+  const int32_t col_in = column_read(type, w0, w1), row_in = row_read(type, w0, w1);
+  const double xc = col_in >= 0 ? x[col_in] : 0.0;
+  const double zc = col_in >= 0 && z ? z[col_in] : 0.0;
+  const bool col_set = type == 12 && dual && zret ? zret[col_in] != 0 : true;
+  const double yr = dual && row_in >= 0 && y ? y[row_in] : 0.0;
+  const int32_t cost = type == 13 ? w0 : type == 5 ? w1 : -1;
+  const double cc = dual && has_orig && cost >= 0 ? O.c[cost] : 0.0;
+
+  // A bound change's row: its z and whether each is set.
+  bool on[kRecChunks];
+  double zk[kRecChunks];
+  if (dual && type == 12) {
+#pragma unroll
+    for (int c = 0; c < kRecChunks; ++c) {
+      const bool other = r.j[c] >= 0 && r.j[c] != w0;
+      zk[c] = other ? z[r.j[c]] : 0.0;
+      on[c] = other && (!zret || zret[r.j[c]]);
     }
-    if (dual && z) { z[from] = r * z[to]; if (zret) zret[from] = 1; }
+  }
+
+  // The sum over the line with x (types 2 and 4) or y, in order.
+  const int kind = line_kind(h);
+  double sum = type == 0 ? W1 : type == 5 ? cc : 0.0;
+  if (ln.n > 0 && type != 12) {
+    const double* vec = type == 2 || type == 4 ? x : y;
+    const double sign = type == 0 || type == 5 ? -1.0 : 1.0;
+    const int32_t skip = type == 5 ? w0 : type == 13 && kind == LINE_COL ? w2 : -1;
+    double p[kRecChunks];
+#pragma unroll
+    for (int c = 0; c < kRecChunks; ++c)
+      p[c] = r.j[c] >= 0 && r.j[c] != skip ? sign * (r.a[c] * vec[r.j[c]]) : -0.0;
+#pragma unroll
+    for (int c = 0; c < kRecChunks; ++c)
+      if (ln.n > c * kRecLanes) sum = row_add(sum, p[c]);
+    constexpr int kHave = kRecChunks * kRecLanes;
+    if (ln.n > kHave)
+      sum = dot_in_order(sum, sign, line_idx(T, O, kind) + ln.qi + kHave, line_val(T, O, kind) + ln.qv + kHave, vec,
+                         ln.n - kHave, skip);
+  }
+
+  if (type == 3) {  // DuplicateColumn
+    const int32_t from = w0, to = w1;
+    if (primal) {
+      double xf = 0.0, xt = xc;
+      recover_dup_col(xc, zc, W0, W1, W2, W3, W4, tol, &xf, &xt);
+      if (first) { x[from] = xf; x[to] = xt; }
+    }
+    if (dual && z && first) { z[from] = W0 * zc; if (zret) zret[from] = 1; }
   } else if (type == 13) {  // DoubletonEquation
-    const int32_t ec = h.a0, kc = h.a1, row = h.a2;
-    const double ecoef = V[v0], kcoef = V[v0 + 1], rhs = V[v0 + 2], eobj = V[v0 + 9];
+    const int32_t ec = w0, kc = w1, row = w2;
+    const double ecoef = W0, kcoef = W1, rhs = W2, eobj = row_lane<9>(r.v);
     const double al = -kcoef / ecoef, be = rhs / ecoef;
-    if (primal) x[ec] = be + al * x[kc];
+    if (primal && first) x[ec] = be + al * xc;
     if (dual && z && y && has_orig) {
-      // The column bounds and c[ec] load together with x[kc] and z[kc].
-      const int32_t qb = O.at_ptr[ec], qe = O.at_ptr[ec + 1];
-      const double cec = O.c[ec];
-      const double ls = v1 >= v0 + 10 ? V[v0 + 10] : 0.0;
-      const double us = v1 >= v0 + 11 ? V[v0 + 11] : 0.0;
       double zk = 0.0, ze = 0.0;
-      dbl_recover_z(x[kc], z[kc], al, V[v0 + 5], V[v0 + 6], V[v0 + 7], V[v0 + 8], ls, us, tol, &zk, &ze);
-      const bool payload = i1 >= i0 + 3 && v1 >= v0 + 11;
-      double so = 0.0;
-      double yrow;
-      if (payload) {
-        so = dot_in_order<false, kRecDotU>(so, I + i0 + 4, V + v0 + 12, y, I[i0 + 3], -1);
-        yrow = (eobj - so - ze) / ecoef;
-      } else {
-        so = dot_in_order<false, kRecDotU>(so, O.at_idx + qb, O.at_val + qb, y, qe - qb, row);
-        yrow = (cec - so - ze) / ecoef;
+      dbl_recover_z(xc, zc, al, W5, row_lane<6>(r.v), row_lane<7>(r.v), row_lane<8>(r.v), row_lane<10>(r.v),
+                    row_lane<11>(r.v), tol, &zk, &ze);
+      const double yrow = ((kind == LINE_TAPE ? eobj : cc) - sum - ze) / ecoef;
+      if (first) {
+        y[row] = yrow;
+        z[kc] = zk;
+        z[ec] = ze;
+        if (zret) { zret[kc] = 1; zret[ec] = 1; }
       }
-      y[row] = yrow;
-      z[kc] = zk;
-      z[ec] = ze;
-      if (zret) { zret[kc] = 1; zret[ec] = 1; }
-    } else if (dual) {
+    } else if (dual && first) {
       if (z) { z[ec] = 0.0; if (zret) zret[ec] = 1; }
       if (y && row >= 0) y[row] = eobj / ecoef;
     }
   } else if (type == 2) {  // SubCol
-    const int32_t ec = h.a0, row = h.a1, sc = h.a2;
-    const double piv = V[v0], rhs = V[v0 + 1], eobj = V[v0 + 4];
-    const bool row_deleted = V[v0 + 5] != 0.0;
-    const double part = dot_in_order<false, kRecDotU>(0.0, I + i0 + 3, V + v0 + 6, x, sc, -1);
-    if (primal) x[ec] = (rhs - part) / piv;
-    if (dual && y && row >= 0) {
-      if (row_deleted) y[row] = eobj / piv; else y[row] += eobj / piv;
-    }
-    if (dual && z) {
-      z[ec] = (row_deleted || !y) ? 0.0 : eobj - piv * y[row];
+    const int32_t ec = w0, row = w1;
+    const double piv = W0, rhs = W1, eobj = W4;
+    const bool row_deleted = W5 != 0.0;
+    if (primal && first) x[ec] = (rhs - sum) / piv;
+    const double y_new = row_deleted ? eobj / piv : yr + eobj / piv;
+    if (dual && y && row >= 0 && first) y[row] = y_new;
+    if (dual && z && first) {
+      z[ec] = (row_deleted || !y) ? 0.0 : eobj - piv * (row >= 0 ? y_new : 0.0);
       if (zret) zret[ec] = 1;
     }
   } else if (type == 0) {  // FixedCol
-    const int32_t col = h.a0;
-    if (primal) x[col] = V[v0];
-    if (dual && z) {
-      double zj = V[v0 + 1];
-      if (y) zj = dot_in_order<true, kRecDotU>(zj, I + i0 + 1, V + v0 + 2, y, i1 - i0, -1);
-      z[col] = zj;
+    const int32_t col = w0;
+    if (primal && first) x[col] = W0;
+    if (dual && z && first) {
+      z[col] = sum;
       if (zret) zret[col] = 1;
     }
-  } else if (type == 1) {  // FixedColInf
+  } else if (type == 1 && first) {  // FixedColInf
     const bool pos_inf = I[i0] > 0;
     const int32_t col = I[i0 + 1];
     const int32_t nrows = static_cast<int32_t>(llround(V[v0]));
@@ -291,7 +423,7 @@ __device__ void replay_one(const gp_tape_dev& T, const gp_orig_dev& O, double* x
       x[col] = ext;
     }
     if (dual && z) { z[col] = 0.0; if (zret) zret[col] = 1; }
-  } else if (type == 14) {  // FmeCol
+  } else if (type == 14 && first) {  // FmeCol
     const int32_t K = I[i0], ec = I[i0 + 1];
     const int32_t L = static_cast<int32_t>(llround(V[v0]));
     int32_t cc = i0 + 3 + K, vp = v0 + 1;
@@ -312,40 +444,40 @@ __device__ void replay_one(const gp_tape_dev& T, const gp_orig_dev& O, double* x
     if (dual && z) { z[ec] = 0.0; if (zret) zret[ec] = 1; }
     if (dual && y) for (int32_t t = 0; t < K; ++t) y[I[i0 + 2 + t]] = 0.0;
   } else if (dual && type == 10) {  // EqToIneq
-    if (y) y[I[i0]] += V[v0];
-  } else if (dual && type == 4 && i1 >= i0 + 1 && v1 >= v0 + 4) {  // DuplicateRow
-    const int32_t kr = I[i0], dr = I[i0 + 1];
-    const double r = V[v0], kal = V[v0 + 1], kau = V[v0 + 2], dal = V[v0 + 3], dau = V[v0 + 4];
-    if (fabs(r) <= tol || !y) return;
-    const double a = dal * r, b = dau * r;
-    const double dsl = r >= 0.0 ? a : b, dsu = r >= 0.0 ? b : a;
-    if (dsl <= kal + tol && kau <= dsu + tol) { y[dr] = 0.0; return; }
+    if (y && first) y[w0] = yr + W0;
+  } else if (dual && type == 4 && w1 >= 0 && h.v1 >= v0 + 4) {  // DuplicateRow
+    const int32_t kr = w0, dr = w1;
+    const double q = W0, kal = W1, kau = W2, dal = W3, dau = W4;
+    if (fabs(q) <= tol || !y) return;
+    const double a = dal * q, b = dau * q;
+    const double dsl = q >= 0.0 ? a : b, dsu = q >= 0.0 ? b : a;
+    if (dsl <= kal + tol && kau <= dsu + tol) {
+      if (first) y[dr] = 0.0;
+      return;
+    }
     if (has_orig) {
-      const int32_t kb = O.a_ptr[kr], db = O.a_ptr[dr];
-      const double ap = dot_in_order<false, kRecDotU>(0.0, O.a_idx + kb, O.a_val + kb, x, O.a_ptr[kr + 1] - kb, -1);
-      const double ad = dot_in_order<false, kRecDotU>(0.0, O.a_idx + db, O.a_val + db, x, O.a_ptr[dr + 1] - db, -1);
+      const int32_t db = O.a_ptr[dr], de = O.a_ptr[dr + 1];
+      const double ap = sum;
+      const double ad = dot_in_order(0.0, 1.0, O.a_idx + db, O.a_val + db, x, de - db, -1);
       const uint8_t ks = row_state(ap, kal, kau, tol), ds = row_state(ad, dal, dau, tol);
       double ydl, ydh, ypl, yph;
       state_interval(ds, &ydl, &ydh);
-      deleted_dual_interval(y[kr], r, ks, &ypl, &yph);
+      deleted_dual_interval(yr, q, ks, &ypl, &yph);
       const double sl = fmax(ydl, ypl), sh = fmin(ydh, yph);
       if (sl <= sh + tol) {
         const double ydn = clamp_inf(0.0, sl, sh);
-        y[kr] = y[kr] - ydn / r;
-        y[dr] = ydn;
+        if (first) { y[kr] = yr - ydn / q; y[dr] = ydn; }
         return;
       }
-      double ypd = y[kr], ydd = 0.0;
-      if (doc_dual_split(y[kr], r, kal, kau, dsl, dsu, tol, &ypd, &ydd)) { y[kr] = ypd; y[dr] = ydd; }
+      double ypd = yr, ydd = 0.0;
+      if (doc_dual_split(yr, q, kal, kau, dsl, dsu, tol, &ypd, &ydd) && first) { y[kr] = ypd; y[dr] = ydd; }
     }
-  } else if (dual && type == 5 && has_orig && i1 >= i0 + 1 && v1 >= v0 + 2) {  // DeletedRow
-    const int32_t row = h.a0, col = h.a1;
-    const double oal = V[v0], oau = V[v0 + 1], aij = V[v0 + 2];
-    const int32_t qb = O.at_ptr[col], qe = O.at_ptr[col + 1];
+  } else if (dual && type == 5 && has_orig && w1 >= 0 && h.v1 >= v0 + 2) {  // DeletedRow
+    const int32_t row = w0, col = w1;
+    const double oal = W0, oau = W1, aij = W2;
     if (fabs(aij) <= tol) return;
-    double gamma = O.c[col];
-    if (y) gamma = dot_in_order<true, kRecDotU>(gamma, O.at_idx + qb, O.at_val + qb, y, qe - qb, row);
-    const double xj = x[col], zbar = z[col];
+    const double gamma = sum;
+    const double xj = xc, zbar = zc;
     const double act = aij * xj;
     const bool ral = pfin(oal) && act <= oal + tol;
     const bool rau = pfin(oau) && act >= oau - tol;
@@ -367,17 +499,14 @@ __device__ void replay_one(const gp_tape_dev& T, const gp_orig_dev& O, double* x
     }
     if (pfin(zl) && pfin(zh) && zl > zh + tol) return;
     const double zn = clamp_inf(zbar, zl, zh);
+    if (!first) return;
     z[col] = zn;
     if (y) y[row] = (gamma - zn) / aij;
     if (zret) zret[col] = 1;
-  } else if (dual && type == 12 && has_orig && i1 >= i0 + 1) {  // BoundChangeTheRow
-    const int32_t col = h.a0, row = h.a1;
-    // Every load that depends only on the record goes out at once; the
-    // decisions below then read registers.
-    const uint8_t col_set = zret ? zret[col] : 1;
-    const double ol = V[v0], ou = V[v0 + 1], nl = V[v0 + 2], nu = V[v0 + 3];
-    const double xj = x[col], zj = z[col];
-    const int32_t qb = O.a_ptr[row], qe = O.a_ptr[row + 1];
+  } else if (dual && type == 12 && has_orig && w1 >= 0) {  // BoundChangeTheRow
+    const int32_t col = w0, row = w1;
+    const double ol = W0, ou = W1, nl = W2, nu = W3;
+    const double xj = xc, zj = zc;
     if (!col_set) return;
     const bool lc = nl > ol + tol, uc = nu < ou - tol;
     if (lc == uc) return;
@@ -389,138 +518,126 @@ __device__ void replay_one(const gp_tape_dev& T, const gp_orig_dev& O, double* x
       if (ok) return;
     }
     if (fabs(xj - implied) > tol) return;
-    // The row's entries are read U at a time with every load in flight
-    // together (the columns of a row are distinct, so the updates of one
-    // chunk are independent); the results are those of the entry-by-entry
-    // loops.  A row of at most U entries is loaded once for both passes.
-    constexpr int U = 16;
-    if (qe <= qb) return;  // an empty row holds no a_ij
-    if (qe - qb <= U) {
-      int32_t kc[U];
-      double a[U];
-#pragma unroll
-      for (int k = 0; k < U; ++k) {
-        const int32_t q = min(qb + k, qe - 1);
-        kc[k] = O.a_idx[q];
-        a[k] = O.a_val[q];
-      }
-      double aij = 0.0;
-#pragma unroll
-      for (int k = U - 1; k >= 0; --k)
-        if (qb + k < qe && kc[k] == col) aij = a[k];
-      if (fabs(aij) <= tol) return;
-      bool on[U];
-      double zk[U];
-#pragma unroll
-      for (int k = 0; k < U; ++k) on[k] = qb + k < qe && kc[k] != col && (!zret || zret[kc[k]]);
-#pragma unroll
-      for (int k = 0; k < U; ++k) zk[k] = z[kc[k]];
-      if (y) y[row] += zj / aij;
-#pragma unroll
-      for (int k = 0; k < U; ++k)
-        if (on[k]) z[kc[k]] = zk[k] - (a[k] / aij) * zj;
-      z[col] = 0.0;
-      if (zret) zret[col] = 1;
-      return;
-    }
+    if (ln.n <= 0) return;  // an empty row holds no a_ij
+    // a_ij is the row's first entry in the column.
     double aij = 0.0;
-    for (int32_t q0 = qb; q0 < qe; q0 += U) {
-      int32_t j[U];
-      double a[U];
-#pragma unroll
-      for (int k = 0; k < U; ++k) {
-        const int32_t q = min(q0 + k, qe - 1);
-        j[k] = O.a_idx[q];
-        a[k] = O.a_val[q];
-      }
-      bool hit = false;
-#pragma unroll
-      for (int k = U - 1; k >= 0; --k)
-        if (q0 + k < qe && j[k] == col) {
-          aij = a[k];
-          hit = true;
-        }
-      if (hit) break;
+    const int g0 = lane_id() & ~(kRecLanes - 1);
+    for (int32_t q = 0; q < ln.n; q += kRecLanes) {
+      const int32_t e = ln.qi + min(q + t, ln.n - 1);
+      const int32_t j = q == 0 ? r.j[0] : q == kRecLanes ? r.j[1] : O.a_idx[e];
+      const uint32_t hit = static_cast<uint32_t>(__ballot(j == col) >> g0) & 0xffffu;
+      if (hit == 0) continue;
+      const double a = q == 0 ? r.a[0] : q == kRecLanes ? r.a[1] : O.a_val[e];
+      aij = __shfl(a, __ffs(hit) - 1, kRecLanes);
+      break;
     }
     if (fabs(aij) <= tol) return;
-    if (y) y[row] += zj / aij;
-    for (int32_t q0 = qb; q0 < qe; q0 += U) {
-      int32_t kc[U];
-      double a[U], zk[U];
-      bool on[U];
+    if (y && first) y[row] = yr + zj / aij;
+    // The row's columns are distinct, so its updates are independent: the
+    // results are those of the entry-by-entry loop.
+    for (int32_t q = 0;;) {
 #pragma unroll
-      for (int k = 0; k < U; ++k) {
-        const int32_t q = min(q0 + k, qe - 1);
-        kc[k] = O.a_idx[q];
-        a[k] = O.a_val[q];
+      for (int c = 0; c < kRecChunks; ++c)
+        if (on[c]) z[r.j[c]] = zk[c] - (r.a[c] / aij) * zj;
+      q += kRecChunks * kRecLanes;
+      if (q >= ln.n) break;
+#pragma unroll
+      for (int c = 0; c < kRecChunks; ++c) {
+        const int32_t e = q + c * kRecLanes + t;
+        r.j[c] = e < ln.n ? O.a_idx[ln.qi + e] : -1;
+        r.a[c] = e < ln.n ? O.a_val[ln.qi + e] : 0.0;
+        const bool other = r.j[c] >= 0 && r.j[c] != col;
+        zk[c] = other ? z[r.j[c]] : 0.0;
+        on[c] = other && (!zret || zret[r.j[c]]);
       }
-#pragma unroll
-      for (int k = 0; k < U; ++k) on[k] = q0 + k < qe && kc[k] != col && (!zret || zret[kc[k]]);
-#pragma unroll
-      for (int k = 0; k < U; ++k) zk[k] = z[kc[k]];
-#pragma unroll
-      for (int k = 0; k < U; ++k)
-        if (on[k]) z[kc[k]] = zk[k] - (a[k] / aij) * zj;
     }
+    if (!first) return;
     z[col] = 0.0;
     if (zret) zret[col] = 1;
   }
 }
 
-// Records begin..end-1 in reverse, one lane (the reference's order).
+// Record k in one go.
+template <bool kDual>
+__device__ __forceinline__ void replay_record(const gp_tape_dev& T, const gp_orig_dev& O, double* x, double* y,
+                                              double* z, uint8_t* zret, int32_t k, double tol) {
+  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
+  const RecHead h = load_head(T, k);
+  const int32_t word = load_word(T, h, t);
+  const RecLine ln = load_line<kDual>(O, h, word, y != nullptr);
+  replay_one<kDual>(T, O, x, y, z, zret, h, word, ln, load_entries(T, O, h, ln, t), tol);
+}
+
+// Records begin..end-1 in reverse, one after the other (the reference's order).
 __global__ void k_replay(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret,
                          int32_t begin, int32_t end, int32_t primal, int32_t dual, double tol) {
-  if (blockIdx.x != 0 || threadIdx.x != 0) return;
-  for (int32_t k = end - 1; k >= begin; --k)
-    replay_one(T, O, x, y, z, zret, load_head(T, k), primal != 0, dual != 0, tol);
+  if (blockIdx.x != 0 || threadIdx.x >= kRecLanes) return;
+  for (int32_t k = end - 1; k >= begin; --k) {
+    if (primal) replay_record<false>(T, O, x, y, z, zret, k, tol);
+    __threadfence_block();  // one lane's stores before the others' loads
+    if (dual) replay_record<true>(T, O, x, y, z, zret, k, tol);
+    __threadfence_block();
+  }
 }
 
 // One level of a dependency-level schedule: its records touch disjoint
-// variables and are replayed one per thread.
-__global__ void __launch_bounds__(kBlock) k_replay_list(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret,
-                              const int32_t* records, int32_t count, int32_t primal, int32_t dual, double tol) {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) replay_one(T, O, x, y, z, zret, load_head(T, records[i]), primal != 0, dual != 0, tol);
+// variables, sixteen lanes each.  Four chains of loads and little else: 6 us
+// for 1,000 to 30,000 records (16 us with a lane per record).
+template <bool kDual>
+__global__ void __launch_bounds__(kBlock)
+    k_replay_list(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret, const int32_t* records,
+                  int32_t count, double tol) {
+  const int32_t i = static_cast<int32_t>(blockIdx.x * (kBlock / kRecLanes) + threadIdx.x / kRecLanes);
+  if (i < count) replay_record<kDual>(T, O, x, y, z, zret, records[i], tol);
 }
 
-// A run of small levels in one workgroup: the threads share each level's
-// records and meet at a barrier before the next level.  All waves of the
-// workgroup run on one CU, so the barrier's workgroup-scope fence makes one
-// level's global stores visible to the next level's loads.
-// The level bounds of up to kLevelChunk levels sit in LDS, and each thread
-// loads the header of its record of the next level while the current level
-// runs, so a level's critical path starts at the tape's indices and values.
-constexpr int kLevelBlock = 512;
-constexpr int kLevelChunk = 4096;
-__global__ void __launch_bounds__(kLevelBlock)
+// A run of small levels in one workgroup, which meets at a barrier after each.
+// All waves of the workgroup run on one CU, so the barrier's workgroup-scope
+// fence makes one level's global stores visible to the next level's loads.
+// A group of lanes has the records of its slot of the next five levels on their
+// way, each a step further than the one of the level after it, so that a level
+// waits only for its x, y, z and zret, and for its stores at the barrier.
+// Bound by that chain: 1,207 dual levels, most of about 31 records, take 4.2 ms
+// (3.5 us each; 11.4 ms with a lane per record and each chain in its turn).
+// Reading x, y, z and zret once a level ahead, to have them in the CU's cache,
+// cost 0.4 ms more.
+template <bool kDual>
+__global__ void __launch_bounds__(GPK_REPLAY_SLOTS * kRecLanes)
     k_replay_levels(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret,
-                    const int32_t* records, const int32_t* level_start, int32_t nlevels, int32_t primal,
-                    int32_t dual, double tol) {
-  __shared__ int32_t s_start[kLevelChunk + 2];
-  const int32_t tid = static_cast<int32_t>(threadIdx.x);
-  for (int32_t c0 = 0; c0 < nlevels; c0 += kLevelChunk) {
-    const int32_t cl = min(kLevelChunk, nlevels - c0);
-    // level_start[c0 .. c0 + cl + 1]: the bounds of this chunk's levels and of the next level
-    const int32_t have = min(cl + 2, nlevels + 1 - c0);
-    for (int32_t t = tid; t < have; t += kLevelBlock) s_start[t] = level_start[c0 + t];
-    __syncthreads();
-    int32_t b = s_start[0], e = s_start[1];
-    RecHead cur{};
-    if (b + tid < e) cur = load_head(T, records[b + tid]);
-    for (int32_t l = 0; l < cl; ++l) {
-      const bool more = l + 1 < have - 1;  // the next level's bounds are in LDS
-      const int32_t nb = more ? s_start[l + 1] : 0, ne = more ? s_start[l + 2] : 0;
-      RecHead nxt{};
-      if (nb + tid < ne) nxt = load_head(T, records[nb + tid]);
-      if (b + tid < e) replay_one(T, O, x, y, z, zret, cur, primal != 0, dual != 0, tol);
-      for (int32_t i = b + tid + kLevelBlock; i < e; i += kLevelBlock)
-        replay_one(T, O, x, y, z, zret, load_head(T, records[i]), primal != 0, dual != 0, tol);
+                    const int32_t* __restrict__ records, const int32_t* __restrict__ level_start, int32_t nlevels,
+                    double tol) {
+  constexpr int kAhead = 5;
+  const int32_t slot = static_cast<int32_t>(threadIdx.x) / kRecLanes;
+  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
+  int32_t begin = level_start[0], end = level_start[min(1, nlevels)];  // of level l + 5
+  RecHead h4 = load_head(T, -1), h3 = h4, h2 = h4, h1 = h4, h0 = h4;
+  int32_t w3 = -1, w2 = -1, w1 = -1, w0 = -1;
+  RecLine n2{0, 0, 0}, n1 = n2, n0 = n2;
+  RecEntries r0 = load_entries(T, O, h0, n0, t);
+#pragma unroll 1
+  for (int32_t l = -kAhead; l < nlevels; ++l) {
+    const int32_t next_end = level_start[min(l + kAhead + 2, nlevels)];
+    const int32_t rec = begin + slot < end ? records[begin + slot] : -1;
+    w3 = load_word(T, h3, t);
+    n2 = load_line<kDual>(O, h2, w2, y != nullptr);
+    const RecEntries r1 = load_entries(T, O, h1, n1, t);
+    if (l >= 0) {
+      replay_one<kDual>(T, O, x, y, z, zret, h0, w0, n0, r0, tol);
       __syncthreads();
-      b = nb;
-      e = ne;
-      cur = nxt;
     }
-    __syncthreads();  // s_start is reloaded for the next chunk
+    h0 = h1;
+    h1 = h2;
+    h2 = h3;
+    h3 = h4;
+    w0 = w1;
+    w1 = w2;
+    w2 = w3;
+    n0 = n1;
+    n1 = n2;
+    r0 = r1;
+    h4 = load_head(T, rec);
+    begin = end;
+    end = next_end;
   }
 }
 
@@ -545,6 +662,31 @@ __device__ inline double project_dual(const gp_orig_dev& O, int32_t col, double 
   return zj;
 }
 
+// The sum over q in [0, count) of val[q] * vec[idx[q]] in q order.  The loads of
+// eight terms go out together, past the end the last term again.
+__device__ inline double column_dot(const int32_t* __restrict__ idx, const double* __restrict__ val,
+                                    const double* __restrict__ vec, int32_t count) {
+  constexpr int U = 8;
+  double s = 0.0;
+#pragma unroll 1
+  for (int32_t q = 0; q < count; q += U) {
+    int32_t j[U];
+    double a[U], v[U];
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      const int32_t p = min(q + k, count - 1);
+      j[k] = idx[p];
+      a[k] = val[p];
+    }
+#pragma unroll
+    for (int k = 0; k < U; ++k) v[k] = vec[j[k]];
+#pragma unroll
+    for (int k = 0; k < U; ++k)
+      if (q + k < count) s += a[k] * v[k];
+  }
+  return s;
+}
+
 __global__ void k_project_duals(gp_orig_dev O, const uint8_t* prot, const double* x, const double* y, double* z,
                                 int32_t n, double tol, int32_t* long_count, int32_t* long_cols) {
   const int32_t col = blockIdx.x * blockDim.x + threadIdx.x;
@@ -554,7 +696,7 @@ __global__ void k_project_duals(gp_orig_dev O, const uint8_t* prot, const double
     long_cols[atomicAdd(long_count, 1)] = col;
     return;
   }
-  const double aty = dot_in_order<false>(0.0, O.at_idx + b, O.at_val + b, y, e - b, -1);
+  const double aty = column_dot(O.at_idx + b, O.at_val + b, y, e - b);
   z[col] = project_dual(O, col, aty, x, tol);
 }
 
@@ -672,16 +814,26 @@ hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double
                            const int32_t* records, int32_t count, int32_t primal, int32_t dual, double tol,
                            hipStream_t stream) {
   if (count <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_replay_list, dim3(grid_for(count)), dim3(kBlock), 0, stream, tape, orig, x, y, z, zret, records,
-                     count, primal, dual, tol);
+  if ((primal != 0) == (dual != 0)) return hipErrorInvalidValue;  // one pass at a time
+  if (dual)
+    hipLaunchKernelGGL(k_replay_list<true>, dim3(grid_for(count, kBlock / kRecLanes)), dim3(kBlock), 0, stream, tape, orig, x, y, z, zret,
+                       records, count, tol);
+  else
+    hipLaunchKernelGGL(k_replay_list<false>, dim3(grid_for(count, kBlock / kRecLanes)), dim3(kBlock), 0, stream, tape, orig, x, y, z, zret,
+                       records, count, tol);
   return hipGetLastError();
 }
 hipError_t gpk_replay_levels(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
                              const int32_t* records, const int32_t* level_start, int32_t nlevels, int32_t primal,
                              int32_t dual, double tol, hipStream_t stream) {
   if (nlevels <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_replay_levels, dim3(1), dim3(kLevelBlock), 0, stream, tape, orig, x, y, z, zret, records,
-                     level_start, nlevels, primal, dual, tol);
+  if ((primal != 0) == (dual != 0)) return hipErrorInvalidValue;
+  if (dual)
+    hipLaunchKernelGGL(k_replay_levels<true>, dim3(1), dim3(GPK_REPLAY_SLOTS * kRecLanes), 0, stream, tape, orig, x, y, z, zret, records,
+                       level_start, nlevels, tol);
+  else
+    hipLaunchKernelGGL(k_replay_levels<false>, dim3(1), dim3(GPK_REPLAY_SLOTS * kRecLanes), 0, stream, tape, orig, x, y, z, zret,
+                       records, level_start, nlevels, tol);
   return hipGetLastError();
 }
 hipError_t gpk_seg_lengths(const int32_t* ptr, const int32_t* list, int32_t count, int32_t* len, hipStream_t stream) {

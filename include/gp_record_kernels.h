@@ -54,9 +54,12 @@ hipError_t gpk_restore_fixed(const int32_t* idx, const double* val, int32_t coun
 hipError_t gpk_replay(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
                       int32_t begin, int32_t end, int32_t primal, int32_t dual, double tol, hipStream_t stream);
 /* Dependency-level replay (the reverse tape order split into levels whose
- * records touch disjoint variables).  gpk_replay_list: the records of one
- * level, one per thread.  gpk_replay_levels: nlevels consecutive levels in one
- * workgroup, level lv being records[level_start[lv] .. level_start[lv+1]). */
+ * records touch disjoint variables), one pass at a time (primal or dual).
+ * gpk_replay_list: the records of one level.  gpk_replay_levels: nlevels
+ * consecutive levels in one workgroup, level lv being
+ * records[level_start[lv] .. level_start[lv+1]), at most GPK_REPLAY_SLOTS of
+ * them (a longer level is given as several); a record of -1 is an empty slot. */
+#define GPK_REPLAY_SLOTS 64
 hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
                            const int32_t* records, int32_t count, int32_t primal, int32_t dual, double tol,
                            hipStream_t stream);

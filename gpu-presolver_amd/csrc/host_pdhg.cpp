@@ -88,24 +88,35 @@ PdhgReport pdhg_solve(const LPInfoGpu& lp, const PdhgOptions& opt, double* x_out
   check_lp_arrays(lp, "pdhg input");
 
   // ---- row blocks of A and AT (from the host copies of the row pointers) ---
-  const auto row_blocks = [&](const presolve::DeviceCsrMatrix& M, DBuf<int32_t>& blk) {
-    const std::vector<int32_t> ptr = cx.to_host(M.rowPtr, static_cast<int64_t>(M.rows) + 1, where);
-    std::vector<int32_t> b(static_cast<size_t>(M.rows) + 1);
-    const int32_t nb = gpk_pdhg_row_blocks(ptr.data(), M.rows, b.data());
-    blk.alloc(static_cast<int64_t>(nb) + 1, where);
-    cx.to_device(blk.get(), b.data(), static_cast<int64_t>(nb) + 1, where);
-    return nb;
+  struct RowPlan {
+    DBuf<gpk_row_block> blk;
+    DBuf<double> part_sum;
+    DBuf<int32_t> part_count;
+    int32_t blocks = 0;
+    gpk_rows rows(gpk_csr M) const { return gpk_rows{M, blk, blocks, part_sum, part_count}; }
   };
-  DBuf<int32_t> blk_a, blk_at;
-  const int32_t nb_a = row_blocks(lp.A, blk_a), nb_at = row_blocks(lp.AT, blk_at);
+  const auto plan_rows = [&](const presolve::DeviceCsrMatrix& M, RowPlan& plan) {
+    const std::vector<int32_t> ptr = cx.to_host(M.rowPtr, static_cast<int64_t>(M.rows) + 1, where);
+    std::vector<gpk_row_block> b(static_cast<size_t>(gpk_pdhg_row_plan(ptr.data(), M.rows, nullptr)) + 1);
+    plan.blocks = gpk_pdhg_row_plan(ptr.data(), M.rows, b.data());
+    plan.blk.alloc(static_cast<int64_t>(b.size()), where);
+    plan.part_sum.alloc(plan.blocks, where);
+    plan.part_count.alloc(plan.blocks, where);
+    cx.to_device(plan.blk.get(), b.data(), static_cast<int64_t>(b.size()), where);
+    CopyBatch().zero(plan.part_count.get(), plan.blocks).run(where);
+  };
+  RowPlan plan_a, plan_at;
+  plan_rows(lp.A, plan_a);
+  plan_rows(lp.AT, plan_at);
+  const int32_t nb_a = plan_a.blocks, nb_at = plan_at.blocks;
 
   // ---- Ruiz equilibration: As = Dr A Dc, ATs = Dc AT Dr ------------------
   DBuf<double> As(nnz, where), ATs(nnz, where), dr(m, where), dc(n, where);
   check(gpk_fill_f64(dr, 1.0, m, s), where);
   check(gpk_fill_f64(dc, 1.0, n, s), where);
   CopyBatch().copy(As.get(), lp.A.nzVal, nnz).copy(ATs.get(), lp.AT.nzVal, nnz).run(where);
-  const gpk_rows A0{view(lp.A, lp.A.nzVal), blk_a, nb_a}, AT0{view(lp.AT, lp.AT.nzVal), blk_at, nb_at};
-  const gpk_rows A{view(lp.A, As), blk_a, nb_a}, AT{view(lp.AT, ATs), blk_at, nb_at};
+  const gpk_rows A0 = plan_a.rows(view(lp.A, lp.A.nzVal)), AT0 = plan_at.rows(view(lp.AT, lp.AT.nzVal));
+  const gpk_rows A = plan_a.rows(view(lp.A, As)), AT = plan_at.rows(view(lp.AT, ATs));
   for (int32_t k = 0; k < opt.ruiz_iters && nnz > 0; ++k) {
     check(gpk_pdhg_ruiz(A, dr, s), where);
     check(gpk_pdhg_ruiz(AT, dc, s), where);
@@ -137,10 +148,8 @@ PdhgReport pdhg_solve(const LPInfoGpu& lp, const PdhgOptions& opt, double* x_out
     DBuf<double> v(n, where), w(m, where);
     check(gpk_pdhg_seed(v, n, s), where);
     for (int32_t k = 0; k < opt.power_iters; ++k) {
-      check(gpk_pdhg_spmv(A, v, w, s), where);
-      check(gpk_pdhg_spmv(AT, w, v, s), where);
-      check(gpk_pdhg_sq_terms(v, nullptr, n, partial, res, s), where);
-      check(gpk_pdhg_normalize(v, res, n, s), where);
+      check(gpk_pdhg_spmv(A, v, k > 0 ? res.get() : nullptr, w, s), where);
+      check(gpk_pdhg_spmv_sq(AT, w, v, partial, res, s), where);
     }
     // ||As^T As v|| with ||v|| = 1 tends to ||As||^2
     norm = std::sqrt(std::sqrt(cx.to_host(res.get(), 1, where)[0]));

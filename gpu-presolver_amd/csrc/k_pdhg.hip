@@ -4,16 +4,29 @@
 // norm estimate, and the residual sums of the KKT check.
 //
 // Every kernel that walks the rows of a CSR matrix (A, or AT for the
-// columns) runs over row blocks built once per solve: either one row,
-// reduced by the whole workgroup (every row of more than
-// GPK_PDHG_LONG_ROW entries gets such a block), or up to 256 consecutive
-// short rows holding at most GPK_PDHG_ENTRY_BUDGET entries, whose products
-// are staged in LDS by coalesced loads and then summed one row per thread.
-// A column of AT with thousands of entries therefore never runs on a single
-// lane.  Each row's sum has a fixed order (given by the blocks, which depend
-// only on the matrix), and every sum over a vector goes through per-block
-// partial sums reduced in block order by one workgroup, so a solve is
-// deterministic run to run.
+// columns) runs over row blocks built once per solve, of at most
+// GPK_PDHG_ENTRY_BUDGET entries each: up to 256 consecutive short rows, whose
+// products are staged in LDS by coalesced loads and then summed one row per
+// thread, or a row of more than GPK_PDHG_LONG_ROW entries or a part of one,
+// reduced by the whole workgroup; the workgroup that finishes a row's last
+// part combines the parts in their order.  A column of AT with thousands of
+// entries therefore runs neither on one lane nor on one workgroup.  Each row's
+// sum has a fixed order (given by the blocks, which depend only on the
+// matrix), and every sum over a vector goes through per-block partial sums
+// reduced in block order by one workgroup, so a solve is deterministic run to
+// run.
+//
+// What bounds them is a chain of memory round trips, a microsecond and more
+// each under load: the block's bounds, its entries (with the row pointers and
+// the vectors of its rows, which need nothing but the bounds), the gathers
+// and, for a split row, the meeting of its parts; on large LPs the gathers
+// (a 128-byte line into the CU's cache for 8 bytes).  A reduced LP of 300,000
+// rows x 450,000 columns, 2.4 million entries: primal half step 31.5 -> 25.2
+// us, dual 18.8 -> 18.1; of 13,000 x 27,000, 33,000 entries: 4.7 -> 3.8 us
+// (a row of up to 256 entries on one thread, the block's row pointers and the
+// rows' vectors in trips of their own before).  Entries or gathers loaded
+// without a place in the caches were 1.2 to 2 times slower: the matrix stays
+// there from launch to launch.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -28,8 +41,10 @@ namespace {
 
 constexpr int kEntryBudget = GPK_PDHG_ENTRY_BUDGET;
 constexpr int kStage = kEntryBudget / kBlock;  // staged entries per thread
-constexpr int kUnroll = 4;                     // chains per thread on a long row
 constexpr int kPartials = 4;
+// A thread sums a row of up to this many entries by itself (about 15 ns each, one
+// after the other); its wave takes a longer one, at about 200 ns a row.
+constexpr int kThreadRow = 32;
 static_assert(kEntryBudget % kBlock == 0, "entry budget in whole strides");
 
 __device__ inline double clampd(double v, double lo, double hi) { return fmin(fmax(v, lo), hi); }
@@ -43,42 +58,85 @@ struct MaxOp {
   static __device__ double combine(double a, double b) { return fmax(a, b); }
 };
 
-// Combination of v over the block in a fixed order (lanes by shuffle tree,
-// waves in index order); every thread gets the result.
-template <class C>
-__device__ inline double block_combine(double v, double* s_w) {
+// Combination of kN values over the block in a fixed order (lanes by shuffle
+// tree, waves in index order); every thread gets the results.
+template <class C, int kN>
+__device__ inline void block_combine(double (&v)[kN], double (*s_w)[kBlock / 64]) {
 #pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v = C::combine(v, __shfl_down(v, d, 64));
-  if (lane_id() == 0) s_w[threadIdx.x >> 6] = v;
+  for (int d = 32; d >= 1; d >>= 1)
+#pragma unroll
+    for (int k = 0; k < kN; ++k) v[k] = C::combine(v[k], __shfl_down(v[k], d, 64));
+  if (lane_id() == 0)
+#pragma unroll
+    for (int k = 0; k < kN; ++k) s_w[k][threadIdx.x >> 6] = v[k];
   __syncthreads();
-  double t = s_w[0];
-  for (int w = 1; w < kBlock / 64; ++w) t = C::combine(t, s_w[w]);
+#pragma unroll
+  for (int k = 0; k < kN; ++k) {
+    v[k] = s_w[k][0];
+#pragma unroll
+    for (int w = 1; w < kBlock / 64; ++w) v[k] = C::combine(v[k], s_w[k][w]);
+  }
   __syncthreads();
-  return t;
+}
+template <class C>
+__device__ inline double block_combine(double v, double (*s_w)[kBlock / 64]) {
+  double t[1] = {v};
+  block_combine<C>(t, s_w);
+  return t[0];
 }
 
 // ---- row operations --------------------------------------------------------
-// elem(p, col, val): the term entry p contributes; row(r, acc, t): consumes
-// the row's combined terms (and, with kTerms, adds its KKT terms to t).
+// elem(col, val, f): the term of an entry, f = factor() the same for all; load(r): the row's own vector entries,
+// loaded before its terms are known; row(r, acc, own, t): consumes the row's
+// combined terms (and, with kTerms, adds its KKT terms to t).
+struct NoOwn {};
 
-// y = M v.
+// y = M v, v scaled by 1 / sqrt(sumsq[0]) where that is given and positive
+// (the power iteration's normalisation, read from device memory so the host
+// need not wait).
 struct OpSpmv {
   using Comb = SumOp;
+  using Own = NoOwn;
   static constexpr bool kTerms = false;
   const double* v;
+  const double* sumsq;
   double* out;
-  __device__ double elem(int32_t, int32_t col, double val) const { return val * v[col]; }
-  __device__ void row(int32_t r, double acc, double*) const { out[r] = acc; }
+  __device__ double factor() const {
+    const double s = sumsq ? sumsq[0] : 0.0;
+    return s > 0.0 ? 1.0 / sqrt(s) : 1.0;
+  }
+  __device__ double elem(int32_t col, double val, double f) const { return val * (v[col] * f); }
+  __device__ Own load(int32_t) const { return {}; }
+  __device__ void row(int32_t r, double acc, Own, double*) const { out[r] = acc; }
+};
+
+// y = M v and, term [0], the sum of y^2.
+struct OpSpmvSq {
+  using Comb = SumOp;
+  using Own = NoOwn;
+  static constexpr bool kTerms = true;
+  const double* v;
+  double* out;
+  __device__ double factor() const { return 1.0; }
+  __device__ double elem(int32_t col, double val, double) const { return val * v[col]; }
+  __device__ Own load(int32_t) const { return {}; }
+  __device__ void row(int32_t r, double acc, Own, double* t) const {
+    out[r] = acc;
+    t[0] += acc * acc;
+  }
 };
 
 // Ruiz: d[r] /= sqrt(max |entry| of row r) (rows without a nonzero keep d).
 struct OpRuiz {
   using Comb = MaxOp;
+  using Own = double;
   static constexpr bool kTerms = false;
   double* d;
-  __device__ double elem(int32_t, int32_t, double val) const { return fabs(val); }
-  __device__ void row(int32_t r, double acc, double*) const {
-    if (acc > 0.0) d[r] /= sqrt(acc);
+  __device__ double factor() const { return 1.0; }
+  __device__ double elem(int32_t, double val, double) const { return fabs(val); }
+  __device__ Own load(int32_t r) const { return d[r]; }
+  __device__ void row(int32_t r, double acc, Own o, double*) const {
+    if (acc > 0.0) d[r] = o / sqrt(acc);
   }
 };
 
@@ -108,20 +166,25 @@ struct OpPrimal {
   double* x_acc;
   const double* x0;
   int32_t j;
-  __device__ double elem(int32_t, int32_t col, double val) const { return val * y[col]; }
-  __device__ void row(int32_t r, double aty, double*) const {
-    const double g = c[r] - aty;
-    const double xo = x[r];
-    const double xn = clampd(xo - step[0] * g, l[r], u[r]);
+  struct Own {
+    double c, l, u, x, acc;  // acc: x0 (Halpern) or the running sum
+  };
+  __device__ double factor() const { return 1.0; }
+  __device__ double elem(int32_t col, double val, double) const { return val * y[col]; }
+  __device__ Own load(int32_t r) const { return {c[r], l[r], u[r], x[r], kHalpern ? x0[r] : x_acc[r]}; }
+  __device__ void row(int32_t r, double aty, const Own& o, double*) const {
+    const double g = o.c - aty;
+    const double xo = o.x;
+    const double xn = clampd(xo - step[0] * g, o.l, o.u);
     const double xb = 2.0 * xn - xo;
     xbar[r] = xb;
     if (kHalpern) {
       const double w = halpern_weight(step, j);
       x_acc[r] = xn;
-      x[r] = w * xb + (1.0 - w) * x0[r];
+      x[r] = w * xb + (1.0 - w) * o.acc;
     } else {
       x[r] = xn;
-      x_acc[r] += xn;
+      x_acc[r] = o.acc + xn;
     }
   }
 };
@@ -142,19 +205,24 @@ struct OpDual {
   double* y_acc;
   const double* y0;
   int32_t j;
-  __device__ double elem(int32_t, int32_t col, double val) const { return val * xbar[col]; }
-  __device__ void row(int32_t i, double ax, double*) const {
+  struct Own {
+    double AL, AU, y, acc;
+  };
+  __device__ double factor() const { return 1.0; }
+  __device__ double elem(int32_t col, double val, double) const { return val * xbar[col]; }
+  __device__ Own load(int32_t i) const { return {AL[i], AU[i], y[i], kHalpern ? y0[i] : y_acc[i]}; }
+  __device__ void row(int32_t i, double ax, const Own& o, double*) const {
     const double sigma = step[1];
-    const double yo = y[i];
+    const double yo = o.y;
     const double yt = yo - sigma * ax;
-    const double yn = yt + sigma * clampd(-yt / sigma, AL[i], AU[i]);
+    const double yn = yt + sigma * clampd(-yt / sigma, o.AL, o.AU);
     if (kHalpern) {
       const double w = halpern_weight(step, j);
       y_acc[i] = yn;
-      y[i] = w * (2.0 * yn - yo) + (1.0 - w) * y0[i];
+      y[i] = w * (2.0 * yn - yo) + (1.0 - w) * o.acc;
     } else {
       y[i] = yn;
-      y_acc[i] += yn;
+      y_acc[i] = o.acc + yn;
     }
   }
 };
@@ -170,12 +238,17 @@ struct OpRowTerms {
   const double* AL;
   const double* AU;
   const double* y;
-  __device__ double elem(int32_t, int32_t col, double val) const { return val * x[col]; }
-  __device__ void row(int32_t i, double ax, double* t) const {
-    const double lo = AL[i], hi = AU[i];
+  struct Own {
+    double AL, AU, y;
+  };
+  __device__ double factor() const { return 1.0; }
+  __device__ double elem(int32_t col, double val, double) const { return val * x[col]; }
+  __device__ Own load(int32_t i) const { return {AL[i], AU[i], y[i]}; }
+  __device__ void row(int32_t, double ax, const Own& o, double* t) const {
+    const double lo = o.AL, hi = o.AU;
     const double viol = ax - clampd(ax, lo, hi);
     t[0] += viol * viol;
-    const double yi = y[i];
+    const double yi = o.y;
     if (yi > 0.0) {
       if (isfinite(lo)) t[1] += yi * lo;
       else t[3] += yi * yi;
@@ -202,144 +275,193 @@ struct OpColTerms {
   const double* u;
   const double* x;
   double* z;
-  __device__ double elem(int32_t, int32_t col, double val) const { return val * y[col]; }
-  __device__ void row(int32_t j, double aty, double* t) const {
-    const double g = c[j] - aty;
-    const bool lo_fin = isfinite(l[j]), hi_fin = isfinite(u[j]);
+  struct Own {
+    double c, l, u, x;
+  };
+  __device__ double factor() const { return 1.0; }
+  __device__ double elem(int32_t col, double val, double) const { return val * y[col]; }
+  __device__ Own load(int32_t j) const { return {c[j], l[j], u[j], x[j]}; }
+  __device__ void row(int32_t j, double aty, const Own& o, double* t) const {
+    const double g = o.c - aty;
+    const bool lo_fin = isfinite(o.l), hi_fin = isfinite(o.u);
     const double lam = clampd(g, hi_fin ? -INFINITY : 0.0, lo_fin ? INFINITY : 0.0);
     if (z) z[j] = lam;
     t[0] += (g - lam) * (g - lam);
-    if (lam > 0.0) t[1] += lam * l[j];
-    else if (lam < 0.0) t[1] += lam * u[j];
-    t[2] += c[j] * c[j];
-    t[3] += c[j] * x[j];
+    if (lam > 0.0) t[1] += lam * o.l;
+    else if (lam < 0.0) t[1] += lam * o.u;
+    t[2] += o.c * o.c;
+    t[3] += o.c * o.x;
   }
 };
 
+// acc with s[b .. e) combined one after the other, four at a time on their way.
+template <class C>
+__device__ inline double combine_in_order(const double* s, int32_t b, int32_t e) {
+  double acc = C::identity();
+  for (int32_t q = b; q < e; q += 4) {
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = s[min(q + k, e - 1)];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      if (q + k < e) acc = C::combine(acc, v[k]);
+  }
+  return acc;
+}
+
 template <class Op>
-__global__ __launch_bounds__(kBlock) void k_rows(gpk_csr M, const int32_t* __restrict__ blk, Op op,
-                                                 double* __restrict__ partial) {
+__global__ __launch_bounds__(kBlock) void k_rows(const int32_t* __restrict__ ptr, const int32_t* __restrict__ idx,
+                                                 const double* __restrict__ val,
+                                                 const gpk_row_block* __restrict__ blk, double* part_sum,
+                                                 int32_t* part_count, double* __restrict__ partial, Op op) {
   using C = typename Op::Comb;
   __shared__ double s_val[kEntryBudget];
-  __shared__ int32_t s_ptr[kBlock + 1];
-  __shared__ double s_w[kBlock / 64];
-  const int32_t r0 = blk[blockIdx.x], r1 = blk[blockIdx.x + 1];
-  const int32_t nr = r1 - r0;
-  const int tid = threadIdx.x;
+  __shared__ double s_w[kPartials][kBlock / 64];
+  __shared__ int32_t s_last;
+  const int32_t bid = static_cast<int32_t>(blockIdx.x);
+  const gpk_row_block b = blk[bid], next = blk[bid + 1];
+  const int32_t nr = next.row - b.row, cnt = next.entry - b.entry;
+  const int tid = static_cast<int>(threadIdx.x);
+  const double factor = op.factor();
   double t[kPartials] = {0.0, 0.0, 0.0, 0.0};
-  if (nr == 1) {
-    // one (long) row: kUnroll independent strided chains per thread (their
-    // loads in flight together), combined in a fixed order, then the tree
-    const int32_t b = M.ptr[r0], e = M.ptr[r0 + 1];
-    double acc[kUnroll];
+  int32_t ci[kStage];
+  double cv[kStage];
+  const int32_t* __restrict__ bi = idx + b.entry;
+  const double* __restrict__ bv = val + b.entry;
 #pragma unroll
-    for (int k = 0; k < kUnroll; ++k) acc[k] = C::identity();
-    int32_t p = b + tid;
-    for (; p + (kUnroll - 1) * kBlock < e; p += kUnroll * kBlock) {
-      int32_t ci[kUnroll];
-      double cv[kUnroll];
-#pragma unroll
-      for (int k = 0; k < kUnroll; ++k) {
-        ci[k] = M.idx[p + k * kBlock];
-        cv[k] = M.val[p + k * kBlock];
-      }
-#pragma unroll
-      for (int k = 0; k < kUnroll; ++k) acc[k] = C::combine(acc[k], op.elem(p + k * kBlock, ci[k], cv[k]));
+  for (int k = 0; k < kStage; ++k) {
+    const int32_t q = tid + k * kBlock;
+    if (q < cnt) {
+      ci[k] = bi[q];
+      cv[k] = bv[q];
     }
-#pragma unroll
-    for (int k = 0; k < kUnroll - 1; ++k) {
-      const int32_t q = p + k * kBlock;
-      if (q < e) acc[k] = C::combine(acc[k], op.elem(q, M.idx[q], M.val[q]));
+  }
+  const bool mine = tid < (b.parts > 0 ? 1 : nr);
+  const int32_t r = b.row + (mine ? tid : 0);
+  typename Op::Own own{};
+  int32_t pb = 0, pe = 0;
+  if (mine) {
+    own = op.load(r);
+    if (b.parts == 0) {
+      pb = ptr[r] - b.entry;
+      pe = ptr[r + 1] - b.entry;
     }
-    double a = acc[0];
+  }
 #pragma unroll
-    for (int k = 1; k < kUnroll; ++k) a = C::combine(a, acc[k]);
+  for (int k = 0; k < kStage; ++k)
+    if (tid + k * kBlock < cnt) cv[k] = op.elem(ci[k], cv[k], factor);
+  if (b.parts == 0) {
+#pragma unroll
+    for (int k = 0; k < kStage; ++k)
+      if (tid + k * kBlock < cnt) s_val[tid + k * kBlock] = cv[k];
+    __syncthreads();
+    double acc = C::identity();
+    const bool by_wave = pe - pb > kThreadRow;
+    if (!by_wave) acc = combine_in_order<C>(s_val, pb, pe);
+    for (uint64_t todo = __ballot(by_wave); todo != 0; todo &= todo - 1) {
+      const int q = __ffsll(static_cast<unsigned long long>(todo)) - 1;
+      const int32_t rb = __shfl(pb, q, 64), re = __shfl(pe, q, 64);
+      double a = C::identity();
+      for (int32_t p = rb + lane_id(); p < re; p += 64) a = C::combine(a, s_val[p]);
+#pragma unroll
+      for (int d = 32; d >= 1; d >>= 1) a = C::combine(a, __shfl_xor(a, d, 64));
+      if (lane_id() == q) acc = a;
+    }
+    if (mine) op.row(r, acc, own, t);
+  } else {
+    // one row or a part of one: each thread its entries, then the tree
+    double a = C::identity();
+#pragma unroll
+    for (int k = 0; k < kStage; ++k)
+      if (tid + k * kBlock < cnt) a = C::combine(a, cv[k]);
     a = block_combine<C>(a, s_w);
-    if (tid == 0) op.row(r0, a, t);
-  } else if (nr > 1) {
-    const int32_t e0 = M.ptr[r0];
-    const int32_t cnt = M.ptr[r1] - e0;
-    if (nr <= kBlock && cnt <= kEntryBudget) {
-      if (tid < nr) s_ptr[tid] = M.ptr[r0 + tid] - e0;
-      if (tid == 0) s_ptr[nr] = cnt;
-      // every load of the thread's (up to kStage) entries issued before the
-      // gathers, every gather before the LDS stores
-      int32_t ci[kStage];
-      double cv[kStage];
-#pragma unroll
-      for (int k = 0; k < kStage; ++k) {
-        const int32_t q = tid + k * kBlock;
-        if (q < cnt) {
-          ci[k] = M.idx[e0 + q];
-          cv[k] = M.val[e0 + q];
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < kStage; ++k) {
-        const int32_t q = tid + k * kBlock;
-        if (q < cnt) cv[k] = op.elem(e0 + q, ci[k], cv[k]);
-      }
-#pragma unroll
-      for (int k = 0; k < kStage; ++k) {
-        const int32_t q = tid + k * kBlock;
-        if (q < cnt) s_val[q] = cv[k];
+    bool whole = b.parts == 1;
+    if (!whole) {
+      // The sum is exchanged, and counted once the exchange has answered (the
+      // count's increment is made to depend on it): it is then where every
+      // XCD's atomic loads see it, and the sums are all that the last part
+      // reads of the others.  A release instead writes back the L2's dirty lines
+      // at every part: 57 us for a primal half step that takes 27 this way.
+      if (tid == 0) {
+        const long long old = __hip_atomic_exchange(reinterpret_cast<long long*>(part_sum) + bid,
+                                                    __double_as_longlong(a), __ATOMIC_RELAXED,
+                                                    __HIP_MEMORY_SCOPE_AGENT);
+        int32_t one = 1;
+        asm volatile("" : "+v"(one) : "v"(old) : "memory");
+        s_last = __hip_atomic_fetch_add(part_count + (bid - b.part), one, __ATOMIC_RELAXED,
+                                        __HIP_MEMORY_SCOPE_AGENT) == b.parts - 1;
       }
       __syncthreads();
-      if (tid < nr) {
-        double acc = C::identity();
-        for (int32_t q = s_ptr[tid]; q < s_ptr[tid + 1]; ++q) acc = C::combine(acc, s_val[q]);
-        op.row(r0 + tid, acc, t);
+      whole = s_last != 0;
+      if (whole) {
+        a = C::identity();
+        for (int32_t k = tid; k < b.parts; k += kBlock)
+          a = C::combine(a, __hip_atomic_load(part_sum + (bid - b.part + k), __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT));
+        a = block_combine<C>(a, s_w);
+        if (tid == 0)  // for the next launch
+          __hip_atomic_store(part_count + (bid - b.part), 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-    } else {
-      // not a block the host builds (more rows or entries than the block
-      // stages): still correct, one row per thread from global memory
-      for (int32_t r = r0 + tid; r < r1; r += kBlock) {
-        double acc = C::identity();
-        for (int32_t p = M.ptr[r]; p < M.ptr[r + 1]; ++p) acc = C::combine(acc, op.elem(p, M.idx[p], M.val[p]));
-        op.row(r, acc, t);
+    }
+    if (whole && tid == 0) op.row(r, a, own, t);
+    if constexpr (Op::kTerms) {
+      // A row's terms stand in its first part's place, whichever block was
+      // the last; the other places are empty.
+      if (tid < kPartials) {
+        if (b.part > 0) partial[static_cast<int64_t>(bid) * kPartials + tid] = 0.0;
       }
+      if (whole && tid == 0)
+#pragma unroll
+        for (int k = 0; k < kPartials; ++k) partial[static_cast<int64_t>(bid - b.part) * kPartials + k] = t[k];
+      return;
     }
   }
   if constexpr (Op::kTerms) {
-    for (int k = 0; k < kPartials; ++k) {
-      const double v = block_combine<SumOp>(t[k], s_w);
-      if (tid == 0) partial[static_cast<int64_t>(blockIdx.x) * kPartials + k] = v;
-    }
+    block_combine<SumOp>(t, s_w);
+    if (tid == 0)
+#pragma unroll
+      for (int k = 0; k < kPartials; ++k) partial[static_cast<int64_t>(bid) * kPartials + k] = t[k];
   }
 }
 
 // out[p] = M.val[p] * drow[row(p)] * dcol[idx[p]], over the same row blocks
-// (entries strided over the block; the row of an entry of a multi-row block
-// by binary search in the block's row pointers).
-__global__ __launch_bounds__(kBlock) void k_rows_scale(gpk_csr M, const int32_t* __restrict__ blk,
+// (the threads of a block's rows write each entry's row into LDS).
+__global__ __launch_bounds__(kBlock) void k_rows_scale(const int32_t* __restrict__ ptr,
+                                                       const int32_t* __restrict__ idx,
+                                                       const double* __restrict__ val,
+                                                       const gpk_row_block* __restrict__ blk,
                                                        const double* __restrict__ drow,
                                                        const double* __restrict__ dcol, double* __restrict__ out) {
-  __shared__ int32_t s_ptr[kBlock + 1];
-  const int32_t r0 = blk[blockIdx.x], r1 = blk[blockIdx.x + 1];
-  const int32_t nr = r1 - r0;
-  const int tid = threadIdx.x;
-  if (nr == 1) {
-    const double dr = drow[r0];
-    for (int32_t p = M.ptr[r0] + tid; p < M.ptr[r0 + 1]; p += kBlock) out[p] = M.val[p] * dr * dcol[M.idx[p]];
-  } else if (nr > 1 && nr <= kBlock) {
-    const int32_t e0 = M.ptr[r0];
-    const int32_t cnt = M.ptr[r1] - e0;
-    if (tid < nr) s_ptr[tid] = M.ptr[r0 + tid] - e0;
-    if (tid == 0) s_ptr[nr] = cnt;
-    __syncthreads();
-    for (int32_t q = tid; q < cnt; q += kBlock) {
-      int32_t lo = 0, hi = nr - 1;  // last k with s_ptr[k] <= q
-      while (lo < hi) {
-        const int32_t mid = (lo + hi + 1) >> 1;
-        if (s_ptr[mid] <= q) lo = mid;
-        else hi = mid - 1;
-      }
-      const int32_t p = e0 + q;
-      out[p] = M.val[p] * drow[r0 + lo] * dcol[M.idx[p]];
+  __shared__ uint8_t s_row[kEntryBudget];
+  __shared__ double s_d[kBlock];
+  const gpk_row_block b = blk[blockIdx.x], next = blk[blockIdx.x + 1];
+  const int32_t nr = b.parts > 0 ? 1 : next.row - b.row, cnt = next.entry - b.entry;
+  const int tid = static_cast<int>(threadIdx.x);
+  int32_t ci[kStage];
+  double cv[kStage];
+#pragma unroll
+  for (int k = 0; k < kStage; ++k) {
+    const int32_t q = tid + k * kBlock;
+    if (q < cnt) {
+      ci[k] = idx[b.entry + q];
+      cv[k] = val[b.entry + q];
     }
-  } else if (nr > kBlock) {
-    for (int32_t r = r0 + tid; r < r1; r += kBlock)
-      for (int32_t p = M.ptr[r]; p < M.ptr[r + 1]; ++p) out[p] = M.val[p] * drow[r] * dcol[M.idx[p]];
+  }
+  if (tid < nr) {
+    s_d[tid] = drow[b.row + tid];
+    if (b.parts == 0)
+      for (int32_t q = ptr[b.row + tid] - b.entry, e = ptr[b.row + tid + 1] - b.entry; q < e; ++q)
+        s_row[q] = static_cast<uint8_t>(tid);
+  }
+  double g[kStage];
+#pragma unroll
+  for (int k = 0; k < kStage; ++k)
+    if (tid + k * kBlock < cnt) g[k] = dcol[ci[k]];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kStage; ++k) {
+    const int32_t q = tid + k * kBlock;
+    if (q < cnt) out[b.entry + q] = cv[k] * s_d[b.parts > 0 ? 0 : s_row[q]] * g[k];
   }
 }
 
@@ -362,32 +484,23 @@ __global__ void k_pdhg_scale_vec(const double* __restrict__ v, const double* __r
   if (i < n) out[i] = mul ? v[i] * d[i] : v[i] / d[i];
 }
 
-// v *= 1 / sqrt(sumsq[0]) when sumsq[0] > 0 (the power iteration's
-// normalisation, read from device memory so the host need not wait).
-__global__ void k_pdhg_normalize(double* __restrict__ v, const double* __restrict__ sumsq, int32_t n) {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  const double s = sumsq[0];
-  if (i < n && s > 0.0) v[i] *= 1.0 / sqrt(s);
-}
-
 // Sum of (a - b)^2 and of a^2 (b may be null) into partials [0], [1].
 __global__ __launch_bounds__(kBlock) void k_pdhg_sq_terms(const double* __restrict__ a,
                                                           const double* __restrict__ b, int32_t n,
                                                           double* __restrict__ partial) {
-  __shared__ double s_w[kBlock / 64];
+  __shared__ double s_w[2][kBlock / 64];
   const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  double d2 = 0.0, a2 = 0.0;
+  double t[2] = {0.0, 0.0};
   if (i < n) {
     const double d = a[i] - (b ? b[i] : 0.0);
-    d2 = d * d;
-    a2 = a[i] * a[i];
+    t[0] = d * d;
+    t[1] = a[i] * a[i];
   }
-  d2 = block_combine<SumOp>(d2, s_w);
-  a2 = block_combine<SumOp>(a2, s_w);
+  block_combine<SumOp>(t, s_w);
   if (threadIdx.x == 0) {
     double* o = partial + static_cast<int64_t>(blockIdx.x) * kPartials;
-    o[0] = d2;
-    o[1] = a2;
+    o[0] = t[0];
+    o[1] = t[1];
     o[2] = 0.0;
     o[3] = 0.0;
   }
@@ -397,13 +510,26 @@ __global__ __launch_bounds__(kBlock) void k_pdhg_sq_terms(const double* __restri
 // workgroup: thread t sums blocks t, t + 256, ..., then the block tree).
 __global__ __launch_bounds__(kBlock) void k_pdhg_reduce(const double* __restrict__ partial, int32_t blocks,
                                                         double* __restrict__ out) {
-  __shared__ double s_w[kBlock / 64];
-  for (int k = 0; k < kPartials; ++k) {
-    double t = 0.0;
-    for (int32_t b = threadIdx.x; b < blocks; b += kBlock) t += partial[static_cast<int64_t>(b) * kPartials + k];
-    const double v = block_combine<SumOp>(t, s_w);
-    if (threadIdx.x == 0) out[k] = v;
+  __shared__ double s_w[kPartials][kBlock / 64];
+  constexpr int kLook = 4;
+  double t[kPartials] = {};
+  for (int32_t b = threadIdx.x; b < blocks; b += kLook * kBlock) {
+    double v[kLook][kPartials];
+#pragma unroll
+    for (int u = 0; u < kLook; ++u)
+#pragma unroll
+      for (int k = 0; k < kPartials; ++k)
+        if (b + u * kBlock < blocks) v[u][k] = partial[static_cast<int64_t>(b + u * kBlock) * kPartials + k];
+#pragma unroll
+    for (int u = 0; u < kLook; ++u)
+#pragma unroll
+      for (int k = 0; k < kPartials; ++k)
+        if (b + u * kBlock < blocks) t[k] += v[u][k];
   }
+  block_combine<SumOp>(t, s_w);
+  if (threadIdx.x == 0)
+#pragma unroll
+    for (int k = 0; k < kPartials; ++k) out[k] = t[k];
 }
 
 // Start vector of the power iteration: 0.5 + frac(i * golden ratio).
@@ -431,11 +557,25 @@ __global__ void k_pdhg_project_zero(const double* __restrict__ l, const double* 
   if (j < n) x[j] = clampd(0.0, l[j], u[j]);
 }
 
+// The row after the last of the block that starts at row r.
+int32_t block_end(const int32_t* ptr, int32_t rows, int32_t r) {
+  if (ptr[r + 1] - ptr[r] > GPK_PDHG_LONG_ROW) return r + 1;
+  const int32_t start = r;
+  int32_t cnt = 0;
+  while (r < rows && r - start < kBlock) {
+    const int32_t len = ptr[r + 1] - ptr[r];
+    if (len > GPK_PDHG_LONG_ROW || cnt + len > kEntryBudget) break;
+    cnt += len;
+    ++r;
+  }
+  return r;
+}
+
 template <class Op>
 hipError_t launch_rows(const gpk_rows& R, const Op& op, double* partial, hipStream_t s) {
   if (R.blocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rows<Op>, dim3(static_cast<unsigned>(R.blocks)), dim3(kBlock), 0, s, R.M, R.blk, op,
-                     partial);
+  hipLaunchKernelGGL(k_rows<Op>, dim3(static_cast<unsigned>(R.blocks)), dim3(kBlock), 0, s, R.M.ptr, R.M.idx, R.M.val,
+                     R.blk, R.part_sum, R.part_count, partial, op);
   return hipGetLastError();
 }
 
@@ -449,24 +589,26 @@ hipError_t launch_reduce(const double* partial, int32_t blocks, double* out, hip
 extern "C" {
 
 int32_t gpk_pdhg_row_blocks(const int32_t* ptr, int32_t rows, int32_t* blk) {
-  int32_t nb = 0, r = 0;
+  int32_t nb = 0;
   if (blk) blk[0] = 0;
-  while (r < rows) {
-    if (ptr[r + 1] - ptr[r] > GPK_PDHG_LONG_ROW) {
-      ++r;
-    } else {
-      const int32_t r_start = r;
-      int32_t cnt = 0;
-      while (r < rows && r - r_start < kBlock) {
-        const int32_t len = ptr[r + 1] - ptr[r];
-        if (len > GPK_PDHG_LONG_ROW || cnt + len > kEntryBudget) break;
-        cnt += len;
-        ++r;
-      }
-    }
+  for (int32_t r = 0; r < rows;) {
+    r = block_end(ptr, rows, r);
     ++nb;
     if (blk) blk[nb] = r;
   }
+  return nb;
+}
+
+int32_t gpk_pdhg_row_plan(const int32_t* ptr, int32_t rows, gpk_row_block* out) {
+  int32_t nb = 0;
+  for (int32_t r = 0; r < rows;) {
+    const int32_t end = block_end(ptr, rows, r), entries = ptr[end] - ptr[r];
+    const int32_t parts = end - r > 1 ? 0 : entries > kEntryBudget ? (entries - 1) / kEntryBudget + 1 : 1;
+    for (int32_t k = 0; k < (parts > 0 ? parts : 1); ++k, ++nb)
+      if (out) out[nb] = gpk_row_block{r, ptr[r] + k * kEntryBudget, k, parts};
+    r = end;
+  }
+  if (out) out[nb] = gpk_row_block{rows, rows > 0 ? ptr[rows] : 0, 0, 0};
   return nb;
 }
 
@@ -501,28 +643,28 @@ hipError_t gpk_pdhg_mul(const double* x, const double* d, double* out, int32_t n
   return hipGetLastError();
 }
 
-hipError_t gpk_pdhg_spmv(gpk_rows M, const double* x, double* y, hipStream_t s) {
-  return launch_rows(M, OpSpmv{x, y}, nullptr, s);
+hipError_t gpk_pdhg_spmv(gpk_rows M, const double* x, const double* sumsq, double* y, hipStream_t s) {
+  return launch_rows(M, OpSpmv{x, sumsq, y}, nullptr, s);
+}
+
+hipError_t gpk_pdhg_spmv_sq(gpk_rows M, const double* x, double* y, double* partial, double* out, hipStream_t s) {
+  const hipError_t e = launch_rows(M, OpSpmvSq{x, y}, partial, s);
+  if (e != hipSuccess) return e;
+  return launch_reduce(partial, M.blocks > 0 ? M.blocks : 0, out, s);
 }
 
 hipError_t gpk_pdhg_ruiz(gpk_rows M, double* d, hipStream_t s) { return launch_rows(M, OpRuiz{d}, nullptr, s); }
 
 hipError_t gpk_pdhg_scale_csr(gpk_rows M, const double* drow, const double* dcol, double* out, hipStream_t s) {
   if (M.blocks <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_rows_scale, dim3(static_cast<unsigned>(M.blocks)), dim3(kBlock), 0, s, M.M, M.blk, drow, dcol,
-                     out);
+  hipLaunchKernelGGL(k_rows_scale, dim3(static_cast<unsigned>(M.blocks)), dim3(kBlock), 0, s, M.M.ptr, M.M.idx, M.M.val,
+                     M.blk, drow, dcol, out);
   return hipGetLastError();
 }
 
 hipError_t gpk_pdhg_scale_vec(const double* v, const double* d, double* out, int32_t n, int32_t mul, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_pdhg_scale_vec, dim3(grid_for(n)), dim3(kBlock), 0, s, v, d, out, n, mul);
-  return hipGetLastError();
-}
-
-hipError_t gpk_pdhg_normalize(double* v, const double* sumsq, int32_t n, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_pdhg_normalize, dim3(grid_for(n)), dim3(kBlock), 0, s, v, sumsq, n);
   return hipGetLastError();
 }
 

@@ -654,23 +654,34 @@ hipError_t gpk_screen_structural_prefix(const int32_t* ptr, const int32_t* idx, 
  * step[0] = tau (primal), step[1] = sigma (dual) are read from device memory
  * so a captured run of iterations can be replayed after the host changes
  * them.  Row kernels take a gpk_rows: the CSR matrix (A, or AT for the
- * columns) and its row blocks, built on the host from the row pointers by
- * gpk_pdhg_row_blocks: a block is one row (every row of more than
- * GPK_PDHG_LONG_ROW entries is alone, reduced by the whole workgroup) or up
- * to 256 consecutive shorter rows with at most GPK_PDHG_ENTRY_BUDGET entries
- * in all (staged in LDS).
+ * columns) and its row blocks, built on the host from the row pointers: a
+ * block is one row (every row of more than GPK_PDHG_LONG_ROW entries is alone,
+ * reduced by the whole workgroup) or up to 256 consecutive shorter rows with at
+ * most GPK_PDHG_ENTRY_BUDGET entries in all (staged in LDS); gpk_pdhg_row_plan
+ * gives a row of more than that in parts, to a workgroup each.
  * ====================================================================== */
 #define GPK_PDHG_LONG_ROW 256
 #define GPK_PDHG_ENTRY_BUDGET 2048
+/* Block k: entries [entry, blk[k + 1].entry) of M, those of the rows
+ * [row, blk[k + 1].row) where parts is 0, otherwise part `part` of the `parts`
+ * parts of row `row`, whose blocks follow each other. */
+typedef struct gpk_row_block {
+  int32_t row, entry, part, parts;
+} gpk_row_block;
 typedef struct gpk_rows {
   gpk_csr M;
-  const int32_t* blk; /* device: blocks + 1 row starts, blk[blocks] = M.rows */
+  const gpk_row_block* blk; /* device: blocks + 1, the last {M.rows, M.nnz, 0, 0} */
   int32_t blocks;
+  double* part_sum;    /* device: blocks words of scratch, for one launch at a time */
+  int32_t* part_count; /* device: blocks words, 0 before the first launch and after each */
 } gpk_rows;
 /* Host: the row blocks of a CSR from its host row pointers (rows + 1);
  * writes blocks + 1 starts to blk (room for rows + 1; NULL only counts) and
  * returns the block count. */
 int32_t gpk_pdhg_row_blocks(const int32_t* ptr, int32_t rows, int32_t* blk);
+/* Host: those blocks with the long rows in parts, blocks + 1 entries (NULL only
+ * counts). */
+int32_t gpk_pdhg_row_plan(const int32_t* ptr, int32_t rows, gpk_row_block* out);
 /* `iterations` PDHG steps from z = (x, y): the PDHG point T(z) is
  * xn = proj_[l,u](x - tau (c - A^T y)), xbar = 2 xn - x, yn the projected
  * dual step on xbar.  halpern == 0 (averaged PDHG): z <- T(z) and x_acc,
@@ -686,7 +697,12 @@ hipError_t gpk_pdhg_iterations(gpk_rows A, gpk_rows AT, const double* c, const d
 hipError_t gpk_pdhg_axpby(double a, const double* x, double b, const double* y, double* out, int32_t n,
                           hipStream_t stream);
 hipError_t gpk_pdhg_mul(const double* x, const double* d, double* out, int32_t n, hipStream_t stream);
-hipError_t gpk_pdhg_spmv(gpk_rows M, const double* x, double* y, hipStream_t stream);
+/* y = M x, x times 1 / sqrt(sumsq[0]) where sumsq (device memory, may be null)
+ * is given and positive. */
+hipError_t gpk_pdhg_spmv(gpk_rows M, const double* x, const double* sumsq, double* y, hipStream_t stream);
+/* y = M x and out[0] = the sum of y^2 (partial as for the *_terms). */
+hipError_t gpk_pdhg_spmv_sq(gpk_rows M, const double* x, double* y, double* partial, double* out,
+                            hipStream_t stream);
 /* One Ruiz step: d[i] /= sqrt(max |M.val[p]| over row i) (rows with no
  * nonzero keep d). */
 hipError_t gpk_pdhg_ruiz(gpk_rows M, double* d, hipStream_t stream);
@@ -695,8 +711,6 @@ hipError_t gpk_pdhg_scale_csr(gpk_rows M, const double* drow, const double* dcol
 /* out = v * d (mul != 0) or v / d. */
 hipError_t gpk_pdhg_scale_vec(const double* v, const double* d, double* out, int32_t n, int32_t mul,
                               hipStream_t stream);
-/* v *= 1 / sqrt(sumsq[0]) when sumsq[0] > 0 (sumsq in device memory). */
-hipError_t gpk_pdhg_normalize(double* v, const double* sumsq, int32_t n, hipStream_t stream);
 /* Doubles of partial sums a *_terms launch over `blocks` workgroups needs
  * (row blocks for row/col terms, ceil(n / 256) for sq_terms). */
 int32_t gpk_pdhg_partials(int32_t blocks);

@@ -315,6 +315,46 @@ class CopyBatch {
 };
 
 // ---- prepared postsolve ------------------------------------------------------
+// A host array of the caller's.
+template <class T>
+struct HostSpan {
+  const T* p = nullptr;
+  size_t n = 0;
+  HostSpan() = default;
+  HostSpan(const T* data, size_t count) : p(data), n(count) {}
+  HostSpan(const std::vector<T>& v) : p(v.data()), n(v.size()) {}
+  size_t size() const { return n; }
+  bool empty() const { return n == 0; }
+  const T* data() const { return p; }
+  const T* begin() const { return p; }
+  const T* end() const { return p + n; }
+  const T& operator[](size_t k) const { return p[k]; }
+  const T& back() const { return p[n - 1]; }
+};
+struct TapeView {
+  HostSpan<int32_t> types, index_starts, value_starts, indices;
+  HostSpan<double> vals;
+};
+// What a postsolve reads of a record, where it stands.
+struct RecordView {
+  int32_t m0 = 0, n0 = 0, m1 = 0, n1 = 0;
+  HostSpan<int32_t> row_red2org, col_red2org, fixed_idx;
+  HostSpan<double> fixed_val;
+  TapeView tape;
+  size_t dual_modes = 0;
+  HostSpan<presolve::StructuralL1PrimalRecoveryStep> structural_primal_recoveries;
+  HostSpan<presolve::AntipodalComponentPrimalRecoveryStep> antipodal_component_recoveries;
+  HostSpan<presolve::PrimalRecoveryCheckpoint> primal_recovery_timeline;
+  RecordView() = default;
+  RecordView(const presolve::PresolveRecordGpu& r)
+      : m0(r.m0), n0(r.n0), m1(r.m1), n1(r.n1), row_red2org(r.row_red2org), col_red2org(r.col_red2org),
+        fixed_idx(r.fixed_idx), fixed_val(r.fixed_val),
+        tape{r.tape.types, r.tape.index_starts, r.tape.value_starts, r.tape.indices, r.tape.vals},
+        dual_modes(r.tape.dual_modes.size()), structural_primal_recoveries(r.structural_primal_recoveries),
+        antipodal_component_recoveries(r.antipodal_component_recoveries),
+        primal_recovery_timeline(r.primal_recovery_timeline) {}
+};
+
 // Everything a postsolve of one record needs that does not depend on the
 // reduced point: the validated, uploaded tape and record maps, the two replay
 // schedules (built on the host and uploaded), the protected-column mask and
@@ -324,11 +364,10 @@ class PostsolvePlan {
  public:
   // Throws std::runtime_error when the record or the original LP cannot be
   // postsolved (the checks of postsolve_gpu).
-  static void validate(const presolve::PresolveRecordGpu& record, const presolve::LPInfoGpu* original);
+  static void validate(const RecordView& record, const presolve::LPInfoGpu* original);
   // original_l: the original lower bounds the max-slack recovery reads
   // (null: original->l, or none).
-  PostsolvePlan(const presolve::PresolveRecordGpu& record, const presolve::LPInfoGpu* original,
-                const double* original_l = nullptr);
+  PostsolvePlan(const RecordView& record, const presolve::LPInfoGpu* original, const double* original_l = nullptr);
   ~PostsolvePlan();
   PostsolvePlan(const PostsolvePlan&) = delete;
   PostsolvePlan& operator=(const PostsolvePlan&) = delete;

@@ -239,6 +239,36 @@ std::vector<T> host_vec(const T* p, int32_t n, const char* what) {
   return n > 0 ? std::vector<T>(p, p + n) : std::vector<T>{};
 }
 
+template <class T>
+amd::HostSpan<T> host_span(const T* p, int32_t n, const char* what) {
+  if (n < 0) throw InvalidArgument(std::string(what) + ": negative length");
+  if (n > 0 && p == nullptr) throw InvalidArgument(std::string(what) + ": null pointer");
+  return amd::HostSpan<T>(p, static_cast<size_t>(n));
+}
+
+// The caller's record where it stands, for a call that is done with it when it
+// returns (the maps and fixed columns of a large LP are tens of megabytes).
+amd::RecordView view_record(const gp_record_view& v) {
+  require(v.m0 >= 0 && v.n0 >= 0 && v.m1 >= 0 && v.n1 >= 0 && v.m1 <= v.m0 && v.n1 <= v.n0,
+          "record: invalid dimensions");
+  amd::RecordView r;
+  r.m0 = v.m0;
+  r.n0 = v.n0;
+  r.m1 = v.m1;
+  r.n1 = v.n1;
+  r.row_red2org = host_span(v.row_red2org, v.m1, "record.row_red2org");
+  r.col_red2org = host_span(v.col_red2org, v.n1, "record.col_red2org");
+  r.fixed_idx = host_span(v.fixed_idx, v.fixed_count, "record.fixed_idx");
+  r.fixed_val = host_span(v.fixed_val, v.fixed_count, "record.fixed_val");
+  r.tape.types = host_span(v.tape_types, v.tape_count, "record.tape_types");
+  r.tape.index_starts = host_span(v.tape_index_starts, v.tape_count + 1, "record.tape_index_starts");
+  r.tape.value_starts = host_span(v.tape_value_starts, v.tape_count + 1, "record.tape_value_starts");
+  r.dual_modes = static_cast<size_t>(v.tape_count);
+  r.tape.indices = host_span(v.tape_indices, v.tape_index_count, "record.tape_indices");
+  r.tape.vals = host_span(v.tape_vals, v.tape_value_count, "record.tape_vals");
+  return r;
+}
+
 PresolveRecordGpu to_record(const gp_record_view& v) {
   require(v.m0 >= 0 && v.n0 >= 0 && v.m1 >= 0 && v.n1 >= 0 && v.m1 <= v.m0 && v.n1 <= v.n0,
           "record: invalid dimensions");
@@ -863,7 +893,7 @@ gp_status gp_postsolve(const gp_record_view* record, const double* x_red, const 
                        const gp_lp* original, double* x_org, double* y_org, double* z_org) {
   return guarded([&] {
     require(record != nullptr, "null record");
-    const PresolveRecordGpu rec = to_record(*record);
+    const amd::RecordView rec = view_record(*record);
     require(rec.n0 == 0 || (x_org && z_org), "null x_org/z_org");
     require(rec.m0 == 0 || y_org, "null y_org");
     LPInfoGpu orig;

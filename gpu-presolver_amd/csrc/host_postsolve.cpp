@@ -2,6 +2,7 @@
 // scatter of the reduced solution, fixed-value restore, reverse tape replay
 // (primal pass, then dual pass) and the final column-dual projection.
 #include <hip/hip_runtime_api.h>
+#include <sys/mman.h>
 
 #include <algorithm>
 #include <chrono>
@@ -10,8 +11,10 @@
 #include <cstdlib>
 #include <limits>
 #include <memory>
+#include <new>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "gp_host.hpp"
@@ -42,7 +45,7 @@ struct DeviceTape {
   DBuf<int32_t> types, index_starts, value_starts, indices;
   DBuf<double> vals;
   gp_tape_dev view{};
-  explicit DeviceTape(const PostsolveTape& t) {
+  explicit DeviceTape(const amd::TapeView& t) {
     auto& c = ctx();
     const int32_t count = static_cast<int32_t>(t.types.size());
     if (t.index_starts.size() != t.types.size() + 1 || t.value_starts.size() != t.types.size() + 1 ||
@@ -88,13 +91,54 @@ gp_orig_dev orig_view(const LPInfoGpu* o) {
 // the serial order, so the results are the serial replay's, bit for bit.
 // Variables: column c (x, z and z_retrieved) -> c, row r (y) -> n0 + r.
 
+// Zeroed words of which few are touched: pages of the kernel's, cleared when
+// they are first touched, two megabytes at a time where the system does that
+// (a vector clears them all, a page fault for each four kilobytes).
+class HostWords {
+ public:
+  HostWords() = default;
+  explicit HostWords(size_t words) : bytes_(words * sizeof(int32_t)) {
+    if (bytes_ == 0) return;
+    void* p = mmap(nullptr, bytes_, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+    if (p == MAP_FAILED) throw std::bad_alloc();
+    (void)madvise(p, bytes_, MADV_HUGEPAGE);
+    p_ = static_cast<int32_t*>(p);
+  }
+  HostWords(HostWords&& o) noexcept : p_(std::exchange(o.p_, nullptr)), bytes_(std::exchange(o.bytes_, 0)) {}
+  HostWords& operator=(HostWords&& o) noexcept {
+    std::swap(p_, o.p_);
+    std::swap(bytes_, o.bytes_);
+    return *this;
+  }
+  ~HostWords() {
+    if (p_) (void)munmap(p_, bytes_);
+  }
+  int32_t& operator[](size_t k) { return p_[k]; }
+  int32_t operator[](size_t k) const { return p_[k]; }
+
+ private:
+  int32_t* p_ = nullptr;
+  size_t bytes_ = 0;
+};
+
+// The last level that wrote and the last that read each variable, for one pass
+// after the other: a pass counts its levels from where the one before it
+// stopped, so nothing is cleared between them (two vectors filled for each pass
+// took 10 and 6 ms for the 1M x 1.5M LP's two passes, this 2 and 4.4).
+struct VarLevels {
+  HostWords last;  // written, read: of each variable, 0 none
+  int32_t base = 0;
+  explicit VarLevels(size_t variables) : last(2 * variables) {}
+};
+
 // Index lists of the original rows of A (columns of AT) that the dual
 // recoveries walk, gathered on the device and copied to the host: line l is
 // idx[off[slot[l]] .. off[slot[l] + 1]).
 struct Lines {
-  std::vector<int32_t> slot, off, idx;
-  const int32_t* begin(int32_t l) const { return idx.data() + off[slot[l]]; }
-  const int32_t* end(int32_t l) const { return idx.data() + off[slot[l] + 1]; }
+  HostWords slot;  // 1 + the line's slot, 0 where it has none
+  std::vector<int32_t> off, idx;
+  const int32_t* begin(int32_t l) const { return idx.data() + off[slot[l] - 1]; }
+  const int32_t* end(int32_t l) const { return idx.data() + off[slot[l]]; }
 };
 
 struct OrigPattern {
@@ -103,12 +147,12 @@ struct OrigPattern {
 
 Lines gather_lines(const int32_t* ptr, const int32_t* idx, int32_t lines_total, const std::vector<int32_t>& wanted) {
   Lines L;
-  L.slot.assign(static_cast<size_t>(lines_total), -1);
+  if (!wanted.empty()) L.slot = HostWords(static_cast<size_t>(lines_total));
   std::vector<int32_t> list;
   for (int32_t l : wanted)
-    if (L.slot[l] < 0) {
-      L.slot[l] = static_cast<int32_t>(list.size());
+    if (L.slot[l] == 0) {
       list.push_back(l);
+      L.slot[l] = static_cast<int32_t>(list.size());
     }
   const int32_t k = static_cast<int32_t>(list.size());
   L.off.assign(1, 0);
@@ -152,7 +196,7 @@ constexpr int32_t kWaveRecords = 4;  // sixteen lanes each
 
 class TapeScanner {
  public:
-  TapeScanner(const PostsolveTape& t, int32_t n0, int32_t m0) : t_(t), n0_(n0), m0_(m0) {}
+  TapeScanner(const amd::TapeView& t, int32_t n0, int32_t m0) : t_(t), n0_(n0), m0_(m0) {}
 
   // Read and write sets of record k in the primal (primal = true) or dual
   // pass; returns false when the record does nothing in that pass.
@@ -343,28 +387,35 @@ class TapeScanner {
     if (r < 0 || r >= m0_) bad_tape(k, "row index out of range");
     return n0_ + r;
   }
-  const PostsolveTape& t_;
+  const amd::TapeView t_;
   int32_t n0_, m0_;
 };
 
 // Records [lo, hi) of the tape, replayed in reverse.
-Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, int32_t n0, int32_t m0, bool primal,
-                        bool has_orig, bool has_y, const OrigPattern* op) {
-  std::vector<int32_t> lw(static_cast<size_t>(n0) + m0, -1), lr(static_cast<size_t>(n0) + m0, -1);
+Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, VarLevels& vars, bool primal, bool has_orig,
+                        bool has_y, const OrigPattern* op) {
+  HostWords& last = vars.last;
+  const int32_t base = vars.base;
   const int32_t span = hi > lo ? hi - lo : 0;
   std::vector<int32_t> level(span, -1);
   std::vector<int32_t> rd, wr;
   int32_t levels = 0;
   for (int32_t k = hi - 1; k >= lo; --k) {
     if (!scan.sets(k, primal, has_orig, has_y, op, rd, wr)) continue;
-    int32_t lv = 0;
-    for (int32_t v : rd) lv = std::max(lv, lw[v] + 1);
-    for (int32_t v : wr) lv = std::max(lv, std::max(lw[v], lr[v]) + 1);
-    for (int32_t v : wr) lw[v] = lv;
-    for (int32_t v : rd) lr[v] = std::max(lr[v], lv);
-    level[k - lo] = lv;
-    levels = std::max(levels, lv + 1);
+    int32_t lv = base;  // past base + the levels that it has to follow
+    for (int32_t v : rd) lv = std::max(lv, last[2 * static_cast<size_t>(v)]);
+    for (int32_t v : wr)
+      lv = std::max({lv, last[2 * static_cast<size_t>(v)], last[2 * static_cast<size_t>(v) + 1]});
+    ++lv;
+    for (int32_t v : wr) last[2 * static_cast<size_t>(v)] = lv;
+    for (int32_t v : rd) {
+      int32_t& r = last[2 * static_cast<size_t>(v) + 1];
+      r = std::max(r, lv);
+    }
+    level[k - lo] = lv - base - 1;
+    levels = std::max(levels, lv - base);
   }
+  vars.base += levels;
   // Records of a level in the order of their types, and in a level that one
   // workgroup replays each type from a new wave on (empty slots, -1, between):
   // a wave runs the branches of its records' types one after the other.  Such
@@ -434,9 +485,10 @@ void enqueue_schedule(const Schedule& sch, const int32_t* buf, const gp_tape_dev
   }
 }
 
-void upload_map(DBuf<int32_t>& dst, const std::vector<int32_t>& src, int32_t bound, const char* what) {
-  for (int32_t v : src)
-    if (v < 0 || v >= bound) throw std::runtime_error(std::string(what) + ": index out of range");
+void upload_map(DBuf<int32_t>& dst, const amd::HostSpan<int32_t>& src, int32_t bound, const char* what) {
+  bool bad = false;
+  for (int32_t v : src) bad |= v < 0 || v >= bound;
+  if (bad) throw std::runtime_error(std::string(what) + ": index out of range");
   dst.alloc(static_cast<int64_t>(src.size()));
   ctx().to_device(dst.get(), src.data(), static_cast<int64_t>(src.size()), what);
 }
@@ -460,7 +512,7 @@ void check_recovery_col(int32_t col, int32_t n0, const char* what) {
 // validate_primal_recovery_timeline (gpu_postsolve.cu:1485-1616): the
 // checkpoints are chronological, each payload has exactly one checkpoint
 // and every column a payload names is an original column.
-void validate_recovery_timeline(const PresolveRecordGpu& r) {
+void validate_recovery_timeline(const RecordView& r) {
   const auto limit = static_cast<size_t>(std::numeric_limits<int32_t>::max());
   if (r.structural_primal_recoveries.size() > limit || r.antipodal_component_recoveries.size() > limit)
     throw std::runtime_error("primal recovery payload exceeds 32-bit checkpoint range");
@@ -607,7 +659,7 @@ struct RecoveryStep {
 
 }  // namespace
 
-void PostsolvePlan::validate(const PresolveRecordGpu& record, const LPInfoGpu* original) {
+void PostsolvePlan::validate(const RecordView& record, const LPInfoGpu* original) {
   validate_recovery_timeline(record);
   if (static_cast<int32_t>(record.col_red2org.size()) != record.n1 ||
       static_cast<int32_t>(record.row_red2org.size()) != record.m1)
@@ -641,7 +693,7 @@ struct PostsolvePlan::Impl {
   int64_t records = 0, tape_bytes = 0;
 };
 
-PostsolvePlan::PostsolvePlan(const PresolveRecordGpu& record, const LPInfoGpu* original, const double* original_l)
+PostsolvePlan::PostsolvePlan(const RecordView& record, const LPInfoGpu* original, const double* original_l)
     : d_(new Impl) {
   AbandonOnThrow abandon_guard;
   validate(record, original);
@@ -656,11 +708,11 @@ PostsolvePlan::PostsolvePlan(const PresolveRecordGpu& record, const LPInfoGpu* o
   d.n1 = record.n1;
   d.m1 = record.m1;
   {
-    const presolve::PostsolveTape& t = record.tape;
+    const TapeView& t = record.tape;
     d.records = static_cast<int64_t>(t.types.size());
     d.tape_bytes = static_cast<int64_t>(sizeof(int32_t) * (t.types.size() + t.index_starts.size() +
                                                             t.value_starts.size() + t.indices.size()) +
-                                        t.dual_modes.size() + sizeof(double) * t.vals.size());
+                                        record.dual_modes + sizeof(double) * t.vals.size());
   }
   // GP_PRESOLVE_PROFILE=1: host time of the preparation steps on stderr.
   const bool prof = std::getenv("GP_PRESOLVE_PROFILE") != nullptr;
@@ -699,11 +751,12 @@ PostsolvePlan::PostsolvePlan(const PresolveRecordGpu& record, const LPInfoGpu* o
   // postsolve_gpu (gpu_postsolve.cu:1691-1713): the primal pass replays the
   // tape from its end down to each recovery checkpoint, in reverse
   // chronological order, and applies that checkpoint's recovery step there.
+  presolve::VarLevels vars(static_cast<size_t>(d.n0) + d.m0);
   int32_t range_end = count;
-  for (auto it = record.primal_recovery_timeline.rbegin(); it != record.primal_recovery_timeline.rend(); ++it) {
+  for (size_t cp = record.primal_recovery_timeline.size(); cp-- > 0;) {
+    const presolve::PrimalRecoveryCheckpoint* it = &record.primal_recovery_timeline[cp];
     Impl::Stage st;
-    st.sched = presolve::level_schedule(scanner, it->tape_position, range_end, d.n0, d.m0, true, has_orig, has_y,
-                                        &pattern);
+    st.sched = presolve::level_schedule(scanner, it->tape_position, range_end, vars, true, has_orig, has_y, &pattern);
     st.buf = presolve::upload_schedule(st.sched);
     if (it->kind == presolve::PrimalRecoveryKind::StructuralL1)
       st.step = std::make_unique<RecoveryStep>(record.structural_primal_recoveries[it->payload_index]);
@@ -714,12 +767,12 @@ PostsolvePlan::PostsolvePlan(const PresolveRecordGpu& record, const LPInfoGpu* o
   }
   {
     Impl::Stage st;
-    st.sched = presolve::level_schedule(scanner, 0, range_end, d.n0, d.m0, true, has_orig, has_y, &pattern);
+    st.sched = presolve::level_schedule(scanner, 0, range_end, vars, true, has_orig, has_y, &pattern);
     st.buf = presolve::upload_schedule(st.sched);
     d.primal.push_back(std::move(st));
   }
   lap("primal schedule");
-  d.dual = presolve::level_schedule(scanner, 0, count, d.n0, d.m0, false, has_orig, has_y, &pattern);
+  d.dual = presolve::level_schedule(scanner, 0, count, vars, false, has_orig, has_y, &pattern);
   d.dual_buf = presolve::upload_schedule(d.dual);
   lap("dual schedule");
   // project_column_duals_from_original (gpu_postsolve.cu:1370-1435): the

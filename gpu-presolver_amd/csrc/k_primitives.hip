@@ -1219,6 +1219,281 @@ __global__ void k_transpose_gather(const int32_t* __restrict__ perm, const gpk_r
   at_val[k] = __hiloint2double(w.w, w.z);
 }
 
+// The transpose by buckets of 2^low columns (at most kTbBuckets of them): the
+// entries are moved once, with their rows and values, into the buckets, and
+// once more, by a workgroup for each bucket, to their columns.  Both moves keep
+// the order of A, so every row of the transpose comes out sorted.  (The sort of
+// the column indices alone reads and writes (key, position) three times and
+// then gathers 16 bytes from a line of 128 for each entry: 493 us a call for the
+// 1M x 1.5M LP's 8 million entries, of which 154 the gather; this takes 290: 32
+// the counts, 90 the first move, 105 the second, the rest the host's look at
+// the largest bucket, allocations and the call.)  The moves are bound by their
+// stores, a request to the L2 for each 16 bytes and for each 4 and 8.
+constexpr int kTbBlock = 512;
+constexpr int kTbWaves = kTbBlock / 64;
+constexpr int kTbSteps = 8;  // of 64 consecutive entries, for a wave
+constexpr int kTbTile = kTbBlock * kTbSteps;
+constexpr int kTbBuckets = 1024;
+constexpr int kTbLowMax = 11;
+constexpr int kTbCols = 1 << kTbLowMax;
+
+// Blocks go to the XCDs in turn; neighbouring tiles write neighbouring words, so
+// an XCD gets a stretch of tiles and its L2 joins them into whole lines.
+constexpr int kXcds = 8;
+__device__ __forceinline__ int32_t tb_tile(int32_t tiles) {
+  const int32_t b = static_cast<int32_t>(blockIdx.x), x = b % kXcds, q = tiles / kXcds, r = tiles % kXcds;
+  return x * q + min(x, r) + b / kXcds;
+}
+
+// A column outside the matrix counts as one of the last bucket.
+__device__ __forceinline__ int tb_bucket(int32_t col, int low, int buckets) {
+  return static_cast<int>(min(static_cast<uint32_t>(col) >> low, static_cast<uint32_t>(buckets - 1)));
+}
+
+// The place of each valid lane's entry among those of its digit that the wave
+// has ranked so far, counted in cnt[digit].
+__device__ __forceinline__ int tb_rank(uint16_t* cnt, int digit, int bits, bool valid, uint64_t below) {
+  uint64_t match = __ballot(valid);
+  for (int b = 0; b < bits; ++b) {
+    const bool bit = (digit >> b) & 1;
+    const uint64_t bal = __ballot(bit);
+    match &= bit ? bal : ~bal;
+  }
+  int rank = 0;
+  if (valid) {
+    const int r = __popcll(match & below);
+    const int prev = cnt[digit];
+    rank = prev + r;
+    if (r == 0) cnt[digit] = static_cast<uint16_t>(prev + __popcll(match));
+  }
+  __builtin_amdgcn_wave_barrier();
+  return rank;
+}
+
+__global__ __launch_bounds__(kTbBlock) void k_tb_hist(const int32_t* __restrict__ col, int32_t nnz, int low,
+                                                      int32_t buckets, int32_t tiles, int32_t* __restrict__ hist) {
+  __shared__ int32_t s_h[kTbBuckets];
+  const int tid = static_cast<int>(threadIdx.x);
+  const int32_t tile = tb_tile(tiles);
+  for (int d = tid; d < buckets; d += kTbBlock) s_h[d] = 0;
+  const int64_t c0 = static_cast<int64_t>(tile) * kTbTile;
+  int32_t j[kTbSteps];
+#pragma unroll
+  for (int k = 0; k < kTbSteps; ++k) j[k] = c0 + k * kTbBlock + tid < nnz ? col[c0 + k * kTbBlock + tid] : 0;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kTbSteps; ++k)
+    if (c0 + k * kTbBlock + tid < nnz) atomicAdd(&s_h[tb_bucket(j[k], low, buckets)], 1);
+  __syncthreads();
+  for (int d = tid; d < buckets; d += kTbBlock) hist[static_cast<int64_t>(d) * tiles + tile] = s_h[d];
+}
+
+// largest[0] = the most entries of a bucket.
+__global__ __launch_bounds__(kTbBuckets) void k_tb_largest(const int32_t* __restrict__ offs, int32_t buckets,
+                                                           int32_t tiles, int32_t* __restrict__ largest) {
+  __shared__ int32_t s_most[kTbBuckets / 64];
+  const int d = static_cast<int>(threadIdx.x);
+  int32_t v = d < buckets ? offs[static_cast<int64_t>(d + 1) * tiles] - offs[static_cast<int64_t>(d) * tiles] : 0;
+#pragma unroll
+  for (int k = 32; k >= 1; k >>= 1) v = max(v, __shfl_xor(v, k, 64));
+  if ((d & 63) == 0) s_most[d >> 6] = v;
+  __syncthreads();
+  if (d == 0) {
+    for (int w = 1; w < kTbBuckets / 64; ++w) v = max(v, s_most[w]);
+    largest[0] = v;
+  }
+}
+
+// The last row that starts at or before entry p, by a wave: a 64th of the rows
+// is left after each look.
+__device__ inline int32_t wave_row_of(const int32_t* __restrict__ ptr, int32_t m, int32_t p) {
+  int32_t lo = 0, n = m;  // the row is one of [lo, lo + n)
+  while (n > 1) {
+    const int32_t step = (n + 63) / 64;
+    const int64_t r = static_cast<int64_t>(lo) + static_cast<int64_t>(lane_id()) * step;
+    const uint64_t before = __ballot(r < static_cast<int64_t>(lo) + n && ptr[r < m ? r : m] <= p);
+    const int32_t at = max(static_cast<int32_t>(__popcll(before)) - 1, 0) * step;
+    lo += at;
+    n = min(step, n - at);
+  }
+  return lo;
+}
+
+__global__ __launch_bounds__(kTbBlock) void k_tb_partition(const int32_t* __restrict__ ptr,
+                                                           const int32_t* __restrict__ col,
+                                                           const double* __restrict__ val, int32_t m, int32_t nnz,
+                                                           int low, int32_t buckets, int bits, int32_t tiles,
+                                                           const int32_t* __restrict__ offs, int4* __restrict__ rec) {
+  __shared__ uint16_t s_cnt[kTbWaves][kTbBuckets];
+  __shared__ int32_t s_base[kTbBuckets];
+  __shared__ int32_t s_row[kTbTile];  // row - first, of each entry
+  __shared__ int32_t s_w[kTbWaves];
+  __shared__ int32_t s_first;
+  const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6, lane = tid & 63;
+  const int32_t tile = tb_tile(tiles);
+  const int32_t c0 = tile * kTbTile;
+  const int32_t cnt = min(kTbTile, nnz - c0);
+  const int32_t mine = wave * (64 * kTbSteps) + lane;
+  int32_t j[kTbSteps];
+  double v[kTbSteps];
+#pragma unroll
+  for (int k = 0; k < kTbSteps; ++k) {
+    const int32_t p = c0 + min(mine + 64 * k, cnt - 1);
+    j[k] = col[p];
+    v[k] = val[p];
+  }
+  for (int i = tid; i < kTbWaves * kTbBuckets / 2; i += kTbBlock) reinterpret_cast<uint32_t*>(&s_cnt[0][0])[i] = 0;
+  for (int i = tid; i < kTbTile; i += kTbBlock) s_row[i] = 0;
+  for (int d = tid; d < buckets; d += kTbBlock) s_base[d] = offs[static_cast<int64_t>(d) * tiles + tile];
+  if (wave == 0) {
+    const int32_t r = wave_row_of(ptr, m, c0);
+    if (lane == 0) s_first = r;
+  }
+  __syncthreads();
+  // Each further row marks its first entry (of rows that start together the
+  // last one holds it); the running maximum is then every entry's row.
+  const int32_t first = s_first;
+  for (int64_t r = static_cast<int64_t>(first) + 1 + tid; r < m; r += kTbBlock) {
+    const int32_t p = ptr[r] - c0;
+    if (p >= cnt) break;
+    if (p >= 0) atomicMax(&s_row[p], static_cast<int32_t>(r - first));
+  }
+  __syncthreads();
+  int32_t run[kTbSteps];
+  int32_t most = 0;
+#pragma unroll
+  for (int k = 0; k < kTbSteps; ++k) {
+    most = max(most, s_row[tid * kTbSteps + k]);
+    run[k] = most;
+  }
+  int32_t upto = most;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int32_t o = __shfl_up(upto, d, 64);
+    if (lane >= d) upto = max(upto, o);
+  }
+  if (lane == 63) s_w[wave] = upto;
+  int32_t before = __shfl_up(upto, 1, 64);
+  if (lane == 0) before = 0;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) before = max(before, s_w[w]);
+#pragma unroll
+  for (int k = 0; k < kTbSteps; ++k) s_row[tid * kTbSteps + k] = max(before, run[k]);
+  const uint64_t below = lanemask_lt(lane);
+  int digit[kTbSteps], rank[kTbSteps];
+#pragma unroll
+  for (int k = 0; k < kTbSteps; ++k) {
+    digit[k] = tb_bucket(j[k], low, buckets);
+    rank[k] = tb_rank(s_cnt[wave], digit[k], bits, mine + 64 * k < cnt, below);
+  }
+  __syncthreads();
+  for (int d = tid; d < buckets; d += kTbBlock) {
+    int32_t sum = 0;
+#pragma unroll
+    for (int w = 0; w < kTbWaves; ++w) {
+      const int32_t c = s_cnt[w][d];
+      s_cnt[w][d] = static_cast<uint16_t>(sum);
+      sum += c;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < kTbSteps; ++k)
+    if (mine + 64 * k < cnt)
+      rec[s_base[digit[k]] + s_cnt[wave][digit[k]] + rank[k]] =
+          make_int4(j[k], first + s_row[mine + 64 * k], __double2loint(v[k]), __double2hiint(v[k]));
+}
+
+// One bucket: its entries counted by column, which gives the columns' row
+// pointers of the transpose, then placed tile by tile in their order.
+__global__ __launch_bounds__(kTbBlock) void k_tb_columns(const int4* __restrict__ rec, int32_t n, int32_t nnz, int low,
+                                                         int32_t tiles, const int32_t* __restrict__ offs,
+                                                         int32_t* __restrict__ at_ptr, int32_t* __restrict__ at_idx,
+                                                         double* __restrict__ at_val) {
+  __shared__ uint16_t s_cnt[kTbWaves][kTbCols];
+  __shared__ int32_t s_next[kTbCols];  // where a column's next entry goes
+  __shared__ int32_t s_w[kTbWaves];
+  constexpr int kPer = kTbCols / kTbBlock;
+  const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6, lane = tid & 63;
+  const int cols = 1 << low;
+  const int32_t bucket = static_cast<int32_t>(blockIdx.x);
+  const int32_t b = offs[static_cast<int64_t>(bucket) * tiles], e = offs[static_cast<int64_t>(bucket + 1) * tiles];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) s_next[tid * kPer + k] = 0;
+  __syncthreads();
+  for (int32_t p0 = b; p0 < e; p0 += kTbTile) {
+    int32_t j[kTbSteps];
+#pragma unroll
+    for (int k = 0; k < kTbSteps; ++k) j[k] = rec[min(p0 + k * kTbBlock + tid, e - 1)].x;
+#pragma unroll
+    for (int k = 0; k < kTbSteps; ++k)
+      if (p0 + k * kTbBlock + tid < e) atomicAdd(&s_next[j[k] & (cols - 1)], 1);
+  }
+  __syncthreads();
+  int32_t c[kPer], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    c[k] = s_next[tid * kPer + k];
+    sum += c[k];
+  }
+  const int32_t inc = wave_inclusive_sum(sum);
+  if (lane == 63) s_w[wave] = inc;
+  __syncthreads();
+  int32_t at = b + inc - sum;
+  for (int w = 0; w < wave; ++w) at += s_w[w];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int64_t col = (static_cast<int64_t>(bucket) << low) + tid * kPer + k;
+    if (tid * kPer + k < cols && col < n) at_ptr[col] = at;
+    s_next[tid * kPer + k] = at;
+    at += c[k];
+  }
+  if (bucket == 0 && tid == 0) at_ptr[n] = nnz;
+  const uint64_t below = lanemask_lt(lane);
+  const int32_t mine = wave * (64 * kTbSteps) + lane;
+  for (int32_t p0 = b; p0 < e; p0 += kTbTile) {
+    const int32_t cnt = min(kTbTile, e - p0);
+    int4 w4[kTbSteps];
+    int rank[kTbSteps];
+#pragma unroll
+    for (int k = 0; k < kTbSteps; ++k) w4[k] = rec[p0 + min(mine + 64 * k, cnt - 1)];
+    for (int w = 0; w < kTbWaves; ++w)
+      for (int i = tid; i < (cols + 1) / 2; i += kTbBlock) reinterpret_cast<uint32_t*>(s_cnt[w])[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kTbSteps; ++k)
+      rank[k] = tb_rank(s_cnt[wave], w4[k].x & (cols - 1), low, mine + 64 * k < cnt, below);
+    __syncthreads();
+    int32_t total[kPer];
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      total[k] = 0;
+      const int col = tid + k * kTbBlock;
+      if (col < cols)
+#pragma unroll
+        for (int w = 0; w < kTbWaves; ++w) {
+          const int32_t t = s_cnt[w][col];
+          s_cnt[w][col] = static_cast<uint16_t>(total[k]);
+          total[k] += t;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kTbSteps; ++k)
+      if (mine + 64 * k < cnt) {
+        const int col = w4[k].x & (cols - 1);
+        const int32_t to = s_next[col] + s_cnt[wave][col] + rank[k];
+        at_idx[to] = w4[k].y;
+        at_val[to] = __hiloint2double(w4[k].w, w4[k].z);
+      }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kPer; ++k)
+      if (tid + k * kTbBlock < cols) s_next[tid + k * kTbBlock] += total[k];
+    __syncthreads();
+  }
+}
+
 // CSR checks.  The row pointers are checked first, one row a thread
 // (flags[0]: not monotone, not from 0 to nnz), and leave the chunk rows of the
 // matrix (its last row past the last chunk); then chunks of 2048 entries are
@@ -1752,6 +2027,50 @@ hipError_t gpk_transpose_sort(const int32_t* col, int32_t nnz, int32_t key_bits,
     vout = to_b ? vb : va;
   }
   *result_in_b = kin == kb ? 1 : 0;
+  return hipGetLastError();
+}
+
+int32_t gpk_transpose_buckets(int32_t n, int32_t nnz, int32_t* low) {
+  // At 1,048,576 entries the buckets take 99 to 107 us where the sort takes 117
+  // to 147 (128 against 190 at twice that); below, the wait for the largest
+  // bucket's size is most of it.  Up to 256 columns the sort has one pass.
+  *low = 0;
+  if (nnz < GPK_TRANSPOSE_BUCKETS_MIN_NNZ || nnz > INT_MAX - 2 * kTbTile || n <= 256) return 0;
+  while (*low < kTbLowMax && ((n - 1) >> *low) >= kTbBuckets) ++*low;
+  const int32_t buckets = ((n - 1) >> *low) + 1;
+  return buckets <= kTbBuckets ? buckets : 0;
+}
+
+int64_t gpk_transpose_buckets_scratch_ints(int32_t buckets, int32_t nnz) {
+  const int64_t words = static_cast<int64_t>(buckets) * grid_for(nnz, kTbTile);
+  return words + 1 + gpk_scan_scratch_ints(words) + 1;
+}
+
+hipError_t gpk_transpose_buckets_count(const int32_t* col, int32_t nnz, int32_t low, int32_t buckets, int32_t* scratch,
+                                       int32_t* largest, hipStream_t s) {
+  if (nnz <= 0 || buckets <= 0 || buckets > kTbBuckets || low < 0 || low > kTbLowMax) return hipErrorInvalidValue;
+  const int32_t tiles = static_cast<int32_t>(grid_for(nnz, kTbTile));
+  const int64_t words = static_cast<int64_t>(buckets) * tiles;
+  hipLaunchKernelGGL(k_tb_hist, dim3(tiles), dim3(kTbBlock), 0, s, col, nnz, low, buckets, tiles, scratch);
+  const hipError_t e = scan_impl<int32_t>(scratch, scratch, words, scratch + words + 1, s);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_tb_largest, dim3(1), dim3(kTbBuckets), 0, s, static_cast<const int32_t*>(scratch), buckets,
+                     tiles, largest);
+  return hipGetLastError();
+}
+
+hipError_t gpk_transpose_buckets_move(const int32_t* ptr, const int32_t* col, const double* val, int32_t m, int32_t n,
+                                      int32_t nnz, int32_t low, int32_t buckets, const int32_t* scratch,
+                                      gpk_row_val* rec, int32_t* at_ptr, int32_t* at_idx, double* at_val,
+                                      hipStream_t s) {
+  if (nnz <= 0 || buckets <= 0 || buckets > kTbBuckets || low < 0 || low > kTbLowMax) return hipErrorInvalidValue;
+  const int32_t tiles = static_cast<int32_t>(grid_for(nnz, kTbTile));
+  int bits = 0;
+  while ((1 << bits) < buckets) ++bits;
+  hipLaunchKernelGGL(k_tb_partition, dim3(tiles), dim3(kTbBlock), 0, s, ptr, col, val, m, nnz, low,
+                     buckets, bits, tiles, scratch, reinterpret_cast<int4*>(rec));
+  hipLaunchKernelGGL(k_tb_columns, dim3(buckets), dim3(kTbBlock), 0, s, reinterpret_cast<const int4*>(rec), n,
+                     nnz, low, tiles, scratch, at_ptr, at_idx, at_val);
   return hipGetLastError();
 }
 

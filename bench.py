@@ -18,9 +18,9 @@ Extra objects on the JSON line:
                      stream: k_pack_lu then k_row_activity_lu), algorithmic
                      bytes 4(m+1) + 12 nnz + 16 n + 24 m, with both kernels
                      also timed apart;
-  roofline_transpose the transpose of the full A (three LSD sort passes over
-                     the column indices, row pointers from the sorted keys,
-                     one gather), algorithmic bytes
+  roofline_transpose the transpose of the full A (its entries counted by bucket
+                     of columns, moved into the buckets, then to their
+                     columns), algorithmic bytes
                      4(m+1) + 12 nnz + 4(n+1) + 12 nnz + 8 n;
   roofline_postsolve the prepared postsolve of the last record: tape records,
                      dependency levels of the two replay passes, time per level
@@ -355,68 +355,65 @@ def transpose_bytes(m, n, nnz):
 
 
 def measure_transpose(gp_ffi, dlp, lp, stream, launches):
-    """Times the library's transpose (stable sort of the column indices
-    carrying entry positions, row pointers from the sorted keys, rows of the
-    entries, one gather of rows and values) on the full A, back to back on
-    one stream, each kernel group also timed apart; the result must equal
-    the LP's own AT."""
+    """Times the library's transpose by buckets of columns (the entries counted
+    by bucket, moved into the buckets, then to their columns) on the full A,
+    back to back on one stream, the counts also timed apart; the result must
+    equal the LP's own AT."""
     import ctypes as C
 
     import numpy as np
 
     m, n, nnz = lp["m"], lp["n"], len(lp["A_idx"])
     L = gp_ffi.lib()
-    vp = C.c_void_p
-    L.gpk_radix_scratch_ints.restype = C.c_int64
-    L.gpk_radix_scratch_ints.argtypes = [C.c_int64]
-    L.gpk_transpose_sort.argtypes = [vp, C.c_int32, C.c_int32, vp, vp, vp, vp, vp, C.POINTER(C.c_int32), vp]
-    L.gpk_col_bounds.argtypes = [vp, C.c_int32, C.c_int32, vp, vp]
-    L.gpk_expand_rows.argtypes = [vp, vp, C.c_int32, vp, vp]
-    L.gpk_transpose_gather.argtypes = [vp, vp, C.c_int32, vp, vp, vp]
-    bits = max(1, int(n - 1).bit_length())
-    ka, kb = gp_ffi.DeviceArray(size=nnz, dtype=np.uint32), gp_ffi.DeviceArray(size=nnz, dtype=np.uint32)
-    va, vb = gp_ffi.DeviceArray(size=nnz, dtype=np.int32), gp_ffi.DeviceArray(size=nnz, dtype=np.int32)
-    scratch = gp_ffi.DeviceArray(size=L.gpk_radix_scratch_ints(nnz), dtype=np.int32)
+    vp, i32 = C.c_void_p, C.c_int32
+    L.gpk_transpose_buckets.argtypes = [i32, i32, C.POINTER(i32)]
+    L.gpk_transpose_buckets_scratch_ints.restype = C.c_int64
+    L.gpk_transpose_buckets_scratch_ints.argtypes = [i32, i32]
+    L.gpk_transpose_buckets_count.argtypes = [vp, i32, i32, i32, vp, vp, vp]
+    L.gpk_transpose_buckets_move.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp]
+    low = i32(0)
+    buckets = L.gpk_transpose_buckets(n, nnz, C.byref(low))
+    if buckets <= 0:
+        raise SystemExit("bench.py: the LP is too small for the transpose by buckets")
+    scratch = gp_ffi.DeviceArray(size=L.gpk_transpose_buckets_scratch_ints(buckets, nnz), dtype=np.int32)
+    largest = gp_ffi.DeviceArray(size=1, dtype=np.int32)
     ptr = gp_ffi.DeviceArray(size=n + 1, dtype=np.int32)
     idx, val = gp_ffi.DeviceArray(size=nnz, dtype=np.int32), gp_ffi.DeviceArray(size=nnz)
-    rv = gp_ffi.DeviceArray(size=2 * nnz)  # 16-byte (row, value) pairs
+    rec = gp_ffi.DeviceArray(size=2 * nnz)  # 16-byte entries
     A = dlp.A.g
-    in_b = C.c_int32(0)
     ck = gp_ffi.hip_check
 
-    def sort():
-        ck(L.gpk_transpose_sort(A.col_idx, nnz, bits, ka.ptr, va.ptr, kb.ptr, vb.ptr, scratch.ptr, C.byref(in_b),
-                                stream.ptr), "transpose sort")
+    def count():
+        ck(L.gpk_transpose_buckets_count(A.col_idx, nnz, low.value, buckets, scratch.ptr, largest.ptr, stream.ptr),
+           "bucket sizes")
 
-    def finish():
-        keys, perm = (kb, vb) if in_b.value else (ka, va)
-        ck(L.gpk_col_bounds(keys.ptr, nnz, n, ptr.ptr, stream.ptr), "col bounds")
-        ck(L.gpk_expand_rows(A.row_ptr, A.val, m, rv.ptr, stream.ptr), "expand rows")
-        ck(L.gpk_transpose_gather(perm.ptr, rv.ptr, nnz, idx.ptr, val.ptr, stream.ptr), "gather")
+    def move():
+        ck(L.gpk_transpose_buckets_move(A.row_ptr, A.col_idx, A.val, m, n, nnz, low.value, buckets, scratch.ptr,
+                                        rec.ptr, ptr.ptr, idx.ptr, val.ptr, stream.ptr), "bucket moves")
 
     for _ in range(2):
-        sort()
-        finish()
+        count()
+        move()
     stream.sync()
     e = [gp_ffi.Event() for _ in range(3)]
     e[0].record(stream)
     for _ in range(launches):
-        sort()
-        finish()
+        count()
+        move()
     e[1].record(stream)
     for _ in range(launches):
-        sort()
+        count()
     e[2].record(stream)
     us = 1e3 * e[0].elapsed_ms(e[1]) / launches
-    sort_us = 1e3 * e[1].elapsed_ms(e[2]) / launches
+    count_us = 1e3 * e[1].elapsed_ms(e[2]) / launches
     if not (np.array_equal(ptr.numpy(), lp["AT_ptr"]) and np.array_equal(idx.numpy(), lp["AT_idx"])
             and np.array_equal(val.numpy(), lp["AT_val"])):
         raise SystemExit("bench.py: the transpose differs from the LP's AT")
     b = transpose_bytes(m, n, nnz)
-    log(f"transpose: {us:.1f} us/call ({b / (us * 1e-6) / 1e9:.0f} GB/s); sort {sort_us:.1f} us, "
-        f"bounds + rows + gather {us - sort_us:.1f} us")
+    log(f"transpose: {us:.1f} us/call ({b / (us * 1e-6) / 1e9:.0f} GB/s); counts {count_us:.1f} us, "
+        f"moves {us - count_us:.1f} us")
     return {"us": us, "bytes": b, "achieved": b / (us * 1e-6) / 1e9,
-            "kernels_us": {"sort (3 LSD passes)": sort_us, "bounds + rows + gather": us - sort_us},
+            "kernels_us": {"bucket counts": count_us, "two moves": us - count_us},
             "workload": f"A of the LP ({m}x{n}, {nnz} nnz) -> AT ({n}x{m})"}
 
 
@@ -529,12 +526,9 @@ def activity_traffic():
 
 def transpose_traffic():
     """HBM bytes of one transpose from the committed PMC summary, or None."""
-    per_pass = [profiled_traffic(k) for k in ("k_radix_hist<unsigned int>", "k_scan_tiles<int>", "k_scan_tile_sums",
-                                              "k_scan_down<int>", "k_radix_scatter<unsigned int, false>")]
-    once = [profiled_traffic(k) for k in ("k_col_bounds", "k_expand_rows", "k_transpose_gather")]
-    if any(p is None for p in per_pass + once):
-        return None
-    return 3 * sum(per_pass) + sum(once)
+    parts = [profiled_traffic(k) for k in ("k_tb_hist", "k_scan_tiles<int>", "k_scan_tile_sums", "k_scan_down<int>",
+                                           "k_tb_largest", "k_tb_partition", "k_tb_columns")]
+    return None if any(p is None for p in parts) else sum(parts)
 
 
 def compaction_traffic():
@@ -1208,8 +1202,7 @@ def main():
                               "us_per_call": act["us"], "algorithmic_bytes": act["bytes"],
                               "effective_bytes": act["effective_bytes"],
                               "effective_frac": act["effective_achieved"] / HBM_PEAK_GBS, **act["kernels"]},
-        "roofline_transpose": {"bound": "hbm", "kernel": "transpose: 3 LSD sort passes + row pointers from the "
-                                                          "sorted keys + entry rows + gather",
+        "roofline_transpose": {"bound": "hbm", "kernel": "transpose: counts by bucket of columns + two moves",
                                "achieved": tr["achieved"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                "frac": tr["achieved"] / HBM_PEAK_GBS, "traffic": transpose_traffic(),
                                "us_per_call": tr["us"], "algorithmic_bytes": tr["bytes"],

@@ -440,24 +440,26 @@ def measure_pdhg_iterations(gp_ffi, dlp, lp, stream, launches, per_launch=64):
     import gp_types as T
 
     class GpkRows(C.Structure):
-        _fields_ = [("M", T.GpCsr), ("blk", C.c_void_p), ("blocks", C.c_int32)]
+        _fields_ = [("M", T.GpCsr), ("blk", C.c_void_p), ("blocks", C.c_int32), ("part_sum", C.c_void_p),
+                    ("part_count", C.c_void_p)]
 
     m, n, nnz = lp["m"], lp["n"], len(lp["A_idx"])
     L = gp_ffi.lib()
     vp = C.c_void_p
-    L.gpk_pdhg_row_blocks.restype = C.c_int32
-    L.gpk_pdhg_row_blocks.argtypes = [vp, C.c_int32, vp]
+    L.gpk_pdhg_row_plan.restype = C.c_int32
+    L.gpk_pdhg_row_plan.argtypes = [vp, C.c_int32, vp]
     L.gpk_pdhg_iterations.argtypes = [GpkRows, GpkRows] + [vp] * 13 + [C.c_int32, C.c_int32, vp]
-    L.gpk_pdhg_spmv.argtypes = [GpkRows, vp, vp, vp]
+    L.gpk_pdhg_spmv.argtypes = [GpkRows, vp, vp, vp, vp]
     keep = []
 
     def rows(g, host_ptr):
         ptr = np.ascontiguousarray(host_ptr, np.int32)
-        blk = np.zeros(len(ptr), np.int32)
-        nb = L.gpk_pdhg_row_blocks(ptr.ctypes.data, len(ptr) - 1, blk.ctypes.data)
-        d = gp_ffi.DeviceArray(blk[:nb + 1])
+        nb = L.gpk_pdhg_row_plan(ptr.ctypes.data, len(ptr) - 1, None)
+        blk = np.zeros(4 * (nb + 1), np.int32)
+        L.gpk_pdhg_row_plan(ptr.ctypes.data, len(ptr) - 1, blk.ctypes.data)
+        d = [gp_ffi.DeviceArray(blk), gp_ffi.DeviceArray(np.zeros(nb)), gp_ffi.DeviceArray(np.zeros(nb, np.int32))]
         keep.append(d)
-        return GpkRows(g, d.ptr, nb)
+        return GpkRows(g, d[0].ptr, nb, d[1].ptr, d[2].ptr)
 
     A, AT = rows(dlp.A.g, lp["A_ptr"]), rows(dlp.AT.g, lp["AT_ptr"])
     v = dlp.vec
@@ -472,8 +474,8 @@ def measure_pdhg_iterations(gp_ffi, dlp, lp, stream, launches, per_launch=64):
            "iterations")
 
     def products():
-        ck(L.gpk_pdhg_spmv(A, x.ptr, y.ptr, stream.ptr), "spmv A")
-        ck(L.gpk_pdhg_spmv(AT, y.ptr, x.ptr, stream.ptr), "spmv AT")
+        ck(L.gpk_pdhg_spmv(A, x.ptr, None, y.ptr, stream.ptr), "spmv A")
+        ck(L.gpk_pdhg_spmv(AT, y.ptr, None, x.ptr, stream.ptr), "spmv AT")
 
     iterate()
     stream.sync()

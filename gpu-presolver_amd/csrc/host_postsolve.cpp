@@ -453,34 +453,44 @@ Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, VarLeve
   return sch;
 }
 
-// The schedule's record order and level bounds in one device block.
-DBuf<int32_t> upload_schedule(const Schedule& sch) {
+// The schedule's level bounds and its records' packets.
+struct DeviceSchedule {
+  DBuf<int32_t> starts, packets;
+};
+DeviceSchedule upload_schedule(const Schedule& sch, const gp_tape_dev& tape, const gp_orig_dev& orig, bool has_y,
+                               bool primal) {
   const int64_t nr = static_cast<int64_t>(sch.order.size()), nl = static_cast<int64_t>(sch.level_start.size());
-  DBuf<int32_t> buf(nr + nl);
+  DeviceSchedule d;
+  DBuf<int32_t> order(nr);
+  d.starts.alloc(nl);
+  d.packets.alloc(nr * GPK_PACKET_WORDS);
   amd::Ctx& c = ctx();
   c.begin_copy_group();
-  c.to_device(buf.get(), sch.order.data(), nr, "replay schedule upload");
-  c.to_device(buf.get() + nr, sch.level_start.data(), nl, "replay schedule upload");
+  c.to_device(order.get(), sch.order.data(), nr, "replay schedule upload");
+  c.to_device(d.starts.get(), sch.level_start.data(), nl, "replay schedule upload");
   c.end_copy_group("replay schedule upload");
-  return buf;
+  check(gpk_pack_records(tape, orig, order, static_cast<int32_t>(nr), has_y ? 1 : 0, primal ? 0 : 1, d.packets,
+                         c.stream()),
+        "replay packets");
+  return d;
 }
 
 // Launches only: no allocation, copy or wait, so it can be captured.
-void enqueue_schedule(const Schedule& sch, const int32_t* buf, const gp_tape_dev& tape, const gp_orig_dev& orig,
+void enqueue_schedule(const Schedule& sch, const DeviceSchedule& dev, const gp_tape_dev& tape, const gp_orig_dev& orig,
                       double* x, double* y, double* z, uint8_t* zret, bool primal, double tol) {
   if (sch.order.empty()) return;
   hipStream_t s = ctx().stream();
-  const int32_t* order = buf;
-  const int32_t* starts = buf + sch.order.size();
-  const int32_t p = primal ? 1 : 0;
+  const int32_t dual = primal ? 0 : 1;
   const char* what = primal ? "replay primal" : "replay dual";
   for (const Segment& g : sch.segs) {
     if (g.grid) {
       const int32_t b = sch.level_start[g.first];
-      check(gpk_replay_list(tape, orig, x, y, z, zret, order + b, sch.level_start[g.first + 1] - b, p, 1 - p, tol, s),
+      check(gpk_replay_list(tape, orig, x, y, z, zret, dev.packets + static_cast<int64_t>(b) * GPK_PACKET_WORDS,
+                            sch.level_start[g.first + 1] - b, dual, tol, s),
             what);
     } else {
-      check(gpk_replay_levels(tape, orig, x, y, z, zret, order, starts + g.first, g.count, p, 1 - p, tol, s), what);
+      check(gpk_replay_levels(tape, orig, x, y, z, zret, dev.packets, dev.starts + g.first, g.count, dual, tol, s),
+            what);
     }
   }
 }
@@ -680,12 +690,12 @@ struct PostsolvePlan::Impl {
   DBuf<uint8_t> zret, prot;
   DBuf<int32_t> long_cols, long_count;
   presolve::Schedule dual;
-  DBuf<int32_t> dual_buf;
+  presolve::DeviceSchedule dual_dev;
   // The primal pass in replay order: a schedule over a tape range, then the
   // recovery step at that range's start (none after the last range).
   struct Stage {
     presolve::Schedule sched;
-    DBuf<int32_t> buf;
+    presolve::DeviceSchedule dev;
     std::unique_ptr<RecoveryStep> step;
   };
   std::vector<Stage> primal;
@@ -757,7 +767,7 @@ PostsolvePlan::PostsolvePlan(const RecordView& record, const LPInfoGpu* original
     const presolve::PrimalRecoveryCheckpoint* it = &record.primal_recovery_timeline[cp];
     Impl::Stage st;
     st.sched = presolve::level_schedule(scanner, it->tape_position, range_end, vars, true, has_orig, has_y, &pattern);
-    st.buf = presolve::upload_schedule(st.sched);
+    st.dev = presolve::upload_schedule(st.sched, d.tape->view, d.orig, has_y, true);
     if (it->kind == presolve::PrimalRecoveryKind::StructuralL1)
       st.step = std::make_unique<RecoveryStep>(record.structural_primal_recoveries[it->payload_index]);
     else
@@ -768,12 +778,12 @@ PostsolvePlan::PostsolvePlan(const RecordView& record, const LPInfoGpu* original
   {
     Impl::Stage st;
     st.sched = presolve::level_schedule(scanner, 0, range_end, vars, true, has_orig, has_y, &pattern);
-    st.buf = presolve::upload_schedule(st.sched);
+    st.dev = presolve::upload_schedule(st.sched, d.tape->view, d.orig, has_y, true);
     d.primal.push_back(std::move(st));
   }
   lap("primal schedule");
   d.dual = presolve::level_schedule(scanner, 0, count, vars, false, has_orig, has_y, &pattern);
-  d.dual_buf = presolve::upload_schedule(d.dual);
+  d.dual_dev = presolve::upload_schedule(d.dual, d.tape->view, d.orig, has_y, false);
   lap("dual schedule");
   // project_column_duals_from_original (gpu_postsolve.cu:1370-1435): the
   // columns the tape recovers duals for keep them.
@@ -808,10 +818,10 @@ void PostsolvePlan::enqueue(const double* x_red, const double* y_red, const doub
   check(gpk_mark(d.col_map, d.n1, d.zret, s), "mark retrieved");
   check(gpk_restore_fixed(d.fidx, d.fval, d.nf, x_org, s), "restore fixed");
   for (const Impl::Stage& st : d.primal) {
-    presolve::enqueue_schedule(st.sched, st.buf, d.tape->view, d.orig, x_org, y, z_org, d.zret, true, kPostsolveTol);
+    presolve::enqueue_schedule(st.sched, st.dev, d.tape->view, d.orig, x_org, y, z_org, d.zret, true, kPostsolveTol);
     if (st.step) st.step->enqueue(x_org, d.original_l, s);
   }
-  presolve::enqueue_schedule(d.dual, d.dual_buf, d.tape->view, d.orig, x_org, y, z_org, d.zret, false,
+  presolve::enqueue_schedule(d.dual, d.dual_dev, d.tape->view, d.orig, x_org, y, z_org, d.zret, false,
                              kPostsolveTol);
   if (d.project)
     check(gpk_project_duals(d.orig, d.prot, x_org, y, z_org, d.n0, kPostsolveTol, d.long_count, d.long_cols, s),

@@ -290,6 +290,28 @@ __device__ inline int32_t row_read(int32_t type, int32_t w0, int32_t w1) {
   return type == 2 || type == 12 ? w1 : type == 10 || type == 4 ? w0 : -1;
 }
 
+// A record's packet, a word to a lane: all of its operands that are not values,
+// in the order of a schedule, so that a turn is three chained loads (packet,
+// line and values, x and y and z) instead of six.
+enum : int { PK_TYPE = 0, PK_I0 = 1, PK_I1 = 2, PK_V0 = 3, PK_V1 = 4, PK_W0 = 5, PK_QI = 9, PK_QV = 10, PK_N = 11 };
+static_assert(GPK_PACKET_WORDS == kRecLanes, "a word to a lane");
+__device__ __forceinline__ RecHead packet_head(int32_t p) {
+  return RecHead{row_lane<PK_TYPE>(p), row_lane<PK_I0>(p), row_lane<PK_I1>(p), row_lane<PK_V0>(p),
+                 row_lane<PK_V1>(p)};
+}
+__device__ __forceinline__ RecLine packet_line(int32_t p) {
+  return RecLine{row_lane<PK_QI>(p), row_lane<PK_QV>(p), row_lane<PK_N>(p)};
+}
+// The word of lane t of an empty slot's packet.
+__device__ __forceinline__ int32_t packet_none(int t) {
+  return t == PK_TYPE || t == PK_I1 || t == PK_V1 ? -1 : 0;
+}
+
+// The record's first index words.
+struct RecVars {
+  int32_t w0, w1, w2;
+};
+
 // One record of the reverse replay (_kernel_replay_postsolve_tape,
 // gpu_postsolve.cu:605-1046); all sixteen lanes come with the same record.
 // kDual picks the pass.  All loads of x, y, z and zret that the record's type
@@ -297,7 +319,7 @@ __device__ inline int32_t row_read(int32_t type, int32_t w0, int32_t w1) {
 // where a decision comes before a row is read.
 template <bool kDual>
 __device__ __forceinline__ void replay_one(const gp_tape_dev& T, const gp_orig_dev& O, double* x, double* y, double* z,
-                                           uint8_t* zret, const RecHead& h, int32_t word, const RecLine& ln,
+                                           uint8_t* zret, const RecHead& h, const RecVars& rv, const RecLine& ln,
                                            RecEntries r, double tol) {
   const bool has_orig = O.present != 0;
   const int32_t type = h.type;
@@ -310,7 +332,7 @@ __device__ __forceinline__ void replay_one(const gp_tape_dev& T, const gp_orig_d
   const int32_t* I = T.indices;
   const double* V = T.vals;
   // The record's first index words and values.
-  const int32_t w0 = row_lane<0>(word), w1 = row_lane<1>(word), w2 = row_lane<2>(word);
+  const int32_t w0 = rv.w0, w1 = rv.w1, w2 = rv.w2;
   const double W0 = row_lane<0>(r.v), W1 = row_lane<1>(r.v), W2 = row_lane<2>(r.v), W3 = row_lane<3>(r.v),
                W4 = row_lane<4>(r.v), W5 = row_lane<5>(r.v);
 
@@ -565,7 +587,8 @@ __device__ __forceinline__ void replay_record(const gp_tape_dev& T, const gp_ori
   const RecHead h = load_head(T, k);
   const int32_t word = load_word(T, h, t);
   const RecLine ln = load_line<kDual>(O, h, word, y != nullptr);
-  replay_one<kDual>(T, O, x, y, z, zret, h, word, ln, load_entries(T, O, h, ln, t), tol);
+  const RecVars rv{row_lane<0>(word), row_lane<1>(word), row_lane<2>(word)};
+  replay_one<kDual>(T, O, x, y, z, zret, h, rv, ln, load_entries(T, O, h, ln, t), tol);
 }
 
 // Records begin..end-1 in reverse, one after the other (the reference's order).
@@ -580,62 +603,78 @@ __global__ void k_replay(gp_tape_dev T, gp_orig_dev O, double* x, double* y, dou
   }
 }
 
+// The packets of `count` slots of a schedule.
+template <bool kDual>
+__global__ void __launch_bounds__(kBlock) k_pack_records(gp_tape_dev T, gp_orig_dev O, const int32_t* records,
+                                                         int32_t count, int32_t has_y, int32_t* packets) {
+  const int32_t i = static_cast<int32_t>(blockIdx.x * (kBlock / kRecLanes) + threadIdx.x / kRecLanes);
+  if (i >= count) return;
+  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
+  const RecHead h = load_head(T, records[i]);
+  const int32_t word = load_word(T, h, t);
+  const RecLine ln = load_line<kDual>(O, h, word, has_y != 0);
+  const int32_t w = __shfl(word, t >= PK_W0 && t < PK_QI ? t - PK_W0 : 0, kRecLanes);
+  const int32_t p = t == PK_TYPE ? h.type : t == PK_I0 ? h.i0 : t == PK_I1 ? h.i1 : t == PK_V0 ? h.v0
+                    : t == PK_V1 ? h.v1 : t < PK_QI ? w : t == PK_QI ? ln.qi : t == PK_QV ? ln.qv
+                    : t == PK_N ? ln.n : 0;
+  packets[static_cast<int64_t>(i) * GPK_PACKET_WORDS + t] = p;
+}
+
 // One level of a dependency-level schedule: its records touch disjoint
-// variables, sixteen lanes each.  Four chains of loads and little else: 6 us
-// for 1,000 to 30,000 records (16 us with a lane per record).
+// variables, sixteen lanes each.  Three chains of loads and little else:
+// 5.6 us for 1,000 to 30,000 records (16 us with a lane per record, 6.5 with
+// six chains).
 template <bool kDual>
 __global__ void __launch_bounds__(kBlock)
-    k_replay_list(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret, const int32_t* records,
+    k_replay_list(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret, const int32_t* packets,
                   int32_t count, double tol) {
   const int32_t i = static_cast<int32_t>(blockIdx.x * (kBlock / kRecLanes) + threadIdx.x / kRecLanes);
-  if (i < count) replay_record<kDual>(T, O, x, y, z, zret, records[i], tol);
+  if (i >= count) return;
+  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
+  const int32_t p = packets[static_cast<int64_t>(i) * GPK_PACKET_WORDS + t];
+  const RecHead h = packet_head(p);
+  const RecLine ln = packet_line(p);
+  const RecEntries r = load_entries(T, O, h, ln, t);
+  const RecVars rv{row_lane<PK_W0>(p), row_lane<PK_W0 + 1>(p), row_lane<PK_W0 + 2>(p)};
+  replay_one<kDual>(T, O, x, y, z, zret, h, rv, ln, r, tol);
 }
 
 // A run of small levels in one workgroup, which meets at a barrier after each.
 // All waves of the workgroup run on one CU, so the barrier's workgroup-scope
 // fence makes one level's global stores visible to the next level's loads.
-// A group of lanes has the records of its slot of the next five levels on their
-// way, each a step further than the one of the level after it, so that a level
-// waits only for its x, y, z and zret, and for its stores at the barrier.
-// Bound by that chain: 1,207 dual levels, most of about 31 records, take 4.2 ms
-// (3.5 us each; 11.4 ms with a lane per record and each chain in its turn).
-// Reading x, y, z and zret once a level ahead, to have them in the CU's cache,
-// cost 0.4 ms more.
+// A group of lanes has the packet of its slot two levels ahead and the line and
+// values of its record one level ahead on their way, so that a level waits only
+// for its x, y, z and zret, and for its stores at the barrier.  Bound by that
+// chain: 1,207 dual levels, most of about 31 records, take 3.2 ms (2.6 us
+// each; 11.4 ms with a lane per record and each chain in its turn, 4.2 with a
+// record's six chains five levels ahead in place of packets).  Reading x, y, z and zret
+// once a level ahead, to have them in the CU's cache, cost 0.4 ms more.
 template <bool kDual>
 __global__ void __launch_bounds__(GPK_REPLAY_SLOTS * kRecLanes)
     k_replay_levels(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret,
-                    const int32_t* __restrict__ records, const int32_t* __restrict__ level_start, int32_t nlevels,
+                    const int32_t* __restrict__ packets, const int32_t* __restrict__ level_start, int32_t nlevels,
                     double tol) {
-  constexpr int kAhead = 5;
   const int32_t slot = static_cast<int32_t>(threadIdx.x) / kRecLanes;
   const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
-  int32_t begin = level_start[0], end = level_start[min(1, nlevels)];  // of level l + 5
-  RecHead h4 = load_head(T, -1), h3 = h4, h2 = h4, h1 = h4, h0 = h4;
-  int32_t w3 = -1, w2 = -1, w1 = -1, w0 = -1;
-  RecLine n2{0, 0, 0}, n1 = n2, n0 = n2;
-  RecEntries r0 = load_entries(T, O, h0, n0, t);
+  const int32_t none = packet_none(t);
+  const auto packet = [&](int32_t begin, int32_t end) {
+    return begin + slot < end ? packets[static_cast<int64_t>(begin + slot) * GPK_PACKET_WORDS + t] : none;
+  };
+  const int32_t b0 = level_start[0], b1 = level_start[min(1, nlevels)], b2 = level_start[min(2, nlevels)];
+  int32_t end = level_start[min(3, nlevels)], begin = b2;  // of level l + 2
+  int32_t p0 = packet(b0, b1), p1 = packet(b1, b2);
+  RecEntries r0 = load_entries(T, O, packet_head(p0), packet_line(p0), t);
 #pragma unroll 1
-  for (int32_t l = -kAhead; l < nlevels; ++l) {
-    const int32_t next_end = level_start[min(l + kAhead + 2, nlevels)];
-    const int32_t rec = begin + slot < end ? records[begin + slot] : -1;
-    w3 = load_word(T, h3, t);
-    n2 = load_line<kDual>(O, h2, w2, y != nullptr);
-    const RecEntries r1 = load_entries(T, O, h1, n1, t);
-    if (l >= 0) {
-      replay_one<kDual>(T, O, x, y, z, zret, h0, w0, n0, r0, tol);
-      __syncthreads();
-    }
-    h0 = h1;
-    h1 = h2;
-    h2 = h3;
-    h3 = h4;
-    w0 = w1;
-    w1 = w2;
-    w2 = w3;
-    n0 = n1;
-    n1 = n2;
+  for (int32_t l = 0; l < nlevels; ++l) {
+    const int32_t next_end = level_start[min(l + 4, nlevels)];
+    const int32_t p2 = packet(begin, end);
+    const RecEntries r1 = load_entries(T, O, packet_head(p1), packet_line(p1), t);
+    const RecVars rv{row_lane<PK_W0>(p0), row_lane<PK_W0 + 1>(p0), row_lane<PK_W0 + 2>(p0)};
+    replay_one<kDual>(T, O, x, y, z, zret, packet_head(p0), rv, packet_line(p0), r0, tol);
+    __syncthreads();
+    p0 = p1;
+    p1 = p2;
     r0 = r1;
-    h4 = load_head(T, rec);
     begin = end;
     end = next_end;
   }
@@ -810,30 +849,37 @@ hipError_t gpk_replay(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, 
   hipLaunchKernelGGL(k_replay, dim3(1), dim3(64), 0, stream, tape, orig, x, y, z, zret, begin, end, primal, dual, tol);
   return hipGetLastError();
 }
-hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                           const int32_t* records, int32_t count, int32_t primal, int32_t dual, double tol,
-                           hipStream_t stream) {
+hipError_t gpk_pack_records(gp_tape_dev tape, gp_orig_dev orig, const int32_t* records, int32_t count, int32_t has_y,
+                            int32_t dual, int32_t* packets, hipStream_t stream) {
   if (count <= 0) return hipSuccess;
-  if ((primal != 0) == (dual != 0)) return hipErrorInvalidValue;  // one pass at a time
+  const dim3 grid(grid_for(count, kBlock / kRecLanes));
   if (dual)
-    hipLaunchKernelGGL(k_replay_list<true>, dim3(grid_for(count, kBlock / kRecLanes)), dim3(kBlock), 0, stream, tape, orig, x, y, z, zret,
-                       records, count, tol);
+    hipLaunchKernelGGL(k_pack_records<true>, grid, dim3(kBlock), 0, stream, tape, orig, records, count, has_y, packets);
   else
-    hipLaunchKernelGGL(k_replay_list<false>, dim3(grid_for(count, kBlock / kRecLanes)), dim3(kBlock), 0, stream, tape, orig, x, y, z, zret,
-                       records, count, tol);
+    hipLaunchKernelGGL(k_pack_records<false>, grid, dim3(kBlock), 0, stream, tape, orig, records, count, has_y, packets);
+  return hipGetLastError();
+}
+hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
+                           const int32_t* packets, int32_t count, int32_t dual, double tol, hipStream_t stream) {
+  if (count <= 0) return hipSuccess;
+  const dim3 grid(grid_for(count, kBlock / kRecLanes));
+  if (dual)
+    hipLaunchKernelGGL(k_replay_list<true>, grid, dim3(kBlock), 0, stream, tape, orig, x, y, z, zret, packets, count, tol);
+  else
+    hipLaunchKernelGGL(k_replay_list<false>, grid, dim3(kBlock), 0, stream, tape, orig, x, y, z, zret, packets, count, tol);
   return hipGetLastError();
 }
 hipError_t gpk_replay_levels(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                             const int32_t* records, const int32_t* level_start, int32_t nlevels, int32_t primal,
-                             int32_t dual, double tol, hipStream_t stream) {
+                             const int32_t* packets, const int32_t* level_start, int32_t nlevels, int32_t dual,
+                             double tol, hipStream_t stream) {
   if (nlevels <= 0) return hipSuccess;
-  if ((primal != 0) == (dual != 0)) return hipErrorInvalidValue;
+  const dim3 block(GPK_REPLAY_SLOTS * kRecLanes);
   if (dual)
-    hipLaunchKernelGGL(k_replay_levels<true>, dim3(1), dim3(GPK_REPLAY_SLOTS * kRecLanes), 0, stream, tape, orig, x, y, z, zret, records,
-                       level_start, nlevels, tol);
+    hipLaunchKernelGGL(k_replay_levels<true>, dim3(1), block, 0, stream, tape, orig, x, y, z, zret, packets, level_start,
+                       nlevels, tol);
   else
-    hipLaunchKernelGGL(k_replay_levels<false>, dim3(1), dim3(GPK_REPLAY_SLOTS * kRecLanes), 0, stream, tape, orig, x, y, z, zret,
-                       records, level_start, nlevels, tol);
+    hipLaunchKernelGGL(k_replay_levels<false>, dim3(1), block, 0, stream, tape, orig, x, y, z, zret, packets,
+                       level_start, nlevels, tol);
   return hipGetLastError();
 }
 hipError_t gpk_seg_lengths(const int32_t* ptr, const int32_t* list, int32_t count, int32_t* len, hipStream_t stream) {

@@ -54,18 +54,23 @@ hipError_t gpk_restore_fixed(const int32_t* idx, const double* val, int32_t coun
 hipError_t gpk_replay(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
                       int32_t begin, int32_t end, int32_t primal, int32_t dual, double tol, hipStream_t stream);
 /* Dependency-level replay (the reverse tape order split into levels whose
- * records touch disjoint variables), one pass at a time (primal or dual).
+ * records touch disjoint variables), one pass at a time (dual or primal).
+ * gpk_pack_records: the packets (GPK_PACKET_WORDS words each) of a schedule's
+ * records for a pass (-1: an empty slot; has_y: the replay has a y), which hold
+ * places in the tape and in the original model's row pointers, no values.
  * gpk_replay_list: the records of one level.  gpk_replay_levels: nlevels
- * consecutive levels in one workgroup, level lv being
- * records[level_start[lv] .. level_start[lv+1]), at most GPK_REPLAY_SLOTS of
- * them (a longer level is given as several); a record of -1 is an empty slot. */
+ * consecutive levels in one workgroup, level lv being slots [level_start[lv],
+ * level_start[lv+1]), at most GPK_REPLAY_SLOTS of them (a longer level is given
+ * as several). */
 #define GPK_REPLAY_SLOTS 64
+#define GPK_PACKET_WORDS 16
+hipError_t gpk_pack_records(gp_tape_dev tape, gp_orig_dev orig, const int32_t* records, int32_t count, int32_t has_y,
+                            int32_t dual, int32_t* packets, hipStream_t stream);
 hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                           const int32_t* records, int32_t count, int32_t primal, int32_t dual, double tol,
-                           hipStream_t stream);
+                           const int32_t* packets, int32_t count, int32_t dual, double tol, hipStream_t stream);
 hipError_t gpk_replay_levels(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                             const int32_t* records, const int32_t* level_start, int32_t nlevels, int32_t primal,
-                             int32_t dual, double tol, hipStream_t stream);
+                             const int32_t* packets, const int32_t* level_start, int32_t nlevels, int32_t dual,
+                             double tol, hipStream_t stream);
 /* len[i] = ptr[list[i] + 1] - ptr[list[i]]; gpk_seg_copy packs line
  * list[i]'s idx entries at out + off[i]. */
 hipError_t gpk_seg_lengths(const int32_t* ptr, const int32_t* list, int32_t count, int32_t* len, hipStream_t stream);

@@ -162,6 +162,61 @@ def test_presolve_with_dense_rows(lengths, kw):
     assert_same_lp(lg, lo)
 
 
+def with_dense_columns(lp, lengths, seed):
+    """The LP with further columns of the given lengths, every third one a
+    scaled copy of the one before it, and an equality of every sixth with a
+    column of the LP."""
+    rng = np.random.default_rng(seed)
+    m, n, k = lp["m"], lp["n"], len(lengths)
+    rows, cols, vals, c = [], [], [], []
+    for j, length in enumerate(lengths):
+        if j % 3 == 2:
+            r, v, cost = rows[-1], -2.0 * vals[-1], -2.0 * c[-1]
+        else:
+            r = np.sort(rng.choice(m, size=min(length, m), replace=False))
+            v = np.round(rng.uniform(0.5, 2.0, len(r)) * 8) / 8 * rng.choice([-1.0, 1.0], len(r))
+            cost = float(rng.integers(-8, 9)) / 8
+        rows.append(r)
+        cols.append(np.full(len(r), n + j))
+        vals.append(v)
+        c.append(cost)
+    pairs = rng.choice(n, size=k, replace=False)
+    eq = np.arange(0, k, 6)
+    r0 = np.repeat(np.arange(m), np.diff(lp["A_ptr"]))
+    M, N = m + len(eq), n + k
+    ptr, idx, val = lp_synth.csr_from_coo(
+        M, N, np.concatenate([r0] + rows + [m + np.arange(len(eq)), m + np.arange(len(eq))]),
+        np.concatenate([lp["A_idx"]] + cols + [n + eq, pairs[eq]]),
+        np.concatenate([lp["A_val"]] + vals + [np.full(len(eq), 2.0), np.full(len(eq), -1.0)]))
+    tptr, tidx, tval = lp_synth.transpose_csr(M, N, ptr, idx, val)
+    big = 2.0 ** 24
+    return dict(lp, m=M, n=N, A_ptr=ptr, A_idx=idx, A_val=val, AT_ptr=tptr, AT_idx=tidx, AT_val=tval,
+                c=np.concatenate([lp["c"], c]), l=np.concatenate([lp["l"], np.full(k, -big)]),
+                u=np.concatenate([lp["u"], np.full(k, big)]), AL=np.concatenate([lp["AL"], np.zeros(len(eq))]),
+                AU=np.concatenate([lp["AU"], np.zeros(len(eq))]))
+
+
+@pytest.mark.parametrize("lengths,kw", [
+    ([127, 128, 128, 129, 130, 130, 255, 256, 256, 8, 9, 9] * 2, {}),
+    ([2500, 2500, 2500, 600, 300, 300] * 4, dict(doubleton_equations_max_fill_in_proxy=100000)),
+    ([2900, 7, 7, 16, 17, 17, 1000, 1000, 1000] * 3, dict(record_postsolve_tape_cpu=1)),
+])
+def test_presolve_with_dense_columns(lengths, kw):
+    lp = lp_synth.generate(3000, 4500, seed=51, mean_row_len=4.0, frac_doubleton=0.25, frac_fixed_cols=0.05,
+                           frac_singleton_cols=0.15, frac_dup_rows=0.0, frac_eq=0.0)
+    lp = with_dense_columns(lp, lengths, 52)
+    kw = dict(kw, enable_structure_specific_rules=0)
+    sg, rg, lg = gp_ffi.presolve(lp, gp_ffi.params(**kw), True)
+    so, ro, lo = O.presolve(lp, O.params(**kw), True)
+    assert (sg["reduced_rows"], sg["reduced_cols"], sg["reduced_nnz"]) == (so["reduced_rows"], so["reduced_cols"],
+                                                                           so["reduced_nnz"])
+    assert sg["obj_constant_delta"] == so["obj_constant_delta"]
+    assert_same_record(rg, ro)
+    if not so["has_infeasible"]:  # the first LP's rules end at a contradiction, after doubletons and duplicates
+        assert_same_lp(lg, lo)
+    assert sg["has_infeasible"] == so["has_infeasible"]
+
+
 @pytest.mark.parametrize("n", [4097, 2048 * 16, 2048 * 16 + 1, 2048 * 17 - 1, 2048 * 64, 2048 * 64 + 1])
 def test_radix_sort_at_histogram_batches(n):
     rng = np.random.default_rng(n)

@@ -5,6 +5,8 @@
 
 #include <cstdint>
 
+#include "gp_walk.hpp"
+
 namespace gpdev {
 
 constexpr int kBlock = 256;  // 4 waves of 64 lanes
@@ -150,27 +152,27 @@ constexpr int kRowPitch = kRowChunk + 2;  // the kinds start in different banks
 template <int kSums, class G, class Load, class Term>
 __device__ __forceinline__ double wave_row_sums(const int32_t* __restrict__ idx, const double* __restrict__ val,
                                                 int32_t b, int32_t e, double* s_t, Load&& load, Term&& term) {
-  const int lane = lane_id();
+  const uint32_t lane = static_cast<uint32_t>(lane_id()), n = row_length(b, e);
   double a[kRowSteps], acc = 0.0;
   int32_t j[kRowSteps];
 #pragma unroll
   for (int k = 0; k < kRowSteps; ++k) {
-    const int32_t p = min(b + 64 * k + lane, e - 1);
+    const int32_t p = row_entry(b, e, 64 * k + lane);
     a[k] = val[p];
     j[k] = idx[p];
   }
 #pragma unroll 1
-  for (int32_t c = b; c < e; c += kRowChunk) {
+  for (uint32_t c = 0; c < n; c += kRowChunk) {
     G g[kRowSteps];
 #pragma unroll
-    for (int k = 0; k < kRowSteps; ++k) g[k] = load(j[k], a[k], c + 64 * k + lane < e);
+    for (int k = 0; k < kRowSteps; ++k) g[k] = load(j[k], a[k], c + 64 * k + lane < n);
     double t[kRowSteps][kSums];
     bool any = false;
 #pragma unroll
-    for (int k = 0; k < kRowSteps; ++k) any = term(a[k], g[k], c + 64 * k + lane < e, t[k]) || any;
+    for (int k = 0; k < kRowSteps; ++k) any = term(a[k], g[k], c + 64 * k + lane < n, t[k]) || any;
 #pragma unroll
     for (int k = 0; k < kRowSteps; ++k) {  // the last entry again past the row's end
-      const int32_t p = min(c + kRowChunk + 64 * k + lane, e - 1);
+      const int32_t p = row_entry(b, e, c + kRowChunk + 64 * k + lane);
       a[k] = val[p];
       j[k] = idx[p];
     }
@@ -180,7 +182,7 @@ __device__ __forceinline__ double wave_row_sums(const int32_t* __restrict__ idx,
 #pragma unroll
       for (int q = 0; q < kSums; ++q) s_t[q * kRowPitch + 64 * k + lane] = t[k][q];
     wave_lds_fence();
-    if (lane < kSums) acc = add_in_order(acc, s_t + lane * kRowPitch, min(kRowChunk, e - c));
+    if (lane < kSums) acc = add_in_order(acc, s_t + lane * kRowPitch, static_cast<int>(min(static_cast<uint32_t>(kRowChunk), n - c)));
     wave_lds_fence();
   }
   return acc;

@@ -188,7 +188,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
   const bool any_long = __syncthreads_or(is_long) != 0;
   double mn = 0.0, mx = 0.0;
   int32_t ni = 0, pi = 0;
-  for (int32_t w = seg_b; w < seg_e; w += kActCap) {
+  for (int32_t w = seg_b, we; w < seg_e; w = we) {
     if (any_long) {  // on to the next entry of a row that is added here
       if (tid == 0) s_next = seg_e;
       __syncthreads();
@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
       w = s_next;
       if (w >= seg_e) break;
     }
-    const int32_t we = min(w + kActCap, seg_e);
+    we = row_length(w, seg_e) > kActCap ? w + kActCap : seg_e;
     const int32_t rb = max(my_b, w), re = min(my_e, we);
     double a[kActItems];
     double2 b[kActItems];
@@ -207,22 +207,22 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
     // back to back and then the 8 gathers, with no wait in between.
 #pragma unroll
     for (int k = 0; k < kActItems; ++k) {
-      const int32_t pc = min(w + tid + k * kBlock, we - 1);
+      const int32_t pc = row_entry(w, we, tid + k * kBlock);
       a[k] = val[pc];
       j[k] = col_idx[pc];
     }
 #pragma unroll
     for (int k = 0; k < kActItems; ++k) {
-      if (w + tid + k * kBlock >= we) a[k] = 0.0;
+      if (tid + k * kBlock >= we - w) a[k] = 0.0;
       b[k] = lu[fabs(a[k]) > ztol ? j[k] : 0];
     }
     double tmx[kActItems];  // the max terms wait in registers while the min terms are summed
 #pragma unroll
     for (int k = 0; k < kActItems; ++k) {
-      const int32_t p = w + tid + k * kBlock;
+      const int t = tid + k * kBlock;
       const bool on = fabs(a[k]) > ztol;
       tmx[k] = act_max(a[k], b[k], on);
-      if (p < we) s_t[p - w] = act_min(a[k], b[k], on);
+      if (t < we - w) s_t[t] = act_min(a[k], b[k], on);
     }
     __syncthreads();
     for (int32_t p = rb; p < re; ++p) {
@@ -232,8 +232,8 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kActItems; ++k) {
-      const int32_t p = w + tid + k * kBlock;
-      if (p < we) s_t[p - w] = tmx[k];
+      const int t = tid + k * kBlock;
+      if (t < we - w) s_t[t] = tmx[k];
     }
     __syncthreads();
     for (int32_t p = rb; p < re; ++p) {
@@ -1192,7 +1192,9 @@ __global__ __launch_bounds__(kBlock) void k_expand_rows(const int32_t* __restric
   const int nr = min(kBlock, m - r0);
   for (int t = threadIdx.x; t <= nr; t += kBlock) s_ptr[t] = ptr[r0 + t];
   __syncthreads();
-  for (int32_t p = s_ptr[0] + threadIdx.x; p < s_ptr[nr]; p += kBlock) {
+  const int32_t b = s_ptr[0];
+  for (uint32_t o = threadIdx.x, n = row_length(b, s_ptr[nr]); o < n; o += kBlock) {
+    const int32_t p = b + static_cast<int32_t>(o);
     const double v = val[p];
     reinterpret_cast<int4*>(rv)[p] =
         make_int4(r0 + find_row(s_ptr, nr, p), 0, __double2loint(v), __double2hiint(v));
@@ -1580,8 +1582,11 @@ __global__ __launch_bounds__(kBlock) void k_csr_unsorted(const int32_t* __restri
   for (int t = tid; t <= nr; t += kBlock) s_ptr[t] = ptr[r0 + t];
   __syncthreads();
   bool desc = false;
-  for (int32_t p = s_ptr[0] + tid; p < s_ptr[nr]; p += kBlock)
+  const int32_t b = s_ptr[0];
+  for (uint32_t o = tid, n = row_length(b, s_ptr[nr]); o < n; o += kBlock) {
+    const int32_t p = b + static_cast<int32_t>(o);
     if (p > s_ptr[find_row(s_ptr, nr, p)]) desc = desc || idx[p] < idx[p - 1];
+  }
   if (desc) wave_set_flag(flag);
 }
 

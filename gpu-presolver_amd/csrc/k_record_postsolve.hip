@@ -763,25 +763,26 @@ __global__ void k_project_duals_long(gp_orig_dev O, const double* x, const doubl
     const int32_t col = long_cols[w];
     const int32_t b = O.at_ptr[col], e = O.at_ptr[col + 1];
     double aty = 0.0;
-    for (int32_t base = b; base < e; base += 64 * kLongSlices) {
+    for (uint32_t base = 0, n = row_length(b, e); base < n; base += 64 * kLongSlices) {
       int32_t j[kLongSlices];
       double a[kLongSlices], p[kLongSlices];
 #pragma unroll
       for (int u = 0; u < kLongSlices; ++u) {
-        const int32_t q = base + 64 * u + lane;
-        j[u] = q < e ? O.at_idx[q] : -1;
-        a[u] = q < e ? O.at_val[q] : 0.0;
+        const uint32_t o = base + 64 * u + lane;
+        const int32_t q = row_entry(b, e, o);
+        j[u] = o < n ? O.at_idx[q] : -1;
+        a[u] = o < n ? O.at_val[q] : 0.0;
       }
 #pragma unroll
       for (int u = 0; u < kLongSlices; ++u) p[u] = j[u] >= 0 ? a[u] * y[j[u]] : 0.0;
 #pragma unroll
       for (int u = 0; u < kLongSlices; ++u) {
-        const int32_t s0 = base + 64 * u;
-        if (s0 + 64 <= e) {
+        const uint32_t s0 = base + 64 * u;
+        if (s0 + 64 <= n) {
 #pragma unroll
           for (int t = 0; t < 64; ++t) aty += lane_f64(p[u], t);
         } else {
-          for (int t = 0; t < e - s0; ++t) aty += lane_f64(p[u], t);
+          for (uint32_t t = s0; t < n; ++t) aty += lane_f64(p[u], static_cast<int>(t - s0));
         }
       }
     }

@@ -219,12 +219,12 @@ __global__ __launch_bounds__(kBlock) void k_cs_activity_cache(int32_t row_blocks
   int32_t mn = 0, mp = 0, xn = 0, xp = 0;
   bool invalid = false;
   if (p.keep_row[i]) {
-    for (int32_t q0 = qb; q0 < qe; q0 += U) {
+    for (uint32_t q0 = 0, n = row_length(qb, qe); q0 < n; q0 += U) {
       int32_t cc[U];
       double av[U];
 #pragma unroll
       for (int k = 0; k < U; ++k) {
-        const int32_t q = min(q0 + k, qe - 1);
+        const int32_t q = row_entry(qb, qe, q0 + k);
         cc[k] = A.idx[q];
         av[k] = A.val[q];
       }
@@ -238,7 +238,7 @@ __global__ __launch_bounds__(kBlock) void k_cs_activity_cache(int32_t row_blocks
       }
 #pragma unroll
       for (int k = 0; k < U; ++k) {
-        if (q0 + k >= qe || !kept[k]) continue;
+        if (q0 + k >= n || !kept[k]) continue;
         const double a = av[k];
         const double tmin = a >= 0.0 ? a * lv[k] : a * uv[k];
         const double tmax = a >= 0.0 ? a * uv[k] : a * lv[k];
@@ -384,10 +384,10 @@ __global__ __launch_bounds__(kBlock) void k_cs_objective(int32_t row_blocks, gpk
     wave_long_rows(AT.ptr, n, kLongRow, row_blocks, [&](int64_t col, int32_t b, int32_t e) {
       double upd = p.c[col];
       if (p.keep_col[col] && !col_del[col]) {
-        for (int32_t c = b; c < e; c += 64) {
-          const int32_t q = min(c + lane_id(), e - 1);
+        for (uint32_t c = lane_id(), len = row_length(b, e); c - lane_id() < len; c += 64) {
+          const int32_t q = row_entry(b, e, c);
           const int32_t ow = owner[AT.idx[q]];
-          const bool on = c + lane_id() < e && ow >= 0 && ow < n && col_del[ow];
+          const bool on = c < len && ow >= 0 && ow < n && col_del[ow];
           const double v = on ? -(p.c[ow] * AT.val[q] / sval[ow]) : 0.0;
           for (uint64_t m = __ballot(on); m != 0; m &= m - 1)
             upd += __shfl(v, __ffsll(static_cast<unsigned long long>(m)) - 1, 64);
@@ -592,10 +592,11 @@ __global__ __launch_bounds__(kBlock) void k_dup_col_hash(int32_t row_blocks, gpk
       if (p.keep_col[col]) {
         int32_t live = 0;
         double piv = 0.0;
-        for (int32_t c = b; c < e; c += 64) {
-          const int32_t q = min(c + lane_id(), e - 1);
+        const uint32_t len = row_length(b, e), lane = static_cast<uint32_t>(lane_id());
+        for (uint32_t c = 0; c < len; c += 64) {
+          const int32_t q = row_entry(b, e, c + lane);
           const double a = AT.val[q];
-          const uint64_t on = __ballot(c + lane_id() < e && p.keep_row[AT.idx[q]] && fabs(a) > zt);
+          const uint64_t on = __ballot(c + lane < len && p.keep_row[AT.idx[q]] && fabs(a) > zt);
           if (live == 0 && on != 0) piv = __shfl(a, __ffsll(static_cast<unsigned long long>(on)) - 1, 64);
           live += static_cast<int32_t>(__popcll(on));
         }
@@ -603,15 +604,15 @@ __global__ __launch_bounds__(kBlock) void k_dup_col_hash(int32_t row_blocks, gpk
           h = fnv_mix(kFnvOffset, h);
         } else {
           h = fnv_mix(kFnvOffset, static_cast<uint64_t>(live));
-          int32_t j = AT.idx[min(b + lane_id(), e - 1)];
-          double a = AT.val[min(b + lane_id(), e - 1)];
+          int32_t j = AT.idx[row_entry(b, e, lane)];
+          double a = AT.val[row_entry(b, e, lane)];
 #pragma unroll 1
-          for (int32_t c = b; c < e; c += 64) {
-            uint64_t on = __ballot(c + lane_id() < e && p.keep_row[j] && fabs(a) > zt);
+          for (uint32_t c = 0; c < len; c += 64) {
+            uint64_t on = __ballot(c + lane < len && p.keep_row[j] && fabs(a) > zt);
             const uint64_t w = dbits(a / piv);
             const int lo = static_cast<int>(w), hi = static_cast<int>(w >> 32), row = j;
-            j = AT.idx[min(c + 64 + lane_id(), e - 1)];
-            a = AT.val[min(c + 64 + lane_id(), e - 1)];
+            j = AT.idx[row_entry(b, e, c + 64 + lane)];
+            a = AT.val[row_entry(b, e, c + 64 + lane)];
             for (; on != 0; on &= on - 1) {
               const int t = __ffsll(static_cast<unsigned long long>(on)) - 1;
               h = fnv_mix(h, static_cast<uint64_t>(static_cast<int64_t>(__builtin_amdgcn_readlane(row, t))));
@@ -845,13 +846,13 @@ struct LiveWalk {
       double a[8];
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
-        const int32_t q = min(base + k, stop - 1);
+        const int32_t q = row_entry(base, stop, k);
         row[k] = AT.idx[q];
         a[k] = AT.val[q];
       }
 #pragma unroll
       for (int k = 0; k < 8; ++k)
-        if (base + k < stop && keep_row[row[k]] && fabs(a[k]) > zt) live |= 1u << k;
+        if (k < stop - base && keep_row[row[k]] && fabs(a[k]) > zt) live |= 1u << k;
     }
     const int at = __ffs(live) - 1;
     int32_t r = row[0];
@@ -909,12 +910,12 @@ __global__ __launch_bounds__(kBlock) void k_dbl_live_nnz(int32_t row_blocks, gpk
     wave_long_rows(AT.ptr, AT.rows, kLongRow, row_blocks, [&](int64_t col, int32_t b, int32_t e) {
       int32_t cnt = 0;
       if (p.keep_col[col]) {
-        for (int32_t c = b; c < e; c += 256) {
+        for (uint32_t c = lane_id(), len = row_length(b, e); c - lane_id() < len; c += 256) {
           int32_t r[4];
           double a[4];
 #pragma unroll
           for (int k = 0; k < 4; ++k) {
-            const int32_t q = min(c + 64 * k + lane_id(), e - 1);
+            const int32_t q = row_entry(b, e, c + 64 * k);
             r[k] = AT.idx[q];
             a[k] = AT.val[q];
           }
@@ -923,7 +924,7 @@ __global__ __launch_bounds__(kBlock) void k_dbl_live_nnz(int32_t row_blocks, gpk
           for (int k = 0; k < 4; ++k) keep[k] = p.keep_row[r[k]] != 0;
 #pragma unroll
           for (int k = 0; k < 4; ++k)
-            cnt += static_cast<int32_t>(__popcll(__ballot(c + 64 * k + lane_id() < e && keep[k] && fabs(a[k]) > zt)));
+            cnt += static_cast<int32_t>(__popcll(__ballot(c + 64 * k < len && keep[k] && fabs(a[k]) > zt)));
         }
       }
       if (lane_id() == 0) nnz[col] = cnt;
@@ -1095,8 +1096,10 @@ __global__ __launch_bounds__(kBlock) void k_dbl_delta_count(int32_t row_blocks, 
       int32_t cnt = 0;
       if (p.keep_row[i])
 #pragma unroll 4
-        for (int32_t q = b + lane_id(); q < e; q += 64)
+        for (uint32_t o = lane_id(), len = row_length(b, e); o < len; o += 64) {
+          const int32_t q = b + static_cast<int32_t>(o);
           cnt += dbl_is_delta(cols, static_cast<int32_t>(i), A.idx[q], A.val[q], zt) ? 1 : 0;
+        }
       cnt = __shfl(wave_inclusive_sum(cnt), 63, 64);
       if (lane_id() == 0) counts[i] = cnt;
     });
@@ -1136,10 +1139,10 @@ __global__ __launch_bounds__(kBlock) void k_dbl_shift(int32_t row_blocks, gpk_cs
               return v.x != 0.0;
             });
         if (include_subst && __ballot(subst) != 0) {
-          for (int32_t c = b; c < e; c += 64) {
-            const int32_t q = min(c + lane_id(), e - 1), j = A.idx[q];
+          for (uint32_t c = lane_id(), len = row_length(b, e); c - lane_id() < len; c += 64) {
+            const int32_t q = row_entry(b, e, c), j = A.idx[q];
             const double a = A.val[q];
-            const bool on = c + lane_id() < e && dbl_is_delta(cols, static_cast<int32_t>(i), j, a, zt);
+            const bool on = c < len && dbl_is_delta(cols, static_cast<int32_t>(i), j, a, zt);
             const double v = on ? a * cols.beta_of[j] : 0.0;
             for (uint64_t m = __ballot(on); m; m &= m - 1) {
               const double x = __shfl(v, __ffsll(static_cast<unsigned long long>(m)) - 1, 64);
@@ -1222,10 +1225,10 @@ __global__ __launch_bounds__(kBlock) void k_dbl_delta_fill(int32_t row_blocks, g
       }
       int32_t n = 0;
 #pragma unroll 1
-      for (int32_t c = b; c < e; c += 64) {
-        const int32_t q = min(c + lane, e - 1), j = A.idx[q];
+      for (uint32_t c = lane, len = row_length(b, e); c - lane < len; c += 64) {
+        const int32_t q = row_entry(b, e, c), j = A.idx[q];
         const double a = A.val[q];
-        const bool on = c + lane < e && dbl_is_delta(cols, static_cast<int32_t>(i), j, a, zt);
+        const bool on = c < len && dbl_is_delta(cols, static_cast<int32_t>(i), j, a, zt);
         const uint64_t m = __ballot(on);
         if (on) {
           const int at = n + static_cast<int>(__popcll(m & lanemask_lt(lane)));
@@ -1307,7 +1310,10 @@ __device__ __forceinline__ void dbl_merge_wave(const gpk_csr& A, int32_t qb, int
   const uint64_t below = lanemask_lt(lane);
   bool ascending = true;
 #pragma unroll 1
-  for (int32_t q = qb + 1 + lane; q < qe; q += 64) ascending = ascending && A.idx[q - 1] < A.idx[q];
+  for (uint32_t o = 1 + lane, len = row_length(qb, qe); o < len; o += 64) {
+    const int32_t q = qb + static_cast<int32_t>(o);
+    ascending = ascending && A.idx[q - 1] < A.idx[q];
+  }
   if (qe - qb > kDblRowMax || re - rb > kDblLds || __ballot(!ascending) != 0) {
     if (lane == 0) dbl_merge_serial(A, qb, qe, rb, re, dcol, dval, zt, w, count, out_idx, out_val);
     return;
@@ -1315,10 +1321,11 @@ __device__ __forceinline__ void dbl_merge_wave(const gpk_csr& A, int32_t qb, int
   // The columns of the deltas that the row does not have.
   int32_t fresh = 0;
 #pragma unroll 1
-  for (int32_t r0 = rb; r0 < re; r0 += 64) {
-    const int32_t r = r0 + lane;
+  for (int32_t o = 0; o < re - rb; o += 64) {  // at most kDblLds
+    const bool in = o + lane < re - rb;
+    const int32_t r = rb + (in ? o + lane : 0);
     bool keep = false;
-    if (r < re) {
+    if (in) {
       const int32_t c = dcol[r];
       if (r == rb || dcol[r - 1] != c) {
         const int32_t q = lower_bound(A.idx, qb, qe, c);
@@ -1328,7 +1335,7 @@ __device__ __forceinline__ void dbl_merge_wave(const gpk_csr& A, int32_t qb, int
           keep = fabs(merged) > zt;
         }
       }
-      if (r - rb < kDblLds) s_new[r - rb] = fresh + static_cast<int32_t>(__popcll(__ballot(keep) & below)) + (keep ? (1 << 30) : 0);
+      s_new[r - rb] = fresh + static_cast<int32_t>(__popcll(__ballot(keep) & below)) + (keep ? (1 << 30) : 0);
     }
     const uint64_t m = __ballot(keep);
     fresh += static_cast<int32_t>(__popcll(m));
@@ -1336,12 +1343,12 @@ __device__ __forceinline__ void dbl_merge_wave(const gpk_csr& A, int32_t qb, int
   wave_lds_fence();
   int32_t kept = 0;
 #pragma unroll 1
-  for (int32_t q0 = qb; q0 < qe; q0 += 64) {
-    const int32_t q = q0 + lane;
+  for (int32_t o = 0; o < qe - qb; o += 64) {  // at most kDblRowMax
     bool keep = false;
     double merged = 0.0;
     int32_t c = 0, r = rb;
-    if (q < qe) {
+    if (o + lane < qe - qb) {
+      const int32_t q = qb + o + lane;
       c = A.idx[q];
       merged += A.val[q];
       r = lower_bound(dcol, rb, re, c);
@@ -1351,8 +1358,8 @@ __device__ __forceinline__ void dbl_merge_wave(const gpk_csr& A, int32_t qb, int
     const uint64_t m = __ballot(keep);
     if (out_idx) {
       if (lane == 0) {
-        s_bits[(q0 - qb) >> 6] = m;
-        s_pre[(q0 - qb) >> 6] = kept;
+        s_bits[o >> 6] = m;
+        s_pre[o >> 6] = kept;
       }
       if (keep) {
         const int32_t at = w + kept + static_cast<int32_t>(__popcll(m & below)) +
@@ -1369,8 +1376,9 @@ __device__ __forceinline__ void dbl_merge_wave(const gpk_csr& A, int32_t qb, int
   }
   wave_lds_fence();
 #pragma unroll 1
-  for (int32_t r = rb + lane; r < re; r += 64) {
-    if ((s_new[r - rb] >> 30) == 0) continue;
+  for (int32_t o = lane; o < re - rb; o += 64) {
+    if ((s_new[o] >> 30) == 0) continue;
+    const int32_t r = rb + o;
     const int32_t c = dcol[r], q = lower_bound(A.idx, qb, qe, c) - qb;
     double merged = 0.0;
     for (int32_t t = r; t < re && dcol[t] == c; ++t) merged += dval[t];

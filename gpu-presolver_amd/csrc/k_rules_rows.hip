@@ -299,12 +299,12 @@ __device__ inline void implied_walk(const gpk_csr& AT, const gpk_implied_row* __
                                     int32_t j, double ol, double ou, F&& f) {
   constexpr int U = 4;
   const int32_t qb = AT.ptr[j], qe = AT.ptr[j + 1];
-  for (int32_t q0 = qb; q0 < qe; q0 += U) {
+  for (uint32_t q0 = 0, n = row_length(qb, qe); q0 < n; q0 += U) {
     int32_t ri[U];
     double av[U];
 #pragma unroll
     for (int k = 0; k < U; ++k) {
-      const int32_t q = min(q0 + k, qe - 1);
+      const int32_t q = row_entry(qb, qe, q0 + k);
       ri[k] = AT.idx[q];
       av[k] = AT.val[q];
     }
@@ -313,7 +313,7 @@ __device__ inline void implied_walk(const gpk_csr& AT, const gpk_implied_row* __
     for (int k = 0; k < U; ++k) r[k] = rows[ri[k]];
 #pragma unroll
     for (int k = 0; k < U; ++k) {
-      if (q0 + k >= qe || !r[k].live) continue;
+      if (q0 + k >= n || !r[k].live) continue;
       const double a = av[k];
       if (fabs(a) <= ztol) continue;
       double tmin, tmax;
@@ -577,15 +577,16 @@ __global__ __launch_bounds__(kBlock) void k_dup_row_hash(int32_t row_blocks, gpk
         h = fnv_mix(kFnvOffset, static_cast<uint64_t>(i));
       } else {
         h = fnv_mix(kFnvOffset, static_cast<uint64_t>(e - b));
-        int32_t j = A.idx[min(b + lane_id(), e - 1)];
-        double a = A.val[min(b + lane_id(), e - 1)];
+        const uint32_t len = row_length(b, e), lane = static_cast<uint32_t>(lane_id());
+        int32_t j = A.idx[row_entry(b, e, lane)];
+        double a = A.val[row_entry(b, e, lane)];
 #pragma unroll 1
-        for (int32_t c = b; c < e; c += 64) {
+        for (uint32_t c = 0; c < len; c += 64) {
           const uint64_t w = dbits(a / piv);
           const int lo = static_cast<int>(w), hi = static_cast<int>(w >> 32), col = j;
-          j = A.idx[min(c + 64 + lane_id(), e - 1)];
-          a = A.val[min(c + 64 + lane_id(), e - 1)];
-          const int n = min(64, e - c);
+          j = A.idx[row_entry(b, e, c + 64 + lane)];
+          a = A.val[row_entry(b, e, c + 64 + lane)];
+          const int n = static_cast<int>(min(64u, len - c));
 #pragma unroll 1
           for (int t = 0; t < n; ++t) {
             h = fnv_mix(h, static_cast<uint64_t>(static_cast<int64_t>(__builtin_amdgcn_readlane(col, t))));
@@ -638,8 +639,10 @@ __global__ void k_dup_row_hash_wide(gpk_csr A, const uint8_t* keep_row, double c
   }
   const double piv = A.val[b];
   uint64_t agg = 0;
-  for (int32_t q = b + lane; q < e; q += 64)
+  for (uint32_t o = lane, n = row_length(b, e); o < n; o += 64) {
+    const int32_t q = b + static_cast<int32_t>(o);
     agg ^= fnv_mix(fnv_mix(kFnvOffset, static_cast<uint64_t>(static_cast<int64_t>(A.idx[q]))), dbits(A.val[q] / piv));
+  }
 #pragma unroll
   for (int d = 32; d >= 1; d >>= 1) agg ^= static_cast<uint64_t>(__shfl_xor(static_cast<unsigned long long>(agg), d, 64));
   if (lane == 0) hash[i] = fnv_mix(fnv_mix(kFnvOffset, static_cast<uint64_t>(e - b)), agg);

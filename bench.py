@@ -209,7 +209,7 @@ def compaction_case(gp_ffi, dlp, lp, frac, seed, with_at):
         _fields_ = [("m", C.c_int32), ("n", C.c_int32), ("keep_row", vp), ("keep_col", vp), ("l", vp), ("u", vp),
                     ("row_map", vp), ("col_map", vp), ("fixed_mask", vp), ("fixed_tiles", vp), ("counts", vp),
                     ("row_rank", vp), ("col_rank", vp), ("a_ptr", vp), ("at_ptr", vp), ("a_chunk", vp),
-                    ("at_chunk", vp), ("tile_counts", vp), ("chunk_shift", C.c_int32)]
+                    ("at_chunk", vp), ("tile_counts", vp), ("chunk_shift", C.c_int32), ("chunks", C.c_int32)]
 
     m, n, nnz = lp["m"], lp["n"], len(lp["A_idx"])
     rng = np.random.default_rng(seed)
@@ -250,7 +250,7 @@ def compaction_case(gp_ffi, dlp, lp, frac, seed, with_at):
     margs = Maps(m, n, keep["row"].ptr, keep["col"].ptr, None, None, maps["row"].ptr, maps["col"].ptr, None, None,
                  counts.ptr, ranks["row"].ptr, ranks["col"].ptr, dlp.A.g.row_ptr,
                  dlp.AT.g.row_ptr if with_at else None, sides[0]["chunk"].ptr,
-                 sides[1]["chunk"].ptr if with_at else None, tile_counts.ptr, shift)
+                 sides[1]["chunk"].ptr if with_at else None, tile_counts.ptr, shift, chunks)
     cnt = D(size=2 * chunks + 1, dtype=np.int32)
     status = D(np.zeros(max(tiles, L.gpk_lookback_tiles(2 * chunks)), np.uint64))
     tickets = D(np.zeros(1 << 16, np.int32))

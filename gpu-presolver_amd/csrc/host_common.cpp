@@ -660,6 +660,7 @@ DeviceCsrMatrix compact_csr(const DeviceCsrMatrix& A, const uint8_t* keep_row, c
   maps.a_chunk = chunk_row;
   maps.tile_counts = tile_counts;
   maps.chunk_shift = gpk_compact_shift(A.nnz);
+  maps.chunks = gpk_compact_chunks(A.nnz);
   check(gpk_apply_maps(maps, c.lookback(tiles), c.stream()), "keep maps");
   CompactStart st = compact_start(A, row_map, col_rank, chunk_row, counts + 4, nullptr, nullptr, nullptr, nullptr);
   int32_t h[5];

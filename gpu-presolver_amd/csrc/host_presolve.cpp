@@ -475,7 +475,7 @@ void apply_plan(WorkLp& cur, const PresolvePlanGpu& p, RecordState& rs, const De
   const gpk_apply_maps_args maps{m, n, p.keep_row_mask, p.keep_col_mask, p.new_l, p.new_u, row_map, col_map,
                                  fixed.mask, fixed.tiles, counts, row_rank.get(), col_rank.get(),
                                  src.rowPtr, at != nullptr ? at->rowPtr : nullptr, a_chunk, at_chunk, tile_counts,
-                                 gpk_compact_shift(src.nnz)};
+                                 gpk_compact_shift(src.nnz), chunks};
   check(gpk_apply_maps(maps, c.lookback(tiles), s), "keep maps");
   // The caller's AT (first change) is compacted like a working AT when its
   // rows are sorted; the flag comes back with the counts.

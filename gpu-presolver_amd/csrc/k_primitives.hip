@@ -534,13 +534,18 @@ __global__ __launch_bounds__(kBlock) void k_apply_maps(gpk_apply_maps_args a, in
     const int shift = a.chunk_shift;
     int64_t r = i0;
 #pragma unroll 1
-    for (int64_t q = (pb + (int64_t{1} << shift) - 1) >> shift; q << shift < pe; ++q) {
+    for (int64_t q = (pb + (int64_t{1} << shift) - 1) >> shift; q << shift < pe && q < a.chunks; ++q) {
 #pragma unroll 1
       while (r + 1 < i1 && ptr[r + 1] <= q << shift) ++r;
       chunk_row[q] = static_cast<int32_t>(r);
     }
-    if (tile == last && i1 == n && any)
-      chunk_row[(pe >> shift) + ((pe & ((1 << shift) - 1)) != 0 ? 1 : 0)] = static_cast<int32_t>(n) - 1;
+    // Chunks that start before the first row's entries or past the last row's.
+    const int64_t round = (int64_t{1} << shift) - 1;
+    if (tile == first)
+      for (int64_t q = tid, lead = (ptr[0] + round) >> shift; q < lead && q < a.chunks; q += kBlock) chunk_row[q] = 0;
+    if (tile == last)
+      for (int64_t q = ((ptr[n] + round) >> shift) + tid; q <= a.chunks; q += kBlock)
+        chunk_row[q] = static_cast<int32_t>(n) - 1;
   }
   if (!rows && a.l != nullptr) {
     // Removed, both bounds finite and within 1e-9 of each other.
@@ -763,7 +768,8 @@ __device__ __forceinline__ void compact_map_chunk(int32_t q, const gpk_compact_s
         const int32_t mid = lo + (hi - lo) / 2;
         if (s.ptr[mid] <= c0 + p) lo = mid; else hi = mid;
       }
-      if (s.row_map[lo] >= 0) atomicOr(&s_live[p >> 5], 1u << (p & 31));
+      const bool held = s.ptr[lo] <= c0 + p && c0 + p < s.ptr[lo + 1];
+      if (held && s.row_map[lo] >= 0) atomicOr(&s_live[p >> 5], 1u << (p & 31));
     }
   }
   __syncthreads();

@@ -83,8 +83,10 @@ typedef struct __attribute__((aligned(16))) gpk_rank_word {
  * 1e-9), fixed_tiles[t] counts those of columns [2048 t, 2048 (t + 1)) and
  * counts[2] all of them (the caller zeroes it).  a_chunk / at_chunk, when a_ptr
  * / at_ptr (row pointers over the m rows / n columns) are given, receive the
- * chunk rows of a compaction: entry q << chunk_shift lies in row a_chunk[q],
- * and the word after the last chunk's holds the last row.
+ * chunk rows of a compaction of `chunks` chunks: entry q << chunk_shift lies in
+ * row a_chunk[q], and a_chunk[chunks] is the last row.  The rows may hold fewer
+ * entries than the chunks (rows of a larger matrix): an entry before the first
+ * row's is given row 0, one past the last row's the last row.
  * The look-back workspace and tile_counts cover gpk_apply_maps_tiles(m, n)
  * tiles, fixed_tiles gpk_apply_maps_tiles(0, n). */
 typedef struct gpk_apply_maps_args {
@@ -106,6 +108,7 @@ typedef struct gpk_apply_maps_args {
   int32_t* at_chunk;
   int32_t* tile_counts;
   int32_t chunk_shift;
+  int32_t chunks;
 } gpk_apply_maps_args;
 int64_t gpk_apply_maps_tiles(int32_t m, int32_t n);
 hipError_t gpk_apply_maps(gpk_apply_maps_args args, gpk_lookback lb, hipStream_t stream);

@@ -225,3 +225,28 @@ def test_radix_sort_at_histogram_batches(n):
     order = np.argsort(keys, kind="stable")
     assert_same_array("keys", k, keys[order])
     assert_same_array("vals", v, order.astype(np.int32))
+
+
+@pytest.mark.parametrize("lengths,first,last", [
+    ([3] * 9000, 700, 8000), ([3] * 9000, 0, 8000), ([3] * 9000, 700, 9000),  # small chunks
+    ([5000] + [2] * 3000 + [4000] * 3, 1, 3001), ([2048] * 700, 2, 690),  # large chunks, whole ones before and after
+    ([40] * 300 + [0] * 20000 + [7] + [0] * 9000 + [40] * 300, 200, 29350),  # a chunk that spans many empty rows
+])
+def test_compaction_of_rows_of_a_larger_matrix(lengths, first, last):
+    """Row pointers that begin past entry 0 or end before the matrix's nnz."""
+    n = 5001
+    ptr, idx, val = csr_of_lengths(lengths, n, 17)
+    rng = np.random.default_rng(18)
+    m = last - first
+    kr, kc = (rng.random(m) < 0.7).astype(np.uint8), (rng.random(n) < 0.7).astype(np.uint8)
+    A = gp_ffi.DeviceCsr(len(lengths), n, ptr, idx, val)
+    view = gp_ffi.T.GpCsr(m, n, len(idx), A.g.row_ptr + 4 * first, A.g.col_idx, A.g.val)
+    dr, dc = gp_ffi.DeviceArray(kr), gp_ffi.DeviceArray(kc)
+    out = gp_ffi.T.GpCsr()
+    gp_ffi._check(gp_ffi.lib().gp_compact_csr(C.byref(view), dr.ptr, dc.ptr, C.byref(out)))
+    got = (out.rows, out.cols) + gp_ffi._take_csr(out)
+    b, e = ptr[first], ptr[last]
+    want = O.compact_csr(m, n, ptr[first:last + 1] - b, idx[b:e], val[b:e], kr, kc)
+    assert got[:2] == want[:2]
+    for name, a, w in zip(("ptr", "idx", "val"), got[2:], want[2:]):
+        assert_same_array(name, a, w)

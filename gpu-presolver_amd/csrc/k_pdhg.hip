@@ -37,6 +37,15 @@
 
 using namespace gpdev;
 
+// The parts of a split row meet through relaxed atomics whose order an empty
+// asm statement gives (k_rows): that the exchange's answer comes back only once
+// the sum is where every XCD's atomic loads see it is a property of this chip's
+// device-scope atomics, not of the memory model.  Another target needs
+// a release and an acquire there.
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "k_pdhg.hip orders the parts of a row as gfx950 does"
+#endif
+
 namespace {
 
 constexpr int kEntryBudget = GPK_PDHG_ENTRY_BUDGET;

@@ -4,6 +4,9 @@ thread to a wave, to a workgroup, to parts: each sum within its rounding bound
 of the exact one and the same bits every time."""
 import ctypes as C
 import math
+import os
+import shutil
+import subprocess
 
 import numpy as np
 import pytest
@@ -47,6 +50,19 @@ def test_plan_covers_every_entry_once(case):
     for k in np.nonzero(parts > 1)[0]:
         assert ptr[row[k]] + part[k] * BUDGET == entry[k] and row[k - part[k]] == row[k]
         assert parts[k] == -(-int(ptr[row[k] + 1] - ptr[row[k]]) // BUDGET)
+
+
+@pytest.mark.parametrize("arch,compiles", [("gfx950", True), ("gfx942", False)])
+def test_split_rows_are_tied_to_their_target(arch, compiles):
+    """The order of a row's parts is gfx950's: no other target may compile it."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    csrc = os.path.join(root, "gpu-presolver_amd", "csrc")
+    hipcc = shutil.which("hipcc") or "/opt/rocm/bin/hipcc"
+    r = subprocess.run([hipcc, f"--offload-arch={arch}", "--cuda-device-only", "-fsyntax-only", "-std=c++17",
+                        "-I" + os.path.join(root, "include"), "-I" + csrc, os.path.join(csrc, "k_pdhg.hip")],
+                       capture_output=True, text=True, timeout=100)
+    assert (r.returncode == 0) == compiles, r.stderr
+    assert compiles or "as gfx950 does" in r.stderr
 
 
 @pytest.mark.gpu

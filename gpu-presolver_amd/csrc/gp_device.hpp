@@ -86,6 +86,11 @@ __device__ inline double add_in_order(double s, const double* t, int n) {
   return s;
 }
 
+// Rows of more entries than this get a wave each in the kernels that otherwise
+// give a row to a thread: a thread walks a row at a few hundred ns an entry
+// (1.3 ms for 3,000), a wave needs about 3 us for a row and 10 ns an entry.
+constexpr int kLongRow = 128;
+
 // Calls f(row, begin, end) in all lanes of a wave for every row of more than
 // `longer` entries that falls to it, in a launch whose blocks from
 // `first_block` on are given to long rows.  A wave looks at every waves-th group of g
@@ -94,17 +99,17 @@ __device__ inline double add_in_order(double s, const double* t, int n) {
 // in all), past that the 16 rows of a line.  The row pointers of kLook groups
 // are loaded together: without a long row these blocks are gone in a few
 // memory round trips.
-// One such block a CU, or eight where rows are long on average (100,000 rows
-// of 200 entries are 12 for each wave then).
+// There are waves for as many long rows as the entries can make, up to eight
+// blocks a CU: 50,000 rows of 200 to 300 entries among a million short ones
+// are six for each wave (row activity 386 us, presolve 20.7 ms; 470 us and 25 ms
+// with one block a CU, 525 us and 26 ms with a thread or tile for every row).  On
+// 1M rows with no long one the blocks cost 2 us of 170.  nnz only sets the
+// number: every long row is found by one block as well.
 inline unsigned long_row_blocks(int32_t m, int64_t nnz) {
-  const unsigned b = grid_for(m, kWaves), most = nnz >= 32 * static_cast<int64_t>(m) ? 2048u : 256u;
-  return b < most ? b : most;
+  const int64_t most = nnz / (kLongRow + 1) + 1;
+  const unsigned b = grid_for(most < m ? most : m, kWaves);
+  return b < 2048 ? b : 2048;
 }
-
-// Rows of more entries than this get a wave each in the kernels that otherwise
-// give a row to a thread: a thread walks a row at a few hundred ns an entry
-// (1.3 ms for 3,000), a wave needs about 3 us for a row and 10 ns an entry.
-constexpr int kLongRow = 128;
 
 template <class F>
 __device__ __forceinline__ void wave_long_rows(const int32_t* __restrict__ ptr, int32_t m, int32_t longer,

@@ -106,7 +106,10 @@ __global__ void k_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t
 // thread would add thousands of terms from LDS while the other 255 wait, and
 // neighbouring long rows (linking rows come last in most models) would queue
 // in one block.  200 adjacent rows of 3,000 entries behind 80,000 short rows
-// took 67 ms per call that way, and 42 us with a wave each.
+// took 67 ms per call that way, and 42 us with a wave each.  The windows of a
+// block with long rows skip them (their entries were read by the tile and
+// by the wave before: 50,000 rows of 200 to 300 entries scattered among a million
+// short ones 570 -> 386 us, 100,000 rows of 129 580 -> 395).
 constexpr int kActRows = kBlock;
 constexpr int kActCap = 2048;
 constexpr int kActItems = kActCap / kBlock;
@@ -169,7 +172,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
   // One term array (the min terms, then the max terms): 16 KB of LDS per
   // block, so eight blocks fit a CU and their load phases overlap.
   __shared__ __align__(16) double s_t[kActCap + 16];
-  __shared__ int32_t s_next;
+  __shared__ int32_t s_run[kActRows], s_at[kActRows];
   if (static_cast<int32_t>(blockIdx.x) >= tiles) {
     double* s_row = s_t + (threadIdx.x >> 6) * 2 * kRowPitch;
     wave_long_rows(row_ptr, m, kLongRow, tiles, [&](int64_t row, int32_t b, int32_t e) {
@@ -181,35 +184,55 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
   const int32_t rows = min(kActRows, m - r0);
   const int tid = threadIdx.x;
   const int32_t seg_b = row_ptr[r0], seg_e = row_ptr[r0 + rows];
-  const int32_t my_b = row_ptr[r0 + min(tid, rows)];
-  int32_t my_e = row_ptr[r0 + min(tid + 1, rows)];
-  const bool is_long = my_e - my_b > kLongRow;
-  if (is_long) my_e = my_b;  // no entry of it is added here
-  const bool any_long = __syncthreads_or(is_long) != 0;
+  const int32_t row_b = row_ptr[r0 + min(tid, rows)], row_e = row_ptr[r0 + min(tid + 1, rows)];
+  const bool is_long = row_e - row_b > kLongRow;
+  // The windows go over the block's entries less those of its long rows: entry
+  // t of them stands at t + seg_b, or where there are long rows at t + s_at of
+  // the last run of rows between them that begins at or before t (s_run).
+  int32_t my_b = row_b - seg_b, my_e = row_e - seg_b, total = seg_e - seg_b, runs = 0;
+  if (__syncthreads_or(is_long) != 0) {
+    const int32_t len = is_long ? 0 : row_e - row_b;
+    my_b = block_exclusive_sum(len, &total);
+    my_e = my_b + len;
+    const bool head = tid < rows && !is_long && (tid == 0 || row_b - row_ptr[r0 + tid - 1] > kLongRow);
+    const int32_t run = block_exclusive_sum(head ? 1 : 0, &runs);
+    if (head) {
+      s_run[run] = my_b;
+      s_at[run] = row_b - my_b;
+    }
+    __syncthreads();
+  }
   double mn = 0.0, mx = 0.0;
   int32_t ni = 0, pi = 0;
-  for (int32_t w = seg_b, we; w < seg_e; w = we) {
-    if (any_long) {  // on to the next entry of a row that is added here
-      if (tid == 0) s_next = seg_e;
-      __syncthreads();
-      if (my_e > w && my_e > my_b) atomicMin(&s_next, max(my_b, w));
-      __syncthreads();
-      w = s_next;
-      if (w >= seg_e) break;
-    }
-    we = row_length(w, seg_e) > kActCap ? w + kActCap : seg_e;
+  for (int32_t w = 0, we; w < total; w = we) {
+    we = total - w > kActCap ? w + kActCap : total;
     const int32_t rb = max(my_b, w), re = min(my_e, we);
     double a[kActItems];
     double2 b[kActItems];
-    int32_t j[kActItems];
+    int32_t j[kActItems], pc[kActItems];
+#pragma unroll
+    for (int k = 0; k < kActItems; ++k) pc[k] = row_entry(w, we, tid + k * kBlock);
+    if (runs > 0) {
+#pragma unroll
+      for (int k = 0; k < kActItems; ++k) {
+        int lo = 0, hi = runs;  // s_run[lo] <= pc[k] < s_run[hi]
+        while (hi - lo > 1) {
+          const int mid = (lo + hi) >> 1;
+          if (s_run[mid] <= pc[k]) lo = mid; else hi = mid;
+        }
+        pc[k] += s_at[lo];
+      }
+    } else {
+#pragma unroll
+      for (int k = 0; k < kActItems; ++k) pc[k] += seg_b;
+    }
     // Every load is issued unconditionally (positions past the window read
     // its last entry and are discarded), so the compiler emits the 16 loads
     // back to back and then the 8 gathers, with no wait in between.
 #pragma unroll
     for (int k = 0; k < kActItems; ++k) {
-      const int32_t pc = row_entry(w, we, tid + k * kBlock);
-      a[k] = val[pc];
-      j[k] = col_idx[pc];
+      a[k] = val[pc[k]];
+      j[k] = col_idx[pc[k]];
     }
 #pragma unroll
     for (int k = 0; k < kActItems; ++k) {
@@ -240,7 +263,7 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
       const double t = s_t[p - w];
       if (isfinite(t)) mx += t; else if (t > 0.0) ++pi;
     }
-    if (we < seg_e) __syncthreads();  // the next window restages
+    if (we < total) __syncthreads();  // the next window restages
   }
   if (tid < rows && !is_long) {
     min_fin[r0 + tid] = mn;

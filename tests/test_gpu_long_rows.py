@@ -35,8 +35,18 @@ def lengths_with_long_rows(seed):
     return out
 
 
+def scattered_lengths(seed):
+    """Long rows between short and empty ones in every tile of 256, at its ends
+    and alone in it."""
+    rng = np.random.default_rng(seed)
+    out = [129, 0, 1] * 85 + [129]
+    out += [0, 300] * 128 + [5] * 255 + [140] + [140] + [5] * 255 + [200] * 256 + [0] * 255 + [131] + [0] * 256
+    out += [int(k) for k in np.where(rng.random(3000) < 0.05, rng.integers(120, 300, 3000), rng.integers(0, 60, 3000))]
+    return out
+
+
 @pytest.mark.parametrize("lengths", [[129], [128], [0, 3000, 0], lengths_with_long_rows(1),
-                                     [1500] * 257 + [3] * 9000 + [400] * 3])
+                                     [1500] * 257 + [3] * 9000 + [400] * 3, scattered_lengths(2)])
 def test_row_activity_long_rows(lengths):
     m, n = len(lengths), 3000
     ptr, idx, val = csr_of_lengths(lengths, n, 5)
@@ -45,6 +55,38 @@ def test_row_activity_long_rows(lengths):
     l, u = -np.round(rng.uniform(0, 4, n) * 1024) / 1024, np.round(rng.uniform(0, 4, n) * 1024) / 1024
     l[rng.random(n) < 0.1], u[rng.random(n) < 0.1] = -np.inf, np.inf
     val *= 1.0 + rng.random(len(val)) * 2.0 ** -20  # sums that round: the order of the terms shows
+    got = gp_ffi.row_activity(m, n, ptr, idx, val, l, u, 1e-10)
+    want = O.row_activity(m, n, ptr, idx, val, l, u, 1e-10)
+    for name, a, b in zip(("min_fin", "max_fin", "neg_inf", "pos_inf"), got, want):
+        assert_same_array(name, a, b)
+
+
+@pytest.mark.parametrize("m", [262_144, 262_145, 600_000, 1_200_001])
+def test_long_rows_of_large_matrices(m):
+    """Long rows where the waves' shares of the rows change: single rows up to
+    262,144 of them, groups of 16 past that; first and last row, neighbours in a
+    group, both sides of a group's end and of the rows that one look covers."""
+    n, group = 3000, 1 if m <= 262_144 else 16
+    longs = [129, 130, 255, 256, 257, 500, 3000, 1000, 200, 300]
+    at = {0, 1, m - 1, m - 2, 1603, 1604, 1615, 1616, m // 2 // 16 * 16 - 1, m // 2 // 16 * 16}
+    while True:  # the looks' length follows the entries: 8 x 64 rows for each wave
+        rows = sorted(at)
+        lengths = np.zeros(m, np.int64)
+        lengths[::37] = 2
+        lengths[rows] = np.resize(longs, len(rows))
+        most = min(m, int(lengths.sum()) // 129 + 1)
+        waves = 4 * min(2048, -(-most // 4))
+        look = 8 * 64 * waves
+        more = {r for k in range(1, m // look + 1) for r in (k * look - 1, k * look) if r < m}
+        more |= {r for r in (group * waves - 1, group * waves, 524_287, 524_288) if r < m}
+        if more <= at or len(at) > 200:
+            break
+        at |= more
+    ptr, idx, val = csr_of_lengths(lengths[lengths > 0], n, 19)
+    ptr = np.concatenate([[0], np.cumsum(lengths)]).astype(np.int32)
+    val *= 1.0 + np.random.default_rng(20).random(len(val)) * 2.0 ** -20
+    l, u = np.full(n, -1.0), np.full(n, 2.0)
+    u[::11] = np.inf
     got = gp_ffi.row_activity(m, n, ptr, idx, val, l, u, 1e-10)
     want = O.row_activity(m, n, ptr, idx, val, l, u, 1e-10)
     for name, a, b in zip(("min_fin", "max_fin", "neg_inf", "pos_inf"), got, want):
@@ -215,6 +257,19 @@ def test_presolve_with_dense_columns(lengths, kw):
     if not so["has_infeasible"]:  # the first LP's rules end at a contradiction, after doubletons and duplicates
         assert_same_lp(lg, lo)
     assert sg["has_infeasible"] == so["has_infeasible"]
+
+
+def test_presolve_with_long_columns_past_262144():
+    """More columns than the waves share one by one, some of them long."""
+    lp = lp_synth.generate(60_000, 264_000, seed=61, mean_row_len=5.0, frac_doubleton=0.1, frac_singleton_cols=0.1)
+    lp = with_dense_columns(lp, [129, 300, 300, 128, 2500, 2500, 700, 140, 140] * 3, 62)
+    kw = dict(enable_structure_specific_rules=0)
+    sg, rg, lg = gp_ffi.presolve(lp, gp_ffi.params(**kw), True)
+    so, ro, lo = O.presolve(lp, O.params(**kw), True)
+    assert lp["n"] > 262_144 and not so["has_infeasible"]
+    assert sg["obj_constant_delta"] == so["obj_constant_delta"]
+    assert_same_record(rg, ro)
+    assert_same_lp(lg, lo)
 
 
 @pytest.mark.parametrize("n", [4097, 2048 * 16, 2048 * 16 + 1, 2048 * 17 - 1, 2048 * 64, 2048 * 64 + 1])

@@ -369,14 +369,13 @@ def measure_transpose(gp_ffi, dlp, lp, stream, launches):
     L.gpk_transpose_buckets.argtypes = [i32, i32, C.POINTER(i32)]
     L.gpk_transpose_buckets_scratch_ints.restype = C.c_int64
     L.gpk_transpose_buckets_scratch_ints.argtypes = [i32, i32]
-    L.gpk_transpose_buckets_count.argtypes = [vp, i32, i32, i32, vp, vp, vp]
+    L.gpk_transpose_buckets_count.argtypes = [vp, i32, i32, i32, vp, vp]
     L.gpk_transpose_buckets_move.argtypes = [vp, vp, vp, i32, i32, i32, i32, i32, vp, vp, vp, vp, vp, vp]
     low = i32(0)
     buckets = L.gpk_transpose_buckets(n, nnz, C.byref(low))
     if buckets <= 0:
         raise SystemExit("bench.py: the LP is too small for the transpose by buckets")
     scratch = gp_ffi.DeviceArray(size=L.gpk_transpose_buckets_scratch_ints(buckets, nnz), dtype=np.int32)
-    largest = gp_ffi.DeviceArray(size=1, dtype=np.int32)
     ptr = gp_ffi.DeviceArray(size=n + 1, dtype=np.int32)
     idx, val = gp_ffi.DeviceArray(size=nnz, dtype=np.int32), gp_ffi.DeviceArray(size=nnz)
     rec = gp_ffi.DeviceArray(size=2 * nnz)  # 16-byte entries
@@ -384,8 +383,7 @@ def measure_transpose(gp_ffi, dlp, lp, stream, launches):
     ck = gp_ffi.hip_check
 
     def count():
-        ck(L.gpk_transpose_buckets_count(A.col_idx, nnz, low.value, buckets, scratch.ptr, largest.ptr, stream.ptr),
-           "bucket sizes")
+        ck(L.gpk_transpose_buckets_count(A.col_idx, nnz, low.value, buckets, scratch.ptr, stream.ptr), "bucket sizes")
 
     def move():
         ck(L.gpk_transpose_buckets_move(A.row_ptr, A.col_idx, A.val, m, n, nnz, low.value, buckets, scratch.ptr,

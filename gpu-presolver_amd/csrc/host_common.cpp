@@ -687,25 +687,22 @@ DeviceCsrMatrix transpose_csr(const DeviceCsrMatrix& A) {
     return T;
   }
   const int32_t nnz = A.nnz;
-  // Large matrices by buckets of columns.  A bucket that holds far more than
-  // the others (a few long columns next to each other) would leave the rest of
-  // the chip waiting for its workgroup, at about 1 us for 1,000 entries.
-  constexpr int32_t kMostInBucket = 65536;
+  // Large matrices by buckets of columns.
   int32_t low = 0;
   const int32_t buckets = gpk_transpose_buckets(A.cols, nnz, &low);
   if (buckets > 0) {
-    DBuf<int32_t> scratch(gpk_transpose_buckets_scratch_ints(buckets, nnz)), largest(1);
-    check(gpk_transpose_buckets_count(A.colVal, nnz, low, buckets, scratch, largest, s), "transpose bucket sizes");
+    DBuf<int32_t> scratch(gpk_transpose_buckets_scratch_ints(buckets, nnz));
+    check(gpk_transpose_buckets_count(A.colVal, nnz, low, buckets, scratch, s), "transpose bucket sizes");
     DBuf<gpk_row_val> rec(nnz, "transpose rows and values");
     DBuf<int32_t> idx(nnz, "transpose colVal");
     DBuf<double> val(nnz, "transpose nzVal");
-    if (c.scalar_to_host(largest.get(), "transpose bucket sizes") <= kMostInBucket) {
-      check(gpk_transpose_buckets_move(A.rowPtr, A.colVal, A.nzVal, A.rows, A.cols, nnz, low, buckets, scratch, rec, ptr, idx, val, s), "transpose buckets");
-      T.rowPtr = ptr.release();
-      T.colVal = idx.release();
-      T.nzVal = val.release();
-      return T;
-    }
+    check(gpk_transpose_buckets_move(A.rowPtr, A.colVal, A.nzVal, A.rows, A.cols, nnz, low, buckets, scratch, rec, ptr,
+                                     idx, val, s),
+          "transpose buckets");
+    T.rowPtr = ptr.release();
+    T.colVal = idx.release();
+    T.nzVal = val.release();
+    return T;
   }
   int32_t bits = 1;
   while (bits < 31 && (int64_t{1} << bits) < A.cols) ++bits;

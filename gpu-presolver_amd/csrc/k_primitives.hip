@@ -1256,9 +1256,10 @@ __global__ void k_transpose_gather(const int32_t* __restrict__ perm, const gpk_r
 // the order of A, so every row of the transpose comes out sorted.  (The sort of
 // the column indices alone reads and writes (key, position) three times and
 // then gathers 16 bytes from a line of 128 for each entry: 493 us a call for the
-// 1M x 1.5M LP's 8 million entries, of which 154 the gather; this takes 290: 32
-// the counts, 90 the first move, 105 the second, the rest the host's look at
-// the largest bucket, allocations and the call.)  The moves are bound by their
+// 1M x 1.5M LP's 8 million entries, of which 154 the gather; this takes 281: 34
+// the counts and pieces, 90 the first move, 105 the second, the rest allocations
+// and the call.  8 million entries with 100,000 to a million of them in one
+// column: 395 to 402, 480 by the sort; 80 million 3.2 ms against 4.9.)  The moves are bound by their
 // stores, a request to the L2 for each 16 bytes and for each 4 and 8.
 constexpr int kTbBlock = 512;
 constexpr int kTbWaves = kTbBlock / 64;
@@ -1319,20 +1320,57 @@ __global__ __launch_bounds__(kTbBlock) void k_tb_hist(const int32_t* __restrict_
   for (int d = tid; d < buckets; d += kTbBlock) hist[static_cast<int64_t>(d) * tiles + tile] = s_h[d];
 }
 
-// largest[0] = the most entries of a bucket.
-__global__ __launch_bounds__(kTbBuckets) void k_tb_largest(const int32_t* __restrict__ offs, int32_t buckets,
-                                                           int32_t tiles, int32_t* __restrict__ largest) {
-  __shared__ int32_t s_most[kTbBuckets / 64];
-  const int d = static_cast<int>(threadIdx.x);
-  int32_t v = d < buckets ? offs[static_cast<int64_t>(d + 1) * tiles] - offs[static_cast<int64_t>(d) * tiles] : 0;
-#pragma unroll
-  for (int k = 32; k >= 1; k >>= 1) v = max(v, __shfl_xor(v, k, 64));
-  if ((d & 63) == 0) s_most[d >> 6] = v;
-  __syncthreads();
-  if (d == 0) {
-    for (int w = 1; w < kTbBuckets / 64; ++w) v = max(v, s_most[w]);
-    largest[0] = v;
+// The second move takes a bucket by one workgroup, at about 1 us for 1,000
+// entries, unless it holds more than tb_share(nnz): then by several, each a
+// piece of its entries.  The share keeps a workgroup's time at what the whole
+// chip needs for the others, so a bucket of ordinary size has one piece (8
+// million entries: 62,500), and at most nnz / share + 1 buckets are split.
+constexpr int32_t kTbShareMin = 16384;
+constexpr int kTbMore = 128;              // pieces beyond one a bucket
+constexpr int kTbSplit = 2 * kTbMore;     // pieces of split buckets
+inline int32_t tb_share(int32_t nnz) {
+  const int32_t part = nnz / kTbMore + 1;
+  return part > kTbShareMin ? part : kTbShareMin;
+}
+struct TbPiece {
+  int32_t bucket;      // -1: none
+  int32_t begin, end;  // its entries
+  int32_t piece, pieces;
+  int32_t slot;  // of its column counts, the bucket's others next to it
+};
+static_assert(sizeof(TbPiece) == 6 * sizeof(int32_t), "laid out in 32-bit scratch");
+
+// The pieces of all buckets, in their order; entries past them have no bucket.
+// split[s]: the piece with slot s, -1 past the last.
+__global__ __launch_bounds__(kTbBuckets) void k_tb_pieces(const int32_t* __restrict__ offs, int32_t buckets,
+                                                          int32_t tiles, int32_t share, TbPiece* __restrict__ piece,
+                                                          int32_t* __restrict__ split) {
+  __shared__ int32_t s_all[kTbBuckets / 64], s_slots[kTbBuckets / 64];
+  const int d = static_cast<int>(threadIdx.x), wave = d >> 6;
+  const int32_t b = d < buckets ? offs[static_cast<int64_t>(d) * tiles] : 0;
+  const int32_t e = d < buckets ? offs[static_cast<int64_t>(d + 1) * tiles] : 0;
+  const int32_t n = d >= buckets ? 0 : e - b > share ? (e - b - 1) / share + 1 : 1;
+  const int32_t many = n > 1 ? n : 0;
+  const int32_t all = wave_inclusive_sum(n), slots = wave_inclusive_sum(many);
+  if ((d & 63) == 63) {
+    s_all[wave] = all;
+    s_slots[wave] = slots;
   }
+  __syncthreads();
+  int32_t at = all - n, slot = slots - many, total = 0, total_slots = 0;
+  for (int w = 0; w < kTbBuckets / 64; ++w) {
+    at += w < wave ? s_all[w] : 0;
+    slot += w < wave ? s_slots[w] : 0;
+    total += s_all[w];
+    total_slots += s_slots[w];
+  }
+  for (int32_t k = 0; k < n; ++k) {
+    const int32_t from = b + k * share;
+    piece[at + k] = TbPiece{d, from, k + 1 < n ? from + share : e, k, n, slot + k};
+    if (many != 0) split[slot + k] = at + k;
+  }
+  for (int32_t k = total + d; k < buckets + kTbMore; k += kTbBuckets) piece[k] = TbPiece{-1, 0, 0, 0, 0, 0};
+  for (int32_t k = total_slots + d; k < kTbSplit; k += kTbBuckets) split[k] = -1;
 }
 
 // The last row that starts at or before entry p, by a wave: a 64th of the rows
@@ -1435,10 +1473,42 @@ __global__ __launch_bounds__(kTbBlock) void k_tb_partition(const int32_t* __rest
           make_int4(j[k], first + s_row[mine + 64 * k], __double2loint(v[k]), __double2hiint(v[k]));
 }
 
-// One bucket: its entries counted by column, which gives the columns' row
-// pointers of the transpose, then placed tile by tile in their order.
+// s_count[c] = the entries of column c of the bucket among rec[b, e).
+__device__ __forceinline__ void tb_count_columns(const int4* __restrict__ rec, int32_t b, int32_t e, int cols,
+                                                 int32_t* s_count) {
+  const int tid = static_cast<int>(threadIdx.x);
+  for (int i = tid; i < kTbCols; i += kTbBlock) s_count[i] = 0;
+  __syncthreads();
+  for (int32_t p0 = b; p0 < e; p0 += kTbTile) {
+    int32_t j[kTbSteps];
+#pragma unroll
+    for (int k = 0; k < kTbSteps; ++k) j[k] = rec[min(p0 + k * kTbBlock + tid, e - 1)].x;
+#pragma unroll
+    for (int k = 0; k < kTbSteps; ++k)
+      if (p0 + k * kTbBlock + tid < e) atomicAdd(&s_count[j[k] & (cols - 1)], 1);
+  }
+  __syncthreads();
+}
+
+// The column counts of the split buckets' pieces, kTbCols words a slot.
+__global__ __launch_bounds__(kTbBlock) void k_tb_piece_counts(const int4* __restrict__ rec, int low,
+                                                              const TbPiece* __restrict__ piece,
+                                                              const int32_t* __restrict__ split,
+                                                              int32_t* __restrict__ counts) {
+  __shared__ int32_t s_count[kTbCols];
+  const int32_t at = split[blockIdx.x];
+  if (at < 0) return;
+  tb_count_columns(rec, piece[at].begin, piece[at].end, 1 << low, s_count);
+  for (int i = static_cast<int>(threadIdx.x); i < kTbCols; i += kTbBlock)
+    counts[static_cast<int64_t>(blockIdx.x) * kTbCols + i] = s_count[i];
+}
+
+// A piece (mostly a whole bucket): the bucket's entries counted by column, which
+// gives the columns' row pointers of the transpose, then the piece's placed tile
+// by tile in their order, after those of the pieces before it.
 __global__ __launch_bounds__(kTbBlock) void k_tb_columns(const int4* __restrict__ rec, int32_t n, int32_t nnz, int low,
-                                                         int32_t tiles, const int32_t* __restrict__ offs,
+                                                         int32_t share, const TbPiece* __restrict__ piece,
+                                                         const int32_t* __restrict__ counts,
                                                          int32_t* __restrict__ at_ptr, int32_t* __restrict__ at_idx,
                                                          double* __restrict__ at_val) {
   __shared__ uint16_t s_cnt[kTbWaves][kTbCols];
@@ -1447,39 +1517,46 @@ __global__ __launch_bounds__(kTbBlock) void k_tb_columns(const int4* __restrict_
   constexpr int kPer = kTbCols / kTbBlock;
   const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6, lane = tid & 63;
   const int cols = 1 << low;
-  const int32_t bucket = static_cast<int32_t>(blockIdx.x);
-  const int32_t b = offs[static_cast<int64_t>(bucket) * tiles], e = offs[static_cast<int64_t>(bucket + 1) * tiles];
+  const TbPiece me = piece[blockIdx.x];
+  if (me.bucket < 0) return;
+  const int32_t b = me.begin, e = me.end;
+  int32_t c[kPer], before[kPer], sum = 0;  // of the whole bucket, of the pieces before
+  if (me.pieces == 1) {
+    tb_count_columns(rec, b, e, cols, s_next);
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) s_next[tid * kPer + k] = 0;
-  __syncthreads();
-  for (int32_t p0 = b; p0 < e; p0 += kTbTile) {
-    int32_t j[kTbSteps];
-#pragma unroll
-    for (int k = 0; k < kTbSteps; ++k) j[k] = rec[min(p0 + k * kTbBlock + tid, e - 1)].x;
-#pragma unroll
-    for (int k = 0; k < kTbSteps; ++k)
-      if (p0 + k * kTbBlock + tid < e) atomicAdd(&s_next[j[k] & (cols - 1)], 1);
+    for (int k = 0; k < kPer; ++k) {
+      c[k] = s_next[tid * kPer + k];
+      before[k] = 0;
+    }
+  } else {
+    static_assert(kPer == 4, "a thread's columns in one load");
+    const int4* __restrict__ of = reinterpret_cast<const int4*>(counts + static_cast<int64_t>(me.slot - me.piece) * kTbCols) + tid;
+    int4 t{0, 0, 0, 0}, f{0, 0, 0, 0};
+#pragma unroll 8
+    for (int32_t k = 0; k < me.pieces; ++k) {
+      const int4 v = of[static_cast<int64_t>(k) * (kTbCols / 4)];
+      const int32_t on = k < me.piece ? 1 : 0;
+      t.x += v.x, t.y += v.y, t.z += v.z, t.w += v.w;
+      f.x += on * v.x, f.y += on * v.y, f.z += on * v.z, f.w += on * v.w;
+    }
+    c[0] = t.x, c[1] = t.y, c[2] = t.z, c[3] = t.w;
+    before[0] = f.x, before[1] = f.y, before[2] = f.z, before[3] = f.w;
   }
-  __syncthreads();
-  int32_t c[kPer], sum = 0;
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    c[k] = s_next[tid * kPer + k];
-    sum += c[k];
-  }
+  for (int k = 0; k < kPer; ++k) sum += c[k];
   const int32_t inc = wave_inclusive_sum(sum);
   if (lane == 63) s_w[wave] = inc;
   __syncthreads();
-  int32_t at = b + inc - sum;
+  int32_t at = b - me.piece * share + inc - sum;  // from where the bucket begins
   for (int w = 0; w < wave; ++w) at += s_w[w];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    const int64_t col = (static_cast<int64_t>(bucket) << low) + tid * kPer + k;
-    if (tid * kPer + k < cols && col < n) at_ptr[col] = at;
-    s_next[tid * kPer + k] = at;
+    const int64_t col = (static_cast<int64_t>(me.bucket) << low) + tid * kPer + k;
+    if (me.piece == 0 && tid * kPer + k < cols && col < n) at_ptr[col] = at;
+    s_next[tid * kPer + k] = at + before[k];
     at += c[k];
   }
-  if (bucket == 0 && tid == 0) at_ptr[n] = nnz;
+  if (me.bucket == 0 && me.piece == 0 && tid == 0) at_ptr[n] = nnz;
   const uint64_t below = lanemask_lt(lane);
   const int32_t mine = wave * (64 * kTbSteps) + lane;
   for (int32_t p0 = b; p0 < e; p0 += kTbTile) {
@@ -2066,8 +2143,8 @@ hipError_t gpk_transpose_sort(const int32_t* col, int32_t nnz, int32_t key_bits,
 
 int32_t gpk_transpose_buckets(int32_t n, int32_t nnz, int32_t* low) {
   // At 1,048,576 entries the buckets take 99 to 107 us where the sort takes 117
-  // to 147 (128 against 190 at twice that); below, the wait for the largest
-  // bucket's size is most of it.  Up to 256 columns the sort has one pass.
+  // to 147 (128 against 190 at twice that).  Up to 256 columns the sort has one
+  // pass.
   *low = 0;
   if (nnz < GPK_TRANSPOSE_BUCKETS_MIN_NNZ || nnz > INT_MAX - 2 * kTbTile || n <= 256) return 0;
   while (*low < kTbLowMax && ((n - 1) >> *low) >= kTbBuckets) ++*low;
@@ -2075,36 +2152,69 @@ int32_t gpk_transpose_buckets(int32_t n, int32_t nnz, int32_t* low) {
   return buckets <= kTbBuckets ? buckets : 0;
 }
 
-int64_t gpk_transpose_buckets_scratch_ints(int32_t buckets, int32_t nnz) {
+namespace {
+// The scratch of a transpose by buckets, 16 bytes to a line of counts.
+struct TbScratch {
+  int32_t* offs;  // buckets x tiles counts, then their exclusive scan and total
+  int32_t* scan;
+  TbPiece* piece;
+  int32_t* split;
+  int32_t* counts;
+  int64_t ints;
+};
+TbScratch tb_scratch(int32_t* base, int32_t buckets, int32_t nnz) {
   const int64_t words = static_cast<int64_t>(buckets) * grid_for(nnz, kTbTile);
-  return words + 1 + gpk_scan_scratch_ints(words) + 1;
+  int64_t used = 0;
+  const auto take = [&](int64_t ints) {
+    int32_t* p = base + used;
+    used += (ints + 3) / 4 * 4;
+    return p;
+  };
+  TbScratch t{};
+  t.offs = take(words + 1);
+  t.scan = take(gpk_scan_scratch_ints(words));
+  t.piece = reinterpret_cast<TbPiece*>(take((buckets + kTbMore) * static_cast<int64_t>(sizeof(TbPiece) / sizeof(int32_t))));
+  t.split = take(kTbSplit);
+  t.counts = take(static_cast<int64_t>(kTbSplit) * kTbCols);
+  t.ints = used;
+  return t;
+}
+}  // namespace
+
+int64_t gpk_transpose_buckets_scratch_ints(int32_t buckets, int32_t nnz) {
+  return tb_scratch(nullptr, buckets, nnz).ints;
 }
 
 hipError_t gpk_transpose_buckets_count(const int32_t* col, int32_t nnz, int32_t low, int32_t buckets, int32_t* scratch,
-                                       int32_t* largest, hipStream_t s) {
+                                       hipStream_t s) {
   if (nnz <= 0 || buckets <= 0 || buckets > kTbBuckets || low < 0 || low > kTbLowMax) return hipErrorInvalidValue;
   const int32_t tiles = static_cast<int32_t>(grid_for(nnz, kTbTile));
   const int64_t words = static_cast<int64_t>(buckets) * tiles;
-  hipLaunchKernelGGL(k_tb_hist, dim3(tiles), dim3(kTbBlock), 0, s, col, nnz, low, buckets, tiles, scratch);
-  const hipError_t e = scan_impl<int32_t>(scratch, scratch, words, scratch + words + 1, s);
+  const TbScratch t = tb_scratch(scratch, buckets, nnz);
+  hipLaunchKernelGGL(k_tb_hist, dim3(tiles), dim3(kTbBlock), 0, s, col, nnz, low, buckets, tiles, t.offs);
+  const hipError_t e = scan_impl<int32_t>(t.offs, t.offs, words, t.scan, s);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_tb_largest, dim3(1), dim3(kTbBuckets), 0, s, static_cast<const int32_t*>(scratch), buckets,
-                     tiles, largest);
+  hipLaunchKernelGGL(k_tb_pieces, dim3(1), dim3(kTbBuckets), 0, s, static_cast<const int32_t*>(t.offs), buckets, tiles,
+                     tb_share(nnz), t.piece, t.split);
   return hipGetLastError();
 }
 
 hipError_t gpk_transpose_buckets_move(const int32_t* ptr, const int32_t* col, const double* val, int32_t m, int32_t n,
-                                      int32_t nnz, int32_t low, int32_t buckets, const int32_t* scratch,
+                                      int32_t nnz, int32_t low, int32_t buckets, int32_t* scratch,
                                       gpk_row_val* rec, int32_t* at_ptr, int32_t* at_idx, double* at_val,
                                       hipStream_t s) {
   if (nnz <= 0 || buckets <= 0 || buckets > kTbBuckets || low < 0 || low > kTbLowMax) return hipErrorInvalidValue;
   const int32_t tiles = static_cast<int32_t>(grid_for(nnz, kTbTile));
   int bits = 0;
   while ((1 << bits) < buckets) ++bits;
+  const TbScratch t = tb_scratch(scratch, buckets, nnz);
   hipLaunchKernelGGL(k_tb_partition, dim3(tiles), dim3(kTbBlock), 0, s, ptr, col, val, m, nnz, low,
-                     buckets, bits, tiles, scratch, reinterpret_cast<int4*>(rec));
-  hipLaunchKernelGGL(k_tb_columns, dim3(buckets), dim3(kTbBlock), 0, s, reinterpret_cast<const int4*>(rec), n,
-                     nnz, low, tiles, scratch, at_ptr, at_idx, at_val);
+                     buckets, bits, tiles, static_cast<const int32_t*>(t.offs), reinterpret_cast<int4*>(rec));
+  hipLaunchKernelGGL(k_tb_piece_counts, dim3(kTbSplit), dim3(kTbBlock), 0, s, reinterpret_cast<const int4*>(rec), low,
+                     static_cast<const TbPiece*>(t.piece), static_cast<const int32_t*>(t.split), t.counts);
+  hipLaunchKernelGGL(k_tb_columns, dim3(buckets + kTbMore), dim3(kTbBlock), 0, s, reinterpret_cast<const int4*>(rec), n,
+                     nnz, low, tb_share(nnz), static_cast<const TbPiece*>(t.piece),
+                     static_cast<const int32_t*>(t.counts), at_ptr, at_idx, at_val);
   return hipGetLastError();
 }
 

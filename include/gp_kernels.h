@@ -275,16 +275,16 @@ hipError_t gpk_expand_rows(const int32_t* ptr, const double* val, int32_t m, gpk
 /* The transpose by buckets of 2^low columns, for matrices of at least
  * GPK_TRANSPOSE_BUCKETS_MIN_NNZ entries and 257 to 2,097,152 columns:
  * gpk_transpose_buckets gives the buckets (0: another matrix) and low;
- * _count counts the entries of the buckets into scratch and leaves the most
- * of a bucket in largest[0]; _move moves them through rec (A.nnz, 16-byte
- * aligned) to the transpose, a bucket's by one workgroup. */
+ * _count counts the entries of the buckets into scratch (16-byte aligned) and
+ * splits large buckets into pieces; _move moves them through rec (A.nnz, 16-byte
+ * aligned) to the transpose, a piece's by one workgroup. */
 #define GPK_TRANSPOSE_BUCKETS_MIN_NNZ 1048576
 int32_t gpk_transpose_buckets(int32_t n, int32_t nnz, int32_t* low);
 int64_t gpk_transpose_buckets_scratch_ints(int32_t buckets, int32_t nnz);
 hipError_t gpk_transpose_buckets_count(const int32_t* col, int32_t nnz, int32_t low, int32_t buckets, int32_t* scratch,
-                                       int32_t* largest, hipStream_t stream);
+                                       hipStream_t stream);
 hipError_t gpk_transpose_buckets_move(const int32_t* ptr, const int32_t* col, const double* val, int32_t m, int32_t n,
-                                      int32_t nnz, int32_t low, int32_t buckets, const int32_t* scratch,
+                                      int32_t nnz, int32_t low, int32_t buckets, int32_t* scratch,
                                       gpk_row_val* rec, int32_t* at_ptr, int32_t* at_idx, double* at_val,
                                       hipStream_t stream);
 hipError_t gpk_transpose_gather(const int32_t* perm, const gpk_row_val* rv, int32_t nnz, int32_t* at_idx,

@@ -1269,6 +1269,13 @@ constexpr int kTbBuckets = 1024;
 constexpr int kTbLowMax = 11;
 constexpr int kTbCols = 1 << kTbLowMax;
 
+// Rows that a tile spans (its entries' and the empty ones between) up to which
+// each marks its first entry; past that every entry looks its row up by
+// bisection.  With 900,000 empty rows in one tile's span a transpose of 8 million
+// entries takes 375 us, 1,190 with a mark for each of them (9 million: 375 against
+// 8,670).
+constexpr int32_t kTbMarkRows = 16 * kTbBlock;
+
 // Blocks go to the XCDs in turn; neighbouring tiles write neighbouring words, so
 // an XCD gets a stretch of tiles and its L2 joins them into whole lines.
 constexpr int kXcds = 8;
@@ -1397,7 +1404,7 @@ __global__ __launch_bounds__(kTbBlock) void k_tb_partition(const int32_t* __rest
   __shared__ int32_t s_base[kTbBuckets];
   __shared__ int32_t s_row[kTbTile];  // row - first, of each entry
   __shared__ int32_t s_w[kTbWaves];
-  __shared__ int32_t s_first;
+  __shared__ int32_t s_first, s_last;
   const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6, lane = tid & 63;
   const int32_t tile = tb_tile(tiles);
   const int32_t c0 = tile * kTbTile;
@@ -1414,18 +1421,28 @@ __global__ __launch_bounds__(kTbBlock) void k_tb_partition(const int32_t* __rest
   for (int i = tid; i < kTbWaves * kTbBuckets / 2; i += kTbBlock) reinterpret_cast<uint32_t*>(&s_cnt[0][0])[i] = 0;
   for (int i = tid; i < kTbTile; i += kTbBlock) s_row[i] = 0;
   for (int d = tid; d < buckets; d += kTbBlock) s_base[d] = offs[static_cast<int64_t>(d) * tiles + tile];
-  if (wave == 0) {
-    const int32_t r = wave_row_of(ptr, m, c0);
-    if (lane == 0) s_first = r;
+  if (wave < 2) {
+    const int32_t r = wave_row_of(ptr, m, wave == 0 ? c0 : c0 + (cnt - 1));
+    if (lane == 0) (wave == 0 ? s_first : s_last) = r;
   }
   __syncthreads();
-  // Each further row marks its first entry (of rows that start together the
-  // last one holds it); the running maximum is then every entry's row.
-  const int32_t first = s_first;
-  for (int64_t r = static_cast<int64_t>(first) + 1 + tid; r < m; r += kTbBlock) {
-    const int32_t p = ptr[r] - c0;
-    if (p >= cnt) break;
-    if (p >= 0) atomicMax(&s_row[p], static_cast<int32_t>(r - first));
+  const int32_t first = s_first, last = s_last;
+  if (last - first <= kTbMarkRows) {
+    // Each further row marks its first entry (of rows that start together the
+    // last one holds it); the running maximum is then every entry's row.
+    for (int64_t r = static_cast<int64_t>(first) + 1 + tid; r <= last; r += kTbBlock) {
+      const int32_t p = ptr[r] - c0;
+      if (p >= 0) atomicMax(&s_row[p], static_cast<int32_t>(r - first));
+    }
+  } else {
+    for (int i = tid; i < cnt; i += kTbBlock) {
+      int32_t lo = first, hi = last;  // the last row that starts at or before the entry is one of [lo, hi]
+      while (lo < hi) {
+        const int32_t mid = hi - (hi - lo) / 2;
+        if (ptr[mid] <= c0 + i) lo = mid; else hi = mid - 1;
+      }
+      s_row[i] = lo - first;
+    }
   }
   __syncthreads();
   int32_t run[kTbSteps];

@@ -51,6 +51,9 @@ def lengths(kind, nnz):
         lens = np.full(nnz // 3000 + 1, 3000)
     elif kind == "one-row":
         lens = np.array([nnz])
+    elif kind == "gap":  # a tile that spans more empty rows than it marks, others a few more or less
+        lens = np.concatenate([np.full(nnz // 10 - 5040, 5)] + [np.r_[np.zeros(g, np.int64), np.full(700, 6)] for g in
+                               (8186, 8190, 8192, 8193, 8200, 300_000)] + [np.full(nnz // 10 + 2, 5)])
     else:  # empty rows in between, by the thousand
         lens = np.zeros(400_000, np.int64)
         at = np.random.default_rng(1).choice(400_000, nnz // 40 + 1, replace=False)
@@ -73,7 +76,7 @@ KINDS = [
     ("short", 1025, MIN + 1, 0), ("short", 256, MIN + 1, 0), ("short", 257, MIN + 1, 0), ("short", 2_097_152, MIN + 5, 0), ("short", 2_097_153, MIN + 5, 0),
     ("long", 100_003, MIN + 17, 0), ("long", 3000, MIN + 17, 0), ("empty", 70_000, MIN + 3, 0),
     ("short", 200_000, MIN + 7, 15_000), ("short", 200_000, MIN + 7, 65_000), ("short", 200_000, MIN + 7, 120_000),
-    ("one-row", 1_500_000, MIN + 9, 0),
+    ("one-row", 1_500_000, MIN + 9, 0), ("gap", 70_000, MIN + 3, 0),
 ]
 
 

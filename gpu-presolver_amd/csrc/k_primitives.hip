@@ -1630,6 +1630,10 @@ __global__ __launch_bounds__(kTbBlock) void k_tb_columns(const int4* __restrict_
 // entry is compared with the one before it: flags[1] a column outside
 // [0, cols), flags[2] two equal neighbours, flags[3] a descending pair.  No
 // entry is read of a matrix whose pointers are bad.
+// Rows of a chunk (its entries' and the empty ones between) up to which they
+// mark their first entries; past that every entry looks its row up by
+// bisection.
+constexpr int kChkMarkRows = 8192;
 constexpr int kChkItems = 8;
 constexpr int kChkChunk = kBlock * kChkItems;
 
@@ -1666,10 +1670,21 @@ __global__ __launch_bounds__(kBlock) void k_csr_check_entries(gpk_csr_check_side
   const int32_t r_lo = s.chunk_row[q], r_hi = q + 1 < chunks ? s.chunk_row[q + 1] : s.rows - 1;
   if (tid < kChkChunk / 32) s_head[tid] = 0;
   __syncthreads();
+  if (r_hi - r_lo < kChkMarkRows) {
 #pragma unroll 1
-  for (int64_t r = r_lo + tid; r <= r_hi; r += kBlock) {
-    const int32_t b = s.ptr[r] - c0;
-    if (b >= 0 && b < c1) atomicOr(&s_head[b >> 5], 1u << (b & 31));  // empty rows mark their successor's
+    for (int64_t r = static_cast<int64_t>(r_lo) + tid; r <= r_hi; r += kBlock) {
+      const int32_t b = s.ptr[r] - c0;
+      if (b >= 0 && b < c1) atomicOr(&s_head[b >> 5], 1u << (b & 31));  // empty rows mark their successor's
+    }
+  } else {
+    for (int p = tid; p < c1; p += kBlock) {
+      int32_t lo = r_lo, hi = r_hi;  // the last row that starts at or before the entry is one of [lo, hi]
+      while (lo < hi) {
+        const int32_t mid = hi - (hi - lo) / 2;
+        if (s.ptr[mid] <= c0 + p) lo = mid; else hi = mid - 1;
+      }
+      if (s.ptr[lo] == c0 + p) atomicOr(&s_head[p >> 5], 1u << (p & 31));
+    }
   }
   __syncthreads();
   bool range = false, equal = false, desc = false;

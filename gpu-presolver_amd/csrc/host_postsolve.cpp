@@ -93,15 +93,22 @@ gp_orig_dev orig_view(const LPInfoGpu* o) {
 
 // Zeroed words of which few are touched: pages of the kernel's, cleared when
 // they are first touched, two megabytes at a time where the system does that
-// (a vector clears them all, a page fault for each four kilobytes).
+// (a vector clears them all, a page fault for each four kilobytes).  Few words
+// come from the heap: a mapping of their own costs a small LP's postsolve 5 us.
 class HostWords {
  public:
   HostWords() = default;
   explicit HostWords(size_t words) : bytes_(words * sizeof(int32_t)) {
     if (bytes_ == 0) return;
-    void* p = mmap(nullptr, bytes_, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
-    if (p == MAP_FAILED) throw std::bad_alloc();
-    (void)madvise(p, bytes_, MADV_HUGEPAGE);
+    void* p;
+    if (bytes_ < kMapped) {
+      p = std::calloc(words, sizeof(int32_t));
+      if (p == nullptr) throw std::bad_alloc();
+    } else {
+      p = mmap(nullptr, bytes_, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+      if (p == MAP_FAILED) throw std::bad_alloc();
+      (void)madvise(p, bytes_, MADV_HUGEPAGE);
+    }
     p_ = static_cast<int32_t*>(p);
   }
   HostWords(HostWords&& o) noexcept : p_(std::exchange(o.p_, nullptr)), bytes_(std::exchange(o.bytes_, 0)) {}
@@ -111,12 +118,15 @@ class HostWords {
     return *this;
   }
   ~HostWords() {
-    if (p_) (void)munmap(p_, bytes_);
+    if (p_ == nullptr) return;
+    if (bytes_ < kMapped) std::free(p_);
+    else (void)munmap(p_, bytes_);
   }
   int32_t& operator[](size_t k) { return p_[k]; }
   int32_t operator[](size_t k) const { return p_[k]; }
 
  private:
+  static constexpr size_t kMapped = size_t{1} << 20;
   int32_t* p_ = nullptr;
   size_t bytes_ = 0;
 };
@@ -169,26 +179,32 @@ Lines gather_lines(const int32_t* ptr, const int32_t* idx, int32_t lines_total, 
   return L;
 }
 
-// Parts [first, first + count) of levels: one grid launch (a single large
-// level) or one workgroup that steps through a run of smaller levels.
+// Levels that one workgroup replays in a run, as `count` parts from `first` on;
+// or one level in a launch of its own: its line slots [first, first + count) and
+// its simple slots [simple, simple + simples).
 struct Segment {
-  int32_t first, count;
   bool grid;
+  int32_t first, count, simple, simples;
+  int32_t waves;  // of a run: the most that a part fills
+  bool lines;     // of a run: some record walks a line
 };
 
 struct Schedule {
-  std::vector<int32_t> order;        // record indices, level by level
-  std::vector<int32_t> level_start;  // offsets into order of the levels' parts, and its end
+  std::vector<int32_t> line, simple;  // record indices, level by level (-1: an empty slot)
+  std::vector<gpk_replay_part> parts;
   std::vector<Segment> segs;
   int32_t levels = 0;
+  // Where its slots and parts begin among those of the plan.
+  int64_t line_at = 0, simple_at = 0, parts_at = 0;
 };
 
-// Levels of at least this many records get a launch of their own (about 10 us
-// with the gap, and as much to start the next run of levels); in a run, a level
-// takes about 3 us for each 64 records.
-constexpr int32_t kGridLevelMin = 512;
-constexpr int32_t kTypes = 15;       // PostsolveReductionType
-constexpr int32_t kWaveRecords = 4;  // sixteen lanes each
+// Levels of more records than these get a launch of their own: 2.5 to 3 us in a
+// graph where its neighbours have theirs too, 4.5 to 5 launched directly.  In a run
+// a level of up to 511 simple records takes 0.7 to 1 us, of 1,024 1.6, of 2,047
+// 3; of up to 64 line records 2.4, of 128 (in two parts) 4.8.
+constexpr int32_t kRunLines = GPK_REPLAY_WAVES * GPK_WAVE_LINES, kRunSimples = 2 * GPK_REPLAY_WAVES * 64;
+constexpr int32_t kTypes = 15;  // PostsolveReductionType
+constexpr int64_t kMostSlots = std::numeric_limits<int32_t>::max();
 
 [[noreturn]] void bad_tape(int32_t k, const char* what) {
   throw std::runtime_error("postsolve_gpu: tape record " + std::to_string(k) + ": " + what);
@@ -356,8 +372,12 @@ class TapeScanner {
     }
   }
 
-  // The type of a record that takes part in a pass.
+  // The type of a record that takes part in a pass, and whether it walks a line.
   int32_t type(int32_t k) const { return t_.types[k]; }
+  bool walks_line(int32_t k, bool primal, bool has_orig, bool has_y) const {
+    return gpk_record_walks_line(t_.types[k], t_.index_starts[k + 1] - t_.index_starts[k], primal ? 0 : 1,
+                                 has_orig ? 1 : 0, has_y ? 1 : 0) != 0;
+  }
 
   // Original rows (type 12) and columns (types 5 and 13 without a row
   // payload) whose index lists the dual pass walks.
@@ -398,6 +418,14 @@ Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, VarLeve
   const int32_t base = vars.base;
   const int32_t span = hi > lo ? hi - lo : 0;
   std::vector<int32_t> level(span, -1);
+  // Line records by type, then the others by type.
+  constexpr int kKinds = 2 * kTypes;
+  const std::unique_ptr<uint8_t[]> kind(new uint8_t[static_cast<size_t>(span) + 1]);
+  struct Level {
+    int32_t records;
+    uint32_t kinds;  // a bit for each that it has
+  };
+  std::vector<Level> all;
   std::vector<int32_t> rd, wr;
   int32_t levels = 0;
   for (int32_t k = hi - 1; k >= lo; --k) {
@@ -412,86 +440,169 @@ Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, VarLeve
       int32_t& r = last[2 * static_cast<size_t>(v) + 1];
       r = std::max(r, lv);
     }
-    level[k - lo] = lv - base - 1;
-    levels = std::max(levels, lv - base);
+    const int32_t l = lv - base - 1;
+    level[k - lo] = l;
+    if (l == levels) {
+      all.push_back(Level{0, 0});
+      ++levels;
+    }
+    const int t = scan.type(k) + (scan.walks_line(k, primal, has_orig, has_y) ? 0 : kTypes);
+    kind[k - lo] = static_cast<uint8_t>(t);
+    ++all[l].records;
+    all[l].kinds |= 1u << t;
   }
   vars.base += levels;
-  // Records of a level in the order of their types, and in a level that one
-  // workgroup replays each type from a new wave on (empty slots, -1, between):
-  // a wave runs the branches of its records' types one after the other.  Such
-  // a level is given to the workgroup in parts of its slots.
-  std::vector<int32_t> size(static_cast<size_t>(levels) * kTypes, 0);
-  for (int32_t k = lo; k < hi; ++k)
-    if (level[k - lo] >= 0) ++size[static_cast<size_t>(level[k - lo]) * kTypes + scan.type(k)];
+  // Within a level the records that walk a line, then the others, both in the
+  // order of their types (a wave runs the branches of its records' types one after
+  // the other), each type's in reverse.  In a run of levels each type of more than
+  // a wave's line records begins a new wave (empty slots between).
   Schedule sch;
   sch.levels = levels;
-  std::vector<int32_t>& start = sch.level_start;
-  start.push_back(0);
-  std::vector<int32_t> fill(static_cast<size_t>(levels) * kTypes);
-  for (int32_t l = 0; l < levels; ++l) {
-    const size_t f = static_cast<size_t>(l) * kTypes;
-    int32_t records = 0, at = start.back();
-    for (int32_t t = 0; t < kTypes; ++t) records += size[f + t];
-    const bool grid = records >= kGridLevelMin;
-    for (int32_t t = 0; t < kTypes; ++t) {
-      fill[f + t] = at;
-      at += grid ? size[f + t] : (size[f + t] + kWaveRecords - 1) / kWaveRecords * kWaveRecords;
+  sch.parts.reserve(static_cast<size_t>(levels) + 16);
+  // The slots of the next level, which has size[t] records of kind t; size[t] is
+  // then where they begin.
+  const auto add_level = [&](uint32_t kinds, int32_t* size) {
+    int64_t lines = 0, simples = 0;
+    for (uint32_t u = kinds; u != 0; u &= u - 1) (__builtin_ctz(u) < kTypes ? lines : simples) += size[__builtin_ctz(u)];
+    const int64_t line0 = static_cast<int64_t>(sch.line.size()), simple0 = static_cast<int64_t>(sch.simple.size());
+    if (line0 + GPK_WAVE_LINES * (lines + kTypes) > kMostSlots || simple0 + simples > kMostSlots)
+      throw std::runtime_error("postsolve_gpu: the tape's replay schedule has more slots than 32 bits count");
+    const bool grid = lines > kRunLines || simples > kRunSimples;
+    int64_t line_end = line0, simple_end = simple0;
+    for (uint32_t u = kinds; u != 0; u &= u - 1) {
+      const int t = __builtin_ctz(u);
+      int64_t& end = t < kTypes ? line_end : simple_end;
+      if (t < kTypes && !grid && lines > GPK_WAVE_LINES) end += (line0 - end) & (GPK_WAVE_LINES - 1);
+      end += std::exchange(size[t], static_cast<int32_t>(end));
     }
-    const int32_t first = static_cast<int32_t>(start.size()) - 1;
-    if (!grid)
-      while (at - start.back() > GPK_REPLAY_SLOTS) start.push_back(start.back() + GPK_REPLAY_SLOTS);
-    start.push_back(at);
-    const int32_t parts = static_cast<int32_t>(start.size()) - 1 - first;
-    if (!grid && !sch.segs.empty() && !sch.segs.back().grid)
-      sch.segs.back().count += parts;
-    else
-      sch.segs.push_back(Segment{first, parts, grid});
+    sch.line.resize(static_cast<size_t>(line_end), -1);
+    sch.simple.resize(static_cast<size_t>(simple_end));
+    const int32_t count = static_cast<int32_t>(line_end - line0);
+    const int32_t first = static_cast<int32_t>(line0), sfirst = static_cast<int32_t>(simple0);
+    if (grid) {
+      sch.segs.push_back(Segment{true, first, count, sfirst, static_cast<int32_t>(simples), 0, false});
+      return;
+    }
+    if (sch.segs.empty() || sch.segs.back().grid)
+      sch.segs.push_back(Segment{false, static_cast<int32_t>(sch.parts.size()), 0, 0, 0, 1, false});
+    Segment& run = sch.segs.back();
+    run.lines |= count > 0;
+    int32_t at = 0, sat = 0, flags = GPK_PART_NEW_LEVEL;
+    while (at < count || sat < simples) {
+      const int32_t l = std::min<int32_t>(count - at, GPK_REPLAY_WAVES * GPK_WAVE_LINES);
+      const int32_t waves = (l + GPK_WAVE_LINES - 1) / GPK_WAVE_LINES;
+      const int32_t n = std::min<int32_t>(static_cast<int32_t>(simples) - sat, (GPK_REPLAY_WAVES - waves) * 64);
+      sch.parts.push_back(gpk_replay_part{first + at, l, sfirst + sat, (n << GPK_PART_SHIFT) | flags});
+      ++run.count;
+      run.waves = std::max(run.waves, waves + (n + 63) / 64);
+      at += l;
+      sat += n;
+      flags = 0;
+    }
+  };
+  const auto place = [&](int32_t k, int32_t* fill) {
+    const int t = kind[k - lo];
+    (t < kTypes ? sch.line : sch.simple)[static_cast<size_t>(fill[t]++)] = k;
+  };
+  int32_t records = 0;
+  for (Level& a : all) records += a.records;
+  if (levels <= records / 32) {  // the counts of all levels are less than the records
+    std::vector<int32_t> size(static_cast<size_t>(levels) * kKinds, 0);
+    for (int32_t k = 0; k < span; ++k)
+      if (level[k] >= 0) ++size[static_cast<size_t>(level[k]) * kKinds + kind[k]];
+    for (int32_t l = 0; l < levels; ++l) add_level(all[l].kinds, &size[static_cast<size_t>(l) * kKinds]);
+    for (int32_t k = hi - 1; k >= lo; --k)
+      if (level[k - lo] >= 0) place(k, &size[static_cast<size_t>(level[k - lo]) * kKinds]);
+    return sch;
   }
-  sch.order.assign(static_cast<size_t>(start.back()), -1);
+  // Many levels of few records: by level first.
+  const std::unique_ptr<int32_t[]> order(new int32_t[static_cast<size_t>(records) + 1]);
+  records = 0;
+  for (Level& a : all) a.records = std::exchange(records, records + a.records);
   for (int32_t k = hi - 1; k >= lo; --k)
-    if (level[k - lo] >= 0) sch.order[fill[static_cast<size_t>(level[k - lo]) * kTypes + scan.type(k)]++] = k;
+    if (level[k - lo] >= 0) order[all[level[k - lo]].records++] = k;
+  int32_t b = 0, size[kKinds] = {};
+  for (const Level& a : all) {
+    const int32_t e = a.records;
+    if (e - b == 1) {  // a chain
+      size[__builtin_ctz(a.kinds)] = 1;
+      add_level(a.kinds, size);
+      (__builtin_ctz(a.kinds) < kTypes ? sch.line : sch.simple).back() = order[b];
+      size[__builtin_ctz(a.kinds)] = 0;
+      b = e;
+      continue;
+    }
+    for (int32_t q = b; q < e; ++q) ++size[kind[order[q] - lo]];
+    add_level(a.kinds, size);
+    for (int32_t q = b; q < e; ++q) place(order[q], size);
+    for (uint32_t u = a.kinds; u != 0; u &= u - 1) size[__builtin_ctz(u)] = 0;
+    b = e;
+  }
   return sch;
 }
 
-// The schedule's level bounds and its records' packets.
-struct DeviceSchedule {
-  DBuf<int32_t> starts, packets;
+// The packets and parts of a plan's schedules.
+struct DeviceSchedules {
+  DBuf<int32_t> line, simple;
+  DBuf<gpk_replay_part> parts;
 };
-DeviceSchedule upload_schedule(const Schedule& sch, const gp_tape_dev& tape, const gp_orig_dev& orig, bool has_y,
-                               bool primal) {
-  const int64_t nr = static_cast<int64_t>(sch.order.size()), nl = static_cast<int64_t>(sch.level_start.size());
-  DeviceSchedule d;
-  DBuf<int32_t> order(nr);
-  d.starts.alloc(nl);
-  d.packets.alloc(nr * GPK_PACKET_WORDS);
+// all: the primal pass's schedules, then the dual pass's.
+DeviceSchedules upload_schedules(const std::vector<Schedule*>& all, const gp_tape_dev& tape, const gp_orig_dev& orig,
+                                 bool has_y) {
+  int64_t lines = 0, simples = 0, parts = 0, dual_line = 0;
+  for (Schedule* s : all) {
+    s->line_at = dual_line = lines;
+    s->simple_at = simples;
+    s->parts_at = parts;
+    lines += static_cast<int64_t>(s->line.size());
+    simples += static_cast<int64_t>(s->simple.size());
+    parts += static_cast<int64_t>(s->parts.size());
+  }
+  if (lines > kMostSlots || simples > kMostSlots || parts > kMostSlots)
+    throw std::runtime_error("postsolve_gpu: the tape's replay schedules have more slots than 32 bits count");
+  DeviceSchedules d;
+  DBuf<int32_t> line_records(lines), simple_records(simples);
+  d.parts.alloc(parts);
+  d.line.alloc(lines * GPK_PACKET_WORDS);
+  d.simple.alloc(simples * GPK_SIMPLE_WORDS);
   amd::Ctx& c = ctx();
   c.begin_copy_group();
-  c.to_device(order.get(), sch.order.data(), nr, "replay schedule upload");
-  c.to_device(d.starts.get(), sch.level_start.data(), nl, "replay schedule upload");
+  for (const Schedule* s : all) {
+    c.to_device(line_records.get() + s->line_at, s->line.data(), static_cast<int64_t>(s->line.size()),
+                "replay schedule upload");
+    c.to_device(simple_records.get() + s->simple_at, s->simple.data(), static_cast<int64_t>(s->simple.size()),
+                "replay schedule upload");
+    c.to_device(d.parts.get() + s->parts_at, s->parts.data(), static_cast<int64_t>(s->parts.size()),
+                "replay schedule upload");
+  }
   c.end_copy_group("replay schedule upload");
-  check(gpk_pack_records(tape, orig, order, static_cast<int32_t>(nr), has_y ? 1 : 0, primal ? 0 : 1, d.packets,
-                         c.stream()),
+  check(gpk_pack_records(tape, orig,
+                         gpk_replay_slots{static_cast<int32_t>(lines), static_cast<int32_t>(simples), line_records,
+                                          simple_records, d.line, d.simple},
+                         static_cast<int32_t>(dual_line), has_y ? 1 : 0, c.stream()),
         "replay packets");
   return d;
 }
 
 // Launches only: no allocation, copy or wait, so it can be captured.
-void enqueue_schedule(const Schedule& sch, const DeviceSchedule& dev, const gp_tape_dev& tape, const gp_orig_dev& orig,
-                      double* x, double* y, double* z, uint8_t* zret, bool primal, double tol) {
-  if (sch.order.empty()) return;
+void enqueue_schedule(const Schedule& sch, const DeviceSchedules& dev, const gp_tape_dev& tape,
+                      const gp_orig_dev& orig, double* x, double* y, double* z, uint8_t* zret, bool primal,
+                      double tol) {
+  if (sch.segs.empty()) return;
   hipStream_t s = ctx().stream();
   const int32_t dual = primal ? 0 : 1;
   const char* what = primal ? "replay primal" : "replay dual";
+  const int32_t* line = dev.line.get() + sch.line_at * GPK_PACKET_WORDS;
+  const int32_t* simple = dev.simple.get() + sch.simple_at * GPK_SIMPLE_WORDS;
   for (const Segment& g : sch.segs) {
-    if (g.grid) {
-      const int32_t b = sch.level_start[g.first];
-      check(gpk_replay_list(tape, orig, x, y, z, zret, dev.packets + static_cast<int64_t>(b) * GPK_PACKET_WORDS,
-                            sch.level_start[g.first + 1] - b, dual, tol, s),
+    if (g.grid)
+      check(gpk_replay_list(tape, orig, x, y, z, zret, line + static_cast<int64_t>(g.first) * GPK_PACKET_WORDS, g.count,
+                            simple + static_cast<int64_t>(g.simple) * GPK_SIMPLE_WORDS, g.simples, dual, tol, s),
             what);
-    } else {
-      check(gpk_replay_levels(tape, orig, x, y, z, zret, dev.packets, dev.starts + g.first, g.count, dual, tol, s),
+    else
+      check(gpk_replay_levels(tape, orig, x, y, z, zret, line, simple, dev.parts.get() + sch.parts_at + g.first,
+                              g.count, g.waves, g.lines ? 1 : 0, dual, tol, s),
             what);
-    }
   }
 }
 
@@ -690,12 +801,11 @@ struct PostsolvePlan::Impl {
   DBuf<uint8_t> zret, prot;
   DBuf<int32_t> long_cols, long_count;
   presolve::Schedule dual;
-  presolve::DeviceSchedule dual_dev;
+  presolve::DeviceSchedules dev;
   // The primal pass in replay order: a schedule over a tape range, then the
   // recovery step at that range's start (none after the last range).
   struct Stage {
     presolve::Schedule sched;
-    presolve::DeviceSchedule dev;
     std::unique_ptr<RecoveryStep> step;
   };
   std::vector<Stage> primal;
@@ -767,7 +877,6 @@ PostsolvePlan::PostsolvePlan(const RecordView& record, const LPInfoGpu* original
     const presolve::PrimalRecoveryCheckpoint* it = &record.primal_recovery_timeline[cp];
     Impl::Stage st;
     st.sched = presolve::level_schedule(scanner, it->tape_position, range_end, vars, true, has_orig, has_y, &pattern);
-    st.dev = presolve::upload_schedule(st.sched, d.tape->view, d.orig, has_y, true);
     if (it->kind == presolve::PrimalRecoveryKind::StructuralL1)
       st.step = std::make_unique<RecoveryStep>(record.structural_primal_recoveries[it->payload_index]);
     else
@@ -778,12 +887,14 @@ PostsolvePlan::PostsolvePlan(const RecordView& record, const LPInfoGpu* original
   {
     Impl::Stage st;
     st.sched = presolve::level_schedule(scanner, 0, range_end, vars, true, has_orig, has_y, &pattern);
-    st.dev = presolve::upload_schedule(st.sched, d.tape->view, d.orig, has_y, true);
     d.primal.push_back(std::move(st));
   }
   lap("primal schedule");
   d.dual = presolve::level_schedule(scanner, 0, count, vars, false, has_orig, has_y, &pattern);
-  d.dual_dev = presolve::upload_schedule(d.dual, d.tape->view, d.orig, has_y, false);
+  std::vector<presolve::Schedule*> schedules;
+  for (Impl::Stage& st : d.primal) schedules.push_back(&st.sched);
+  schedules.push_back(&d.dual);
+  d.dev = presolve::upload_schedules(schedules, d.tape->view, d.orig, has_y);
   lap("dual schedule");
   // project_column_duals_from_original (gpu_postsolve.cu:1370-1435): the
   // columns the tape recovers duals for keep them.
@@ -818,10 +929,10 @@ void PostsolvePlan::enqueue(const double* x_red, const double* y_red, const doub
   check(gpk_mark(d.col_map, d.n1, d.zret, s), "mark retrieved");
   check(gpk_restore_fixed(d.fidx, d.fval, d.nf, x_org, s), "restore fixed");
   for (const Impl::Stage& st : d.primal) {
-    presolve::enqueue_schedule(st.sched, st.dev, d.tape->view, d.orig, x_org, y, z_org, d.zret, true, kPostsolveTol);
+    presolve::enqueue_schedule(st.sched, d.dev, d.tape->view, d.orig, x_org, y, z_org, d.zret, true, kPostsolveTol);
     if (st.step) st.step->enqueue(x_org, d.original_l, s);
   }
-  presolve::enqueue_schedule(d.dual, d.dual_dev, d.tape->view, d.orig, x_org, y, z_org, d.zret, false,
+  presolve::enqueue_schedule(d.dual, d.dev, d.tape->view, d.orig, x_org, y, z_org, d.zret, false,
                              kPostsolveTol);
   if (d.project)
     check(gpk_project_duals(d.orig, d.prot, x_org, y, z_org, d.n0, kPostsolveTol, d.long_count, d.long_cols, s),

@@ -144,12 +144,18 @@ __device__ void dbl_recover_z(double xk, double zk_hat, double al, double okl, d
   else { *zk = zk_hat; *ze = 0.0; }
 }
 
-// Sixteen lanes (a DPP row) work on a record: its index words, its values and
-// the entries of the line it walks are one to a lane.  A level's time is that
-// of the instructions of one wave and of its round trips to memory: with a lane
-// per record the entries of a line are that many loads, branches and divides
-// one after the other (9.3 us a level even with all of them loaded ahead), so
-// they are side by side instead.
+// A record goes one of two ways (gpk_record_walks_line), at every turn the same.
+//
+// A record that walks a line of entries (a row's or column's dual, a
+// substituted column's primal) is worked on by sixteen lanes (a DPP row): its
+// index words, its values and the entries of its line are one to a lane.  A
+// level's time is that of the instructions of one wave and of its round trips
+// to memory: with a lane per record the entries of a line are that many loads,
+// branches and divides one after the other (9.3 us a level even with all of them
+// loaded ahead), so they are side by side instead.
+//
+// Any other record has one lane: a wave takes 64 of them where sixteen lanes
+// each would take 4 (a level of 256 such records 0.8 us, 6.3 with sixteen).
 constexpr int kRecLanes = 16;
 constexpr int kRecChunks = 2;  // chunks of 16 entries of a line loaded ahead
 
@@ -243,12 +249,11 @@ __device__ inline int line_kind(const RecHead& h) {
 }
 // The lines of types 0, 4, 5 and 13 are walked for y, and a line's place is
 // checked by the host only where there is a y.
-template <bool kDual>
-__device__ inline RecLine load_line(const gp_orig_dev& O, const RecHead& h, int32_t word, bool has_y) {
+__device__ inline RecLine load_line(const gp_orig_dev& O, const RecHead& h, int32_t word, bool has_y, bool dual) {
   const int32_t type = h.type;
-  if (!kDual && type == 2) return RecLine{h.i0 + 3, h.v0 + 6, row_lane<2>(word)};
-  if (kDual && type == 0 && has_y) return RecLine{h.i0 + 1, h.v0 + 2, h.i1 - h.i0};
-  if (kDual && O.present != 0 && (has_y || type == 12)) {
+  if (!dual && type == 2) return RecLine{h.i0 + 3, h.v0 + 6, row_lane<2>(word)};
+  if (dual && type == 0 && has_y) return RecLine{h.i0 + 1, h.v0 + 2, h.i1 - h.i0};
+  if (dual && O.present != 0 && (has_y || type == 12)) {
     const int kind = line_kind(h);
     if (type == 13 && kind == LINE_TAPE) return RecLine{h.i0 + 4, h.v0 + 12, row_lane<3>(word)};
     const int32_t line = type == 13 || type == 4 ? row_lane<0>(word) : row_lane<1>(word);
@@ -284,17 +289,18 @@ __device__ inline RecEntries load_entries(const gp_tape_dev& T, const gp_orig_de
 
 // The column and the row whose values a record reads besides its line's.
 __device__ inline int32_t column_read(int32_t type, int32_t w0, int32_t w1) {
-  return type == 3 || type == 13 || type == 5 ? w1 : type == 12 ? w0 : -1;
+  return type == 13 || type == 5 ? w1 : type == 12 ? w0 : -1;
 }
 __device__ inline int32_t row_read(int32_t type, int32_t w0, int32_t w1) {
-  return type == 2 || type == 12 ? w1 : type == 10 || type == 4 ? w0 : -1;
+  return type == 12 ? w1 : type == 4 ? w0 : -1;
 }
 
-// A record's packet, a word to a lane: all of its operands that are not values,
-// in the order of a schedule, so that a turn is three chained loads (packet,
-// line and values, x and y and z) instead of six.
+// A record's packet: all of its operands that are not values, in the order of a
+// schedule, so that a turn is three chained loads (packet, line and values, x and
+// y and z) instead of six.  A record without a line has the first eight words.
 enum : int { PK_TYPE = 0, PK_I0 = 1, PK_I1 = 2, PK_V0 = 3, PK_V1 = 4, PK_W0 = 5, PK_QI = 9, PK_QV = 10, PK_N = 11 };
 static_assert(GPK_PACKET_WORDS == kRecLanes, "a word to a lane");
+static_assert(GPK_SIMPLE_WORDS == 8 && PK_W0 + 3 == GPK_SIMPLE_WORDS, "two loads of sixteen bytes");
 __device__ __forceinline__ RecHead packet_head(int32_t p) {
   return RecHead{row_lane<PK_TYPE>(p), row_lane<PK_I0>(p), row_lane<PK_I1>(p), row_lane<PK_V0>(p),
                  row_lane<PK_V1>(p)};
@@ -312,13 +318,143 @@ struct RecVars {
   int32_t w0, w1, w2;
 };
 
-// One record of the reverse replay (_kernel_replay_postsolve_tape,
+// A record without a line, a lane to itself.
+struct SimpleRec {
+  int32_t type, i0, i1, v0, v1, w0, w1, w2;  // type -1: none
+};
+// Its values [0, 6) and 9 (0 past its end).
+struct SimpleVals {
+  double v[6], v9;
+};
+// What its turn reads.
+struct SimpleReads {
+  double x, z, y;
+};
+__device__ __forceinline__ SimpleRec simple_none() { return SimpleRec{-1, 0, -1, 0, -1, -1, -1, -1}; }
+__device__ __forceinline__ SimpleRec simple_packet(const int32_t* __restrict__ packets, int64_t slot) {
+  const int4* p = reinterpret_cast<const int4*>(packets) + slot * (GPK_SIMPLE_WORDS / 4);
+  const int4 a = p[0], b = p[1];
+  return SimpleRec{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+}
+__device__ __forceinline__ SimpleVals simple_values(const gp_tape_dev& T, const SimpleRec& h) {
+  SimpleVals r;
+#pragma unroll
+  for (int q = 0; q < 6; ++q) r.v[q] = h.v0 + q <= h.v1 ? T.vals[h.v0 + q] : 0.0;
+  r.v9 = h.v0 + 9 <= h.v1 ? T.vals[h.v0 + 9] : 0.0;
+  return r;
+}
+template <bool kDual>
+__device__ __forceinline__ SimpleReads simple_reads(const SimpleRec& h, const double* x, const double* y,
+                                                    const double* z) {
+  const int32_t col = h.type == 3 || h.type == 13 ? h.w1 : -1;
+  const int32_t row = h.type == 2 ? h.w1 : h.type == 10 ? h.w0 : -1;
+  SimpleReads v;
+  v.x = !kDual && col >= 0 ? x[col] : 0.0;
+  v.z = col >= 0 && z ? z[col] : 0.0;
+  v.y = kDual && row >= 0 && y ? y[row] : 0.0;
+  return v;
+}
+
+template <bool kDual>
+__device__ __forceinline__ void replay_simple(const gp_tape_dev& T, double* x, double* y, double* z, uint8_t* zret,
+                                              const SimpleRec& h, const SimpleVals& r, const SimpleReads& in,
+                                              double tol) {
+  const int32_t type = h.type, w0 = h.w0, w1 = h.w1;
+  if (type < 0) return;
+  constexpr bool primal = !kDual, dual = kDual;
+  const int32_t* I = T.indices;
+  const double* V = T.vals;
+  const int32_t i0 = h.i0, v0 = h.v0;
+  const double xc = in.x, zc = in.z, yr = in.y;
+  if (type == 3) {  // DuplicateColumn
+    if (primal) {
+      double xf = 0.0, xt = xc;
+      recover_dup_col(xc, zc, r.v[0], r.v[1], r.v[2], r.v[3], r.v[4], tol, &xf, &xt);
+      x[w0] = xf;
+      x[w1] = xt;
+    }
+    if (dual && z) { z[w0] = r.v[0] * zc; if (zret) zret[w0] = 1; }
+  } else if (type == 13) {  // DoubletonEquation; dual: without an original model or y
+    const double ecoef = r.v[0], kcoef = r.v[1], rhs = r.v[2], eobj = r.v9;
+    const double al = -kcoef / ecoef, be = rhs / ecoef;
+    if (primal) x[w0] = be + al * xc;
+    if (dual) {
+      if (z) { z[w0] = 0.0; if (zret) zret[w0] = 1; }
+      if (y && h.w2 >= 0) y[h.w2] = eobj / ecoef;
+    }
+  } else if (dual && type == 2) {  // SubCol
+    const double piv = r.v[0], eobj = r.v[4];
+    const bool row_deleted = r.v[5] != 0.0;
+    const double y_new = row_deleted ? eobj / piv : yr + eobj / piv;
+    if (y && w1 >= 0) y[w1] = y_new;
+    if (z) {
+      z[w0] = (row_deleted || !y) ? 0.0 : eobj - piv * (w1 >= 0 ? y_new : 0.0);
+      if (zret) zret[w0] = 1;
+    }
+  } else if (type == 0) {  // FixedCol; dual: without rows or y
+    if (primal) x[w0] = r.v[0];
+    if (dual && z) { z[w0] = r.v[1]; if (zret) zret[w0] = 1; }
+  } else if (type == 1) {  // FixedColInf
+    const bool pos_inf = w0 > 0;
+    const int32_t col = w1;
+    if (primal) {
+      const int32_t nrows = static_cast<int32_t>(llround(r.v[0]));
+      double ext = r.v[1];
+      int32_t ip = i0 + 2, vp = v0 + 2;
+      for (int32_t q = 0; q < nrows; ++q) {
+        const int32_t len = I[ip];
+        double side = V[vp], coef = 0.0;
+        for (int32_t t = 0; t < len; ++t) {
+          const int32_t rc = I[ip + 1 + t];
+          const double rv = V[vp + 1 + t];
+          if (rc == col) coef = rv; else side -= rv * x[rc];
+        }
+        const double cand = side / coef;
+        ext = pos_inf ? fmax(ext, cand) : fmin(ext, cand);
+        ip += len + 1;
+        vp += len + 1;
+      }
+      x[col] = ext;
+    }
+    if (dual && z) { z[col] = 0.0; if (zret) zret[col] = 1; }
+  } else if (type == 14) {  // FmeCol
+    const int32_t K = w0, ec = w1;
+    if (primal) {
+      const int32_t L = static_cast<int32_t>(llround(r.v[0]));
+      int32_t cc = i0 + 3 + K, vp = v0 + 1;
+      double lo = -INFINITY, hi = INFINITY;
+      bool hl = false, hh = false;
+      for (int32_t q = 0; q < L; ++q) {
+        const double orient = V[vp];
+        const int32_t len = static_cast<int32_t>(llround(V[vp + 1]));
+        double cand = V[vp + 2];
+        for (int32_t t = 0; t < len; ++t) cand += V[vp + 3 + t] * x[I[cc++]];
+        if (orient > 0.0) { lo = fmax(lo, cand); hl = true; }
+        else { hi = fmin(hi, cand); hh = true; }
+        vp += 3 + len;
+      }
+      x[ec] = hl ? lo : (hh ? hi : 0.0);
+    }
+    if (dual && z) { z[ec] = 0.0; if (zret) zret[ec] = 1; }
+    if (dual && y) for (int32_t t = 0; t < K; ++t) y[I[i0 + 2 + t]] = 0.0;
+  } else if (dual && type == 10) {  // EqToIneq
+    if (y) y[w0] = yr + r.v[0];
+  } else if (dual && type == 4 && w1 >= 0 && h.v1 >= v0 + 4) {  // DuplicateRow without an original model
+    const double q = r.v[0], kal = r.v[1], kau = r.v[2];
+    if (fabs(q) <= tol || !y) return;
+    const double a = r.v[3] * q, b = r.v[4] * q;
+    const double dsl = q >= 0.0 ? a : b, dsu = q >= 0.0 ? b : a;
+    if (dsl <= kal + tol && kau <= dsu + tol) y[w1] = 0.0;
+  }
+}
+
+// A record with a line of the reverse replay (_kernel_replay_postsolve_tape,
 // gpu_postsolve.cu:605-1046); all sixteen lanes come with the same record.
 // kDual picks the pass.  All loads of x, y, z and zret that the record's type
 // needs go out together at the top: a wave waits for one round trip, for two
 // where a decision comes before a row is read.
 template <bool kDual>
-__device__ __forceinline__ void replay_one(const gp_tape_dev& T, const gp_orig_dev& O, double* x, double* y, double* z,
+__device__ __forceinline__ void replay_line(const gp_tape_dev& T, const gp_orig_dev& O, double* x, double* y, double* z,
                                            uint8_t* zret, const RecHead& h, const RecVars& rv, const RecLine& ln,
                                            RecEntries r, double tol) {
   const bool has_orig = O.present != 0;
@@ -327,10 +463,7 @@ __device__ __forceinline__ void replay_one(const gp_tape_dev& T, const gp_orig_d
   constexpr bool primal = !kDual, dual = kDual;
   const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
   const bool first = t == 0;  // the lane that stores what the record has one of
-  const int32_t i0 = h.i0;
   const int32_t v0 = h.v0;
-  const int32_t* I = T.indices;
-  const double* V = T.vals;
   // The record's first index words and values.
   const int32_t w0 = rv.w0, w1 = rv.w1, w2 = rv.w2;
   const double W0 = row_lane<0>(r.v), W1 = row_lane<1>(r.v), W2 = row_lane<2>(r.v), W3 = row_lane<3>(r.v),
@@ -376,97 +509,26 @@ __device__ __forceinline__ void replay_one(const gp_tape_dev& T, const gp_orig_d
                          ln.n - kHave, skip);
   }
 
-  if (type == 3) {  // DuplicateColumn
-    const int32_t from = w0, to = w1;
-    if (primal) {
-      double xf = 0.0, xt = xc;
-      recover_dup_col(xc, zc, W0, W1, W2, W3, W4, tol, &xf, &xt);
-      if (first) { x[from] = xf; x[to] = xt; }
-    }
-    if (dual && z && first) { z[from] = W0 * zc; if (zret) zret[from] = 1; }
-  } else if (type == 13) {  // DoubletonEquation
+  if (dual && type == 13) {  // DoubletonEquation
     const int32_t ec = w0, kc = w1, row = w2;
-    const double ecoef = W0, kcoef = W1, rhs = W2, eobj = row_lane<9>(r.v);
-    const double al = -kcoef / ecoef, be = rhs / ecoef;
-    if (primal && first) x[ec] = be + al * xc;
-    if (dual && z && y && has_orig) {
-      double zk = 0.0, ze = 0.0;
-      dbl_recover_z(xc, zc, al, W5, row_lane<6>(r.v), row_lane<7>(r.v), row_lane<8>(r.v), row_lane<10>(r.v),
-                    row_lane<11>(r.v), tol, &zk, &ze);
-      const double yrow = ((kind == LINE_TAPE ? eobj : cc) - sum - ze) / ecoef;
-      if (first) {
-        y[row] = yrow;
-        z[kc] = zk;
-        z[ec] = ze;
-        if (zret) { zret[kc] = 1; zret[ec] = 1; }
-      }
-    } else if (dual && first) {
-      if (z) { z[ec] = 0.0; if (zret) zret[ec] = 1; }
-      if (y && row >= 0) y[row] = eobj / ecoef;
+    const double ecoef = W0, al = -W1 / ecoef, eobj = row_lane<9>(r.v);
+    double zk = 0.0, ze = 0.0;
+    dbl_recover_z(xc, zc, al, W5, row_lane<6>(r.v), row_lane<7>(r.v), row_lane<8>(r.v), row_lane<10>(r.v),
+                  row_lane<11>(r.v), tol, &zk, &ze);
+    const double yrow = ((kind == LINE_TAPE ? eobj : cc) - sum - ze) / ecoef;
+    if (first) {
+      y[row] = yrow;
+      z[kc] = zk;
+      z[ec] = ze;
+      if (zret) { zret[kc] = 1; zret[ec] = 1; }
     }
-  } else if (type == 2) {  // SubCol
-    const int32_t ec = w0, row = w1;
-    const double piv = W0, rhs = W1, eobj = W4;
-    const bool row_deleted = W5 != 0.0;
-    if (primal && first) x[ec] = (rhs - sum) / piv;
-    const double y_new = row_deleted ? eobj / piv : yr + eobj / piv;
-    if (dual && y && row >= 0 && first) y[row] = y_new;
-    if (dual && z && first) {
-      z[ec] = (row_deleted || !y) ? 0.0 : eobj - piv * (row >= 0 ? y_new : 0.0);
-      if (zret) zret[ec] = 1;
+  } else if (primal && type == 2) {  // SubCol
+    if (first) x[w0] = (W1 - sum) / W0;
+  } else if (dual && type == 0) {  // FixedCol
+    if (z && first) {
+      z[w0] = sum;
+      if (zret) zret[w0] = 1;
     }
-  } else if (type == 0) {  // FixedCol
-    const int32_t col = w0;
-    if (primal && first) x[col] = W0;
-    if (dual && z && first) {
-      z[col] = sum;
-      if (zret) zret[col] = 1;
-    }
-  } else if (type == 1 && first) {  // FixedColInf
-    const bool pos_inf = I[i0] > 0;
-    const int32_t col = I[i0 + 1];
-    const int32_t nrows = static_cast<int32_t>(llround(V[v0]));
-    double ext = V[v0 + 1];
-    int32_t ip = i0 + 2, vp = v0 + 2;
-    if (primal) {
-      for (int32_t r = 0; r < nrows; ++r) {
-        const int32_t len = I[ip];
-        double side = V[vp], coef = 0.0;
-        for (int32_t t = 0; t < len; ++t) {
-          const int32_t rc = I[ip + 1 + t];
-          const double rv = V[vp + 1 + t];
-          if (rc == col) coef = rv; else side -= rv * x[rc];
-        }
-        const double cand = side / coef;
-        ext = pos_inf ? fmax(ext, cand) : fmin(ext, cand);
-        ip += len + 1;
-        vp += len + 1;
-      }
-      x[col] = ext;
-    }
-    if (dual && z) { z[col] = 0.0; if (zret) zret[col] = 1; }
-  } else if (type == 14 && first) {  // FmeCol
-    const int32_t K = I[i0], ec = I[i0 + 1];
-    const int32_t L = static_cast<int32_t>(llround(V[v0]));
-    int32_t cc = i0 + 3 + K, vp = v0 + 1;
-    double lo = -INFINITY, hi = INFINITY;
-    bool hl = false, hh = false;
-    if (primal) {
-      for (int32_t s = 0; s < L; ++s) {
-        const double orient = V[vp];
-        const int32_t len = static_cast<int32_t>(llround(V[vp + 1]));
-        double cand = V[vp + 2];
-        for (int32_t t = 0; t < len; ++t) cand += V[vp + 3 + t] * x[I[cc++]];
-        if (orient > 0.0) { lo = fmax(lo, cand); hl = true; }
-        else { hi = fmin(hi, cand); hh = true; }
-        vp += 3 + len;
-      }
-      x[ec] = hl ? lo : (hh ? hi : 0.0);
-    }
-    if (dual && z) { z[ec] = 0.0; if (zret) zret[ec] = 1; }
-    if (dual && y) for (int32_t t = 0; t < K; ++t) y[I[i0 + 2 + t]] = 0.0;
-  } else if (dual && type == 10) {  // EqToIneq
-    if (y && first) y[w0] = yr + W0;
   } else if (dual && type == 4 && w1 >= 0 && h.v1 >= v0 + 4) {  // DuplicateRow
     const int32_t kr = w0, dr = w1;
     const double q = W0, kal = W1, kau = W2, dal = W3, dau = W4;
@@ -579,104 +641,164 @@ __device__ __forceinline__ void replay_one(const gp_tape_dev& T, const gp_orig_d
   }
 }
 
-// Record k in one go.
-template <bool kDual>
-__device__ __forceinline__ void replay_record(const gp_tape_dev& T, const gp_orig_dev& O, double* x, double* y,
-                                              double* z, uint8_t* zret, int32_t k, double tol) {
-  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
-  const RecHead h = load_head(T, k);
-  const int32_t word = load_word(T, h, t);
-  const RecLine ln = load_line<kDual>(O, h, word, y != nullptr);
-  const RecVars rv{row_lane<0>(word), row_lane<1>(word), row_lane<2>(word)};
-  replay_one<kDual>(T, O, x, y, z, zret, h, rv, ln, load_entries(T, O, h, ln, t), tol);
-}
-
-// Records begin..end-1 in reverse, one after the other (the reference's order).
-__global__ void k_replay(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret,
-                         int32_t begin, int32_t end, int32_t primal, int32_t dual, double tol) {
-  if (blockIdx.x != 0 || threadIdx.x >= kRecLanes) return;
-  for (int32_t k = end - 1; k >= begin; --k) {
-    if (primal) replay_record<false>(T, O, x, y, z, zret, k, tol);
-    __threadfence_block();  // one lane's stores before the others' loads
-    if (dual) replay_record<true>(T, O, x, y, z, zret, k, tol);
-    __threadfence_block();
+// The packets of a plan's schedules, primal first: line slots from dual_line on
+// are of the dual pass (the others' packets are the same in both).  Blocks: the records with a line, sixteen
+// lanes each, then the others.
+__global__ void __launch_bounds__(kBlock) k_pack_records(gp_tape_dev T, gp_orig_dev O, gpk_replay_slots s,
+                                                         int32_t dual_line, int32_t has_y, int32_t line_blocks) {
+  const int32_t block = static_cast<int32_t>(blockIdx.x);
+  if (block >= line_blocks) {
+    const int32_t i = (block - line_blocks) * kBlock + static_cast<int32_t>(threadIdx.x);
+    if (i >= s.simple_slots) return;
+    const RecHead h = load_head(T, s.simple_records[i]);
+    int4* p = reinterpret_cast<int4*>(s.simple) + static_cast<int64_t>(i) * (GPK_SIMPLE_WORDS / 4);
+    p[0] = make_int4(h.type, h.i0, h.i1, h.v0);
+    p[1] = make_int4(h.v1, load_word(T, h, 0), load_word(T, h, 1), load_word(T, h, 2));
+    return;
   }
-}
-
-// The packets of `count` slots of a schedule.
-template <bool kDual>
-__global__ void __launch_bounds__(kBlock) k_pack_records(gp_tape_dev T, gp_orig_dev O, const int32_t* records,
-                                                         int32_t count, int32_t has_y, int32_t* packets) {
-  const int32_t i = static_cast<int32_t>(blockIdx.x * (kBlock / kRecLanes) + threadIdx.x / kRecLanes);
-  if (i >= count) return;
+  const int32_t i = block * (kBlock / kRecLanes) + static_cast<int32_t>(threadIdx.x) / kRecLanes;
+  if (i >= s.line_slots) return;
   const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
-  const RecHead h = load_head(T, records[i]);
+  const RecHead h = load_head(T, s.line_records[i]);
   const int32_t word = load_word(T, h, t);
-  const RecLine ln = load_line<kDual>(O, h, word, has_y != 0);
+  const RecLine ln = load_line(O, h, word, has_y != 0, i >= dual_line);
   const int32_t w = __shfl(word, t >= PK_W0 && t < PK_QI ? t - PK_W0 : 0, kRecLanes);
   const int32_t p = t == PK_TYPE ? h.type : t == PK_I0 ? h.i0 : t == PK_I1 ? h.i1 : t == PK_V0 ? h.v0
                     : t == PK_V1 ? h.v1 : t < PK_QI ? w : t == PK_QI ? ln.qi : t == PK_QV ? ln.qv
                     : t == PK_N ? ln.n : 0;
-  packets[static_cast<int64_t>(i) * GPK_PACKET_WORDS + t] = p;
+  s.line[static_cast<int64_t>(i) * GPK_PACKET_WORDS + t] = p;
 }
 
 // One level of a dependency-level schedule: its records touch disjoint
-// variables, sixteen lanes each.  Three chains of loads and little else:
-// 5.6 us for 1,000 to 30,000 records (16 us with a lane per record, 6.5 with
-// six chains).
+// variables.  Blocks: line records, sixteen lanes each, then the others, a lane
+// each.  Three chains of loads and little else: 5.6 us for 1,000 to 30,000 line
+// records (16 us with a lane per record, 6.5 with six chains).
 template <bool kDual>
 __global__ void __launch_bounds__(kBlock)
-    k_replay_list(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret, const int32_t* packets,
-                  int32_t count, double tol) {
-  const int32_t i = static_cast<int32_t>(blockIdx.x * (kBlock / kRecLanes) + threadIdx.x / kRecLanes);
-  if (i >= count) return;
+    k_replay_list(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret,
+                  const int32_t* __restrict__ line, int32_t lines, const int32_t* __restrict__ simple, int32_t simples,
+                  int32_t line_blocks, double tol) {
+  const int32_t block = static_cast<int32_t>(blockIdx.x);
+  if (block >= line_blocks) {
+    const int32_t i = (block - line_blocks) * kBlock + static_cast<int32_t>(threadIdx.x);
+    if (i >= simples) return;
+    const SimpleRec h = simple_packet(simple, i);
+    replay_simple<kDual>(T, x, y, z, zret, h, simple_values(T, h), simple_reads<kDual>(h, x, y, z), tol);
+    return;
+  }
+  const int32_t i = block * (kBlock / kRecLanes) + static_cast<int32_t>(threadIdx.x) / kRecLanes;
+  if (i >= lines) return;
   const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
-  const int32_t p = packets[static_cast<int64_t>(i) * GPK_PACKET_WORDS + t];
+  const int32_t p = line[static_cast<int64_t>(i) * GPK_PACKET_WORDS + t];
   const RecHead h = packet_head(p);
   const RecLine ln = packet_line(p);
   const RecEntries r = load_entries(T, O, h, ln, t);
   const RecVars rv{row_lane<PK_W0>(p), row_lane<PK_W0 + 1>(p), row_lane<PK_W0 + 2>(p)};
-  replay_one<kDual>(T, O, x, y, z, zret, h, rv, ln, r, tol);
+  replay_line<kDual>(T, O, x, y, z, zret, h, rv, ln, r, tol);
 }
 
-// A run of small levels in one workgroup, which meets at a barrier after each.
-// All waves of the workgroup run on one CU, so the barrier's workgroup-scope
-// fence makes one level's global stores visible to the next level's loads.
-// A group of lanes has the packet of its slot two levels ahead and the line and
-// values of its record one level ahead on their way, so that a level waits only
-// for its x, y, z and zret, and for its stores at the barrier.  Bound by that
-// chain: 1,207 dual levels, most of about 31 records, take 3.2 ms (2.6 us
-// each; 11.4 ms with a lane per record and each chain in its turn, 4.2 with a
-// record's six chains five levels ahead in place of packets).  Reading x, y, z and zret
-// once a level ahead, to have them in the CU's cache, cost 0.4 ms more.
-template <bool kDual>
-__global__ void __launch_bounds__(GPK_REPLAY_SLOTS * kRecLanes)
+// What a wave holds of a part of a level (gpk_replay_part): its records'
+// packets, and later their values and entries.
+struct PartWords {
+  int4 a, b;  // simple: the packet; line: a.x the lane's word
+};
+struct PartOperands {
+  RecEntries r;
+  SimpleVals s;
+};
+constexpr int kLevelBlock = 64 * GPK_REPLAY_WAVES;
+constexpr int kWaveLines = 64 / kRecLanes;
+static_assert(GPK_WAVE_LINES == kWaveLines, "a wave's line records");
+
+// A run of small levels in one workgroup, which meets at a barrier between
+// levels; it has as many waves as its largest level fills (a chain of single
+// records: one, 0.7 us a level against 1.1 with sixteen).  All waves run on one
+// CU, so the barrier's workgroup-scope fence makes one level's global stores
+// visible to the next level's loads.  A part's first waves take its line records,
+// the next ones the others; the parts of a level follow each other without
+// meeting.  kLine: the run has line records.
+// A wave has the packets of its records two parts ahead and their lines and
+// values one part ahead on their way, so that a level waits only for its x, y, z
+// and zret, and for its stores at the barrier.  Bound by that chain: 1,207 dual
+// levels, most of about 31 records, take 3.2 ms (2.6 us each; 11.4 ms with a
+// lane per record and each chain in its turn, 4.2 with a record's six chains
+// five levels ahead in place of packets).  Reading x, y, z and zret once a level
+// ahead, to have them in the CU's cache, cost 0.4 ms more.
+template <bool kDual, bool kLine>
+__global__ void __launch_bounds__(kLevelBlock)
     k_replay_levels(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret,
-                    const int32_t* __restrict__ packets, const int32_t* __restrict__ level_start, int32_t nlevels,
-                    double tol) {
-  const int32_t slot = static_cast<int32_t>(threadIdx.x) / kRecLanes;
-  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
-  const int32_t none = packet_none(t);
-  const auto packet = [&](int32_t begin, int32_t end) {
-    return begin + slot < end ? packets[static_cast<int64_t>(begin + slot) * GPK_PACKET_WORDS + t] : none;
+                    const int32_t* __restrict__ line, const int32_t* __restrict__ simple,
+                    const gpk_replay_part* __restrict__ parts, int32_t nparts, double tol) {
+  const int32_t wave = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x) >> 6);
+  const int32_t lane = static_cast<int32_t>(threadIdx.x) & 63;
+  const int t = lane & (kRecLanes - 1);
+  // A part is loaded a turn before it is looked at.  With line records by a vector
+  // load: a scalar one would be waited for together with the newest of its kind
+  // (a level of one line record 2.28 us against 2.35; without line records the
+  // scalar load is the better one, 1.18 against 1.22).
+  int32_t zero = 0;
+  if (kLine) asm("" : "+v"(zero));
+  const auto part = [&](int32_t p) {
+    const int4 v = p < nparts ? reinterpret_cast<const int4*>(parts)[p + zero] : make_int4(0, 0, 0, 0);
+    return gpk_replay_part{v.x, v.y, v.z, v.w};
   };
-  const int32_t b0 = level_start[0], b1 = level_start[min(1, nlevels)], b2 = level_start[min(2, nlevels)];
-  int32_t end = level_start[min(3, nlevels)], begin = b2;  // of level l + 2
-  int32_t p0 = packet(b0, b1), p1 = packet(b1, b2);
-  RecEntries r0 = load_entries(T, O, packet_head(p0), packet_line(p0), t);
+  const auto uniform = [](const gpk_replay_part& d) {
+    return gpk_replay_part{__builtin_amdgcn_readfirstlane(d.line), __builtin_amdgcn_readfirstlane(d.lines),
+                           __builtin_amdgcn_readfirstlane(d.simple), __builtin_amdgcn_readfirstlane(d.simples)};
+  };
+  const auto line_waves = [](const gpk_replay_part& d) { return kLine ? (d.lines + kWaveLines - 1) / kWaveLines : 0; };
+  const auto takes_line = [&](const gpk_replay_part& d) { return kLine && wave < line_waves(d); };
+  const auto packets = [&](const gpk_replay_part& d) {
+    PartWords w;
+    if (takes_line(d)) {
+      const int32_t slot = wave * kWaveLines + lane / kRecLanes;
+      w.a.x = slot < d.lines ? line[(static_cast<int64_t>(d.line) + slot) * GPK_PACKET_WORDS + t] : packet_none(t);
+    } else {
+      const int32_t slot = (wave - line_waves(d)) * 64 + lane;
+      const SimpleRec h = slot < d.simples >> GPK_PART_SHIFT
+                              ? simple_packet(simple, static_cast<int64_t>(d.simple) + slot) : simple_none();
+      w.a = make_int4(h.type, h.i0, h.i1, h.v0);
+      w.b = make_int4(h.v1, h.w0, h.w1, h.w2);
+    }
+    return w;
+  };
+  const auto simple_of = [](const PartWords& w) {
+    return SimpleRec{w.a.x, w.a.y, w.a.z, w.a.w, w.b.x, w.b.y, w.b.z, w.b.w};
+  };
+  const auto operands = [&](const gpk_replay_part& d, const PartWords& w) {
+    PartOperands o;
+    if (takes_line(d)) o.r = load_entries(T, O, packet_head(w.a.x), packet_line(w.a.x), t);
+    else o.s = simple_values(T, simple_of(w));
+    return o;
+  };
+  gpk_replay_part d0 = uniform(part(0)), d1 = uniform(part(1)), ahead = part(2);
+  PartWords w0 = packets(d0), w1 = packets(d1);
+  PartOperands o0 = operands(d0, w0);
 #pragma unroll 1
-  for (int32_t l = 0; l < nlevels; ++l) {
-    const int32_t next_end = level_start[min(l + 4, nlevels)];
-    const int32_t p2 = packet(begin, end);
-    const RecEntries r1 = load_entries(T, O, packet_head(p1), packet_line(p1), t);
-    const RecVars rv{row_lane<PK_W0>(p0), row_lane<PK_W0 + 1>(p0), row_lane<PK_W0 + 2>(p0)};
-    replay_one<kDual>(T, O, x, y, z, zret, packet_head(p0), rv, packet_line(p0), r0, tol);
-    __syncthreads();
-    p0 = p1;
-    p1 = p2;
-    r0 = r1;
-    begin = end;
-    end = next_end;
+  for (int32_t p = 0; p < nparts; ++p) {
+    const gpk_replay_part d2 = uniform(ahead), next = part(p + 3);
+    PartWords w2;
+    PartOperands o1;
+    if (takes_line(d0)) {
+      w2 = packets(d2);
+      o1 = operands(d1, w1);
+      const int32_t w = w0.a.x;
+      const RecVars rv{row_lane<PK_W0>(w), row_lane<PK_W0 + 1>(w), row_lane<PK_W0 + 2>(w)};
+      replay_line<kDual>(T, O, x, y, z, zret, packet_head(w), rv, packet_line(w), o0.r, tol);
+    } else {
+      const SimpleRec h = simple_of(w0);
+      const SimpleReads in = simple_reads<kDual>(h, x, y, z);  // on their way before the loads ahead
+      w2 = packets(d2);
+      o1 = operands(d1, w1);
+      replay_simple<kDual>(T, x, y, z, zret, h, o0.s, in, tol);
+    }
+    if (d1.simples & GPK_PART_NEW_LEVEL) __syncthreads();
+    d0 = d1;
+    d1 = d2;
+    ahead = next;
+    w0 = w1;
+    w1 = w2;
+    o0 = o1;
   }
 }
 
@@ -844,43 +966,37 @@ hipError_t gpk_mark(const int32_t* red2org, int32_t n_red, uint8_t* mask, hipStr
 hipError_t gpk_restore_fixed(const int32_t* idx, const double* val, int32_t count, double* x, hipStream_t stream) {
   GPK_LAUNCH(k_restore_fixed, count, idx, val, count, x);
 }
-hipError_t gpk_replay(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                      int32_t begin, int32_t end, int32_t primal, int32_t dual, double tol, hipStream_t stream) {
-  if (end <= begin) return hipSuccess;
-  hipLaunchKernelGGL(k_replay, dim3(1), dim3(64), 0, stream, tape, orig, x, y, z, zret, begin, end, primal, dual, tol);
-  return hipGetLastError();
-}
-hipError_t gpk_pack_records(gp_tape_dev tape, gp_orig_dev orig, const int32_t* records, int32_t count, int32_t has_y,
-                            int32_t dual, int32_t* packets, hipStream_t stream) {
-  if (count <= 0) return hipSuccess;
-  const dim3 grid(grid_for(count, kBlock / kRecLanes));
-  if (dual)
-    hipLaunchKernelGGL(k_pack_records<true>, grid, dim3(kBlock), 0, stream, tape, orig, records, count, has_y, packets);
-  else
-    hipLaunchKernelGGL(k_pack_records<false>, grid, dim3(kBlock), 0, stream, tape, orig, records, count, has_y, packets);
+hipError_t gpk_pack_records(gp_tape_dev tape, gp_orig_dev orig, gpk_replay_slots slots, int32_t dual_line,
+                            int32_t has_y, hipStream_t stream) {
+  const int32_t lb = slots.line_slots > 0 ? static_cast<int32_t>(grid_for(slots.line_slots, kBlock / kRecLanes)) : 0;
+  const int32_t sb = slots.simple_slots > 0 ? static_cast<int32_t>(grid_for(slots.simple_slots)) : 0;
+  if (lb + sb == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_pack_records, dim3(lb + sb), dim3(kBlock), 0, stream, tape, orig, slots, dual_line, has_y, lb);
   return hipGetLastError();
 }
 hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                           const int32_t* packets, int32_t count, int32_t dual, double tol, hipStream_t stream) {
-  if (count <= 0) return hipSuccess;
-  const dim3 grid(grid_for(count, kBlock / kRecLanes));
+                           const int32_t* line, int32_t lines, const int32_t* simple, int32_t simples, int32_t dual,
+                           double tol, hipStream_t stream) {
+  const int32_t lb = lines > 0 ? static_cast<int32_t>(grid_for(lines, kBlock / kRecLanes)) : 0;
+  const int32_t sb = simples > 0 ? static_cast<int32_t>(grid_for(simples)) : 0;
+  if (lb + sb == 0) return hipSuccess;
   if (dual)
-    hipLaunchKernelGGL(k_replay_list<true>, grid, dim3(kBlock), 0, stream, tape, orig, x, y, z, zret, packets, count, tol);
+    hipLaunchKernelGGL(k_replay_list<true>, dim3(lb + sb), dim3(kBlock), 0, stream, tape, orig, x, y, z, zret, line,
+                       lines, simple, simples, lb, tol);
   else
-    hipLaunchKernelGGL(k_replay_list<false>, grid, dim3(kBlock), 0, stream, tape, orig, x, y, z, zret, packets, count, tol);
+    hipLaunchKernelGGL(k_replay_list<false>, dim3(lb + sb), dim3(kBlock), 0, stream, tape, orig, x, y, z, zret, line,
+                       lines, simple, simples, lb, tol);
   return hipGetLastError();
 }
 hipError_t gpk_replay_levels(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                             const int32_t* packets, const int32_t* level_start, int32_t nlevels, int32_t dual,
-                             double tol, hipStream_t stream) {
-  if (nlevels <= 0) return hipSuccess;
-  const dim3 block(GPK_REPLAY_SLOTS * kRecLanes);
-  if (dual)
-    hipLaunchKernelGGL(k_replay_levels<true>, dim3(1), block, 0, stream, tape, orig, x, y, z, zret, packets, level_start,
-                       nlevels, tol);
-  else
-    hipLaunchKernelGGL(k_replay_levels<false>, dim3(1), block, 0, stream, tape, orig, x, y, z, zret, packets,
-                       level_start, nlevels, tol);
+                             const int32_t* line, const int32_t* simple, const gpk_replay_part* parts, int32_t nparts,
+                             int32_t waves, int32_t has_lines, int32_t dual, double tol, hipStream_t stream) {
+  if (nparts <= 0) return hipSuccess;
+  if (waves < 1 || waves > GPK_REPLAY_WAVES) return hipErrorInvalidValue;
+  const auto run = dual ? (has_lines ? k_replay_levels<true, true> : k_replay_levels<true, false>)
+                        : (has_lines ? k_replay_levels<false, true> : k_replay_levels<false, false>);
+  hipLaunchKernelGGL(run, dim3(1), dim3(64 * waves), 0, stream, tape, orig, x, y, z, zret, line, simple, parts, nparts,
+                     tol);
   return hipGetLastError();
 }
 hipError_t gpk_seg_lengths(const int32_t* ptr, const int32_t* list, int32_t count, int32_t* len, hipStream_t stream) {

@@ -51,26 +51,52 @@ hipError_t gpk_map_tape_indices(int32_t count, int32_t* idx, const uint8_t* kind
 hipError_t gpk_scatter(const double* src, const int32_t* red2org, int32_t n_red, double* dst, hipStream_t stream);
 hipError_t gpk_mark(const int32_t* red2org, int32_t n_red, uint8_t* mask, hipStream_t stream);
 hipError_t gpk_restore_fixed(const int32_t* idx, const double* val, int32_t count, double* x, hipStream_t stream);
-hipError_t gpk_replay(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                      int32_t begin, int32_t end, int32_t primal, int32_t dual, double tol, hipStream_t stream);
 /* Dependency-level replay (the reverse tape order split into levels whose
- * records touch disjoint variables), one pass at a time (dual or primal).
- * gpk_pack_records: the packets (GPK_PACKET_WORDS words each) of a schedule's
- * records for a pass (-1: an empty slot; has_y: the replay has a y), which hold
- * places in the tape and in the original model's row pointers, no values.
- * gpk_replay_list: the records of one level.  gpk_replay_levels: nlevels
- * consecutive levels in one workgroup, level lv being slots [level_start[lv],
- * level_start[lv+1]), at most GPK_REPLAY_SLOTS of them (a longer level is given
- * as several). */
-#define GPK_REPLAY_SLOTS 64
+ * records touch disjoint variables), one pass at a time (dual or primal).  A
+ * record that walks a line of entries (gpk_record_walks_line: its type and number
+ * of index words, and whether the replay has an original model and a y) is
+ * replayed by sixteen lanes, any other by one; the two have slots and packets
+ * of their own, in the order of the schedules.  gpk_pack_records writes the
+ * packets of all slots (line_records / simple_records: the slots' records, -1 an
+ * empty slot; line slots from dual_line on belong to the dual pass): places in
+ * the tape and in the original model's row pointers, no values.
+ * gpk_replay_list: the records of one level.  gpk_replay_levels: consecutive
+ * levels in one workgroup of `waves` waves (up to GPK_REPLAY_WAVES), given as
+ * parts: line records `line` .. line + lines - 1, GPK_WAVE_LINES to a wave, and
+ * (simples >> GPK_PART_SHIFT) of the others from `simple` on, 64 to a wave, as many
+ * together as the waves hold; GPK_PART_NEW_LEVEL in simples where the part begins
+ * a level.  has_lines: some part has line records. */
+#define GPK_REPLAY_WAVES 16
+#define GPK_WAVE_LINES 4
 #define GPK_PACKET_WORDS 16
-hipError_t gpk_pack_records(gp_tape_dev tape, gp_orig_dev orig, const int32_t* records, int32_t count, int32_t has_y,
-                            int32_t dual, int32_t* packets, hipStream_t stream);
+#define GPK_SIMPLE_WORDS 8
+#define GPK_PART_NEW_LEVEL 1
+#define GPK_PART_SHIFT 1
+typedef struct __attribute__((aligned(16))) gpk_replay_part {
+  int32_t line, lines, simple, simples;
+} gpk_replay_part;
+typedef struct gpk_replay_slots {
+  int32_t line_slots, simple_slots;
+  const int32_t* line_records;
+  const int32_t* simple_records;
+  int32_t* line;   /* GPK_PACKET_WORDS a slot */
+  int32_t* simple; /* GPK_SIMPLE_WORDS a slot, 16-byte aligned */
+} gpk_replay_slots;
+static inline int32_t gpk_record_walks_line(int32_t type, int32_t indices, int32_t dual, int32_t has_orig,
+                                            int32_t has_y) {
+  if (!dual) return type == 2;
+  if (type == 0) return has_y && indices > 1;
+  if (type == 13 || type == 4) return has_orig && has_y;
+  return type == 5 || type == 12;
+}
+hipError_t gpk_pack_records(gp_tape_dev tape, gp_orig_dev orig, gpk_replay_slots slots, int32_t dual_line,
+                            int32_t has_y, hipStream_t stream);
 hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                           const int32_t* packets, int32_t count, int32_t dual, double tol, hipStream_t stream);
+                           const int32_t* line, int32_t lines, const int32_t* simple, int32_t simples, int32_t dual,
+                           double tol, hipStream_t stream);
 hipError_t gpk_replay_levels(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                             const int32_t* packets, const int32_t* level_start, int32_t nlevels, int32_t dual,
-                             double tol, hipStream_t stream);
+                             const int32_t* line, const int32_t* simple, const gpk_replay_part* parts, int32_t nparts,
+                             int32_t waves, int32_t has_lines, int32_t dual, double tol, hipStream_t stream);
 /* len[i] = ptr[list[i] + 1] - ptr[list[i]]; gpk_seg_copy packs line
  * list[i]'s idx entries at out + off[i]. */
 hipError_t gpk_seg_lengths(const int32_t* ptr, const int32_t* list, int32_t count, int32_t* len, hipStream_t stream);

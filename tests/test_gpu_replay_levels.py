@@ -1,7 +1,9 @@
 """Tapes written by hand for the postsolve replay, against the oracle's
 record-by-record replay, bit for bit: lines around the 16 and 32 entries that
-are loaded ahead, every record type in one level, levels around the 64 slots
-of the workgroup and around the size that takes a launch of its own."""
+are loaded ahead, every record type in one level, levels around a wave's, a
+part's and a workgroup's records of either kind (those that walk a line and the
+others) and around the sizes that take a launch of their own, chains of single
+records, and records without rows or an original model."""
 import numpy as np
 import pytest
 
@@ -100,13 +102,101 @@ def test_random_tapes(count, with_original):
     check(lp, [random_record(rng, lp) for _ in range(count)], 43, with_original)
 
 
-def test_levels_around_the_slots_and_the_launch_of_their_own():
-    lp = original(700, 900, 51)
+def test_levels_of_simple_records():
+    """A wave, a part, two parts, a launch of their own; grid and run in turn."""
+    m = 2100
+    lp = original(m, 900, 51)
     rng = np.random.default_rng(52)
-    sizes = [1, 3, 4, 5, 15, 16, 17, 63, 64, 65, 127, 128, 129, 510, 511, 512, 513, 600]
+    sizes = [1, 3, 4, 5, 63, 64, 65, 127, 128, 129, 511, 512, 513, 1023, 1024, 1025, 2047, 2048, 2049, 1, 2049, 700]
     records = [(10, np.r_[row], np.r_[rng.standard_normal()]) for size in sizes for row in range(size)]
     check(lp, records, 53)
-    rec = record_of(700, 900, records, 53)
+    rec = record_of(m, 900, records, 53)
     plan = gp_ffi.PostsolvePlan(rec, original=lp)
     assert plan.shape()["dual_levels"] == len(sizes)
     plan.free()
+
+
+def disjoint_rows(m, k):
+    """An LP whose row r holds the columns k r .. k r + k - 1, all at 1 there."""
+    rng = np.random.default_rng(m)
+    rows, cols = np.repeat(np.arange(m), k), np.arange(m * k)
+    vals = rng.choice([-2.0, -0.5, 0.5, 2.0], m * k) * (1.0 + rng.random(m * k) * 2.0 ** -20)
+    ptr, idx, val = lp_synth.csr_from_coo(m, m * k, rows, cols, vals)
+    tptr, tidx, tval = lp_synth.transpose_csr(m, m * k, ptr, idx, val)
+    n = m * k
+    return dict(m=m, n=n, A_ptr=ptr, A_idx=idx, A_val=val, AT_ptr=tptr, AT_idx=tidx, AT_val=tval, c=rng.standard_normal(n),
+                l=np.zeros(n), u=np.full(n, INF), AL=np.full(m, -INF), AU=np.full(m, 1e6), obj=0.0)
+
+
+# line records (bound changes: a row of four entries each), then the others (type 10 on further rows) of a level
+MIXED = [(1, 0), (1, 1), (3, 5), (4, 60), (5, 64), (16, 65), (59, 64), (60, 64), (60, 65), (61, 64), (63, 1), (64, 0),
+         (64, 1), (64, 1024), (64, 1100), (1, 960), (1, 961), (4, 1025), (65, 0), (65, 700), (2, 2048), (2, 2049), (64, 64)]
+
+
+def test_levels_of_both_kinds():
+    m, k = 2200, 4
+    lp = disjoint_rows(m, k)
+    rng = np.random.default_rng(71)
+    records = []
+    for level, (lines, others) in enumerate(MIXED):
+        for r in range(lines):
+            records.append((12, np.r_[r * k + level % k, r], np.r_[0.0, INF, 1.0, INF]))
+        for r in range(100, 100 + others):
+            records.append((10, np.r_[r], np.r_[rng.standard_normal()]))
+        records.append((10, np.r_[0], np.r_[0.25]))  # ties the next level's rows to this one's
+    rec = record_of(lp["m"], lp["n"], records, 72)
+    rec.update(n1=lp["n"], col_red2org=np.arange(lp["n"], dtype=np.int32), fixed_idx=np.zeros(0, np.int32),
+               fixed_val=np.zeros(0))
+    point = (np.ones(lp["n"]), rng.standard_normal(m), rng.standard_normal(lp["n"]))
+    want = O.postsolve(rec, *point, original=lp)
+    got = gp_ffi.postsolve(rec, *point, original=lp)
+    for name, a, b in zip("xyz", got, want):
+        assert_same_array(name, a, b)
+
+
+@pytest.mark.parametrize("kind", ["simple", "line", "in-turn"])
+def test_chains_of_single_records(kind):
+    lp = disjoint_rows(50, 4)
+    rng = np.random.default_rng(81)
+    line = [(12, np.r_[q % 4, 0], np.r_[0.0, INF, 1.0, INF]) for q in range(700)]
+    simple = [(10, np.r_[0], np.r_[rng.standard_normal()]) for _ in range(700)]
+    records = {"simple": simple, "line": line, "in-turn": [r for pair in zip(line, simple) for r in pair]}[kind]
+    rec = record_of(lp["m"], lp["n"], records, 82)
+    rec.update(n1=lp["n"], col_red2org=np.arange(lp["n"], dtype=np.int32), fixed_idx=np.zeros(0, np.int32),
+               fixed_val=np.zeros(0))
+    point = (np.ones(lp["n"]), rng.standard_normal(50), rng.standard_normal(lp["n"]))
+    want = O.postsolve(rec, *point, original=lp)
+    got = gp_ffi.postsolve(rec, *point, original=lp)
+    for name, a, b in zip("xyz", got, want):
+        assert_same_array(name, a, b)
+
+
+def test_records_without_rows():
+    """No rows and no original model: every record is a lane's, but for the
+    substituted columns' primal."""
+    n = 3000
+    rng = np.random.default_rng(91)
+    f = lambda size=None: rng.choice([-2.0, -1.0, -0.5, 0.5, 1.0, 2.0], size) * (1 + rng.random(size) * 2.0 ** -20)
+    records = []
+    for _ in range(900):
+        t, cols = int(rng.choice([0, 1, 2, 3, 13, 14])), rng.choice(n, size=20, replace=False)
+        if t == 0:
+            records.append((0, cols[:1], np.r_[1.0, f()]))
+        elif t == 1:
+            records.append((1, np.r_[0, cols[0], 2, cols[:2]], np.r_[1.0, 0.5, 1.0, f(2)]))
+        elif t == 2:
+            records.append((2, np.r_[cols[0], -1, 17, cols[3:]], np.r_[f(), 1.0, 0.0, 0.0, f(), 1.0, f(17) / 64]))
+        elif t == 3:
+            records.append((3, cols[:2], np.r_[f(), 0.0, 1.0, -1.0, INF]))
+        elif t == 13:
+            records.append((13, np.r_[cols[:2], -1], np.r_[4.0, f(), 1.0, 0.0, 0.0, 0.0, 4.0, 0.5, 2.0, f()]))
+        else:
+            records.append((14, np.r_[0, cols[0], 0, cols[1:3]], np.r_[1.0, f(), 2.0, 0.25, rng.standard_normal(2) / 64]))
+    rec = record_of(0, n, records, 92)
+    point = (rng.integers(0, 2, rec["n1"]).astype(float), np.zeros(0), rng.standard_normal(rec["n1"]))
+    with np.errstate(all="ignore"):
+        want = O.postsolve(rec, *point)
+    assert all(np.isfinite(w).all() for w in want)
+    got = gp_ffi.postsolve(rec, *point)
+    for name, a, b in zip("xyz", got, want):
+        assert_same_array(name, a, b)

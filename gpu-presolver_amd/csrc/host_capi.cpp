@@ -674,6 +674,7 @@ gp_status gp_serve_trace(const gp_lp* lps, int32_t lp_count, const int32_t* lp_o
       if (arrival_s) require(k == 0 || arrival_s[k] >= arrival_s[k - 1], "arrival times must be non-decreasing");
     }
     require_device();
+    amd::check(hipDeviceSynchronize(), "gp_serve_trace entry synchronize");
     std::unique_ptr<amd::Server, void (*)(amd::Server*)> srv(amd::server_create(to_params(params), *config),
                                                              amd::server_destroy);
     for (int32_t k = 0; k < jobs; ++k) {
@@ -806,6 +807,7 @@ gp_status gp_synthetic_point(uint64_t seed, const gp_lp* lp, double* x, double* 
     const LPInfoGpu L = to_lp(*lp);
     require((L.A.cols == 0 || (x && z)) && (L.A.rows == 0 || y), "null output vector");
     require_device();
+    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_synthetic_point entry synchronize");
     amd::Ctx& c = amd::ctx();
     amd::check(gpk_synthetic_point(seed, L.A.cols, L.A.rows, L.l, L.u, x, y, z, c.stream()), "synthetic point");
     c.sync("synthetic point");
@@ -817,6 +819,7 @@ gp_status gp_checksum(const double* x, int32_t n, const double* y, int32_t m, co
     require(out != nullptr && n >= 0 && m >= 0, "invalid argument");
     require((n == 0 || (x && z)) && (m == 0 || y), "null vector");
     require_device();
+    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_checksum entry synchronize");
     *out = amd::checksum_xyz(x, n, y, m, z);
   });
 }
@@ -1103,6 +1106,7 @@ gp_status gp_pdhg_solve(const gp_lp* lp, const gp_pdhg_params* params, double* x
     require(L.A.cols == 0 || (L.c && L.l && L.u), "null c/l/u");
     require(L.A.rows == 0 || (L.AL && L.AU), "null AL/AU");
     require_device();
+    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_pdhg_solve entry synchronize");
     const amd::PdhgReport r = amd::pdhg_solve(L, pdhg_options(params), x, y, z);
     amd::ctx().sync("gp_pdhg_solve");
     *out = pdhg_result(r);

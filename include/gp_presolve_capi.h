@@ -13,7 +13,10 @@
  *    the comment says "host".
  *  - Calls are synchronous with respect to the host (like the reference,
  *    which returns after cudaDeviceSynchronize) and run on the library's
- *    internal stream.
+ *    internal stream, after the work that is pending on the device when they
+ *    are entered (a call with a stream argument: on that stream; a submitted
+ *    job's LP must be complete on the device, as its worker waits for no other
+ *    stream).
  *  - Errors: a nonzero gp_status; gp_last_error() gives the message of the
  *    last failure on the calling thread.  LP outcomes (infeasible, unbounded)
  *    are not errors; they are flags in the results, as in the reference.

@@ -141,3 +141,62 @@ def test_postsolve_rejects_original_with_repeated_column():
     bad = _with_rows(lp, dup)
     with pytest.raises(gp_ffi.GpError, match="repeats a column"):
         gp_ffi.postsolve(rec, x, y, z, bad)
+
+
+class _Pending:
+    """Device arrays that a busy stream is still to fill: each holds zeros until
+    some milliseconds of other work on the stream are done."""
+
+    def __init__(self, arrays):
+        H = gp_ffi.hip()
+        H.hipMemsetAsync.argtypes = [C.c_void_p, C.c_int, C.c_size_t, C.c_void_p]
+        H.hipMemcpyAsync.argtypes = [C.c_void_p, C.c_void_p, C.c_size_t, C.c_int, C.c_void_p]
+        self.stream, self.busy = gp_ffi.Stream(), gp_ffi.DeviceArray(size=1 << 28)
+        self.copies = []
+        for ptr, nbytes in arrays:
+            keep = gp_ffi.DeviceArray(size=nbytes, dtype=np.uint8)
+            gp_ffi.hip_check(H.hipMemcpy(keep.ptr, ptr, nbytes, gp_ffi.D2D), "keep")
+            gp_ffi.hip_check(H.hipMemset(ptr, 0, nbytes), "clear")
+            self.copies.append((ptr, keep, nbytes))
+        self.start()
+
+    def start(self):
+        H = gp_ffi.hip()
+        for _ in range(20):
+            gp_ffi.hip_check(H.hipMemsetAsync(self.busy.ptr, 1, self.busy.nbytes, self.stream.ptr), "busy")
+        for ptr, keep, nbytes in self.copies:
+            gp_ffi.hip_check(H.hipMemcpyAsync(ptr, keep.ptr, nbytes, gp_ffi.D2D, self.stream.ptr), "fill")
+
+
+def test_solver_waits_for_the_callers_pending_work():
+    lp = lp_synth.generate(300, 450, seed=26, mean_row_len=5.0)
+    prm = gp_ffi.pdhg_params(max_iters=200, tol=1e-13)
+    d = gp_ffi.DeviceLp(lp)
+    want, out = gp_ffi.pdhg_solve_view(d.g, prm)
+    want_x = out[0].numpy()
+    g, nnz = d.g, len(lp["A_idx"])
+    pending = _Pending([(g.A.row_ptr, 4 * (lp["m"] + 1)), (g.AT.row_ptr, 4 * (lp["n"] + 1)), (g.A.col_idx, 4 * nnz),
+                        (g.A.val, 8 * nnz), (g.AT.val, 8 * nnz)])
+    got, out = gp_ffi.pdhg_solve_view(d.g, prm)
+    assert got["iterations"] == want["iterations"] and got["primal_obj"] == want["primal_obj"]
+    assert np.array_equal(out[0].numpy(), want_x)
+    pending.stream.sync()
+
+
+def test_checksum_and_point_wait_for_the_callers_pending_work():
+    rng = np.random.default_rng(27)
+    x, y, z = rng.standard_normal(1000), rng.standard_normal(700), rng.standard_normal(1000)
+    want = gp_ffi.checksum(x, y, z)
+    dx, dy, dz = (gp_ffi.DeviceArray(v) for v in (x, y, z))
+    pending = _Pending([(dx.ptr, dx.nbytes), (dy.ptr, dy.nbytes), (dz.ptr, dz.nbytes)])
+    out = C.c_uint64()
+    gp_ffi._check(gp_ffi.lib().gp_checksum(dx.ptr, 1000, dy.ptr, 700, dz.ptr, C.byref(out)))
+    assert out.value == want
+    pending.stream.sync()
+    lp = lp_synth.generate(300, 450, seed=28, mean_row_len=5.0)
+    d = gp_ffi.DeviceLp(lp)
+    want_p = gp_ffi.synthetic_point(5, d.g)
+    pending = _Pending([(d.g.l, 8 * lp["n"]), (d.g.u, 8 * lp["n"])])
+    for a, b in zip(gp_ffi.synthetic_point(5, d.g), want_p):
+        assert np.array_equal(a, b)
+    pending.stream.sync()

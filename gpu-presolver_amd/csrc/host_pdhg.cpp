@@ -97,12 +97,12 @@ PdhgReport pdhg_solve(const LPInfoGpu& lp, const PdhgOptions& opt, double* x_out
   };
   const auto plan_rows = [&](const presolve::DeviceCsrMatrix& M, RowPlan& plan) {
     const std::vector<int32_t> ptr = cx.to_host(M.rowPtr, static_cast<int64_t>(M.rows) + 1, where);
-    std::vector<gpk_row_block> b(static_cast<size_t>(gpk_pdhg_row_plan(ptr.data(), M.rows, nullptr)) + 1);
+    std::vector<gpk_row_block> b(static_cast<size_t>(gpk_pdhg_row_plan_most(M.rows, M.nnz)) + 1);
     plan.blocks = gpk_pdhg_row_plan(ptr.data(), M.rows, b.data());
-    plan.blk.alloc(static_cast<int64_t>(b.size()), where);
+    plan.blk.alloc(static_cast<int64_t>(plan.blocks) + 1, where);
     plan.part_sum.alloc(plan.blocks, where);
     plan.part_count.alloc(plan.blocks, where);
-    cx.to_device(plan.blk.get(), b.data(), static_cast<int64_t>(b.size()), where);
+    cx.to_device(plan.blk.get(), b.data(), static_cast<int64_t>(plan.blocks) + 1, where);
     CopyBatch().zero(plan.part_count.get(), plan.blocks).run(where);
   };
   RowPlan plan_a, plan_at;

@@ -51,9 +51,15 @@ namespace {
 constexpr int kEntryBudget = GPK_PDHG_ENTRY_BUDGET;
 constexpr int kStage = kEntryBudget / kBlock;  // staged entries per thread
 constexpr int kPartials = 4;
-// A thread sums a row of up to this many entries by itself (about 15 ns each, one
-// after the other); its wave takes a longer one, at about 200 ns a row.
+// A thread sums a row by itself (about 15 ns an entry, one after the other), or
+// a wave does, at about 200 ns a row.  A block's rows of more than kThreadRow
+// entries go to its waves in turn where those are done first, which the plan says
+// (GPK_ROWS_BY_WAVE).  (With every such row left to the wave of its thread, a
+// block's rows were all one wave's: 128 iterations with rows of 40 entries
+// 10.4 ms, 7.4 with a thread a row and 7.2 this way; of 100 entries 9.0, 7.7 and
+// 7.1; columns of 200 entries 9.2, 9.8 and 7.7.)
 constexpr int kThreadRow = 32;
+bool rows_by_wave(int32_t rows, int32_t longest) { return rows > 0 && 200 * rows < kWaves * 15 * longest; }
 static_assert(kEntryBudget % kBlock == 0, "entry budget in whole strides");
 
 __device__ inline double clampd(double v, double lo, double hi) { return fmin(fmax(v, lo), hi); }
@@ -345,13 +351,18 @@ __global__ __launch_bounds__(kBlock) void k_rows(const int32_t* __restrict__ ptr
       cv[k] = bv[q];
     }
   }
-  const bool mine = tid < (b.parts > 0 ? 1 : nr);
-  const int32_t r = b.row + (mine ? tid : 0);
+  // A block's few rows go to its waves in turn where those sum the longer ones
+  // (more rows are spread as they stand, and load their own vectors in order: 150
+  // entries in each twentieth of rows of 8 are 4.7 ms that way, 4.95 in turn).
+  const bool waves = b.parts == GPK_ROWS_BY_WAVE;
+  const int at = waves && nr <= 64 ? lane_id() * kWaves + (tid >> 6) : tid;
+  const bool mine = at < (b.parts > 0 ? 1 : nr);
+  const int32_t r = b.row + (mine ? at : 0);
   typename Op::Own own{};
   int32_t pb = 0, pe = 0;
   if (mine) {
     own = op.load(r);
-    if (b.parts == 0) {
+    if (b.parts <= 0) {
       pb = ptr[r] - b.entry;
       pe = ptr[r + 1] - b.entry;
     }
@@ -359,13 +370,13 @@ __global__ __launch_bounds__(kBlock) void k_rows(const int32_t* __restrict__ ptr
 #pragma unroll
   for (int k = 0; k < kStage; ++k)
     if (tid + k * kBlock < cnt) cv[k] = op.elem(ci[k], cv[k], factor);
-  if (b.parts == 0) {
+  if (b.parts <= 0) {
 #pragma unroll
     for (int k = 0; k < kStage; ++k)
       if (tid + k * kBlock < cnt) s_val[tid + k * kBlock] = cv[k];
     __syncthreads();
     double acc = C::identity();
-    const bool by_wave = pe - pb > kThreadRow;
+    const bool by_wave = waves && pe - pb > kThreadRow;
     if (!by_wave) acc = combine_in_order<C>(s_val, pb, pe);
     for (uint64_t todo = __ballot(by_wave); todo != 0; todo &= todo - 1) {
       const int q = __ffsll(static_cast<unsigned long long>(todo)) - 1;
@@ -458,7 +469,7 @@ __global__ __launch_bounds__(kBlock) void k_rows_scale(const int32_t* __restrict
   }
   if (tid < nr) {
     s_d[tid] = drow[b.row + tid];
-    if (b.parts == 0)
+    if (b.parts <= 0)
       for (int32_t q = ptr[b.row + tid] - b.entry, e = ptr[b.row + tid + 1] - b.entry; q < e; ++q)
         s_row[q] = static_cast<uint8_t>(tid);
   }
@@ -566,17 +577,24 @@ __global__ void k_pdhg_project_zero(const double* __restrict__ l, const double* 
   if (j < n) x[j] = clampd(0.0, l[j], u[j]);
 }
 
-// The row after the last of the block that starts at row r.
-int32_t block_end(const int32_t* ptr, int32_t rows, int32_t r) {
+// The row after the last of the block that starts at row r; *by_wave: its rows
+// are the waves'.
+int32_t block_end(const int32_t* ptr, int32_t rows, int32_t r, bool* by_wave) {
+  *by_wave = false;
   if (ptr[r + 1] - ptr[r] > GPK_PDHG_LONG_ROW) return r + 1;
   const int32_t start = r;
-  int32_t cnt = 0;
+  int32_t cnt = 0, longs = 0, longest = 0;
   while (r < rows && r - start < kBlock) {
     const int32_t len = ptr[r + 1] - ptr[r];
     if (len > GPK_PDHG_LONG_ROW || cnt + len > kEntryBudget) break;
+    if (__builtin_expect(len > kThreadRow, 0)) {
+      ++longs;
+      longest = len > longest ? len : longest;
+    }
     cnt += len;
     ++r;
   }
+  *by_wave = r - start > 1 && rows_by_wave(longs, longest);
   return r;
 }
 
@@ -601,18 +619,28 @@ int32_t gpk_pdhg_row_blocks(const int32_t* ptr, int32_t rows, int32_t* blk) {
   int32_t nb = 0;
   if (blk) blk[0] = 0;
   for (int32_t r = 0; r < rows;) {
-    r = block_end(ptr, rows, r);
+    bool by_wave;
+    r = block_end(ptr, rows, r, &by_wave);
     ++nb;
     if (blk) blk[nb] = r;
   }
   return nb;
 }
 
+int64_t gpk_pdhg_row_plan_most(int32_t rows, int32_t nnz) {
+  // A block ends at 256 rows, or past the budget less a row, or before a long row
+  // or at the end; a long row's parts are its whole budgets and one.
+  const int64_t e = nnz, longs = e / (GPK_PDHG_LONG_ROW + 1);
+  return rows / kBlock + e / (kEntryBudget - GPK_PDHG_LONG_ROW) + (longs + 1) + (e / kEntryBudget + longs);
+}
+
 int32_t gpk_pdhg_row_plan(const int32_t* ptr, int32_t rows, gpk_row_block* out) {
   int32_t nb = 0;
   for (int32_t r = 0; r < rows;) {
-    const int32_t end = block_end(ptr, rows, r), entries = ptr[end] - ptr[r];
-    const int32_t parts = end - r > 1 ? 0 : entries > kEntryBudget ? (entries - 1) / kEntryBudget + 1 : 1;
+    bool by_wave;
+    const int32_t end = block_end(ptr, rows, r, &by_wave), entries = ptr[end] - ptr[r];
+    const int32_t parts = end - r > 1 ? (by_wave ? GPK_ROWS_BY_WAVE : 0)
+                                      : entries > kEntryBudget ? (entries - 1) / kEntryBudget + 1 : 1;
     for (int32_t k = 0; k < (parts > 0 ? parts : 1); ++k, ++nb)
       if (out) out[nb] = gpk_row_block{r, ptr[r] + k * kEntryBudget, k, parts};
     r = end;

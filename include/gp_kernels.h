@@ -681,8 +681,10 @@ hipError_t gpk_screen_structural_prefix(const int32_t* ptr, const int32_t* idx, 
 #define GPK_PDHG_LONG_ROW 256
 #define GPK_PDHG_ENTRY_BUDGET 2048
 /* Block k: entries [entry, blk[k + 1].entry) of M, those of the rows
- * [row, blk[k + 1].row) where parts is 0, otherwise part `part` of the `parts`
- * parts of row `row`, whose blocks follow each other. */
+ * [row, blk[k + 1].row) where parts is 0 or GPK_ROWS_BY_WAVE (the block's waves
+ * sum its longer rows in turn), otherwise part `part` of the `parts` parts of
+ * row `row`, whose blocks follow each other. */
+#define GPK_ROWS_BY_WAVE (-1)
 typedef struct gpk_row_block {
   int32_t row, entry, part, parts;
 } gpk_row_block;
@@ -698,7 +700,8 @@ typedef struct gpk_rows {
  * returns the block count. */
 int32_t gpk_pdhg_row_blocks(const int32_t* ptr, int32_t rows, int32_t* blk);
 /* Host: those blocks with the long rows in parts, blocks + 1 entries (NULL only
- * counts). */
+ * counts); gpk_pdhg_row_plan_most: no matrix of rows and nnz has more blocks. */
+int64_t gpk_pdhg_row_plan_most(int32_t rows, int32_t nnz);
 int32_t gpk_pdhg_row_plan(const int32_t* ptr, int32_t rows, gpk_row_block* out);
 /* `iterations` PDHG steps from z = (x, y): the PDHG point T(z) is
  * xn = proj_[l,u](x - tau (c - A^T y)), xbar = 2 xn - x, yn the projected

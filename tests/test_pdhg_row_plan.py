@@ -20,6 +20,8 @@ CASES = {
     "neighbours": [2049] * 5 + [257] * 9 + [33] * 70 + [0] * 600 + [1],
     "many-parts": [0, 600_000, 3, 40_000],
     "short": [3] * 1000,
+    "few-rows-by-wave": [100] * 61 + [200, 33, 32, 1, 0] * 30 + [150] * 40,
+    "many-rows-by-wave": [200, 256, 40] + [3] * 240 + [150] + [0] * 30 + [33] + [7] * 150,
     "empty": [0] * 700,
 }
 
@@ -50,6 +52,27 @@ def test_plan_covers_every_entry_once(case):
     for k in np.nonzero(parts > 1)[0]:
         assert ptr[row[k]] + part[k] * BUDGET == entry[k] and row[k - part[k]] == row[k]
         assert parts[k] == -(-int(ptr[row[k] + 1] - ptr[row[k]]) // BUDGET)
+
+
+def test_plan_says_which_blocks_the_waves_sum():
+    """The rows past 32 entries of a block of several rows go to the waves where
+    their 200 ns each on four waves are less than the longest's 15 ns an entry."""
+    for lens, want in (([40] * 51, 0), ([100] * 20, -1), ([33] + [8] * 200, -1), ([32] * 64, 0), ([200, 1], -1),
+                       ([60] * 18 + [8] * 20, 0), ([60] * 17 + [8] * 20, -1)):
+        ptr = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        b = plan(ptr)
+        assert len(b) == 2 and b[0, 3] == want, lens
+
+
+def test_no_plan_has_more_blocks_than_its_bound():
+    f = gp_ffi.lib().gpk_pdhg_row_plan_most
+    f.restype, f.argtypes = C.c_int64, [C.c_int32, C.c_int32]
+    rng = np.random.default_rng(3)
+    shapes = list(CASES.values()) + [[257, 0] * 500, [257] * 999, [256] * 999, [1, 257] * 400, [225] * 777, [0] * 5000]
+    shapes += [rng.integers(0, 600, 3000).tolist(), [], [1], [2048, 2049] * 50]
+    for lens in shapes:
+        ptr = np.concatenate([[0], np.cumsum(np.asarray(lens, np.int64))]).astype(np.int32)
+        assert len(plan(ptr)) - 1 <= f(len(lens), int(ptr[-1]))
 
 
 @pytest.mark.parametrize("arch,compiles", [("gfx950", True), ("gfx942", False)])

@@ -305,3 +305,29 @@ def test_compaction_of_rows_of_a_larger_matrix(lengths, first, last):
     assert got[:2] == want[:2]
     for name, a, w in zip(("ptr", "idx", "val"), got[2:], want[2:]):
         assert_same_array(name, a, w)
+
+
+SPLIT = [127, 128, 128, 129, 130, 130, 255, 256, 256, 8, 9, 9] * 2
+
+
+def columns_at_the_split(seed):
+    lp = lp_synth.generate(3000, 4500, seed=seed, mean_row_len=4.0, frac_doubleton=0.25, frac_fixed_cols=0.05,
+                           frac_singleton_cols=0.15, frac_dup_rows=0.0, frac_eq=0.0)
+    return with_dense_columns(lp, SPLIT, 52)
+
+
+@pytest.mark.parametrize("seed", [53, 60, 72])
+def test_presolve_with_columns_at_the_split(seed):
+    """LPs that the rules leave feasible, so the reduced costs of columns of 127 to
+    130 entries, which the column singletons change, are compared."""
+    lp = columns_at_the_split(seed)
+    kw = dict(enable_structure_specific_rules=0)
+    so, ro, lo = O.presolve(lp, O.params(**kw), True)
+    assert not so["has_infeasible"]
+    length = np.diff(lp["AT_ptr"])[ro["col_red2org"]]
+    changed = set(length[lo["c"] != lp["c"][ro["col_red2org"]]].tolist())
+    assert changed & {127, 128} and changed & {129, 130, 131}, sorted(changed)
+    sg, rg, lg = gp_ffi.presolve(lp, gp_ffi.params(**kw), True)
+    assert sg["obj_constant_delta"] == so["obj_constant_delta"] and not sg["has_infeasible"]
+    assert_same_record(rg, ro)
+    assert_same_lp(lg, lo)

@@ -615,18 +615,6 @@ hipError_t launch_reduce(const double* partial, int32_t blocks, double* out, hip
 
 extern "C" {
 
-int32_t gpk_pdhg_row_blocks(const int32_t* ptr, int32_t rows, int32_t* blk) {
-  int32_t nb = 0;
-  if (blk) blk[0] = 0;
-  for (int32_t r = 0; r < rows;) {
-    bool by_wave;
-    r = block_end(ptr, rows, r, &by_wave);
-    ++nb;
-    if (blk) blk[nb] = r;
-  }
-  return nb;
-}
-
 int64_t gpk_pdhg_row_plan_most(int32_t rows, int32_t nnz) {
   // A block ends at 256 rows, or past the budget less a row, or before a long row
   // or at the end; a long row's parts are its whole budgets and one.

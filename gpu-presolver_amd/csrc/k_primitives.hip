@@ -89,11 +89,6 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(const In* in, int32_t* out
   }
 }
 
-__global__ void k_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t* o2n, int32_t n) {
-  const int32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) o2n[i] = mask[i] != 0 ? prefix[i] : -1;
-}
-
 // -------------------------------------------------------- row activity ----
 // One thread per row, 256 consecutive rows per block.  The block's CSR
 // segment is streamed through LDS in windows: all threads cooperatively load
@@ -169,8 +164,8 @@ __global__ __launch_bounds__(kBlock, 6) void k_row_activity_lu(const int32_t* __
                                                             int32_t* __restrict__ neg_inf,
                                                             int32_t* __restrict__ pos_inf,
                                                             int32_t tiles) {
-  // One term array (the min terms, then the max terms): 16 KB of LDS per
-  // block, so eight blocks fit a CU and their load phases overlap.
+  // One term array (the min terms, then the max terms): with the runs 18 KB of
+  // LDS per block, so LDS has room for eight blocks a CU (the registers for six).
   __shared__ __align__(16) double s_t[kActCap + 16];
   __shared__ int32_t s_run[kActRows], s_at[kActRows];
   if (static_cast<int32_t>(blockIdx.x) >= tiles) {
@@ -1846,6 +1841,9 @@ __global__ __launch_bounds__(kSortSmallBlock) void k_sort_small(K* __restrict__ 
   }
 }
 
+// Words of scratch of a scan of n values.
+int64_t scan_scratch_ints(int64_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
+
 template <class In>
 hipError_t scan_impl(const In* in, int32_t* out, int64_t n, int32_t* scratch, hipStream_t s) {
   if (n <= 0) {
@@ -1933,16 +1931,6 @@ hipError_t gpk_iota_i32(int32_t* dst, int32_t n, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_iota, dim3(grid_for(n)), dim3(kBlock), 0, s, dst, n);
   return hipGetLastError();
-}
-
-int64_t gpk_scan_scratch_ints(int64_t n) { return (n + kScanTile - 1) / kScanTile + 1; }
-
-hipError_t gpk_scan_exclusive_i32(const int32_t* in, int32_t* out, int64_t n, int32_t* scratch, hipStream_t s) {
-  return scan_impl<int32_t>(in, out, n, scratch, s);
-}
-
-hipError_t gpk_scan_mask_u8(const uint8_t* mask, int32_t* out, int64_t n, int32_t* scratch, hipStream_t s) {
-  return scan_impl<uint8_t>(mask, out, n, scratch, s);
 }
 
 int64_t gpk_lookback_tiles(int64_t n) { return n > 0 ? (n + kScanTile - 1) / kScanTile : 1; }
@@ -2035,12 +2023,6 @@ hipError_t gpk_compact_write(gpk_compact_side a, gpk_compact_side t, const int32
   return hipGetLastError();
 }
 
-hipError_t gpk_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t* o2n, int32_t n, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(k_old_to_new, dim3(grid_for(n)), dim3(kBlock), 0, s, mask, prefix, o2n, n);
-  return hipGetLastError();
-}
-
 hipError_t gpk_pack_lu(const double* l, const double* u, int32_t n, double* lu, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL(k_pack_lu, dim3(grid_for(n)), dim3(kBlock), 0, s, l, u, n, reinterpret_cast<double2*>(lu));
@@ -2115,7 +2097,7 @@ hipError_t gpk_gather_i32(const int32_t* map, int32_t n_old, const int32_t* src,
 
 int64_t gpk_radix_scratch_ints(int64_t n) {
   const int64_t tiles = (n + kRsTile - 1) / kRsTile;
-  return 256 * tiles + 1 + gpk_scan_scratch_ints(256 * tiles) + 1;
+  return 256 * tiles + 1 + scan_scratch_ints(256 * tiles) + 1;
 }
 
 hipError_t gpk_radix_sort_u64_i32(uint64_t* keys, int32_t* vals, uint64_t* keys_alt, int32_t* vals_alt, int32_t n,
@@ -2204,7 +2186,7 @@ TbScratch tb_scratch(int32_t* base, int32_t buckets, int32_t nnz) {
   };
   TbScratch t{};
   t.offs = take(words + 1);
-  t.scan = take(gpk_scan_scratch_ints(words));
+  t.scan = take(scan_scratch_ints(words));
   t.piece = reinterpret_cast<TbPiece*>(take((buckets + kTbMore) * static_cast<int64_t>(sizeof(TbPiece) / sizeof(int32_t))));
   t.split = take(kTbSplit);
   t.counts = take(static_cast<int64_t>(kTbSplit) * kTbCols);

@@ -31,15 +31,6 @@ hipError_t gpk_fill_i32(int32_t* dst, int32_t v, int64_t n, hipStream_t stream);
 hipError_t gpk_fill_f64(double* dst, double v, int64_t n, hipStream_t stream);
 hipError_t gpk_iota_i32(int32_t* dst, int32_t n, hipStream_t stream);
 
-/* ---- scans --------------------------------------------------------------
- * Exclusive prefix sum of n int32 values into out[0..n]; out[n] is the total.
- * `scratch` holds gpk_scan_scratch_ints(n) ints.  In-place (out == in) is allowed. */
-int64_t gpk_scan_scratch_ints(int64_t n);
-hipError_t gpk_scan_exclusive_i32(const int32_t* in, int32_t* out, int64_t n, int32_t* scratch,
-                                  hipStream_t stream);
-/* Exclusive scan of (mask[i] != 0): out[0..n], out[n] = popcount. */
-hipError_t gpk_scan_mask_u8(const uint8_t* mask, int32_t* out, int64_t n, int32_t* scratch,
-                            hipStream_t stream);
 /* ---- single-pass scans (decoupled look-back) ----------------------------
  * One launch per scan: each 2048-item tile takes a ticket (dynamic tile id, in
  * dispatch order), publishes its aggregate, walks back over its predecessors'
@@ -208,10 +199,6 @@ hipError_t gpk_copy_many(const gpk_copy_seg* segs, int32_t count, hipStream_t st
  * makes them visible system-wide, then stores seq to mail[0].  mail is the
  * device address of host-mapped, coherent pinned memory. */
 hipError_t gpk_mail(const uint32_t* src, int32_t words, uint32_t* mail, uint32_t seq, hipStream_t stream);
-
-/* old_to_new[i] = mask[i] ? prefix[i] : -1. */
-hipError_t gpk_old_to_new(const uint8_t* mask, const int32_t* prefix, int32_t* old_to_new, int32_t n,
-                          hipStream_t stream);
 
 /* ---- activity primitives ----------------------------------------------- */
 /* Row activity (reference gpu_presolve_kernels.cu:18-111) over bounds packed
@@ -695,12 +682,9 @@ typedef struct gpk_rows {
   double* part_sum;    /* device: blocks words of scratch, for one launch at a time */
   int32_t* part_count; /* device: blocks words, 0 before the first launch and after each */
 } gpk_rows;
-/* Host: the row blocks of a CSR from its host row pointers (rows + 1);
- * writes blocks + 1 starts to blk (room for rows + 1; NULL only counts) and
- * returns the block count. */
-int32_t gpk_pdhg_row_blocks(const int32_t* ptr, int32_t rows, int32_t* blk);
-/* Host: those blocks with the long rows in parts, blocks + 1 entries (NULL only
- * counts); gpk_pdhg_row_plan_most: no matrix of rows and nnz has more blocks. */
+/* Host: the row blocks of a CSR from its host row pointers (rows + 1), blocks + 1
+ * entries (NULL only counts); returns the block count.
+ * gpk_pdhg_row_plan_most: no matrix of rows and nnz has more blocks. */
 int64_t gpk_pdhg_row_plan_most(int32_t rows, int32_t nnz);
 int32_t gpk_pdhg_row_plan(const int32_t* ptr, int32_t rows, gpk_row_block* out);
 /* `iterations` PDHG steps from z = (x, y): the PDHG point T(z) is

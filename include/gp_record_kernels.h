@@ -2,12 +2,11 @@
  * Internal C-ABI launchers for record maintenance and postsolve
  * (part of the same thin layer as gp_kernels.h).
  *
- *       append_removed_fixed_bound_records (reference gpu_presolve.cu:1005-1233)
  *   gpk_map_tape_indices
  *       append_globalized_postsolve_tape (reference gpu_presolve.cu:1363-1533)
  *   gpk_scatter / gpk_mark / gpk_restore_fixed
  *       reference gpu_postsolve.cu:143-190
- *   gpk_replay
+ *   gpk_pack_records / gpk_replay_list / gpk_replay_levels
  *       _kernel_replay_postsolve_tape (reference gpu_postsolve.cu:605-1046)
  *   gpk_protect_columns / gpk_project_duals
  *       reference gpu_postsolve.cu:1370-1435

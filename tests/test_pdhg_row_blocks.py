@@ -1,8 +1,9 @@
-"""Host side of the solver's row kernels (CPU): gpk_pdhg_row_blocks, the
-partition of a CSR's rows into the workgroup blocks the device kernels
-assume -- contiguous, covering every row once, a row of more than
-GPK_PDHG_LONG_ROW entries alone in its block, and any block of several rows
-within 256 rows and GPK_PDHG_ENTRY_BUDGET entries."""
+"""Host side of the solver's row kernels (CPU): gpk_pdhg_row_plan's partition
+of a CSR's rows into the workgroup blocks the device kernels assume --
+contiguous, covering every row once, a row of more than GPK_PDHG_LONG_ROW
+entries alone (in one block or, in parts, in several that follow each other),
+and any block of several rows within 256 rows and GPK_PDHG_ENTRY_BUDGET
+entries."""
 import ctypes as C
 import os
 
@@ -17,15 +18,18 @@ LONG_ROW, BUDGET = 256, 2048
 
 
 def _blocks(ptr):
+    """The first rows of the plan's blocks (a row's parts as one), and the end."""
     L = C.CDLL(LIB)
-    L.gpk_pdhg_row_blocks.restype = C.c_int32
-    L.gpk_pdhg_row_blocks.argtypes = [C.c_void_p, C.c_int32, C.c_void_p]
+    L.gpk_pdhg_row_plan.restype = C.c_int32
+    L.gpk_pdhg_row_plan.argtypes = [C.c_void_p, C.c_int32, C.c_void_p]
     ptr = np.ascontiguousarray(ptr, np.int32)
     rows = len(ptr) - 1
-    blk = np.full(rows + 1, -1, np.int32)
-    nb = L.gpk_pdhg_row_blocks(ptr.ctypes.data, rows, blk.ctypes.data)
-    assert L.gpk_pdhg_row_blocks(ptr.ctypes.data, rows, None) == nb
-    return blk[:nb + 1]
+    nb = L.gpk_pdhg_row_plan(ptr.ctypes.data, rows, None)
+    out = np.full((nb + 1, 4), -7, np.int32)  # row, entry, part, parts
+    assert L.gpk_pdhg_row_plan(ptr.ctypes.data, rows, out.ctypes.data) == nb
+    parts = out[:, 2] > 0
+    assert np.all(out[parts, 0] == out[np.nonzero(parts)[0] - 1, 0])
+    return out[~parts, 0]
 
 
 def _check(ptr):

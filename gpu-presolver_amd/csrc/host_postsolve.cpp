@@ -181,30 +181,28 @@ Lines gather_lines(const int32_t* ptr, const int32_t* idx, int32_t lines_total, 
   return L;
 }
 
-// Levels that one workgroup replays in a run, as `count` parts from `first` on;
-// or one level in a launch of its own: its line slots [first, first + count) and
-// its simple slots [simple, simple + simples).
+// Levels [first, first + count) that one workgroup replays in a run; or one level
+// in a launch of its own: its line slots [first, first + count) and its simple
+// slots [simple, simple + simples).
 struct Segment {
   bool grid;
   int32_t first, count, simple, simples;
-  int32_t waves;  // of a run: the most that a part fills
-  bool lines;     // of a run: some record walks a line
+  int32_t line_waves, simple_waves;  // of a run: the most that a level fills
 };
 
 struct Schedule {
   std::vector<int32_t> line, simple;  // record indices, level by level (-1: an empty slot)
-  std::vector<gpk_replay_part> parts;
+  std::vector<gpk_replay_level> run;  // the levels of the runs
   std::vector<Segment> segs;
   int32_t levels = 0;
-  // Where its slots and parts begin among those of the plan.
-  int64_t line_at = 0, simple_at = 0, parts_at = 0;
+  // Where its slots and levels begin among those of the plan.
+  int64_t line_at = 0, simple_at = 0, run_at = 0;
 };
 
-// Levels of more records than these get a launch of their own: 2.5 to 3 us in a
-// graph where its neighbours have theirs too, 4.5 to 5 launched directly.  In a run
-// a level of up to 511 simple records takes 0.7 to 1 us, of 1,024 1.6, of 2,047
-// 3; of up to 64 line records 2.4, of 128 (in two parts) 4.8.
-constexpr int32_t kRunLines = GPK_REPLAY_WAVES * GPK_WAVE_LINES, kRunSimples = 2 * GPK_REPLAY_WAVES * 64;
+// Levels that fill more waves than a workgroup's get a launch of their own: 2.5 to
+// 3 us in a graph where its neighbours have theirs too, 4.5 to 5 launched
+// directly.  In a run a level of up to 511 simple records takes 0.7 to 1 us, of
+// 1,024 1.6; of up to 64 line records 2.2 to 2.4 (of 128, in two turns, 4.8).
 constexpr int32_t kTypes = 15;  // PostsolveReductionType
 constexpr int64_t kMostSlots = std::numeric_limits<int32_t>::max();
 
@@ -460,7 +458,7 @@ Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, VarLeve
   // a wave's line records begins a new wave (empty slots between).
   Schedule sch;
   sch.levels = levels;
-  sch.parts.reserve(static_cast<size_t>(levels) + 16);
+  sch.run.reserve(static_cast<size_t>(levels));
   // The slots of the next level, which has size[t] records of kind t; size[t] is
   // then where they begin.
   const auto add_level = [&](uint32_t kinds, int32_t* size) {
@@ -469,7 +467,8 @@ Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, VarLeve
     const int64_t line0 = static_cast<int64_t>(sch.line.size()), simple0 = static_cast<int64_t>(sch.simple.size());
     if (line0 + GPK_WAVE_LINES * (lines + kTypes) > kMostSlots || simple0 + simples > kMostSlots)
       throw std::runtime_error("postsolve_gpu: the tape's replay schedule has more slots than 32 bits count");
-    const bool grid = lines > kRunLines || simples > kRunSimples;
+    const int64_t simple_waves = (simples + 63) / 64;
+    bool grid = lines > GPK_REPLAY_WAVES * GPK_WAVE_LINES || simple_waves > GPK_REPLAY_WAVES;
     int64_t line_end = line0, simple_end = simple0;
     for (uint32_t u = kinds; u != 0; u &= u - 1) {
       const int t = __builtin_ctz(u);
@@ -481,26 +480,20 @@ Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, VarLeve
     sch.simple.resize(static_cast<size_t>(simple_end));
     const int32_t count = static_cast<int32_t>(line_end - line0);
     const int32_t first = static_cast<int32_t>(line0), sfirst = static_cast<int32_t>(simple0);
+    const int32_t lw = (count + GPK_WAVE_LINES - 1) / GPK_WAVE_LINES, sw = static_cast<int32_t>(simple_waves);
+    grid = grid || lw + sw > GPK_REPLAY_WAVES;  // empty slots of the padding included
     if (grid) {
-      sch.segs.push_back(Segment{true, first, count, sfirst, static_cast<int32_t>(simples), 0, false});
+      sch.segs.push_back(Segment{true, first, count, sfirst, static_cast<int32_t>(simples), 0, 0});
       return;
     }
-    if (sch.segs.empty() || sch.segs.back().grid)
-      sch.segs.push_back(Segment{false, static_cast<int32_t>(sch.parts.size()), 0, 0, 0, 1, false});
-    Segment& run = sch.segs.back();
-    run.lines |= count > 0;
-    int32_t at = 0, sat = 0, flags = GPK_PART_NEW_LEVEL;
-    while (at < count || sat < simples) {
-      const int32_t l = std::min<int32_t>(count - at, GPK_REPLAY_WAVES * GPK_WAVE_LINES);
-      const int32_t waves = (l + GPK_WAVE_LINES - 1) / GPK_WAVE_LINES;
-      const int32_t n = std::min<int32_t>(static_cast<int32_t>(simples) - sat, (GPK_REPLAY_WAVES - waves) * 64);
-      sch.parts.push_back(gpk_replay_part{first + at, l, sfirst + sat, (n << GPK_PART_SHIFT) | flags});
-      ++run.count;
-      run.waves = std::max(run.waves, waves + (n + 63) / 64);
-      at += l;
-      sat += n;
-      flags = 0;
-    }
+    if (sch.segs.empty() || sch.segs.back().grid ||
+        std::max(sch.segs.back().line_waves, lw) + std::max(sch.segs.back().simple_waves, sw) > GPK_REPLAY_WAVES)
+      sch.segs.push_back(Segment{false, static_cast<int32_t>(sch.run.size()), 0, 0, 0, 0, 0});
+    Segment& seg = sch.segs.back();
+    ++seg.count;
+    seg.line_waves = std::max(seg.line_waves, lw);
+    seg.simple_waves = std::max(seg.simple_waves, sw);
+    sch.run.push_back(gpk_replay_level{first, count, sfirst, static_cast<int32_t>(simples)});
   };
   const auto place = [&](int32_t k, int32_t* fill) {
     const int t = kind[k - lo];
@@ -543,28 +536,28 @@ Schedule level_schedule(const TapeScanner& scan, int32_t lo, int32_t hi, VarLeve
   return sch;
 }
 
-// The packets and parts of a plan's schedules.
+// The packets and run levels of a plan's schedules.
 struct DeviceSchedules {
   DBuf<int32_t> line, simple;
-  DBuf<gpk_replay_part> parts;
+  DBuf<gpk_replay_level> run;
 };
 // all: the primal pass's schedules, then the dual pass's.
 DeviceSchedules upload_schedules(const std::vector<Schedule*>& all, const gp_tape_dev& tape, const gp_orig_dev& orig,
                                  bool has_y) {
-  int64_t lines = 0, simples = 0, parts = 0, dual_line = 0;
+  int64_t lines = 0, simples = 0, run = 0, dual_line = 0;
   for (Schedule* s : all) {
     s->line_at = dual_line = lines;
     s->simple_at = simples;
-    s->parts_at = parts;
+    s->run_at = run;
     lines += static_cast<int64_t>(s->line.size());
     simples += static_cast<int64_t>(s->simple.size());
-    parts += static_cast<int64_t>(s->parts.size());
+    run += static_cast<int64_t>(s->run.size());
   }
-  if (lines > kMostSlots || simples > kMostSlots || parts > kMostSlots)
+  if (lines > kMostSlots || simples > kMostSlots || run > kMostSlots)
     throw std::runtime_error("postsolve_gpu: the tape's replay schedules have more slots than 32 bits count");
   DeviceSchedules d;
   DBuf<int32_t> line_records(lines), simple_records(simples);
-  d.parts.alloc(parts);
+  d.run.alloc(run);
   d.line.alloc(lines * GPK_PACKET_WORDS);
   d.simple.alloc(simples * GPK_SIMPLE_WORDS);
   amd::Ctx& c = ctx();
@@ -574,7 +567,7 @@ DeviceSchedules upload_schedules(const std::vector<Schedule*>& all, const gp_tap
                 "replay schedule upload");
     c.to_device(simple_records.get() + s->simple_at, s->simple.data(), static_cast<int64_t>(s->simple.size()),
                 "replay schedule upload");
-    c.to_device(d.parts.get() + s->parts_at, s->parts.data(), static_cast<int64_t>(s->parts.size()),
+    c.to_device(d.run.get() + s->run_at, s->run.data(), static_cast<int64_t>(s->run.size()),
                 "replay schedule upload");
   }
   c.end_copy_group("replay schedule upload");
@@ -602,8 +595,8 @@ void enqueue_schedule(const Schedule& sch, const DeviceSchedules& dev, const gp_
                             simple + static_cast<int64_t>(g.simple) * GPK_SIMPLE_WORDS, g.simples, dual, tol, s),
             what);
     else
-      check(gpk_replay_levels(tape, orig, x, y, z, zret, line, simple, dev.parts.get() + sch.parts_at + g.first,
-                              g.count, g.waves, g.lines ? 1 : 0, dual, tol, s),
+      check(gpk_replay_levels(tape, orig, x, y, z, zret, line, simple, dev.run.get() + sch.run_at + g.first, g.count,
+                              g.line_waves, g.simple_waves, dual, tol, s),
             what);
   }
 }

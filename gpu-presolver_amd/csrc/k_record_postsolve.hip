@@ -697,109 +697,98 @@ __global__ void __launch_bounds__(kBlock)
   replay_line<kDual>(T, O, x, y, z, zret, h, rv, ln, r, tol);
 }
 
-// What a wave holds of a part of a level (gpk_replay_part): its records'
-// packets, and later their values and entries.
-struct PartWords {
-  int4 a, b;  // simple: the packet; line: a.x the lane's word
-};
-struct PartOperands {
-  RecEntries r;
-  SimpleVals s;
-};
 constexpr int kLevelBlock = 64 * GPK_REPLAY_WAVES;
 constexpr int kWaveLines = 64 / kRecLanes;
 static_assert(GPK_WAVE_LINES == kWaveLines, "a wave's line records");
 
-// A run of small levels in one workgroup, which meets at a barrier between
-// levels; it has as many waves as its largest level fills (a chain of single
-// records: one, 0.7 us a level against 1.1 with sixteen).  All waves run on one
-// CU, so the barrier's workgroup-scope fence makes one level's global stores
-// visible to the next level's loads.  A part's first waves take its line records,
-// the next ones the others; the parts of a level follow each other without
-// meeting.  kLine: the run has line records.
-// A wave has the packets of its records two parts ahead and their lines and
-// values one part ahead on their way, so that a level waits only for its x, y, z
-// and zret, and for its stores at the barrier.  Bound by that chain: 1,207 dual
-// levels, most of about 31 records, take 3.2 ms (2.6 us each; 11.4 ms with a
-// lane per record and each chain in its turn, 4.2 with a record's six chains
-// five levels ahead in place of packets).  Reading x, y, z and zret once a level
-// ahead, to have them in the CU's cache, cost 0.4 ms more.
-template <bool kDual, bool kLine>
+// The line records of a run of levels, by the workgroup's first waves: those of a
+// level, then the barrier.  A wave has the packets of its records two levels
+// ahead and their lines and values one level ahead on their way, so that a level
+// waits only for its x, y, z and zret, and for its stores at the barrier.  Bound
+// by that chain: 1,106 dual levels, most of about 31 records, take 2.7 ms (2.5 us
+// each; 11.4 ms for 1,207 with a lane per record and each chain in its turn, 4.2
+// with a record's six chains five levels ahead in place of packets).  Reading x,
+// y, z and zret once a level ahead, to have them in the CU's cache, cost 0.4 ms
+// more.  The levels' slots come by vector loads: a scalar one would be waited
+// for together with the newest of its kind (2.28 us a level against 2.35).
+template <bool kDual>
+__device__ __forceinline__ void replay_level_lines(const gp_tape_dev& T, const gp_orig_dev& O, double* x, double* y,
+                                                   double* z, uint8_t* zret, const int32_t* __restrict__ line,
+                                                   const gpk_replay_level* __restrict__ levels, int32_t nlevels,
+                                                   double tol) {
+  const int32_t slot = static_cast<int32_t>(threadIdx.x) / kRecLanes;
+  const int t = static_cast<int>(threadIdx.x & (kRecLanes - 1));
+  int32_t zero = 0;
+  asm("" : "+v"(zero));
+  const auto level = [&](int32_t l) {
+    return l < nlevels ? reinterpret_cast<const int2*>(levels)[2 * (l + zero)] : make_int2(0, 0);
+  };
+  const auto packet = [&](int2 d) {
+    return slot < d.y ? line[(static_cast<int64_t>(d.x) + slot) * GPK_PACKET_WORDS + t] : packet_none(t);
+  };
+  int2 d2 = level(2);
+  int32_t p0 = packet(level(0)), p1 = packet(level(1));
+  RecEntries r0 = load_entries(T, O, packet_head(p0), packet_line(p0), t);
+#pragma unroll 1
+  for (int32_t l = 0; l < nlevels; ++l) {
+    const int2 d3 = level(l + 3);
+    const int32_t p2 = packet(d2);
+    const RecEntries r1 = load_entries(T, O, packet_head(p1), packet_line(p1), t);
+    const RecVars rv{row_lane<PK_W0>(p0), row_lane<PK_W0 + 1>(p0), row_lane<PK_W0 + 2>(p0)};
+    replay_line<kDual>(T, O, x, y, z, zret, packet_head(p0), rv, packet_line(p0), r0, tol);
+    __syncthreads();
+    p0 = p1;
+    p1 = p2;
+    r0 = r1;
+    d2 = d3;
+  }
+}
+
+// The other records, by the waves from `first` on, in the same way.
+template <bool kDual>
+__device__ __forceinline__ void replay_level_simples(const gp_tape_dev& T, double* x, double* y, double* z,
+                                                     uint8_t* zret, const int32_t* __restrict__ simple,
+                                                     const gpk_replay_level* __restrict__ levels, int32_t nlevels,
+                                                     int32_t first, double tol) {
+  const int32_t slot = static_cast<int32_t>(threadIdx.x) - 64 * first;
+  const auto level = [&](int32_t l) {
+    return l < nlevels ? reinterpret_cast<const int2*>(levels)[2 * l + 1] : make_int2(0, 0);
+  };
+  const auto packet = [&](int2 d) {
+    return slot < d.y ? simple_packet(simple, static_cast<int64_t>(d.x) + slot) : simple_none();
+  };
+  int2 d2 = level(2);
+  SimpleRec h0 = packet(level(0)), h1 = packet(level(1));
+  SimpleVals v0 = simple_values(T, h0);
+#pragma unroll 1
+  for (int32_t l = 0; l < nlevels; ++l) {
+    const int2 d3 = level(l + 3);
+    const SimpleReads in = simple_reads<kDual>(h0, x, y, z);  // on their way before the loads ahead
+    const SimpleRec h2 = packet(d2);
+    const SimpleVals v1 = simple_values(T, h1);
+    replay_simple<kDual>(T, x, y, z, zret, h0, v0, in, tol);
+    __syncthreads();
+    h0 = h1;
+    h1 = h2;
+    v0 = v1;
+    d2 = d3;
+  }
+}
+
+// A run of small levels in one workgroup, which meets at a barrier after each.
+// Its first waves replay the line records, the others the rest, as many of each
+// as the run's largest level fills (a chain of single records: one wave, 0.7 us a
+// level against 1.1 with sixteen).  All waves run on one CU, so the barrier's
+// workgroup-scope fence makes one level's global stores visible to the next
+// level's loads.  Both kinds of wave come to the barrier once a level.
+template <bool kDual>
 __global__ void __launch_bounds__(kLevelBlock)
     k_replay_levels(gp_tape_dev T, gp_orig_dev O, double* x, double* y, double* z, uint8_t* zret,
                     const int32_t* __restrict__ line, const int32_t* __restrict__ simple,
-                    const gpk_replay_part* __restrict__ parts, int32_t nparts, double tol) {
+                    const gpk_replay_level* __restrict__ levels, int32_t nlevels, int32_t line_waves, double tol) {
   const int32_t wave = __builtin_amdgcn_readfirstlane(static_cast<int32_t>(threadIdx.x) >> 6);
-  const int32_t lane = static_cast<int32_t>(threadIdx.x) & 63;
-  const int t = lane & (kRecLanes - 1);
-  // A part is loaded a turn before it is looked at.  With line records by a vector
-  // load: a scalar one would be waited for together with the newest of its kind
-  // (a level of one line record 2.28 us against 2.35; without line records the
-  // scalar load is the better one, 1.18 against 1.22).
-  int32_t zero = 0;
-  if (kLine) asm("" : "+v"(zero));
-  const auto part = [&](int32_t p) {
-    const int4 v = p < nparts ? reinterpret_cast<const int4*>(parts)[p + zero] : make_int4(0, 0, 0, 0);
-    return gpk_replay_part{v.x, v.y, v.z, v.w};
-  };
-  const auto uniform = [](const gpk_replay_part& d) {
-    return gpk_replay_part{__builtin_amdgcn_readfirstlane(d.line), __builtin_amdgcn_readfirstlane(d.lines),
-                           __builtin_amdgcn_readfirstlane(d.simple), __builtin_amdgcn_readfirstlane(d.simples)};
-  };
-  const auto line_waves = [](const gpk_replay_part& d) { return kLine ? (d.lines + kWaveLines - 1) / kWaveLines : 0; };
-  const auto takes_line = [&](const gpk_replay_part& d) { return kLine && wave < line_waves(d); };
-  const auto packets = [&](const gpk_replay_part& d) {
-    PartWords w;
-    if (takes_line(d)) {
-      const int32_t slot = wave * kWaveLines + lane / kRecLanes;
-      w.a.x = slot < d.lines ? line[(static_cast<int64_t>(d.line) + slot) * GPK_PACKET_WORDS + t] : packet_none(t);
-    } else {
-      const int32_t slot = (wave - line_waves(d)) * 64 + lane;
-      const SimpleRec h = slot < d.simples >> GPK_PART_SHIFT
-                              ? simple_packet(simple, static_cast<int64_t>(d.simple) + slot) : simple_none();
-      w.a = make_int4(h.type, h.i0, h.i1, h.v0);
-      w.b = make_int4(h.v1, h.w0, h.w1, h.w2);
-    }
-    return w;
-  };
-  const auto simple_of = [](const PartWords& w) {
-    return SimpleRec{w.a.x, w.a.y, w.a.z, w.a.w, w.b.x, w.b.y, w.b.z, w.b.w};
-  };
-  const auto operands = [&](const gpk_replay_part& d, const PartWords& w) {
-    PartOperands o;
-    if (takes_line(d)) o.r = load_entries(T, O, packet_head(w.a.x), packet_line(w.a.x), t);
-    else o.s = simple_values(T, simple_of(w));
-    return o;
-  };
-  gpk_replay_part d0 = uniform(part(0)), d1 = uniform(part(1)), ahead = part(2);
-  PartWords w0 = packets(d0), w1 = packets(d1);
-  PartOperands o0 = operands(d0, w0);
-#pragma unroll 1
-  for (int32_t p = 0; p < nparts; ++p) {
-    const gpk_replay_part d2 = uniform(ahead), next = part(p + 3);
-    PartWords w2;
-    PartOperands o1;
-    if (takes_line(d0)) {
-      w2 = packets(d2);
-      o1 = operands(d1, w1);
-      const int32_t w = w0.a.x;
-      const RecVars rv{row_lane<PK_W0>(w), row_lane<PK_W0 + 1>(w), row_lane<PK_W0 + 2>(w)};
-      replay_line<kDual>(T, O, x, y, z, zret, packet_head(w), rv, packet_line(w), o0.r, tol);
-    } else {
-      const SimpleRec h = simple_of(w0);
-      const SimpleReads in = simple_reads<kDual>(h, x, y, z);  // on their way before the loads ahead
-      w2 = packets(d2);
-      o1 = operands(d1, w1);
-      replay_simple<kDual>(T, x, y, z, zret, h, o0.s, in, tol);
-    }
-    if (d1.simples & GPK_PART_NEW_LEVEL) __syncthreads();
-    d0 = d1;
-    d1 = d2;
-    ahead = next;
-    w0 = w1;
-    w1 = w2;
-    o0 = o1;
-  }
+  if (wave < line_waves) replay_level_lines<kDual>(T, O, x, y, z, zret, line, levels, nlevels, tol);
+  else replay_level_simples<kDual>(T, x, y, z, zret, simple, levels, nlevels, line_waves, tol);
 }
 
 // gpu_postsolve.cu:162-180, 568-603: z_j from r = c_j - (A^T y)_j and the
@@ -989,14 +978,15 @@ hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double
   return hipGetLastError();
 }
 hipError_t gpk_replay_levels(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                             const int32_t* line, const int32_t* simple, const gpk_replay_part* parts, int32_t nparts,
-                             int32_t waves, int32_t has_lines, int32_t dual, double tol, hipStream_t stream) {
-  if (nparts <= 0) return hipSuccess;
-  if (waves < 1 || waves > GPK_REPLAY_WAVES) return hipErrorInvalidValue;
-  const auto run = dual ? (has_lines ? k_replay_levels<true, true> : k_replay_levels<true, false>)
-                        : (has_lines ? k_replay_levels<false, true> : k_replay_levels<false, false>);
-  hipLaunchKernelGGL(run, dim3(1), dim3(64 * waves), 0, stream, tape, orig, x, y, z, zret, line, simple, parts, nparts,
-                     tol);
+                             const int32_t* line, const int32_t* simple, const gpk_replay_level* levels,
+                             int32_t nlevels, int32_t line_waves, int32_t simple_waves, int32_t dual, double tol,
+                             hipStream_t stream) {
+  if (nlevels <= 0) return hipSuccess;
+  const int32_t waves = line_waves + simple_waves;
+  if (line_waves < 0 || simple_waves < 0 || waves < 1 || waves > GPK_REPLAY_WAVES) return hipErrorInvalidValue;
+  const auto run = dual ? k_replay_levels<true> : k_replay_levels<false>;
+  hipLaunchKernelGGL(run, dim3(1), dim3(64 * waves), 0, stream, tape, orig, x, y, z, zret, line, simple, levels,
+                     nlevels, line_waves, tol);
   return hipGetLastError();
 }
 hipError_t gpk_seg_lengths(const int32_t* ptr, const int32_t* list, int32_t count, int32_t* len, hipStream_t stream) {

@@ -59,21 +59,18 @@ hipError_t gpk_restore_fixed(const int32_t* idx, const double* val, int32_t coun
  * packets of all slots (line_records / simple_records: the slots' records, -1 an
  * empty slot; line slots from dual_line on belong to the dual pass): places in
  * the tape and in the original model's row pointers, no values.
- * gpk_replay_list: the records of one level.  gpk_replay_levels: consecutive
- * levels in one workgroup of `waves` waves (up to GPK_REPLAY_WAVES), given as
- * parts: line records `line` .. line + lines - 1, GPK_WAVE_LINES to a wave, and
- * (simples >> GPK_PART_SHIFT) of the others from `simple` on, 64 to a wave, as many
- * together as the waves hold; GPK_PART_NEW_LEVEL in simples where the part begins
- * a level.  has_lines: some part has line records. */
+ * gpk_replay_list: the records of one level.  gpk_replay_levels: nlevels
+ * consecutive levels in one workgroup of line_waves + simple_waves waves (up to
+ * GPK_REPLAY_WAVES); a level has the line records `line` .. line + lines - 1, at most
+ * GPK_WAVE_LINES for each of the former, and the others `simple` .. simple +
+ * simples - 1, at most 64 for each of the latter. */
 #define GPK_REPLAY_WAVES 16
 #define GPK_WAVE_LINES 4
 #define GPK_PACKET_WORDS 16
 #define GPK_SIMPLE_WORDS 8
-#define GPK_PART_NEW_LEVEL 1
-#define GPK_PART_SHIFT 1
-typedef struct __attribute__((aligned(16))) gpk_replay_part {
+typedef struct __attribute__((aligned(16))) gpk_replay_level {
   int32_t line, lines, simple, simples;
-} gpk_replay_part;
+} gpk_replay_level;
 typedef struct gpk_replay_slots {
   int32_t line_slots, simple_slots;
   const int32_t* line_records;
@@ -94,8 +91,9 @@ hipError_t gpk_replay_list(gp_tape_dev tape, gp_orig_dev orig, double* x, double
                            const int32_t* line, int32_t lines, const int32_t* simple, int32_t simples, int32_t dual,
                            double tol, hipStream_t stream);
 hipError_t gpk_replay_levels(gp_tape_dev tape, gp_orig_dev orig, double* x, double* y, double* z, uint8_t* zret,
-                             const int32_t* line, const int32_t* simple, const gpk_replay_part* parts, int32_t nparts,
-                             int32_t waves, int32_t has_lines, int32_t dual, double tol, hipStream_t stream);
+                             const int32_t* line, const int32_t* simple, const gpk_replay_level* levels,
+                             int32_t nlevels, int32_t line_waves, int32_t simple_waves, int32_t dual, double tol,
+                             hipStream_t stream);
 /* len[i] = ptr[list[i] + 1] - ptr[list[i]]; gpk_seg_copy packs line
  * list[i]'s idx entries at out + off[i]. */
 hipError_t gpk_seg_lengths(const int32_t* ptr, const int32_t* list, int32_t count, int32_t* len, hipStream_t stream);

@@ -1,7 +1,7 @@
 """Tapes written by hand for the postsolve replay, against the oracle's
 record-by-record replay, bit for bit: lines around the 16 and 32 entries that
-are loaded ahead, every record type in one level, levels around a wave's, a
-part's and a workgroup's records of either kind (those that walk a line and the
+are loaded ahead, every record type in one level, levels around a wave's and a
+workgroup's records of either kind (those that walk a line and the
 others) and around the sizes that take a launch of their own, chains of single
 records, and records without rows or an original model."""
 import numpy as np
@@ -103,7 +103,7 @@ def test_random_tapes(count, with_original):
 
 
 def test_levels_of_simple_records():
-    """A wave, a part, two parts, a launch of their own; grid and run in turn."""
+    """A wave, the workgroup, a launch of their own; launches and runs in turn."""
     m = 2100
     lp = original(m, 900, 51)
     rng = np.random.default_rng(52)

@@ -527,7 +527,7 @@ def activity_traffic():
 def transpose_traffic():
     """HBM bytes of one transpose from the committed PMC summary, or None."""
     parts = [profiled_traffic(k) for k in ("k_tb_hist", "k_scan_tiles<int>", "k_scan_tile_sums", "k_scan_down<int>",
-                                           "k_tb_largest", "k_tb_partition", "k_tb_columns")]
+                                           "k_tb_pieces", "k_tb_partition", "k_tb_piece_counts", "k_tb_columns")]
     return None if any(p is None for p in parts) else sum(parts)
 
 

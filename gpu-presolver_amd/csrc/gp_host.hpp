@@ -414,6 +414,22 @@ struct JobMode {
 };
 JobMode& job_mode();
 
+// Waits for the whole device, outside every graph capture of the library.  The
+// runtime refuses a device-wide wait while any thread captures, and the refused
+// wait spoils that capture as well.
+void device_sync(const char* what);
+
+// Held from hipStreamBeginCapture to hipStreamEndCapture: a device_sync of
+// another thread waits for its end, and its start for those under way.  The
+// holder neither calls device_sync nor waits for a thread that does.
+class CaptureSection {
+ public:
+  CaptureSection();
+  ~CaptureSection();
+  CaptureSection(const CaptureSection&) = delete;
+  CaptureSection& operator=(const CaptureSection&) = delete;
+};
+
 // Serving runtime (host_serve.cpp).
 class Server;
 Server* server_create(const presolve::PresolveParams& prm, const ::gp_serve_config& cfg);

@@ -389,7 +389,7 @@ gp_status gp_row_activity(const gp_csr* A, const double* l, const double* u, dou
       return;
     }
     require_device();
-    amd::check(hipDeviceSynchronize(), "entry synchronize");
+    amd::device_sync("entry synchronize");
     compute_row_activity_summary(row_min_fin, row_max_fin, row_min_neg_inf_count, row_max_pos_inf_count, to_csr(*A),
                                  l, u, zero_tol);
     amd::ctx().sync("gp_row_activity");
@@ -431,7 +431,7 @@ gp_status gp_col_max_abs(const gp_csr* AT, double* col_max_abs, void* stream) {
       return;
     }
     require_device();
-    amd::check(hipDeviceSynchronize(), "entry synchronize");
+    amd::device_sync("entry synchronize");
     compute_col_max_abs(col_max_abs, to_csr(*AT));
     amd::ctx().sync("gp_col_max_abs");
   });
@@ -443,7 +443,7 @@ gp_status gp_compact_csr(const gp_csr* A, const uint8_t* keep_row, const uint8_t
     check_csr(*A, "A");
     require((A->rows == 0 || keep_row) && (A->cols == 0 || keep_col), "null keep mask");
     require_device();
-    amd::check(hipDeviceSynchronize(), "entry synchronize");
+    amd::device_sync("entry synchronize");
     const DeviceCsrMatrix r = amd::compact_csr(to_csr(*A), keep_row, keep_col);
     amd::ctx().sync("gp_compact_csr");
     *out = from_csr(r);
@@ -455,7 +455,7 @@ gp_status gp_transpose_csr(const gp_csr* A, gp_csr* out) {
     require(A != nullptr && out != nullptr, "null argument");
     check_csr(*A, "A");
     require_device();
-    amd::check(hipDeviceSynchronize(), "entry synchronize");
+    amd::device_sync("entry synchronize");
     const DeviceCsrMatrix r = amd::transpose_csr(to_csr(*A));
     amd::ctx().sync("gp_transpose_csr");
     *out = from_csr(r);
@@ -469,7 +469,7 @@ gp_status gp_rule_apply(int32_t rule_id, gp_plan_view* plan, const gp_lp* lp, co
     require(rule_id >= GP_RULE_EMPTY_ROWS && rule_id <= GP_RULE_REDUNDANT_BOUNDS, "unknown rule id");
     const LPInfoGpu L = to_lp(*lp);
     require_device();
-    amd::check(hipDeviceSynchronize(), "entry synchronize");
+    amd::device_sync("entry synchronize");
     PresolvePlanGpu P;
     P.keep_row_mask = plan->keep_row;
     P.keep_col_mask = plan->keep_col;
@@ -674,7 +674,7 @@ gp_status gp_serve_trace(const gp_lp* lps, int32_t lp_count, const int32_t* lp_o
       if (arrival_s) require(k == 0 || arrival_s[k] >= arrival_s[k - 1], "arrival times must be non-decreasing");
     }
     require_device();
-    amd::check(hipDeviceSynchronize(), "gp_serve_trace entry synchronize");
+    amd::device_sync("gp_serve_trace entry synchronize");
     std::unique_ptr<amd::Server, void (*)(amd::Server*)> srv(amd::server_create(to_params(params), *config),
                                                              amd::server_destroy);
     for (int32_t k = 0; k < jobs; ++k) {
@@ -807,7 +807,7 @@ gp_status gp_synthetic_point(uint64_t seed, const gp_lp* lp, double* x, double* 
     const LPInfoGpu L = to_lp(*lp);
     require((L.A.cols == 0 || (x && z)) && (L.A.rows == 0 || y), "null output vector");
     require_device();
-    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_synthetic_point entry synchronize");
+    if (amd::job_mode().device_sync_on_entry) amd::device_sync("gp_synthetic_point entry synchronize");
     amd::Ctx& c = amd::ctx();
     amd::check(gpk_synthetic_point(seed, L.A.cols, L.A.rows, L.l, L.u, x, y, z, c.stream()), "synthetic point");
     c.sync("synthetic point");
@@ -819,7 +819,7 @@ gp_status gp_checksum(const double* x, int32_t n, const double* y, int32_t m, co
     require(out != nullptr && n >= 0 && m >= 0, "invalid argument");
     require((n == 0 || (x && z)) && (m == 0 || y), "null vector");
     require_device();
-    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_checksum entry synchronize");
+    if (amd::job_mode().device_sync_on_entry) amd::device_sync("gp_checksum entry synchronize");
     *out = amd::checksum_xyz(x, n, y, m, z);
   });
 }
@@ -903,7 +903,7 @@ gp_status gp_postsolve(const gp_record_view* record, const double* x_red, const 
     if (original != nullptr) orig = to_lp(*original);
     require_device();
     amd::PostsolvePlan::validate(rec, original ? &orig : nullptr);
-    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_postsolve entry synchronize");
+    if (amd::job_mode().device_sync_on_entry) amd::device_sync("gp_postsolve entry synchronize");
     // Straight into the caller's outputs.
     amd::PostsolvePlan plan(rec, original ? &orig : nullptr);
     plan.enqueue(x_red, y_red, z_red, x_org, y_org, z_org);
@@ -942,18 +942,22 @@ bool capture_postsolve(gp_postsolve_plan& p) {
   p.out_z.alloc(plan.n0());
   hipStream_t s = amd::ctx().stream();
   amd::ctx().sync("postsolve graph capture");  // nothing of this stream's earlier work enters the graph
-  if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) {
-    (void)hipGetLastError();
-    return false;
-  }
   bool ok = true;
-  try {
-    p.plan->enqueue(p.in_x, p.in_y, p.in_z, p.out_x, p.out_y, p.out_z);
-  } catch (...) {
-    ok = false;
-  }
   hipGraph_t g = nullptr;
-  const hipError_t end = hipStreamEndCapture(s, &g);
+  hipError_t end;
+  {
+    amd::CaptureSection section;
+    if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    try {
+      p.plan->enqueue(p.in_x, p.in_y, p.in_z, p.out_x, p.out_y, p.out_z);
+    } catch (...) {
+      ok = false;
+    }
+    end = hipStreamEndCapture(s, &g);
+  }
   if (!ok || end != hipSuccess || g == nullptr) {
     if (g) (void)hipGraphDestroy(g);
     (void)hipGetLastError();
@@ -987,7 +991,7 @@ gp_status gp_postsolve_prepare(const gp_record_view* record, const gp_lp* origin
     p->use_graph = use_graph != 0;
     require_device();
     amd::PostsolvePlan::validate(p->record, p->has_orig ? &p->orig : nullptr);
-    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_postsolve_prepare entry");
+    if (amd::job_mode().device_sync_on_entry) amd::device_sync("gp_postsolve_prepare entry");
     p->plan = std::make_unique<amd::PostsolvePlan>(p->record, p->has_orig ? &p->orig : nullptr);
     amd::ctx().sync("gp_postsolve_prepare");
     *out = p.release();
@@ -1002,7 +1006,7 @@ gp_status gp_postsolve_plan_run(gp_postsolve_plan* p, const double* x_red, const
     require(plan.n0() == 0 || (x_org && z_org), "null x_org/z_org");
     require(plan.m0() == 0 || y_org, "null y_org");
     require_device();
-    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_postsolve_plan_run entry");
+    if (amd::job_mode().device_sync_on_entry) amd::device_sync("gp_postsolve_plan_run entry");
     const bool all_inputs = x_red && (y_red || plan.m1() == 0) && z_red;
     if (p->use_graph && all_inputs && !p->graph_failed && p->exec == nullptr && !capture_postsolve(*p))
       p->graph_failed = true;
@@ -1106,7 +1110,7 @@ gp_status gp_pdhg_solve(const gp_lp* lp, const gp_pdhg_params* params, double* x
     require(L.A.cols == 0 || (L.c && L.l && L.u), "null c/l/u");
     require(L.A.rows == 0 || (L.AL && L.AU), "null AL/AU");
     require_device();
-    if (amd::job_mode().device_sync_on_entry) amd::check(hipDeviceSynchronize(), "gp_pdhg_solve entry synchronize");
+    if (amd::job_mode().device_sync_on_entry) amd::device_sync("gp_pdhg_solve entry synchronize");
     const amd::PdhgReport r = amd::pdhg_solve(L, pdhg_options(params), x, y, z);
     amd::ctx().sync("gp_pdhg_solve");
     *out = pdhg_result(r);

@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <condition_variable>
 #include <cstring>
 #include <limits>
 #include <memory>
@@ -271,6 +272,54 @@ JobMode& job_mode() {
   thread_local JobMode mode;
   return mode;
 }
+
+namespace {
+
+// Device-wide waits go on beside each other and captures beside each other, but
+// not the one beside the other; who comes first goes first, so neither kind is
+// kept out for good.
+class CaptureGate {
+ public:
+  void enter(int kind) {
+    std::unique_lock<std::mutex> lk(mu_);
+    const uint64_t ticket = next_++;
+    cv_.wait(lk, [&] { return ticket == turn_ && inside_[1 - kind] == 0; });
+    ++turn_;
+    ++inside_[kind];
+    cv_.notify_all();
+  }
+  void leave(int kind) {
+    std::lock_guard<std::mutex> lk(mu_);
+    --inside_[kind];
+    cv_.notify_all();
+  }
+
+ private:
+  std::mutex mu_;
+  std::condition_variable cv_;
+  uint64_t next_ = 0, turn_ = 0;
+  int inside_[2] = {0, 0};
+};
+
+constexpr int kWait = 0, kCapture = 1;
+
+// Never destroyed: a thread may still be inside when the process ends.
+CaptureGate& capture_gate() {
+  static CaptureGate* g = new CaptureGate;
+  return *g;
+}
+
+}  // namespace
+
+void device_sync(const char* what) {
+  capture_gate().enter(kWait);
+  const hipError_t st = hipDeviceSynchronize();
+  capture_gate().leave(kWait);
+  check(st, what);
+}
+
+CaptureSection::CaptureSection() { capture_gate().enter(kCapture); }
+CaptureSection::~CaptureSection() { capture_gate().leave(kCapture); }
 
 ScopedCtx::ScopedCtx(Ctx& c) : prev_(t_current) { t_current = &c; }
 ScopedCtx::~ScopedCtx() { t_current = prev_; }

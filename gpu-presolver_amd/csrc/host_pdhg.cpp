@@ -189,10 +189,14 @@ PdhgReport pdhg_solve(const LPInfoGpu& lp, const PdhgOptions& opt, double* x_out
   GraphExec graph;
   if (opt.use_graph) {
     cx.sync("pdhg graph capture");
-    check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "pdhg graph capture");
-    const hipError_t launched = enqueue_period();
     hipGraph_t g = nullptr;
-    const hipError_t end = hipStreamEndCapture(s, &g);
+    hipError_t launched, end;
+    {
+      CaptureSection section;
+      check(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal), "pdhg graph capture");
+      launched = enqueue_period();
+      end = hipStreamEndCapture(s, &g);
+    }
     if ((launched != hipSuccess || end != hipSuccess) && g != nullptr) (void)hipGraphDestroy(g);
     check(launched, "pdhg graph capture");
     check(end, "pdhg graph capture");

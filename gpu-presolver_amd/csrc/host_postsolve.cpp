@@ -954,14 +954,14 @@ void postsolve_restore_structural_primal_gpu(double* x_org, const std::vector<St
                                              const double* original_l) {
   amd::AbandonOnThrow abandon_guard;
   if (!recoveries.empty()) {
-    check(hipDeviceSynchronize(), "structural primal recovery entry synchronize");
+    amd::device_sync("structural primal recovery entry synchronize");
     for (auto it = recoveries.rbegin(); it != recoveries.rend(); ++it) {
       amd::RecoveryStep step(*it);
       step.enqueue(x_org, original_l, ctx().stream());
       ctx().sync("structural primal recovery");
     }
   }
-  check(hipDeviceSynchronize(), "postsolve_restore_structural_primal_gpu synchronize");
+  amd::device_sync("postsolve_restore_structural_primal_gpu synchronize");
 }
 
 GpuPostsolveResult postsolve_gpu(double* x_red, double* y_red, double* z_red, const PresolveRecordGpu& record,
@@ -973,7 +973,7 @@ GpuPostsolveResult postsolve_gpu(double* x_red, double* y_red, double* z_red, co
                                  const LPInfoGpu* original_model, const double* original_l) {
   amd::AbandonOnThrow abandon_guard;
   amd::PostsolvePlan::validate(record, original_model);
-  if (amd::job_mode().device_sync_on_entry) check(hipDeviceSynchronize(), "postsolve entry synchronize");
+  if (amd::job_mode().device_sync_on_entry) amd::device_sync("postsolve entry synchronize");
   auto& c = ctx();
   hipStream_t s = c.stream();
   GpuPostsolveResult res;

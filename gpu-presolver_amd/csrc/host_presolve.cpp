@@ -667,7 +667,7 @@ GpuPresolveSummary run_impl(const LPInfoGpu& lp, const PresolveParams& prm, bool
   amd::AbandonOnThrow abandon_guard;
   DeferObjectiveSums defer_sums;
   validate_lp(lp);
-  if (amd::job_mode().device_sync_on_entry) check(hipDeviceSynchronize(), "presolve entry synchronize");
+  if (amd::job_mode().device_sync_on_entry) amd::device_sync("presolve entry synchronize");
   amd::check_lp_arrays(lp, "presolve input");
   GpuPresolveSummary res;
   res.original_rows = lp.A.rows;

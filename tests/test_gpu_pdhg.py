@@ -10,6 +10,7 @@ from the solver's relative KKT tolerance tol: the reported residuals are
 of the optimum (relative), and the largest row or bound violation is within
 tol * (1 + ||b||)."""
 import ctypes as C
+import threading
 
 import numpy as np
 import pytest
@@ -245,3 +246,62 @@ def test_pipeline_on_an_infeasible_lp():
                                               gp_ffi.pdhg_params())
     assert res["has_infeasible"] == 1 and res["solve"]["status"] == -1
     assert not px.numpy().any() and not py.numpy().any() and not pz.numpy().any()
+
+
+def test_calls_in_several_threads():
+    """A call's wait for the device on entry and another thread's capture (a
+    solve's check period, a prepared postsolve's first run) leave each other
+    alone.  The threads only make the library's calls: the runtime refuses a copy
+    on the legacy stream while any thread captures."""
+    lps = [gp_ffi.DeviceLp(lp_synth.generate(200 + 20 * k, 300 + 30 * k, seed=31 + k, mean_row_len=4.0)) for k in range(3)]
+    prm = gp_ffi.pdhg_params(tol=1e-12, max_iters=256)
+    presolve = gp_ffi.params(enable_structure_specific_rules=0)
+    lp = lp_synth.config0(seed=0)
+    _, rec, red = gp_ffi.presolve(lp, presolve, True)
+    point = [gp_ffi.DeviceArray(v) for v in lp_synth.reduced_solution(1, red["m"], red["n"], red["l"], red["u"])]
+    dlp = gp_ffi.DeviceLp(lp)
+    rounds = 6
+
+    def outputs(m, n):
+        return tuple(gp_ffi.DeviceArray(size=k) for k in (n, m, n))
+
+    def solve(d, out, org):
+        res, _ = gp_ffi.pdhg_solve_view(d.g, prm, out)
+        assert res["graph_launches"] > 0
+        gp_ffi.presolve_solve(d, presolve, prm, org)
+
+    def postsolve(out):
+        plan = gp_ffi.PostsolvePlan(rec, original_dev=dlp, use_graph=True)
+        gp_ffi._check(gp_ffi.lib().gp_postsolve_plan_run(plan.h, *(v.ptr for v in (*point, *out))))
+        assert plan.graph_runs() == 1
+        plans.append(plan)
+
+    plans, calls = [], []  # calls[k]: the outputs of each round, and the call that fills them
+    for d in lps:
+        bufs = [outputs(d.m, d.n) + outputs(d.m, d.n) for _ in range(rounds + 1)]
+        calls.append((bufs, lambda b, d=d: solve(d, b[:3], b[3:])))
+    calls.append(([outputs(rec["m0"], rec["n0"]) for _ in range(rounds + 1)], postsolve))
+    for bufs, call in calls:
+        call(bufs[rounds])
+    errors = []
+
+    def work(bufs, call):
+        try:
+            for b in bufs[:rounds]:
+                call(b)
+        except Exception as e:  # noqa: BLE001 (reported below)
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=c) for c in calls]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for bufs, _ in calls:
+        want = [v.numpy() for v in bufs[rounds]]
+        for b in bufs[:rounds]:
+            for got, w in zip(b, want):
+                assert np.array_equal(got.numpy().view(np.uint64), w.view(np.uint64))
+    for plan in plans:
+        plan.free()
